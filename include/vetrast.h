@@ -375,8 +375,8 @@ int vetrast_adam_step(vetrast_ctx* ctx, const vetrast_adam_args* args, void* str
 /* Byte offset inside the workspace of a uint32 that is 1 after the call if the camera row holds non-zero distortion
  * coefficients (they are ignored, as in vetrast_forward), else 0. */
 #define VETRAST_LIFT_FLAGS_OFFSET 192
-/* Byte offset inside the workspace of a uint32 that holds, after the call, how many cells were too large on screen for
- * one wave and went through the shared path (a diagnostic; nothing has to read it). */
+/* Byte offset inside the workspace of a uint32 that holds, after the call, how many cells have a box of more than 4096
+ * pixels on screen (a diagnostic; nothing has to read it). */
 #define VETRAST_LIFT_QUEUE_LENGTH_OFFSET 176
 typedef struct vetrast_lift_args
 {
@@ -402,7 +402,7 @@ int vetrast_lift_error(vetrast_ctx* ctx, const vetrast_lift_args* args, void* st
 /* vetrast_lift_error for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc). It has no counterpart in the reference. Same arguments, same kernels and
  * same results as vetrast_lift_error, but `workspace` / `workspace_bytes` are ignored: the scratch is an array inside
- * the library (about 12.6 MB of device memory per GPU, held until the process ends), whose address on the context's
+ * the library (about 48 MB of device memory per GPU, held until the process ends), whose address on the context's
  * device vetrast_create looks up once. The call itself allocates and frees nothing, creates no events (it reports no
  * timing scope) and only launches kernels.
  *   - num_cells > VETRAST_LIFT_STATIC_MAX_CELLS is refused with VETRAST_ERR_TOO_LARGE.

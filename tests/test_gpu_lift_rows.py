@@ -1,0 +1,71 @@
+"""Error lifting by rows, where the row bounds can go wrong: faces seen edge-on (lines through pixel centres), cells that
+touch the camera plane (tested pixel by pixel), image widths around the steps of the running sums, images that take
+several bands, pixels that are not finite."""
+import numpy as np
+import pytest
+import torch
+
+from vet_amd import synthetic
+from vet_amd.synthetic import ViewSpec
+
+pytestmark = pytest.mark.gpu
+
+
+def _lift(rasterizer, mn, ln, view, poses, intr, img, border):
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (mn, ln, poses, intr, img)]
+    val = torch.zeros(len(mn), device="cuda")
+    cnt = torch.zeros(len(mn), dtype=torch.int32, device="cuda")
+    rasterizer.lift_error(dev[0], dev[1], val, cnt, view, dev[2], dev[3], dev[4], border_pixels=border)
+    torch.cuda.synchronize()
+    return val.cpu().numpy(), cnt.cpu().numpy()
+
+
+def _both(rasterizer, oracle, mn, ln, view, poses, intr, img, border):
+    val, cnt = _lift(rasterizer, mn, ln, view, poses, intr, img, border)
+    want_v, want_c = np.zeros(len(mn), np.float32), np.zeros(len(mn), np.int32)
+    oracle.lift_error(mn, ln, want_v, want_c, view, poses, intr, img, border_pixels=border, num_threads=16)
+    assert want_c.sum() > 0
+    np.testing.assert_array_equal(cnt, want_c)
+    np.testing.assert_allclose(val, want_v, rtol=1e-6, atol=1e-9)
+
+
+def _camera(w, h, t, yaw=0.0, f=None):
+    poses = np.array([[0.0, np.sin(yaw / 2), 0.0, np.cos(yaw / 2), *t, 0.0]])
+    intr = np.zeros((1, 13), np.float32)
+    intr[0, :4] = [f or 0.8 * w, f or 0.8 * w, w // 2, h // 2]
+    return poses, intr
+
+
+# widths and heights around the 4 pixels of a load, the 512 of a step and the 4 rows of a group; one of several bands
+@pytest.mark.parametrize("w,h,border", [(64, 48, 0), (511, 33, 0), (512, 30, 3), (513, 31, 0), (1027, 66, 32), (3000, 1500, 32)])
+@pytest.mark.parametrize("yaw", [0.0, 0.3])
+def test_edge_on_faces_and_sizes(w, h, border, yaw, rasterizer, oracle):
+    print(f"[case] lift rows {w}x{h} border {border} yaw {yaw}", flush=True)
+    mn, ln = synthetic.cell_grid(np.array([[-1.0, -1.0, -1.0], [0.98, 0.98, 0.98]]) + 0.01, 0.25)  # faces on x = 0, y = 0
+    poses, intr = _camera(w, h, (0.0, 0.0, 2.0), yaw)
+    _both(rasterizer, oracle, mn, ln, ViewSpec(w, h), poses, intr, synthetic.error_image(1, 3, h, w), border)
+
+
+# the camera inside the grid: depths of a cell's nearest corners from 1e-6 on
+@pytest.mark.parametrize("depth", [1e-6, 1e-4, 1e-2, 3e-2])
+def test_cells_next_to_the_camera_plane(depth, rasterizer, oracle):
+    print(f"[case] lift rows, nearest corners at depth {depth}", flush=True)
+    w, h = 320, 200
+    mn, ln = synthetic.cell_grid(np.array([[-1.0, -1.0, -1.0], [0.9, 0.9, 0.9]]), 0.3)
+    poses, intr = _camera(w, h, (0.013, -0.007, depth - float(np.unique(mn[:, 2])[3])), 0.0)
+    _both(rasterizer, oracle, mn, ln, ViewSpec(w, h), poses, intr, synthetic.error_image(2, 2, h, w), 0)
+    poses, intr = _camera(w, h, (0.013, -0.007, depth), 0.4)
+    _both(rasterizer, oracle, mn, ln, ViewSpec(w, h), poses, intr, synthetic.error_image(3, 1, h, w), 8)
+
+
+def test_pixels_that_are_not_finite_stay_with_their_cells(rasterizer, oracle):
+    w, h = 600, 64
+    mn, ln = synthetic.cell_grid(np.array([[-2.0, -0.2, -0.1], [1.9, 0.1, 0.1]]), 0.2)
+    poses, intr = _camera(w, h, (0.0, 0.0, 2.0), 0.1)
+    img = synthetic.error_image(4, 3, h, w)
+    img[0, 32, 100], img[1, 30, 300] = np.inf, 1e30
+    val, cnt = _lift(rasterizer, mn, ln, ViewSpec(w, h), poses, intr, img, 0)
+    want_v, want_c = np.zeros(len(mn), np.float32), np.zeros(len(mn), np.int32)
+    oracle.lift_error(mn, ln, want_v, want_c, ViewSpec(w, h), poses, intr, img, border_pixels=0)
+    np.testing.assert_array_equal(cnt, want_c)
+    np.testing.assert_allclose(val, want_v, rtol=1e-5, atol=1e-9)

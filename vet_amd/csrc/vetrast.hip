@@ -46,13 +46,14 @@ inline size_t align_up(size_t v, size_t a)
     return (v + a - 1) / a * a;
 }
 
-// Bytes of error-lifting scratch for num_cells cells: header (camera constants, queue length, flag word), queue
-// entries, one double per queue slot, chunk prefix sums.
+// Bytes of error-lifting scratch for num_cells cells: header (camera constants, counters, flag word), per cell the sum of
+// the bands so far (images that take several) and the list of cells tested pixel by pixel (number, sum, count, finished
+// shares), the running sums of a band of image rows.
 constexpr size_t align_up_c(size_t v, size_t a) { return (v + a - 1) / a * a; }
 constexpr size_t lift_workspace_bytes_for(size_t num_cells)
 {
-    return kLiftHeader + align_up_c(num_cells * sizeof(uint2), kAlign) + align_up_c(num_cells * sizeof(double), kAlign) +
-           align_up_c((num_cells + 1) * sizeof(unsigned long long), kAlign);
+    return kLiftHeader + 2 * align_up_c(num_cells * sizeof(double), kAlign) + 3 * align_up_c(num_cells * sizeof(uint32_t), kAlign) +
+           kLiftSums * sizeof(double);
 }
 
 #define VET_HIP(ctx, expr)                               \
@@ -372,10 +373,9 @@ int validate_lift(const vetrast_lift_args* a, bool* nothing_to_do)
     return VETRAST_OK;
 }
 
-// The five launches of the error lifting with their scratch at `ws` (lift_workspace_bytes_for(num_cells) bytes,
-// 256-byte aligned). Every word of the scratch a kernel reads has been written by an earlier kernel of the same call
-// (the prepare kernel empties the queue, a slot's sum is cleared when the slot is taken), so nothing needs clearing
-// between calls that share one scratch.
+// The launches of the error lifting (three for an image of up to kLiftSums pixels) with their scratch at `ws`
+// (lift_workspace_bytes_for(num_cells) bytes, 256-byte aligned). Every word of the scratch a kernel reads has been written
+// by an earlier kernel of the same call, so nothing needs clearing between calls that share one scratch.
 void launch_lift(const vetrast_lift_args* a, char* ws, hipStream_t stream)
 {
     const vetrast_view& v = a->view;
@@ -390,13 +390,19 @@ void launch_lift(const vetrast_lift_args* a, char* ws, hipStream_t stream)
     lp.height       = a->height;
     lp.width        = a->width;
     lp.border       = a->border_pixels;
-    lp.view         = reinterpret_cast<const DeviceView*>(ws);
-    lp.queue_length = reinterpret_cast<uint32_t*>(ws + VETRAST_LIFT_QUEUE_LENGTH_OFFSET);
-    lp.queue        = reinterpret_cast<uint2*>(ws + kLiftHeader);
-    lp.sums = reinterpret_cast<double*>(ws + kLiftHeader + align_up((size_t)a->num_cells * sizeof(uint2), kAlign));
-    lp.starts = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(lp.sums) +
-                                                      align_up((size_t)a->num_cells * sizeof(double), kAlign));
-    uint32_t* flags = reinterpret_cast<uint32_t*>(ws + VETRAST_LIFT_FLAGS_OFFSET);
+    lp.view         = reinterpret_cast<DeviceView*>(ws);
+    lp.large_cells  = reinterpret_cast<uint32_t*>(ws + VETRAST_LIFT_QUEUE_LENGTH_OFFSET);
+    lp.flags        = reinterpret_cast<uint32_t*>(ws + VETRAST_LIFT_FLAGS_OFFSET);
+    lp.num_plain    = lp.large_cells + 1;
+    const size_t doubles = align_up((size_t)a->num_cells * sizeof(double), kAlign);
+    const size_t words   = align_up((size_t)a->num_cells * sizeof(uint32_t), kAlign);
+    char* at             = ws + kLiftHeader;
+    lp.cell_sums         = reinterpret_cast<double*>(at);
+    lp.plain_sum         = reinterpret_cast<double*>(at + doubles);
+    lp.plain_cell        = reinterpret_cast<uint32_t*>(at + 2 * doubles);
+    lp.plain_count       = reinterpret_cast<int32_t*>(at + 2 * doubles + words);
+    lp.plain_done        = reinterpret_cast<uint32_t*>(at + 2 * doubles + 2 * words);
+    lp.sums              = reinterpret_cast<double*>(at + 2 * doubles + 3 * words);
 
     ViewSource src;
     src.image_index  = v.image_index;
@@ -406,17 +412,25 @@ void launch_lift(const vetrast_lift_args* a, char* ws, hipStream_t stream)
     for (int j = 0; j < 5; ++j) src.crop[j] = v.crop_transform[j];
     for (int j = 0; j < 4; ++j) src.rot[j] = v.crop_rotation[j];
 
-    hipLaunchKernelGGL(lift_prepare_kernel, dim3(1), dim3(kWave), 0, stream, src, a->poses_se3, a->intrinsics,
-                       reinterpret_cast<DeviceView*>(ws), lp.queue_length, flags);
-    const int waves_per_block = kBlock / kWave;
-    hipLaunchKernelGGL(lift_cells_kernel, dim3((unsigned)((a->num_cells + waves_per_block - 1) / waves_per_block)),
-                       dim3(kBlock), 0, stream, lp);
-    // The queue length stays on the device, so the shared pass is launched at a fixed width and splits the chunks
-    // it finds evenly.
-    hipLaunchKernelGGL(lift_scan_kernel, dim3(1), dim3(kLiftScanBlock), 0, stream, lp);
-    hipLaunchKernelGGL(lift_queued_kernel, dim3(2048), dim3(kBlock), 0, stream, lp);
-    hipLaunchKernelGGL(lift_finish_kernel, dim3((unsigned)std::min<int64_t>(grid_for((size_t)a->num_cells), 256)),
-                       dim3(kBlock), 0, stream, lp);
+    // rows a cell can cover, in bands whose running sums fit their room
+    const int64_t top = std::min<int64_t>(a->border_pixels, a->height), bottom = std::max<int64_t>(top, (int64_t)a->height - a->border_pixels);
+    int64_t band = (int64_t)(kLiftSums / ((size_t)a->width + 1)) / kLiftRows * kLiftRows;
+    if (band == 0) lp.sums = nullptr, band = bottom - top;  // a single row is too long: runs are added up pixel by pixel
+    band = std::max<int64_t>(band, kLiftRows);
+    int64_t y = top;
+    do
+    {
+        lp.y0    = (int)y;
+        lp.y1    = (int)std::min(bottom, y + band);
+        lp.first = y == top ? 1 : 0;
+        lp.last  = lp.y1 == bottom ? 1 : 0;
+        const unsigned groups = lp.sums ? (unsigned)std::max(1, (lp.y1 - lp.y0 + kLiftRows - 1) / kLiftRows) : 1u;
+        hipLaunchKernelGGL(lift_prefix_kernel, dim3(groups), dim3(kLiftPrefixBlock), 0, stream, lp, src, a->poses_se3, a->intrinsics);
+        hipLaunchKernelGGL(lift_cells_kernel, dim3((unsigned)((a->num_cells + kLiftCells - 1) / kLiftCells)), dim3(kLiftBlock), 0,
+                           stream, lp);
+        y += band;
+    } while (y < bottom);
+    hipLaunchKernelGGL(lift_plain_kernel, dim3(kLiftPlainShare, kLiftPlainAtOnce), dim3(kBlock), 0, stream, lp);
 }
 
 }  // namespace
