@@ -140,7 +140,7 @@ void PointRendererCache::PollDeviceFlags()
     flags_pending_ = false;
     if (flags_host_.data_ptr<int32_t>()[0] & 1)
     {
-        checked_intrinsics_ptr_ = nullptr;  // the next call checks the tensor itself again, and blocks for it
+        checked_intrinsics_.clear();  // the next call checks the tensor itself again, and blocks for it
         TORCH_CHECK(false, "an earlier forward call rendered with these intrinsics: ", kDistortionRefused);
     }
 }
@@ -152,22 +152,24 @@ void PointRendererCache::CheckIntrinsics(const torch::Tensor& intrinsics)
     PollDeviceFlags();
     const void* ptr       = intrinsics.data_ptr();
     const int64_t version = (int64_t)intrinsics._version();
-    const auto held = checked_intrinsics_storage_.lock();
-    if (ptr == checked_intrinsics_ptr_ && intrinsics.numel() == checked_intrinsics_numel_ && held &&
-        held.get() == intrinsics.storage().unsafeGetStorageImpl())
+    for (size_t k = 0; k < checked_intrinsics_.size(); ++k)
     {
+        CheckedIntrinsics& c = checked_intrinsics_[k];
+        if (ptr != c.ptr || intrinsics.numel() != c.numel) continue;
+        const auto held = c.storage.lock();
+        if (!held || held.get() != intrinsics.storage().unsafeGetStorageImpl()) continue;
         // known memory: no read here; ask for the device's own verdict on this call where the contents may have changed
-        if (version != checked_intrinsics_version_ || ++calls_since_flags_ >= 64) flags_wanted_ = true;
-        checked_intrinsics_version_ = version;
+        if (version != c.version || ++calls_since_flags_ >= 64) flags_wanted_ = true;
+        c.version = version;
+        if (k > 0) std::rotate(checked_intrinsics_.begin(), checked_intrinsics_.begin() + k, checked_intrinsics_.begin() + k + 1);
         return;
     }
     // blocking: one device -> host read per intrinsics tensor
     const bool distorted = intrinsics.detach().slice(1, 5, 13).ne(0).any().item<bool>();
     TORCH_CHECK(!distorted, kDistortionRefused);
-    checked_intrinsics_ptr_     = ptr;
-    checked_intrinsics_storage_ = intrinsics.storage().getWeakStorageImpl();
-    checked_intrinsics_version_ = version;
-    checked_intrinsics_numel_   = intrinsics.numel();
+    if (checked_intrinsics_.size() >= kCheckedIntrinsicsMax) checked_intrinsics_.pop_back();
+    checked_intrinsics_.insert(checked_intrinsics_.begin(),
+                               {ptr, intrinsics.storage().getWeakStorageImpl(), version, intrinsics.numel()});
     flags_wanted_               = false;
     calls_since_flags_          = 0;
 }
@@ -944,8 +946,10 @@ std::vector<torch::Tensor> blend_point_cloud(torch::Tensor texture, torch::Tenso
     scene.tangent_poses             = pose_tangents;
     scene.intrinsics                = intrinsics;
     scene.confidence_value_of_point = confidence;
-    scene.dynamic_refinement_t      = torch::zeros({1}, points.options());
-    scene.poses_se3                 = poses_se3;
+    // (a placeholder that nothing reads: on the host, so that no call launches a fill kernel for it)
+    static const torch::Tensor no_refinement = torch::zeros({1});
+    scene.dynamic_refinement_t               = no_refinement;
+    scene.poses_se3                          = poses_se3;
     if (t_index.defined() && t_index.numel() > 0) scene.t_index = t_index;
 
     NeuralRenderInfo nri;

@@ -112,7 +112,8 @@ class PointRendererCache
     torch::Tensor train_workspace;
     // Cameras with non-zero distortion coefficients are refused unless RenderParams::allow_distortion is set. The
     // coefficients sit in device memory. The first call for an intrinsics tensor (its memory and size) reads columns
-    // 5..12 of `intrinsics` [num_cameras,13] back, which blocks, and throws if they are not all zero. Later calls never
+    // 5..12 of `intrinsics` [num_cameras,13] back, which blocks, and throws if they are not all zero. Later calls on it (or
+    // on the 15 other tensors seen most recently) never
     // block: when the tensor's version counter has moved (an optimiser step), and every 64th call whatever the counter
     // says (writes through a raw pointer leave it alone), NoteDeviceFlags copies the status word that the forward call
     // raises on the device to pinned memory behind the call, and the next call that finds the copy landed throws.
@@ -166,9 +167,16 @@ class PointRendererCache
 
    private:
     // the storage is held weakly: while it is, no other tensor's memory can pass for it at the same address
-    const void* checked_intrinsics_ptr_ = nullptr;
-    c10::weak_intrusive_ptr<c10::StorageImpl> checked_intrinsics_storage_{c10::intrusive_ptr<c10::StorageImpl>()};
-    int64_t checked_intrinsics_version_ = -1, checked_intrinsics_numel_ = -1;
+    struct CheckedIntrinsics
+    {
+        const void* ptr;
+        c10::weak_intrusive_ptr<c10::StorageImpl> storage;
+        int64_t version, numel;
+    };
+    // Several, most recent first: a program that trains or renders several scenes in turn has an intrinsics tensor for
+    // each, and with room for one every change of scene blocked on the read (19 us per call).
+    static constexpr size_t kCheckedIntrinsicsMax = 16;
+    std::vector<CheckedIntrinsics> checked_intrinsics_;
     bool flags_wanted_ = false, flags_pending_ = false;
     int64_t calls_since_flags_ = 0;
     torch::Tensor flags_host_;
