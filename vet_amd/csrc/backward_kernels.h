@@ -1521,6 +1521,60 @@ __device__ __forceinline__ float sign_of(float x)
 
 constexpr int kCameraRow  = 20;  // doubles per workgroup row: 6 pose tangent, fx, fy, cx, cy, 8 distortion, fragment count, pad
 constexpr int kCameraSums = 18;  // of them sums of per-fragment terms
+constexpr int kCameraUsed = 19;  // column of a row that says whether the workgroup had any fragment (the rest is unset if not)
+constexpr int kCameraTerms     = kCameraSums + 1;
+constexpr int kCameraFoldRows  = 64;    // rows the rows of a view are folded into ...
+constexpr int kCameraFoldAbove = 256;   // ... where there are more than this many
+
+// Sums kCameraTerms doubles over the 64 lanes, all of which must call. Every step a lane hands half of its values to its
+// partner and keeps the sums of the other half, so the whole takes 22 exchanges instead of 6 per value. On return the
+// lanes with an even number and `term` >= 0 hold the sum of that term.
+template <int M>
+__device__ __forceinline__ double lane_xor_double(double v, int lane)
+{
+    const uint64_t u  = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = lane_xor<M>((uint32_t)u, lane), hi = lane_xor<M>((uint32_t)(u >> 32), lane);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+template <int M, int HALF, int N>
+__device__ __forceinline__ void exchange_halves(double (&v)[N], int lane)
+{
+    const bool upper = (lane & M) != 0;
+#pragma unroll
+    for (int k = 0; k < HALF; ++k)
+    {
+        const double other = k + HALF < N ? v[k + HALF < N ? k + HALF : 0] : 0.0;
+        const double got   = lane_xor_double<M>(upper ? v[k] : other, lane);
+        v[k]               = (upper ? other : v[k]) + got;
+    }
+}
+__device__ __forceinline__ double wave_sum_terms(const double (&term_values)[kCameraTerms], int lane, int& term)
+{
+    double v[kCameraTerms];
+#pragma unroll
+    for (int k = 0; k < kCameraTerms; ++k) v[k] = term_values[k];
+    exchange_halves<32, 10, kCameraTerms>(v, lane);
+    double w[10];
+#pragma unroll
+    for (int k = 0; k < 10; ++k) w[k] = v[k];
+    exchange_halves<16, 5, 10>(w, lane);
+    double x[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) x[k] = w[k];
+    exchange_halves<8, 3, 5>(x, lane);
+    double y[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) y[k] = x[k];
+    exchange_halves<4, 2, 3>(y, lane);
+    double z[2] = {y[0], y[1]};
+    exchange_halves<2, 1, 2>(z, lane);
+    const double sum = z[0] + lane_xor_double<1>(z[0], lane);
+    // which term that is, and whether it is one (the halves of 5 and 3 are padded)
+    const int in2 = (lane & 2) ? 1 : 0, in3 = ((lane & 4) ? 2 : 0) + in2, in5 = ((lane & 8) ? 3 : 0) + in3;
+    const int all = ((lane & 32) ? 10 : 0) + ((lane & 16) ? 5 : 0) + in5;
+    term          = ((lane & 1) == 0 && in3 < 3 && in5 < 5 && all < kCameraTerms) ? all : -1;
+    return sum;
+}
 
 // One thread per point: find the pixel the point fell into in every layer (the same projection as the scatter pass), decide
 // whether its fragment survived the top-K cut (its key is not larger than the K-th key of that pixel's sorted list), and
@@ -1664,21 +1718,39 @@ __global__ void __launch_bounds__(kBlock) gather_point_gradients_kernel(GatherPa
     }
     if (a.camera_partial)
     {
-        // workgroup sums in double, one row per workgroup; reduce_camera_kernel adds the rows of a view
+        // Workgroup sums in double, one row per workgroup, added up behind this kernel. A wave without a fragment (most
+        // of the cloud, for a crop) leaves its sums out, a workgroup without one its row.
         __shared__ double cam_red[kBlock / kWave][kCameraRow];
-        const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-#pragma unroll
-        for (int k = 0; k <= kCameraSums; ++k)
+        const int lane  = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+        const bool some = __ballot(view_cnt > 0.f) != 0ull;
+        if (some)
         {
-            double v = (k < kSums) ? (double)cam_sum[k < kSums ? k : 0] : (k == kCameraSums ? (double)view_cnt : 0.0);
+            double v[kCameraTerms];
 #pragma unroll
-            for (int d = kWave / 2; d >= 1; d >>= 1) v += __shfl_xor(v, d, kWave);
-            if (lane == 0) cam_red[wave][k] = v;
+            for (int k = 0; k < kCameraTerms; ++k) v[k] = k < kSums ? (double)cam_sum[k < kSums ? k : 0] : (k == kCameraSums ? (double)view_cnt : 0.0);
+            int term;
+            const double sum = wave_sum_terms(v, lane, term);
+            if (term >= 0) cam_red[wave][term] = sum;
         }
+        if (lane == 0) cam_red[wave][kCameraUsed] = some ? 1.0 : 0.0;
         __syncthreads();
-        if (threadIdx.x <= kCameraSums)
-            a.camera_partial[(size_t)view * a.camera_partial_stride + (size_t)blockIdx.x * kCameraRow + threadIdx.x] =
-                (cam_red[0][threadIdx.x] + cam_red[1][threadIdx.x]) + (cam_red[2][threadIdx.x] + cam_red[3][threadIdx.x]);
+        if (threadIdx.x < kCameraRow)
+        {
+            double* row  = a.camera_partial + (size_t)view * a.camera_partial_stride + (size_t)blockIdx.x * kCameraRow;
+            double total = 0.0;
+            bool used    = false;
+#pragma unroll
+            for (int w = 0; w < kBlock / kWave; ++w)
+                if (cam_red[w][kCameraUsed] != 0.0)
+                {
+                    total += cam_red[w][threadIdx.x];
+                    used = true;
+                }
+            if (threadIdx.x == kCameraUsed)
+                row[kCameraUsed] = used ? 1.0 : 0.0;
+            else if (used)
+                row[threadIdx.x] = total;
+        }
         __syncthreads();  // (the next view of the round uses the array again)
     }
   }
@@ -1769,93 +1841,120 @@ __global__ void __launch_bounds__(kBlock) gather_point_gradients_kernel(GatherPa
     }
 }
 
-// Adds the per-workgroup camera rows of one view to the pose row image_index (double) and the intrinsics row
-// camera_index (fx, fy, cx, cy times K_gradient_factor, the skew column stays zero; the distortion columns where
-// distortion is switched on), and the scaled fragment
-// count to both count arrays, as src/lib/rendering/RenderBackward.cu:1418-1459 does per fragment with atomics.
-__global__ void __launch_bounds__(kBlock) reduce_camera_kernel(const double* __restrict__ rows, int num_rows,
-                                                                int image_index, int camera_index, float k_factor,
-                                                                double* __restrict__ grad_pose,
-                                                                float* __restrict__ grad_pose_count,
-                                                                float* __restrict__ grad_intrinsics,
-                                                                float* __restrict__ grad_intrinsics_count,
-                                                                float pose_count_step, int with_distortion,
-                                                                float distortion_factor)
+// Sums of the camera rows [first, first + step, ...) below num_rows that are in use, by one wave; as wave_sum_terms.
+__device__ __forceinline__ double sum_camera_rows(const double* __restrict__ rows, int first, int step, int num_rows, int lane, int& term)
 {
-    constexpr int kTerms = kCameraSums + 1;
-    __shared__ double red[kBlock / kWave][kCameraRow];
-    double acc[kTerms];
+    double acc[kCameraTerms];
 #pragma unroll
-    for (int k = 0; k < kTerms; ++k) acc[k] = 0.0;
-    for (int r = threadIdx.x; r < num_rows; r += kBlock)
+    for (int k = 0; k < kCameraTerms; ++k) acc[k] = 0.0;
+    for (int r = first; r < num_rows; r += step)
     {
         const double* row = rows + (size_t)r * kCameraRow;
+        if (row[kCameraUsed] == 0.0) continue;
 #pragma unroll
-        for (int k = 0; k < kTerms; ++k) acc[k] += row[k];
+        for (int k = 0; k < kCameraTerms; ++k) acc[k] += row[k];
     }
+    return wave_sum_terms(acc, lane, term);
+}
+
+// Folds the camera rows of every view of a round (blockIdx.y) into kCameraFoldRows rows, one per workgroup, in a fixed
+// order. One workgroup adding up a view's 7 800 rows (2 M points) took 37 us per view; this takes 5 us for four.
+__global__ void __launch_bounds__(kBlock) fold_camera_rows_kernel(const double* __restrict__ rows, int num_rows, size_t rows_stride,
+                                                                   double* __restrict__ folded, size_t folded_stride)
+{
+    __shared__ double part[kBlock / kWave][kCameraRow];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-#pragma unroll
-    for (int k = 0; k < kTerms; ++k)
+    int term;
+    const double sum = sum_camera_rows(rows + (size_t)blockIdx.y * rows_stride, blockIdx.x + kCameraFoldRows * threadIdx.x,
+                                       kCameraFoldRows * kBlock, num_rows, lane, term);
+    if (term >= 0) part[wave][term] = sum;
+    __syncthreads();
+    double* out = folded + (size_t)blockIdx.y * folded_stride + (size_t)blockIdx.x * kCameraRow;
+    if (threadIdx.x < kCameraTerms)
+        out[threadIdx.x] = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
+    if (threadIdx.x == kCameraUsed) out[kCameraUsed] = 1.0;
+}
+
+// Adds the camera rows of the views of a round, a wave per view, to the pose row image_index (double) and the intrinsics row
+// camera_index (fx, fy, cx, cy times K_gradient_factor, the skew column stays zero; the distortion columns where
+// distortion is switched on), and the scaled fragment count to both count arrays, view after view, as
+// src/lib/rendering/RenderBackward.cu:1418-1459 does per fragment with atomics. In the call's last round with
+// `normalize` it also divides the rows by their counts: NormalizeGradientDevTensor<double,6> on the poses and
+// NormalizeGradient<float,13> on the intrinsics (src/lib/rendering/PointRenderer.cu:1092-1109,1253-1308).
+struct CameraPass
+{
+    const double* rows;
+    int num_rows;
+    size_t rows_stride;
+    int view_count;
+    int image_index[kViewLanes], camera_index[kViewLanes];
+    float k_factor;
+    double* grad_pose;
+    float* grad_pose_count;
+    float* grad_intrinsics;
+    float* grad_intrinsics_count;
+    float pose_count_step;
+    int with_distortion;
+    float distortion_factor;
+    int normalize, num_poses, num_cameras;
+};
+static_assert(kViewLanes <= kBlock / kWave, "a wave per view of a round");
+
+__global__ void __launch_bounds__(kBlock) reduce_camera_kernel(CameraPass a)
+{
+    __shared__ double red[kBlock / kWave][kCameraRow];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    if (wave < a.view_count)
     {
-        double v = acc[k];
-#pragma unroll
-        for (int d = kWave / 2; d >= 1; d >>= 1) v += __shfl_xor(v, d, kWave);
-        if (lane == 0) red[wave][k] = v;
+        int term;
+        const double sum = sum_camera_rows(a.rows + (size_t)wave * a.rows_stride, lane, kWave, a.num_rows, lane, term);
+        if (term >= 0) red[wave][term] = sum;
     }
     __syncthreads();
-    if (threadIdx.x < kTerms)
+    for (int v = 0; v < a.view_count && threadIdx.x < kCameraTerms; ++v)
     {
-        const int k    = threadIdx.x;
-        const double s = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+        const int k            = threadIdx.x;
+        const double s         = red[v][k];
+        const int image_index  = a.image_index[v], camera_index = a.camera_index[v];
         if (k < 6)
         {
-            if (grad_pose) grad_pose[6 * (size_t)image_index + k] += s;
+            if (a.grad_pose) a.grad_pose[6 * (size_t)image_index + k] += s;
         }
         else if (k < 10)
         {
-            if (grad_intrinsics)
-                grad_intrinsics[13 * (size_t)camera_index + (k - 6)] += (float)((double)k_factor * s);
+            if (a.grad_intrinsics) a.grad_intrinsics[13 * (size_t)camera_index + (k - 6)] += (float)((double)a.k_factor * s);
         }
         else if (k < kCameraSums)
         {
             // the distortion columns with the weights of src/lib/rendering/RenderBackward.cu:1440-1455:
             // k3 x 0.25, k4..k6 and p1, p2 x 0.1, all x distortion_gradient_factor
-            const int c       = k - 10;
+            const int c     = k - 10;
             const double w8 = c < 2 ? 1.0 : c == 2 ? 0.25 : 0.1;
-            if (grad_intrinsics && with_distortion)
-                grad_intrinsics[13 * (size_t)camera_index + 5 + c] += (float)((double)distortion_factor * (s * w8));
+            if (a.grad_intrinsics && a.with_distortion)
+                a.grad_intrinsics[13 * (size_t)camera_index + 5 + c] += (float)((double)a.distortion_factor * (s * w8));
         }
         else
         {
             // per fragment the reference adds 1/1024 to both counts in FULL_BLEND, but 1 to the pose count in
             // BILINEAR_BLEND (src/lib/rendering/RenderBackward.cu:1425,1458 and :3146,3174)
-            if (grad_pose) grad_pose_count[image_index] += (float)(s * (double)pose_count_step);
-            if (grad_intrinsics) grad_intrinsics_count[camera_index] += (float)(s / 1024.0);
+            if (a.grad_pose) a.grad_pose_count[image_index] += (float)(s * (double)a.pose_count_step);
+            if (a.grad_intrinsics) a.grad_intrinsics_count[camera_index] += (float)(s / 1024.0);
         }
     }
-}
-
-// Rows divided by their counts: NormalizeGradientDevTensor<double,6> on the poses and NormalizeGradient<float,13> on the
-// intrinsics (src/lib/rendering/PointRenderer.cu:1092-1109,1253-1308).
-__global__ void __launch_bounds__(kBlock) normalize_camera_gradients_kernel(double* __restrict__ grad_pose,
-                                                                             const float* __restrict__ pose_count,
-                                                                             int num_poses,
-                                                                             float* __restrict__ grad_intrinsics,
-                                                                             const float* __restrict__ intrinsics_count,
-                                                                             int num_cameras)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (grad_pose && i < num_poses)
+    if (!a.normalize) return;
+    __threadfence_block();
+    __syncthreads();
+    for (int i = threadIdx.x; a.grad_pose && i < a.num_poses; i += kBlock)
     {
-        const float c = pose_count[i];
+        const float c = a.grad_pose_count[i];
         if (c > 0.f)
-            for (int k = 0; k < 6; ++k) grad_pose[6 * (size_t)i + k] = grad_pose[6 * (size_t)i + k] / c;
+            for (int k = 0; k < 6; ++k) a.grad_pose[6 * (size_t)i + k] = a.grad_pose[6 * (size_t)i + k] / c;
     }
-    if (grad_intrinsics && i < num_cameras)
+    for (int i = threadIdx.x; a.grad_intrinsics && i < a.num_cameras; i += kBlock)
     {
-        const float c = intrinsics_count[i];
+        const float c = a.grad_intrinsics_count[i];
         if (c > 0.f)
-            for (int k = 0; k < 13; ++k) grad_intrinsics[13 * (size_t)i + k] = grad_intrinsics[13 * (size_t)i + k] / c;
+            for (int k = 0; k < 13; ++k) a.grad_intrinsics[13 * (size_t)i + k] = a.grad_intrinsics[13 * (size_t)i + k] / c;
     }
 }
 

@@ -1136,14 +1136,41 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             else
                 with_channels(std::integral_constant<int, 4>{});
         }
-        for (int v = first; want_camera && v < last; ++v)
+        if (want_camera)
         {
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_GATHER);
-            hipLaunchKernelGGL(reduce_camera_kernel, dim3(1), dim3(kBlock), 0, stream,
-                               camera_rows + (size_t)(v - first) * (camera_rows_bytes(N) / sizeof(double)), grid_for(N),
-                               a->views[v].image_index, a->views[v].camera_index, p.K_gradient_factor, g->grad_pose,
-                               g->grad_pose_count, g->grad_intrinsics, g->grad_intrinsics_count,
-                               hits == 1 ? 1.f / 1024.f : 1.f, p.allow_distortion, p.distortion_gradient_factor);
+            CameraPass cp;
+            cp.rows        = camera_rows;
+            cp.num_rows    = grid_for(N);
+            cp.rows_stride = camera_rows_bytes(N) / sizeof(double);
+            cp.view_count  = count;
+            if (cp.num_rows > kCameraFoldAbove)
+            {
+                // (into the gradient records of the round, which nothing reads any more)
+                double* folded = ws_ptr<double>(ws, lay.partial_base);
+                hipLaunchKernelGGL(fold_camera_rows_kernel, dim3(kCameraFoldRows, (unsigned)count), dim3(kBlock), 0, stream, cp.rows,
+                                   cp.num_rows, cp.rows_stride, folded, (size_t)kCameraFoldRows * kCameraRow);
+                cp.rows        = folded;
+                cp.num_rows    = kCameraFoldRows;
+                cp.rows_stride = (size_t)kCameraFoldRows * kCameraRow;
+            }
+            for (int v = 0; v < kViewLanes; ++v)
+            {
+                cp.image_index[v]  = v < count ? a->views[first + v].image_index : 0;
+                cp.camera_index[v] = v < count ? a->views[first + v].camera_index : 0;
+            }
+            cp.k_factor              = p.K_gradient_factor;
+            cp.grad_pose             = g->grad_pose;
+            cp.grad_pose_count       = g->grad_pose_count;
+            cp.grad_intrinsics       = g->grad_intrinsics;
+            cp.grad_intrinsics_count = g->grad_intrinsics_count;
+            cp.pose_count_step       = hits == 1 ? 1.f / 1024.f : 1.f;
+            cp.with_distortion       = p.allow_distortion;
+            cp.distortion_factor     = p.distortion_gradient_factor;
+            cp.normalize             = (p.camera_gradient_normalization && last == B) ? 1 : 0;
+            cp.num_poses             = a->num_poses;
+            cp.num_cameras           = a->num_cameras;
+            hipLaunchKernelGGL(reduce_camera_kernel, dim3(1), dim3(kBlock), 0, stream, cp);
         }
         for (int v = first; N == 0 && v < last; ++v)
         {
@@ -1159,14 +1186,6 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
         ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_POST);
         hipLaunchKernelGGL(normalize_point_gradient_kernel, dim3(grid_for(N)), dim3(kBlock), 0, stream,
                            g->grad_points, g->grad_point_count, N, p.point_gradient_normalization);
-    }
-    if (want_camera && p.camera_gradient_normalization)
-    {
-        ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_POST);
-        const int n = std::max(a->num_poses, a->num_cameras);
-        hipLaunchKernelGGL(normalize_camera_gradients_kernel, dim3(grid_for(n)), dim3(kBlock), 0, stream, g->grad_pose,
-                           g->grad_pose_count, a->num_poses, g->grad_intrinsics, g->grad_intrinsics_count,
-                           a->num_cameras);
     }
     VET_HIP(ctx, hipGetLastError());
     return VETRAST_OK;
