@@ -322,6 +322,24 @@ def test_cameras_with_distortion_are_refused_by_the_shim():
     assert len(_plain_call(scene, torch_ops, intrinsics=intr)) == scene.num_layers
 
 
+def test_distortion_is_found_when_two_intrinsics_tensors_take_turns():
+    """A change of tensor reads the coefficients again, so a write that leaves the version counter alone is found however
+    the calls alternate: the very next call with the tensor written to throws, and the other tensor stays usable."""
+    from vet_amd import torch_ops
+
+    scene = synthetic.tiny_scene(num_points=1000, K=8, seed=37)
+    a, b = (torch.from_numpy(scene.intrinsics.copy()).cuda() for _ in range(2))
+    for t in (a, b, a, b):
+        assert len(_plain_call(scene, torch_ops, intrinsics=t)) == scene.num_layers
+    with torch.autograd._unsafe_preserve_version_counter(a):
+        a[0, 5] = 2e-3
+    with pytest.raises(RuntimeError, match="distortion"):
+        _plain_call(scene, torch_ops, intrinsics=a)
+    assert len(_plain_call(scene, torch_ops, intrinsics=b)) == scene.num_layers
+    with pytest.raises(RuntimeError, match="distortion"):
+        _plain_call(scene, torch_ops, intrinsics=a)
+
+
 def test_add_depth_to_network_appends_a_zero_channel(oracle):
     """The blend modes never write the depth tensors (src/lib/rendering/PointRenderer.cu:1061-1066 hands out the zero-filled
     buffers); PointRenderModuleImpl::forward appends them to the images as a channel (RenderModule.cpp:223-232), behind

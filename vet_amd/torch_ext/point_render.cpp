@@ -140,36 +140,49 @@ void PointRendererCache::PollDeviceFlags()
     flags_pending_ = false;
     if (flags_host_.data_ptr<int32_t>()[0] & 1)
     {
-        checked_intrinsics_.clear();  // the next call checks the tensor itself again, and blocks for it
+        checked_intrinsics_ptr_ = nullptr;  // the next call checks the tensor itself again, and blocks for it
         TORCH_CHECK(false, "an earlier forward call rendered with these intrinsics: ", kDistortionRefused);
     }
 }
 
-void PointRendererCache::CheckIntrinsics(const torch::Tensor& intrinsics)
+void PointRendererCache::BeginIntrinsicsCheck(const torch::Tensor& intrinsics)
 {
     TORCH_CHECK(intrinsics.defined() && intrinsics.dim() == 2 && intrinsics.size(1) == 13,
                 "intrinsics must be [num_cameras,13]");
     PollDeviceFlags();
     const void* ptr       = intrinsics.data_ptr();
     const int64_t version = (int64_t)intrinsics._version();
-    for (size_t k = 0; k < checked_intrinsics_.size(); ++k)
+    const auto held       = checked_intrinsics_storage_.lock();
+    if (ptr == checked_intrinsics_ptr_ && intrinsics.numel() == checked_intrinsics_numel_ && held &&
+        held.get() == intrinsics.storage().unsafeGetStorageImpl())
     {
-        CheckedIntrinsics& c = checked_intrinsics_[k];
-        if (ptr != c.ptr || intrinsics.numel() != c.numel) continue;
-        const auto held = c.storage.lock();
-        if (!held || held.get() != intrinsics.storage().unsafeGetStorageImpl()) continue;
         // known memory: no read here; ask for the device's own verdict on this call where the contents may have changed
-        if (version != c.version || ++calls_since_flags_ >= 64) flags_wanted_ = true;
-        c.version = version;
-        if (k > 0) std::rotate(checked_intrinsics_.begin(), checked_intrinsics_.begin() + k, checked_intrinsics_.begin() + k + 1);
+        if (version != checked_intrinsics_version_ || ++calls_since_flags_ >= 64) flags_wanted_ = true;
+        checked_intrinsics_version_ = version;
         return;
     }
-    // blocking: one device -> host read per intrinsics tensor
-    const bool distorted = intrinsics.detach().slice(1, 5, 13).ne(0).any().item<bool>();
-    TORCH_CHECK(!distorted, kDistortionRefused);
-    if (checked_intrinsics_.size() >= kCheckedIntrinsicsMax) checked_intrinsics_.pop_back();
-    checked_intrinsics_.insert(checked_intrinsics_.begin(),
-                               {ptr, intrinsics.storage().getWeakStorageImpl(), version, intrinsics.numel()});
+    torch::NoGradGuard no_grad;
+    if (reading_intrinsics_.defined()) read_event_->synchronize();  // a call that threw in between left its copy under way
+    reading_intrinsics_ = intrinsics.detach();
+    if (!read_host_.defined() || read_host_.numel() < intrinsics.numel())
+        read_host_ = torch::empty({intrinsics.numel()}, torch::TensorOptions().dtype(torch::kFloat32).pinned_memory(true));
+    read_host_.narrow(0, 0, intrinsics.numel()).view(intrinsics.sizes()).copy_(reading_intrinsics_, /*non_blocking=*/true);
+    if (!read_event_) read_event_ = std::make_unique<c10::Event>(c10::DeviceType::CUDA);
+    read_event_->record(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA());
+}
+
+void PointRendererCache::FinishIntrinsicsCheck()
+{
+    if (!reading_intrinsics_.defined()) return;
+    read_event_->synchronize();
+    const torch::Tensor intrinsics = std::move(reading_intrinsics_);
+    reading_intrinsics_            = torch::Tensor();
+    const float* k                 = read_host_.data_ptr<float>();
+    for (int64_t i = 0; i < intrinsics.numel(); ++i) TORCH_CHECK(i % 13 < 5 || k[i] == 0.f, kDistortionRefused);
+    checked_intrinsics_ptr_     = intrinsics.data_ptr();
+    checked_intrinsics_storage_ = intrinsics.storage().getWeakStorageImpl();
+    checked_intrinsics_version_ = (int64_t)intrinsics._version();
+    checked_intrinsics_numel_   = intrinsics.numel();
     flags_wanted_               = false;
     calls_since_flags_          = 0;
 }
@@ -246,7 +259,8 @@ void PointRendererCache::FillSceneGridWithLoss(int batch, const CellTensors& cel
     TORCH_CHECK(is_dev(poses_se3, torch::kFloat64) && is_dev(intrinsics, torch::kFloat32) && is_dev(loss_img, torch::kFloat32),
                 "FillSceneGridWithLoss: poses_se3 (float64), intrinsics and loss_img (float32) must be contiguous CUDA tensors");
     TORCH_CHECK(loss_img.dim() == 3, "FillSceneGridWithLoss: loss_img is [C,h,w]");
-    CheckIntrinsics(intrinsics);
+    BeginIntrinsicsCheck(intrinsics);
+    FinishIntrinsicsCheck();  // (before the launch: it updates the caller's cells in place)
     const int64_t n = cells.t_cell_value.numel();
     TORCH_CHECK(cells.t_cell_bb_min.numel() == 3 * n && cells.t_cell_bb_length.numel() == 3 * n &&
                     cells.t_cell_access_count.numel() == n,
@@ -299,7 +313,7 @@ torch::autograd::variable_list PointRender::forward(torch::autograd::AutogradCon
     const int B = (int)info->images.size(), L = info->num_layers, C = (int)texture.size(0);
     const int64_t N = points.size(0);
     auto f32        = torch::TensorOptions().device(points.device()).dtype(torch::kFloat32);
-    if (!info->params.allow_distortion) info->cache->CheckIntrinsics(intrinsics);
+    if (!info->params.allow_distortion) info->cache->BeginIntrinsicsCheck(intrinsics);
 
     // dropout mask per view, PointRenderer.cu:461-468 (the mask is 1 where a point is dropped)
     torch::Tensor dropout;
@@ -376,7 +390,11 @@ torch::autograd::variable_list PointRender::forward(torch::autograd::AutogradCon
     const torch::Tensor& order = info->cache->PointOrderFor(points);
     a.point_order              = order.defined() ? order.data_ptr<int32_t>() : nullptr;
     check_status(vetrast_forward(info->cache->ctx, &a, current_stream()), "forward");
-    if (!info->params.allow_distortion) info->cache->NoteDeviceFlags(workspace, lay);
+    if (!info->params.allow_distortion)
+    {
+        info->cache->FinishIntrinsicsCheck();  // may throw: nothing of this call has been handed out yet
+        info->cache->NoteDeviceFlags(workspace, lay);
+    }
     if (info->params.size_bins_from_history)
         info->cache->NoteFragmentCounts(workspace, lay, N, L, info->images[0].w, info->images[0].h, a.params.render_mode);
 

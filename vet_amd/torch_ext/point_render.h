@@ -111,13 +111,15 @@ class PointRendererCache
     // training loop then runs in one workspace instead of allocating one per step.
     torch::Tensor train_workspace;
     // Cameras with non-zero distortion coefficients are refused unless RenderParams::allow_distortion is set. The
-    // coefficients sit in device memory. The first call for an intrinsics tensor (its memory and size) reads columns
-    // 5..12 of `intrinsics` [num_cameras,13] back, which blocks, and throws if they are not all zero. Later calls on it (or
-    // on the 15 other tensors seen most recently) never
+    // coefficients sit in device memory. The first call for an intrinsics tensor (its memory and size) reads
+    // `intrinsics` [num_cameras,13] back and throws if columns 5..12 are not all zero: BeginIntrinsicsCheck puts one copy
+    // to pinned memory on the stream in front of the call's kernels, FinishIntrinsicsCheck waits for that copy after the
+    // kernels have been launched, so that they run meanwhile. Later calls never
     // block: when the tensor's version counter has moved (an optimiser step), and every 64th call whatever the counter
     // says (writes through a raw pointer leave it alone), NoteDeviceFlags copies the status word that the forward call
     // raises on the device to pinned memory behind the call, and the next call that finds the copy landed throws.
-    void CheckIntrinsics(const torch::Tensor& intrinsics);
+    void BeginIntrinsicsCheck(const torch::Tensor& intrinsics);
+    void FinishIntrinsicsCheck();
     void NoteDeviceFlags(const torch::Tensor& workspace, const vetrast_workspace_layout& lay);
     // The order in which the binning pass walks the points (vetrast_forward_args.point_order): Morton order with shuffled
     // 256-point blocks, built on the device from the positions, rebuilt when the number of points changes and every
@@ -167,16 +169,11 @@ class PointRendererCache
 
    private:
     // the storage is held weakly: while it is, no other tensor's memory can pass for it at the same address
-    struct CheckedIntrinsics
-    {
-        const void* ptr;
-        c10::weak_intrusive_ptr<c10::StorageImpl> storage;
-        int64_t version, numel;
-    };
-    // Several, most recent first: a program that trains or renders several scenes in turn has an intrinsics tensor for
-    // each, and with room for one every change of scene blocked on the read (19 us per call).
-    static constexpr size_t kCheckedIntrinsicsMax = 16;
-    std::vector<CheckedIntrinsics> checked_intrinsics_;
+    const void* checked_intrinsics_ptr_ = nullptr;
+    c10::weak_intrusive_ptr<c10::StorageImpl> checked_intrinsics_storage_{c10::intrusive_ptr<c10::StorageImpl>()};
+    int64_t checked_intrinsics_version_ = -1, checked_intrinsics_numel_ = -1;
+    torch::Tensor reading_intrinsics_, read_host_;  // the tensor whose copy is under way, and where it lands
+    std::unique_ptr<c10::Event> read_event_;
     bool flags_wanted_ = false, flags_pending_ = false;
     int64_t calls_since_flags_ = 0;
     torch::Tensor flags_host_;
