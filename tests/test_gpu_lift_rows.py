@@ -69,3 +69,14 @@ def test_pixels_that_are_not_finite_stay_with_their_cells(rasterizer, oracle):
     oracle.lift_error(mn, ln, want_v, want_c, ViewSpec(w, h), poses, intr, img, border_pixels=0)
     np.testing.assert_array_equal(cnt, want_c)
     np.testing.assert_allclose(val, want_v, rtol=1e-5, atol=1e-9)
+
+
+# cells next to the camera in an image wide enough for rows with hundreds of open columns: such a cell leaves its rows and
+# is tested pixel by pixel as a whole, unless the image takes several bands
+@pytest.mark.parametrize("w,h", [(1920, 1080), (3000, 1500)])
+@pytest.mark.parametrize("yaw,depth", [(0.02, 0.05), (0.3, 0.002), (-0.45, 0.01)])
+def test_cells_with_many_wide_open_rows(w, h, yaw, depth, rasterizer, oracle):
+    print(f"[case] lift rows {w}x{h} yaw {yaw} depth {depth}", flush=True)
+    mn, ln = synthetic.cell_grid(np.array([[-0.7, -0.7, -0.7], [0.7, 0.7, 0.7]]), 0.25)
+    poses, intr = _camera(w, h, (0.013, -0.007, depth - float(np.unique(mn[:, 2])[3])), yaw, f=0.52 * w)
+    _both(rasterizer, oracle, mn, ln, ViewSpec(w, h), poses, intr, synthetic.error_image(5, 2, h, w), 16)

@@ -36,7 +36,13 @@ constexpr int kLiftPlainAtOnce  = 8;     // cells in work at a time
 constexpr float kLiftThin       = 0.05f; // smallest angle (about) of a triangle that is not a sliver
 constexpr int kLiftOpen         = 8;     // open pixels of a row that go to the list; a row with more is left to a wave
 constexpr int kLiftOpenPixels   = 256;   // the list; it is worked off when half full (a lane tests what does not fit)
-constexpr int kLiftOpenRows     = 64;    // such rows a workgroup keeps (a lane finishes what does not fit)
+constexpr int kLiftOpenRows     = 128;   // such rows a workgroup keeps (a lane finishes what does not fit)
+// A cell whose open rows of more than kLiftWideRow columns add up to more than kLiftWideWork is tested pixel by pixel by
+// lift_plain_kernel: next to the camera the lines of slivers sweep hundreds of columns in hundreds of rows, and the one
+// workgroup that had such a cell held the launch up (three 1080p views, one of them like that: 1.61 ms of kernels, now
+// 0.55 ms; its launch of the rows 1.32 ms, now 0.20 ms).
+constexpr int kLiftWideRow      = 256;
+constexpr int kLiftWideWork     = 2048;
 constexpr size_t kLiftSums      = (size_t)1 << 22;  // running sums that exist at a time (33.5 MB: an image of 4.2 M
                                                     // pixels); taller images take several bands
 static_assert(sizeof(DeviceView) <= VETRAST_LIFT_QUEUE_LENGTH_OFFSET && VETRAST_LIFT_QUEUE_LENGTH_OFFSET + 4 <= VETRAST_LIFT_FLAGS_OFFSET,
@@ -259,6 +265,7 @@ struct LiftCell
     float sliver_width[kLiftSliverMax];  // their half width in columns, or -(half width in rows)
     uint32_t left_mask;                  // bit t: the third bound of triangle t is a left one; bit 8 + k: outline[k] is
     int num_outline, num_tri, num_sliver;
+    int wide;      // columns of the wide open rows; kLiftWideWork + 1 and more: the cell is lift_plain_kernel's
     int count;
     double sum;
 };
@@ -302,6 +309,16 @@ __device__ __forceinline__ double lift_run_sum(const LiftPass& a, int x0, int x1
     double s = 0.0;
     for (int x = x0; x < x1; ++x) s += (double)lift_pixel_error(a, x, y);
     return s;
+}
+
+// Enters a cell, once per call, into the list of lift_plain_kernel (a few cells of a grid).
+__device__ __forceinline__ void leave_to_plain_kernel(const LiftPass& a, int64_t cell)
+{
+    const uint32_t at = atomicAdd(a.num_plain, 1u);
+    a.plain_cell[at]  = (uint32_t)cell;
+    a.plain_sum[at]   = 0.0;
+    a.plain_count[at] = 0;
+    a.plain_done[at]  = 0u;
 }
 
 __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
@@ -381,19 +398,13 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         const bool large = part == 0 && seen && x_size * y_size > kLiftLargeCell;
         if (seen && plain)
         {
-            if (part == 0 && a.first)
-            {
-                const uint32_t at = atomicAdd(a.num_plain, 1u);  // (a few cells of a grid)
-                a.plain_cell[at]  = (uint32_t)cell;
-                a.plain_sum[at]   = 0.0;
-                a.plain_count[at] = 0;
-                a.plain_done[at]  = 0u;
-            }
+            if (part == 0 && a.first) leave_to_plain_kernel(a, cell);
             seen = false;
         }
         if (part == 0)
         {
             s_start[slot] = seen ? y_size : 0;
+            f.wide        = 0;
             f.count       = 0;
             f.sum         = 0.0;
             f.left_mask = 0u;
@@ -672,6 +683,9 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         }
         if (open > kLiftOpen)
         {
+            // (one band only: with several the cell's rows of the other bands may be in its sums already)
+            const int width = x_end - x_first;
+            if (width > kLiftWideRow && a.first && a.last && atomicAdd(&f.wide, width) + width > kLiftWideWork) return;
             const int at = atomicAdd(&s_num_open, 1);
             if (at < kLiftOpenRows)
             {
@@ -723,6 +737,7 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     {
         const int4 row = s_open[k];
         LiftCell& f    = s_cell[row.x];
+        if (f.wide > kLiftWideWork) continue;
         int count      = 0;
         double sum     = 0.0;
         for (int x = row.z + lane; x < row.w; x += kWave)
@@ -743,7 +758,9 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     if (tid < kLiftCells)
     {
         const int64_t cell = (int64_t)tid * gridDim.x + blockIdx.x;
-        if (cell < a.num_cells)
+        if (cell < a.num_cells && s_cell[tid].wide > kLiftWideWork)
+            leave_to_plain_kernel(a, cell);
+        else if (cell < a.num_cells)
         {
             double sum      = s_cell[tid].sum;
             const int count = s_cell[tid].count;
