@@ -720,24 +720,25 @@ __global__ void __launch_bounds__(kBlock) pack_descriptors_kernel(PackJob pack)
 }
 
 // Brings the logged records (rank beyond the bin's own room) to the bin's place in the compact array:
-// binned[bin_offsets[bin] + rank]. Runs after the scan of the bin counts; the log is empty as a rule.
+// binned[bin_offsets[bin] + rank]. Runs after the scan of the bin counts; the log is empty as a rule. The grid is a multiple
+// of kLogSegments workgroups.
 __device__ __forceinline__ void overflow_move(const ScatterTargets& in, const uint32_t* __restrict__ bin_offsets,
                                               uint4* __restrict__ binned, uint32_t capacity)
 {
-    for (uint32_t segment = blockIdx.x; segment < (uint32_t)kLogSegments; segment += gridDim.x)
+    // workgroups beyond the first kLogSegments take their share of a segment
+    const uint32_t share   = gridDim.x / (uint32_t)kLogSegments, part = blockIdx.x / (uint32_t)kLogSegments;
+    const uint32_t segment = blockIdx.x % (uint32_t)kLogSegments;
+    const uint32_t entries = min(in.log_cursor[segment * kLogCursorStride], in.segment_capacity);
+    const size_t first     = (size_t)segment * in.segment_capacity;
+    for (uint32_t e = part * blockDim.x + threadIdx.x; e < entries; e += share * blockDim.x)
     {
-        const uint32_t entries = min(in.log_cursor[segment * kLogCursorStride], in.segment_capacity);
-        const size_t first     = (size_t)segment * in.segment_capacity;
-        for (uint32_t e = threadIdx.x; e < entries; e += blockDim.x)
-        {
-            const uint4 rec    = in.log[first + e];
-            const uint32_t pos = bin_offsets[rec.w] + in.log_rank[first + e];
-            if (pos >= capacity) continue;  // guard: never true
-            if (in.compact)
-                reinterpret_cast<uint2*>(binned)[pos] = make_uint2(rec.y, (rec.x << 8) | rec.z);
-            else
-                binned[pos] = make_uint4(rec.x, rec.y, rec.z, 0u);
-        }
+        const uint4 rec    = in.log[first + e];
+        const uint32_t pos = bin_offsets[rec.w] + in.log_rank[first + e];
+        if (pos >= capacity) continue;  // guard: never true
+        if (in.compact)
+            reinterpret_cast<uint2*>(binned)[pos] = make_uint2(rec.y, (rec.x << 8) | rec.z);
+        else
+            binned[pos] = make_uint4(rec.x, rec.y, rec.z, 0u);
     }
 }
 

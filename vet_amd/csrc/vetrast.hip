@@ -802,9 +802,9 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
             // the few records beyond their bin's own room, if any
             const ScanArgs& sa = scan.v[0];
             if (one)
-                hipLaunchKernelGGL(overflow_move_kernel, dim3(256), blk, 0, stream, sa.in, sa.bin_counts, sa.binned, sa.capacity);
+                hipLaunchKernelGGL(overflow_move_kernel, dim3(kMoveShare * kLogSegments), blk, 0, stream, sa.in, sa.bin_counts, sa.binned, sa.capacity);
             else
-                hipLaunchKernelGGL(overflow_move_views_kernel, dim3(256, views_y), blk, 0, stream, scan);
+                hipLaunchKernelGGL(overflow_move_views_kernel, dim3(kMoveShare * kLogSegments, views_y), blk, 0, stream, scan);
         }
         {
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BUILD);
