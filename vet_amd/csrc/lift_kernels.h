@@ -6,14 +6,15 @@
 // So the work here goes by rows instead of pixels:
 //   1. lift_prefix_kernel: per image row the running sum (double) of sum_c |loss|, so that the sum over a run of pixels is
 //      one difference of two entries.
-//   2. lift_cells_kernel: a workgroup takes 64 cells, projects their corners and sets up, per triangle and for the outline
+//   2. lift_cells_kernel: a workgroup takes 32 cells, projects their corners and sets up, per triangle and for the outline
 //      of the 8 corners, where their edges cross a row; then every lane takes one ROW of one of the cells. Pixels that
 //      lie inside a triangle by more than the rounding error of the test are counted as a run, pixels outside the outline
 //      by more than that are left out, and the few in between get the literal test of the reference. The counts are the
 //      literal ones, pixel for pixel.
-// Measured (146 k cells of 0.25 m, 1080p, 121 M covered pixels): 0.94 ms per call with a test per pixel (bound by its
-// ~200 vector instructions per 64 pixels), 0.17 ms by rows (running sums 17 us, rows 137 us, the handful of cells that touch
-// the camera plane 13 us; 2.2 M rows, bound by their ~400 vector instructions per 64 rows and the tests of open pixels).
+// Measured (146 k cells of 0.25 m, 1080p, 121 M covered pixels, the camera inside the grid): 0.87 ms per call with a test per
+// pixel (bound by its ~200 vector instructions per 64 pixels), 0.29 ms by rows (running sums 17 us, rows 211 us, the
+// cells next to the camera that are tested pixel by pixel 63 us); bound by the ~400 vector instructions per 64 rows and
+// the tests of open pixels.
 #pragma once
 #include "common.h"
 #include "forward_kernels.h"
@@ -40,7 +41,8 @@ constexpr int kLiftOpenRows     = 128;   // such rows a workgroup keeps (a lane 
 // A cell whose open rows of more than kLiftWideRow columns add up to more than kLiftWideWork is tested pixel by pixel by
 // lift_plain_kernel: next to the camera the lines of slivers sweep hundreds of columns in hundreds of rows, and the one
 // workgroup that had such a cell held the launch up (three 1080p views, one of them like that: 1.61 ms of kernels, now
-// 0.55 ms; its launch of the rows 1.32 ms, now 0.20 ms).
+// 0.55 ms; its launch of the rows 1.32 ms, now 0.20 ms; the scene above 6.5 ms, now 0.29 ms). Limits of 64 and 128 columns
+// a row and 1024 and 8192 in all measure the same within 5 %, 32768 in all is slower by half on that scene.
 constexpr int kLiftWideRow      = 256;
 constexpr int kLiftWideWork     = 2048;
 constexpr size_t kLiftSums      = (size_t)1 << 22;  // running sums that exist at a time (33.5 MB: an image of 4.2 M
