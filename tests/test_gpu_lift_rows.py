@@ -80,3 +80,22 @@ def test_cells_with_many_wide_open_rows(w, h, yaw, depth, rasterizer, oracle):
     mn, ln = synthetic.cell_grid(np.array([[-0.7, -0.7, -0.7], [0.7, 0.7, 0.7]]), 0.25)
     poses, intr = _camera(w, h, (0.013, -0.007, depth - float(np.unique(mn[:, 2])[3])), yaw, f=0.52 * w)
     _both(rasterizer, oracle, mn, ln, ViewSpec(w, h), poses, intr, synthetic.error_image(5, 2, h, w), 16)
+
+
+# flat cells with a face next to the camera's height: triangles with two edges so flat that they say nothing about a single
+# row, beside a left or a right one
+@pytest.mark.parametrize("yaw", [0.0, 0.2, -0.7])
+@pytest.mark.parametrize("top", [False, True])
+def test_flat_cells_with_a_face_next_to_the_camera_height(yaw, top, rasterizer, oracle):
+    print(f"[case] lift rows, flat cells, yaw {yaw} top {top}", flush=True)
+    w, h, n = 512, 192, 12_000
+    rng = np.random.default_rng(int(100 * abs(yaw)) + top)
+    width = rng.uniform(0.1, 1.0, (n, 1))
+    height = width * rng.uniform(0.02, 0.4, (n, 1))
+    ln = np.concatenate([width, height, width * rng.uniform(0.5, 1.0, (n, 1))], 1).astype(np.float32)
+    face = np.exp(rng.uniform(np.log(1e-7), np.log(3e-5), (n, 1))) * rng.choice([-1.0, 1.0], (n, 1))
+    depth = rng.uniform(0.5, 6.0, (n, 1))
+    mn = np.concatenate([rng.uniform(-0.7, 0.7, (n, 1)) * depth, face - (height if top else 0.0), depth], 1).astype(np.float32)
+    poses, intr = _camera(w, h, (0.0, 0.0, 0.0), yaw)
+    intr[0, 2:4] = [247.3, 94.18]
+    _both(rasterizer, oracle, mn, ln, ViewSpec(w, h), poses, intr, synthetic.error_image(6, 1, h, w), 0)

@@ -512,11 +512,16 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
                                 r.x0 += is_left ? slack : -slack;
                             else
                             {
-                                // a flat edge: rows beyond it are all right, rows before it are all wrong
+                                // A flat edge: rows beyond it are all right, rows before it are all wrong. It can be a left
+                                // or a right bound alike. It takes the first that is free, so that no bound is lost: at most
+                                // two of the other edges bound from one side, and only one where there is a flat edge (the
+                                // c1 of the three edges sum up to zero, and two of one sign to more than a flat edge has).
                                 const float beyond = (err + flat * reach_x) / fmaxf(fabsf(dx), 1e-12f);
                                 r.slope   = dx < 0.f ? -1e12f : 1e12f;
                                 r.y0      = dx < 0.f ? by + beyond : by - beyond;
                                 r.x0      = 1e7f;  // (beyond any column; one part in 1e5 of a row further it is -infinity)
+                                is_left   = !have_left || have_right;
+                                if (!is_left) r.slope = -r.slope, r.x0 = -r.x0;
                             }
                             if (is_left && !have_left)
                                 bound[0] = r, have_left = true;
