@@ -99,3 +99,36 @@ def test_flat_cells_with_a_face_next_to_the_camera_height(yaw, top, rasterizer, 
     poses, intr = _camera(w, h, (0.0, 0.0, 0.0), yaw)
     intr[0, 2:4] = [247.3, 94.18]
     _both(rasterizer, oracle, mn, ln, ViewSpec(w, h), poses, intr, synthetic.error_image(6, 1, h, w), 0)
+
+
+def _strip_of_cells(w, pixels):
+    """Cells side by side, seen head-on, that each cover `pixels` columns of row 9 of an image of 19 rows."""
+    h = 19
+    poses, intr = _camera(w, h, (0.0, 0.0, 0.0), f=float(w))
+    left = (np.arange(16, w - 16 - pixels, pixels) - w // 2 + 0.5) / w
+    n = len(left)
+    mn = np.stack([left, np.full(n, (8.5 - h // 2) / w), np.ones(n)], 1).astype(np.float32)
+    ln = np.stack([np.full(n, pixels / w), np.full(n, 2.0 / w), np.full(n, 1e-3)], 1).astype(np.float32)
+    return mn, ln, poses, intr, h
+
+
+# A run of dim pixels behind bright ones of its row is a difference of large sums in 64 bits. What is left of it has to be
+# good for the float that the cell's value is: with 38 bits left, one cell in 2^13 or so differs from the sequential sum's
+# float, of the 59 to 246 cells here one at most. (With 26 bits left every tenth does.)
+@pytest.mark.parametrize("bright,dim,w,pixels", [(1000.0, 1e-15, 1100, 10), (4e5, 1e-12, 1100, 10), (1000.0, 1000 * 2.0 ** -26, 2000, 16),
+                                                 (1.0, 2.0 ** -26, 3000, 12), (1.0, 1e-3, 2000, 8), (1.0, 2.0 ** -20, 1100, 18),
+                                                 (1e-3, 0.0, 1100, 10)])
+def test_dim_runs_behind_bright_pixels_keep_their_bits(bright, dim, w, pixels, rasterizer, oracle):
+    print(f"[case] lift rows, runs of {pixels} x {dim} behind {bright}, width {w}", flush=True)
+    mn, ln, poses, intr, h = _strip_of_cells(w, pixels)
+    rng = np.random.default_rng(3)
+    img = (dim * rng.uniform(0.5, 1.5, (1, h, w))).astype(np.float32)
+    img[0, :, :12] = bright * rng.uniform(0.5, 1.5, (h, 12))
+    view = ViewSpec(w, h)
+    val, cnt = _lift(rasterizer, mn, ln, view, poses, intr, img, 0)
+    want_v, want_c = np.zeros(len(mn), np.float32), np.zeros(len(mn), np.int32)
+    oracle.lift_error(mn, ln, want_v, want_c, view, poses, intr, img, border_pixels=0)
+    assert want_c.min() >= pixels - 2
+    np.testing.assert_array_equal(cnt, want_c)
+    np.testing.assert_allclose(val, want_v, rtol=2.0 ** -23, atol=0.0)  # at most one unit in the last place
+    assert (val != want_v).sum() <= 1

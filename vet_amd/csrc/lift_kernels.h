@@ -74,7 +74,8 @@ struct LiftPass
     double* sums;       // running sums of the band, see lift_sum_at; null: the image is too wide for one band to hold a row
 };
 
-// Where the sum of the pixels [0, x) of image row y is, 0 <= x <= width.
+// Where the sum of the pixels [0, x) of image row y is, 0 <= x <= width. The entry of x = 0 is zero, with the sign bit set
+// where rounding has swallowed a pixel of the row.
 __device__ __forceinline__ size_t lift_sum_at(const LiftPass& a, int x, int y)
 {
     const uint32_t r = (uint32_t)(y - a.y0);
@@ -142,8 +143,8 @@ __global__ void __launch_bounds__(kLiftPrefixBlock) lift_prefix_kernel(LiftPass 
             }
         }
     };
-    if (lane == 0) group[wave] = 0.0;  // the empty run
-    double carry = 0.0;
+    double carry  = 0.0;
+    bool faithful = true;  // every pixel with an error has raised the sum, none has lowered it
     float g[kLiftPerLane];
     load(kLiftPerLane * lane, g);
     for (int x0 = 0; x0 < a.width; x0 += kLiftStep)
@@ -162,17 +163,28 @@ __global__ void __launch_bounds__(kLiftPrefixBlock) lift_prefix_kernel(LiftPass 
             const double up = __shfl_up(incl, d, kWave);
             if (lane >= d) incl += up;
         }
-        const double before = carry + (incl - own);
-        carry += __shfl(incl, kWave - 1, kWave);
+        const double in_front = __shfl_up(incl, 1, kWave);
+        const double before   = lane == 0 ? carry : carry + in_front;  // the last entry of the lane in front, to the bit
         __syncthreads();  // the block of the step before has been stored
+        double last = before;
 #pragma unroll
-        for (int k = 0; k < kLiftPerLane; ++k) s_sum[(kLiftPerLane * lane + k) * kLiftRows + wave] = before + p[k];
+        for (int k = 0; k < kLiftPerLane; ++k)
+        {
+            const double sum = k == kLiftPerLane - 1 ? carry + incl : before + p[k];
+            faithful &= g[k] > 0.f ? sum > last : sum >= last;
+            last = sum;
+            s_sum[(kLiftPerLane * lane + k) * kLiftRows + wave] = sum;
+        }
+        carry = __shfl(last, kWave - 1, kWave);
         __syncthreads();
         const int columns = min(kLiftStep, a.width - x0);
         for (int k = threadIdx.x; k < columns * kLiftRows; k += kLiftPrefixBlock) group[(size_t)(x0 + 1) * kLiftRows + k] = s_sum[k];
 #pragma unroll
         for (int k = 0; k < kLiftPerLane; ++k) g[k] = next[k];
     }
+    // the empty run; its sign says whether equal entries of the row mean that there is no error between them
+    const bool all_faithful = __ballot(!faithful) == 0ull;
+    if (lane == 0) group[wave] = all_faithful ? 0.0 : -0.0;
 }
 
 // tris_indices of the reference (src/lib/rendering/RenderForward.cu:665-666): two triangles per face of the box, corner
@@ -298,15 +310,17 @@ __device__ __forceinline__ bool in_any_triangle(const Corners& f, float x, float
     return false;
 }
 
-// Sum of the pixels [x0, x1) of row y.
+// Sum of the pixels [x0, x1) of row y. The difference of two running sums is taken where it keeps its bits: an entry is
+// off by 2^-50 of itself or so, so a run of at least 2^-12 of what lies in front of it is good to 38 bits, 14 more than the
+// float it ends in. Dimmer runs (also those behind a pixel that is not finite) are added up pixel by pixel; a difference
+// of zero is a run without any error where the row says so.
 __device__ __forceinline__ double lift_run_sum(const LiftPass& a, int x0, int x1, int y)
 {
     if (a.sums)
     {
         const double lo = a.sums[lift_sum_at(a, x0, y)], s = a.sums[lift_sum_at(a, x1, y)] - lo;
-        // Taken where the difference has kept its digits: not behind a pixel that is not finite, nor behind sums that
-        // dwarf it (a run without any error is a difference of zero).
-        if (s >= lo * 0x1p-26 || (s == 0.0 && lo < 0x1p20)) return s;
+        if (s >= lo * 0x1p-12) return s;
+        if (s == 0.0 && !__builtin_signbit(a.sums[lift_sum_at(a, 0, y)])) return 0.0;
     }
     double s = 0.0;
     for (int x = x0; x < x1; ++x) s += (double)lift_pixel_error(a, x, y);
