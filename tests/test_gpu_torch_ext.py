@@ -340,6 +340,36 @@ def test_distortion_is_found_when_two_intrinsics_tensors_take_turns():
         _plain_call(scene, torch_ops, intrinsics=a)
 
 
+def _call_that_throws(scene, torch_ops, intrinsics):
+    """A call that is refused behind the start of the distortion check (its textures do not fit its points)."""
+    texture = torch.zeros((scene.texture.shape[0], scene.num_points + 1), device="cuda")
+    with pytest.raises(RuntimeError, match="texture must be"):
+        _plain_call(scene, torch_ops, texture=texture, intrinsics=intrinsics)
+
+
+def test_a_refused_call_leaves_no_distortion_check_behind():
+    """A call with another intrinsics tensor that throws for a reason of its own must neither make the next call with a
+    good tensor throw nor count as a look at its tensor."""
+    from vet_amd import torch_ops
+
+    scene = synthetic.tiny_scene(num_points=500, K=8, seed=43)
+    good, bad = (torch.from_numpy(scene.intrinsics.copy()).cuda() for _ in range(2))
+    bad[0, 5] = 0.25
+    assert len(_plain_call(scene, torch_ops, intrinsics=good)) == scene.num_layers
+    _call_that_throws(scene, torch_ops, bad)
+    assert len(_plain_call(scene, torch_ops, intrinsics=good)) == scene.num_layers
+    with pytest.raises(RuntimeError, match="distortion"):
+        _plain_call(scene, torch_ops, intrinsics=bad)
+    # without distortion when the refused call came, with it afterwards
+    late = torch.from_numpy(scene.intrinsics.copy()).cuda()
+    assert len(_plain_call(scene, torch_ops, intrinsics=good)) == scene.num_layers
+    _call_that_throws(scene, torch_ops, late)
+    late[0, 5] = 0.25
+    assert len(_plain_call(scene, torch_ops, intrinsics=good)) == scene.num_layers
+    with pytest.raises(RuntimeError, match="distortion"):
+        _plain_call(scene, torch_ops, intrinsics=late)
+
+
 def test_add_depth_to_network_appends_a_zero_channel(oracle):
     """The blend modes never write the depth tensors (src/lib/rendering/PointRenderer.cu:1061-1066 hands out the zero-filled
     buffers); PointRenderModuleImpl::forward appends them to the images as a channel (RenderModule.cpp:223-232), behind

@@ -150,6 +150,12 @@ void PointRendererCache::BeginIntrinsicsCheck(const torch::Tensor& intrinsics)
     TORCH_CHECK(intrinsics.defined() && intrinsics.dim() == 2 && intrinsics.size(1) == 13,
                 "intrinsics must be [num_cameras,13]");
     PollDeviceFlags();
+    if (reading_intrinsics_.defined())
+    {
+        // a call that threw before FinishIntrinsicsCheck: its copy lands, and says nothing about this call's cameras
+        read_event_->synchronize();
+        reading_intrinsics_ = torch::Tensor();
+    }
     const void* ptr       = intrinsics.data_ptr();
     const int64_t version = (int64_t)intrinsics._version();
     const auto held       = checked_intrinsics_storage_.lock();
@@ -162,13 +168,13 @@ void PointRendererCache::BeginIntrinsicsCheck(const torch::Tensor& intrinsics)
         return;
     }
     torch::NoGradGuard no_grad;
-    if (reading_intrinsics_.defined()) read_event_->synchronize();  // a call that threw in between left its copy under way
-    reading_intrinsics_ = intrinsics.detach();
+    if (!read_event_) read_event_ = std::make_unique<c10::Event>(c10::DeviceType::CUDA);
     if (!read_host_.defined() || read_host_.numel() < intrinsics.numel())
         read_host_ = torch::empty({intrinsics.numel()}, torch::TensorOptions().dtype(torch::kFloat32).pinned_memory(true));
-    read_host_.narrow(0, 0, intrinsics.numel()).view(intrinsics.sizes()).copy_(reading_intrinsics_, /*non_blocking=*/true);
-    if (!read_event_) read_event_ = std::make_unique<c10::Event>(c10::DeviceType::CUDA);
+    read_host_.narrow(0, 0, intrinsics.numel()).view(intrinsics.sizes()).copy_(intrinsics.detach(), /*non_blocking=*/true);
     read_event_->record(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA());
+    reading_intrinsics_ = intrinsics.detach();
+    reading_version_    = version;  // what is written to the tensor from here on is not in the copy
 }
 
 void PointRendererCache::FinishIntrinsicsCheck()
@@ -181,7 +187,7 @@ void PointRendererCache::FinishIntrinsicsCheck()
     for (int64_t i = 0; i < intrinsics.numel(); ++i) TORCH_CHECK(i % 13 < 5 || k[i] == 0.f, kDistortionRefused);
     checked_intrinsics_ptr_     = intrinsics.data_ptr();
     checked_intrinsics_storage_ = intrinsics.storage().getWeakStorageImpl();
-    checked_intrinsics_version_ = (int64_t)intrinsics._version();
+    checked_intrinsics_version_ = reading_version_;
     checked_intrinsics_numel_   = intrinsics.numel();
     flags_wanted_               = false;
     calls_since_flags_          = 0;
@@ -375,13 +381,14 @@ torch::autograd::variable_list PointRender::forward(torch::autograd::AutogradCon
             a.out_mask[l] = mask[l].data_ptr<float>();
         }
     }
+    std::vector<torch::Tensor> weights;
     if (info->cache->keep_layer_weights)
     {
-        info->cache->layer_weights.resize(L);
+        weights.resize(L);
         for (int l = 0; l < L; ++l)
         {
-            info->cache->layer_weights[l] = torch::empty({B, 1, lay.layer_h[l], lay.layer_w[l]}, f32);
-            a.out_weight[l]               = info->cache->layer_weights[l].data_ptr<float>();
+            weights[l]      = torch::empty({B, 1, lay.layer_h[l], lay.layer_w[l]}, f32);
+            a.out_weight[l] = weights[l].data_ptr<float>();
         }
     }
     a.workspace         = workspace.data_ptr();
@@ -395,6 +402,7 @@ torch::autograd::variable_list PointRender::forward(torch::autograd::AutogradCon
         info->cache->FinishIntrinsicsCheck();  // may throw: nothing of this call has been handed out yet
         info->cache->NoteDeviceFlags(workspace, lay);
     }
+    if (info->cache->keep_layer_weights) info->cache->layer_weights = std::move(weights);
     if (info->params.size_bins_from_history)
         info->cache->NoteFragmentCounts(workspace, lay, N, L, info->images[0].w, info->images[0].h, a.params.render_mode);
 

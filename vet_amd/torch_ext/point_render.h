@@ -173,6 +173,7 @@ class PointRendererCache
     c10::weak_intrusive_ptr<c10::StorageImpl> checked_intrinsics_storage_{c10::intrusive_ptr<c10::StorageImpl>()};
     int64_t checked_intrinsics_version_ = -1, checked_intrinsics_numel_ = -1;
     torch::Tensor reading_intrinsics_, read_host_;  // the tensor whose copy is under way, and where it lands
+    int64_t reading_version_ = -1;                  // its version counter when the copy was put on the stream
     std::unique_ptr<c10::Event> read_event_;
     bool flags_wanted_ = false, flags_pending_ = false;
     int64_t calls_since_flags_ = 0;
