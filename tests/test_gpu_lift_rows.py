@@ -71,9 +71,9 @@ def test_pixels_that_are_not_finite_stay_with_their_cells(rasterizer, oracle):
     np.testing.assert_allclose(val, want_v, rtol=1e-5, atol=1e-9)
 
 
-# cells next to the camera in an image wide enough for rows with hundreds of open columns: such a cell leaves its rows and
-# is tested pixel by pixel as a whole, unless the image takes several bands
-@pytest.mark.parametrize("w,h", [(1920, 1080), (3000, 1500)])
+# cells next to the camera in an image wide enough for rows with hundreds of open columns: such a cell leaves its rows, those
+# of this band and the ones behind it, and is tested pixel by pixel (two bands of rows in the two larger images)
+@pytest.mark.parametrize("w,h", [(1920, 1080), (3000, 1500), (3840, 2160)])
 @pytest.mark.parametrize("yaw,depth", [(0.02, 0.05), (0.3, 0.002), (-0.45, 0.01)])
 def test_cells_with_many_wide_open_rows(w, h, yaw, depth, rasterizer, oracle):
     print(f"[case] lift rows {w}x{h} yaw {yaw} depth {depth}", flush=True)

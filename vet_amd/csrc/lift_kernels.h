@@ -38,13 +38,16 @@ constexpr float kLiftThin       = 0.05f; // smallest angle (about) of a triangle
 constexpr int kLiftOpen         = 8;     // open pixels of a row that go to the list; a row with more is left to a wave
 constexpr int kLiftOpenPixels   = 256;   // the list; it is worked off when half full (a lane tests what does not fit)
 constexpr int kLiftOpenRows     = 128;   // such rows a workgroup keeps (a lane finishes what does not fit)
-// A cell whose open rows of more than kLiftWideRow columns add up to more than kLiftWideWork is tested pixel by pixel by
-// lift_plain_kernel: next to the camera the lines of slivers sweep hundreds of columns in hundreds of rows, and the one
-// workgroup that had such a cell held the launch up (three 1080p views, one of them like that: 1.61 ms of kernels, now
-// 0.55 ms; its launch of the rows 1.32 ms, now 0.20 ms; the scene above 6.5 ms, now 0.29 ms). Limits of 64 and 128 columns
-// a row and 1024 and 8192 in all measure the same within 5 %, 32768 in all is slower by half on that scene.
+// A cell whose open rows of more than kLiftWideRow columns add up to more than kLiftWideWork and more than one in
+// kLiftWideShare of its box's pixels is tested pixel by pixel by lift_plain_kernel: next to the camera the lines of slivers
+// sweep hundreds of columns in hundreds of rows, and the one workgroup that had such a cell held the launch up (three 1080p
+// views, one of them like that: 1.61 ms of kernels, now 0.57 ms; with 1 m cells at 3840x2160, two bands of rows, 3.47 ms,
+// now 1.92 ms). Limits of 64 and 128 columns a row and 1024 and 8192 in all measure the same within 5 % at 1080p, 32768 in
+// all is slower by half there; without the share of the box, 0.25 m cells at 3840x2160 take 1.79 ms instead of 1.49 (a few
+// wide rows are less work than all pixels of a large box), shares of 256 to 1024 measure the same.
 constexpr int kLiftWideRow      = 256;
 constexpr int kLiftWideWork     = 2048;
+constexpr int kLiftWideShare    = 512;
 constexpr size_t kLiftSums      = (size_t)1 << 22;  // running sums that exist at a time (33.5 MB: an image of 4.2 M
                                                     // pixels); taller images take several bands
 static_assert(sizeof(DeviceView) <= VETRAST_LIFT_QUEUE_LENGTH_OFFSET && VETRAST_LIFT_QUEUE_LENGTH_OFFSET + 4 <= VETRAST_LIFT_FLAGS_OFFSET,
@@ -65,12 +68,12 @@ struct LiftPass
     DeviceView* view;
     uint32_t* large_cells;
     uint32_t* flags;
-    uint32_t* num_plain;   // cells left to lift_plain_kernel, then per such cell its number, sum, count and finished shares
-    uint32_t* plain_cell;
-    double* plain_sum;
-    int32_t* plain_count;
-    uint32_t* plain_done;
-    double* cell_sums;  // [num_cells] sums of the bands so far; only with several bands
+    uint32_t* num_plain;    // cells left to lift_plain_kernel
+    uint32_t* plain_cell;   // their numbers
+    // [num_cells] each, written for cells left to lift_plain_kernel and, with several bands, for every cell:
+    double* cell_sums;      // sum of the bands so far
+    uint32_t* plain_state;  // 0, or first image row that is lift_plain_kernel's + 1 in bits 8.., below them its finished shares
+    int32_t* plain_count;   // pixels lift_plain_kernel has counted
     double* sums;       // running sums of the band, see lift_sum_at; null: the image is too wide for one band to hold a row
 };
 
@@ -279,7 +282,7 @@ struct LiftCell
     float sliver_width[kLiftSliverMax];  // their half width in columns, or -(half width in rows)
     uint32_t left_mask;                  // bit t: the third bound of triangle t is a left one; bit 8 + k: outline[k] is
     int num_outline, num_tri, num_sliver;
-    int wide;      // columns of the wide open rows; kLiftWideWork + 1 and more: the cell is lift_plain_kernel's
+    int wide;      // columns of the wide open rows less the limit; above 0: the cell is lift_plain_kernel's
     int count;
     double sum;
 };
@@ -327,14 +330,14 @@ __device__ __forceinline__ double lift_run_sum(const LiftPass& a, int x0, int x1
     return s;
 }
 
-// Enters a cell, once per call, into the list of lift_plain_kernel (a few cells of a grid).
-__device__ __forceinline__ void leave_to_plain_kernel(const LiftPass& a, int64_t cell)
+// Leaves the rows of a cell from this band on to lift_plain_kernel (a few cells of a grid, once per call). `sum`: what the
+// bands in front of it have added up.
+__device__ __forceinline__ void leave_to_plain_kernel(const LiftPass& a, int64_t cell, double sum)
 {
-    const uint32_t at = atomicAdd(a.num_plain, 1u);
-    a.plain_cell[at]  = (uint32_t)cell;
-    a.plain_sum[at]   = 0.0;
-    a.plain_count[at] = 0;
-    a.plain_done[at]  = 0u;
+    a.plain_cell[atomicAdd(a.num_plain, 1u)] = (uint32_t)cell;
+    a.cell_sums[cell]   = sum;
+    a.plain_count[cell] = 0;
+    a.plain_state[cell] = (uint32_t)(a.y0 + 1) << 8;  // (an image has less than 2^24 rows)
 }
 
 __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
@@ -345,6 +348,7 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     __shared__ uint2 s_pixel[kLiftOpenPixels];  // open pixels: x | slot << 24, y
     __shared__ int s_num_open, s_num_pixels;
     __shared__ uint32_t s_large;
+    __shared__ bool s_left[kLiftCells];  // the cell is lift_plain_kernel's
     if (threadIdx.x == 0) s_num_open = s_num_pixels = 0, s_large = 0u;
     __syncthreads();
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -354,7 +358,8 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         const int slot = tid / kLiftSetup, part = tid % kLiftSetup;
         LiftCell& f        = s_cell[slot];
         const int64_t cell = (int64_t)slot * gridDim.x + blockIdx.x;
-        bool behind        = cell >= a.num_cells;
+        const bool left    = !a.first && cell < a.num_cells && a.plain_state[cell] != 0u;  // by an earlier band
+        bool behind        = cell >= a.num_cells || left;
         float max_x = -10000000.f, max_y = -10000000.f, min_x = 10000000.f, min_y = 10000000.f;
         float far = 0.f;  // largest coordinate
         if (!behind)
@@ -412,15 +417,14 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         const int x_size = seen ? (int)(max_x - min_x) : 0, y_size = seen ? (int)(max_y - min_y) : 0;
         seen             = x_size > 0 && y_size > 0;
         const bool large = part == 0 && seen && x_size * y_size > kLiftLargeCell;
-        if (seen && plain)
-        {
-            if (part == 0 && a.first) leave_to_plain_kernel(a, cell);
-            seen = false;
-        }
+        const bool leaves = seen && plain;  // (in the first band: the corners say so)
+        if (leaves) seen = false;
         if (part == 0)
         {
+            if (leaves) leave_to_plain_kernel(a, cell, 0.0);
+            s_left[slot]  = leaves || left;
             s_start[slot] = seen ? y_size : 0;
-            f.wide        = 0;
+            f.wide        = -max(kLiftWideWork, x_size * y_size / kLiftWideShare);
             f.count       = 0;
             f.sum         = 0.0;
             f.left_mask = 0u;
@@ -704,9 +708,8 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         }
         if (open > kLiftOpen)
         {
-            // (one band only: with several the cell's rows of the other bands may be in its sums already)
             const int width = x_end - x_first;
-            if (width > kLiftWideRow && a.first && a.last && atomicAdd(&f.wide, width) + width > kLiftWideWork) return;
+            if (width > kLiftWideRow && atomicAdd(&f.wide, width) + width > 0) return;
             const int at = atomicAdd(&s_num_open, 1);
             if (at < kLiftOpenRows)
             {
@@ -758,7 +761,7 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     {
         const int4 row = s_open[k];
         LiftCell& f    = s_cell[row.x];
-        if (f.wide > kLiftWideWork) continue;
+        if (f.wide > 0) continue;
         int count      = 0;
         double sum     = 0.0;
         for (int x = row.z + lane; x < row.w; x += kWave)
@@ -779,24 +782,26 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     if (tid < kLiftCells)
     {
         const int64_t cell = (int64_t)tid * gridDim.x + blockIdx.x;
-        if (cell < a.num_cells && s_cell[tid].wide > kLiftWideWork)
-            leave_to_plain_kernel(a, cell);
-        else if (cell < a.num_cells)
+        if (cell >= a.num_cells || s_left[tid]) return;
+        const double in_front = a.first ? 0.0 : a.cell_sums[cell];
+        if (s_cell[tid].wide > 0)
         {
-            double sum      = s_cell[tid].sum;
-            const int count = s_cell[tid].count;
-            if (!a.first) sum += a.cell_sums[cell];
-            if (!a.last) a.cell_sums[cell] = sum;
-            if (count > 0) a.access_count[cell] += count;
-            // one rounding per call: the float terms of a cell are summed in double
-            if (a.last && (count > 0 || (!a.first && sum != 0.0))) a.value[cell] = (float)((double)a.value[cell] + sum);
+            leave_to_plain_kernel(a, cell, in_front);
+            return;
         }
+        const double sum = s_cell[tid].sum + in_front;
+        const int count  = s_cell[tid].count;
+        if (!a.last) a.cell_sums[cell] = sum;
+        if (a.first && !a.last) a.plain_state[cell] = 0u;
+        if (count > 0) a.access_count[cell] += count;
+        // one rounding per call: the float terms of a cell are summed in double
+        if (a.last && (count > 0 || in_front != 0.0)) a.value[cell] = (float)((double)a.value[cell] + sum);
     }
 }
 
-// The cells the rows were not made for: kLiftPlainShare workgroups per cell, each every kLiftPlainShare-th row of its box,
-// a thread per pixel. The last one to finish adds the cell's sum, with one rounding, to its value. The list is empty or
-// a few cells long; the launch is fixed.
+// The cells the rows were not made for: kLiftPlainShare workgroups per cell, each every kLiftPlainShare-th row of its box
+// (from the band on that left it here), a thread per pixel. The last one to finish adds the cell's sum, with one rounding,
+// to its value. The list is empty or a few cells long; the launch is fixed.
 __global__ void __launch_bounds__(kBlock) lift_plain_kernel(LiftPass a)
 {
     __shared__ double s_sum[kBlock / kWave];
@@ -807,6 +812,7 @@ __global__ void __launch_bounds__(kBlock) lift_plain_kernel(LiftPass a)
     for (uint32_t k = blockIdx.y; k < cells; k += kLiftPlainAtOnce)
     {
         const int64_t cell = (int64_t)a.plain_cell[k];
+        const int from     = (int)(a.plain_state[cell] >> 8) - 1;  // the rows in front of it are in the sum
         if (wave == 0)
         {
             CellFootprint f;
@@ -820,7 +826,7 @@ __global__ void __launch_bounds__(kBlock) lift_plain_kernel(LiftPass a)
             for (int col = tid; col < s_f.x_size; col += kBlock)
             {
                 const int x = (int)((float)col + s_f.min_x), y = (int)((float)row + s_f.min_y);
-                if (x < 0 || x >= a.width || y < 0 || y >= a.height || !in_any_triangle(s_f, (float)x, (float)y)) continue;
+                if (x < 0 || x >= a.width || y < from || y >= a.height || !in_any_triangle(s_f, (float)x, (float)y)) continue;
                 ++count;
                 sum += (double)lift_pixel_error(a, x, y);
             }
@@ -833,15 +839,15 @@ __global__ void __launch_bounds__(kBlock) lift_plain_kernel(LiftPass a)
             for (int w = 1; w < kBlock / kWave; ++w) sum += s_sum[w], count += s_count[w];
             if (count > 0)
             {
-                atomicAdd(&a.plain_sum[k], sum);
-                atomicAdd(&a.plain_count[k], count);
+                atomicAdd(&a.cell_sums[cell], sum);
+                atomicAdd(&a.plain_count[cell], count);
             }
             __threadfence();
-            if (atomicAdd(&a.plain_done[k], 1u) == (uint32_t)kLiftPlainShare - 1u)
+            if ((atomicAdd(&a.plain_state[cell], 1u) & 0xFFu) == (uint32_t)kLiftPlainShare - 1u)
             {
                 __threadfence();
-                const double all = atomicAdd(&a.plain_sum[k], 0.0);
-                a.access_count[cell] += atomicAdd(&a.plain_count[k], 0);
+                const double all = atomicAdd(&a.cell_sums[cell], 0.0);
+                a.access_count[cell] += atomicAdd(&a.plain_count[cell], 0);
                 a.value[cell] = (float)((double)a.value[cell] + all);
             }
         }

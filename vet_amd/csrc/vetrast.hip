@@ -47,12 +47,12 @@ inline size_t align_up(size_t v, size_t a)
 }
 
 // Bytes of error-lifting scratch for num_cells cells: header (camera constants, counters, flag word), per cell the sum of
-// the bands so far (images that take several) and the list of cells tested pixel by pixel (number, sum, count, finished
-// shares), the running sums of a band of image rows.
+// the bands so far (images that take several) and what lift_plain_kernel needs of the cells that are left to it (their
+// list, rows and finished shares, counted pixels), the running sums of a band of image rows.
 constexpr size_t align_up_c(size_t v, size_t a) { return (v + a - 1) / a * a; }
 constexpr size_t lift_workspace_bytes_for(size_t num_cells)
 {
-    return kLiftHeader + 2 * align_up_c(num_cells * sizeof(double), kAlign) + 3 * align_up_c(num_cells * sizeof(uint32_t), kAlign) +
+    return kLiftHeader + align_up_c(num_cells * sizeof(double), kAlign) + 3 * align_up_c(num_cells * sizeof(uint32_t), kAlign) +
            kLiftSums * sizeof(double);
 }
 
@@ -398,11 +398,10 @@ void launch_lift(const vetrast_lift_args* a, char* ws, hipStream_t stream)
     const size_t words   = align_up((size_t)a->num_cells * sizeof(uint32_t), kAlign);
     char* at             = ws + kLiftHeader;
     lp.cell_sums         = reinterpret_cast<double*>(at);
-    lp.plain_sum         = reinterpret_cast<double*>(at + doubles);
-    lp.plain_cell        = reinterpret_cast<uint32_t*>(at + 2 * doubles);
-    lp.plain_count       = reinterpret_cast<int32_t*>(at + 2 * doubles + words);
-    lp.plain_done        = reinterpret_cast<uint32_t*>(at + 2 * doubles + 2 * words);
-    lp.sums              = reinterpret_cast<double*>(at + 2 * doubles + 3 * words);
+    lp.plain_cell        = reinterpret_cast<uint32_t*>(at + doubles);
+    lp.plain_state       = reinterpret_cast<uint32_t*>(at + doubles + words);
+    lp.plain_count       = reinterpret_cast<int32_t*>(at + doubles + 2 * words);
+    lp.sums              = reinterpret_cast<double*>(at + doubles + 3 * words);
 
     ViewSource src;
     src.image_index  = v.image_index;
