@@ -367,8 +367,9 @@ int vetrast_adam_step(vetrast_ctx* ctx, const vetrast_adam_args* args, void* str
  * (VETRAST_LIFT_BORDER_PIXELS in the reference); every integer pixel of the box that lies in one of the 12 projected
  * face triangles adds sum_c |loss_image[c][y][x]| to cell_value and 1 to cell_access_count.
  *
- * The reference adds the float terms with atomics in arrival order; here the terms of a cell are summed in double and
- * added to cell_value with one rounding, which makes the call reproducible. cell_value and cell_access_count are
+ * The reference adds the float terms with atomics in arrival order; here the terms of a cell are summed in double (also
+ * in arrival order, row by row) and added to cell_value with one rounding: two calls give the same float unless a sum lies
+ * within its last double bits of halfway between two floats. cell_value and cell_access_count are
  * accumulated into, not cleared (ResetCellValues / NormalizeBBCellValue stay with the caller,
  * src/lib/rendering/NeuralPointCloudCuda.h:42-52). */
 #define VETRAST_LIFT_BORDER_PIXELS 32
@@ -393,16 +394,20 @@ typedef struct vetrast_lift_args
     const float* loss_image;     /* device [channels,height,width], e.g. |target - output| of that view */
     int32_t channels, height, width;
     int32_t border_pixels;       /* >= 0; the reference's constant is VETRAST_LIFT_BORDER_PIXELS */
-    void* workspace;             /* device, 256-byte aligned, vetrast_lift_workspace_bytes(num_cells) bytes */
+    void* workspace;             /* device, 256-byte aligned, vetrast_lift_workspace_bytes_for_image(num_cells, width,
+                                  * height) bytes or more */
     size_t workspace_bytes;
 } vetrast_lift_args;
+/* Bytes for an image of that size (20 per cell, 8 per pixel and row, at most 33.6 MB of the latter), and bytes that do for
+ * an image of any size. */
+size_t vetrast_lift_workspace_bytes_for_image(int64_t num_cells, int32_t width, int32_t height);
 size_t vetrast_lift_workspace_bytes(int64_t num_cells);
 int vetrast_lift_error(vetrast_ctx* ctx, const vetrast_lift_args* args, void* stream);
 
 /* vetrast_lift_error for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc). It has no counterpart in the reference. Same arguments, same kernels and
  * same results as vetrast_lift_error, but `workspace` / `workspace_bytes` are ignored: the scratch is an array inside
- * the library (about 48 MB of device memory per GPU, held until the process ends), whose address on the context's
+ * the library (about 27 MB of device memory per GPU, held until the process ends), whose address on the context's
  * device vetrast_create looks up once. The call itself allocates and frees nothing, creates no events (it reports no
  * timing scope) and only launches kernels.
  *   - num_cells > VETRAST_LIFT_STATIC_MAX_CELLS is refused with VETRAST_ERR_TOO_LARGE.

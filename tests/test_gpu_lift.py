@@ -124,6 +124,25 @@ def test_constant_image_gives_channels_times_count(rasterizer):
     assert int(cnt.max()) <= (1920 - 64) * (1080 - 64)
 
 
+def test_workspace_of_the_images_size_is_enough_and_less_is_refused(rasterizer, oracle):
+    mn, ln, view, poses, intr, img = _rotated_view_case(4, W=161, H=119)
+    n = len(mn)
+    need = int(rasterizer.lib.vetrast_lift_workspace_bytes_for_image(n, 161, 119))
+    assert need < 300_000 + 24 * n < int(rasterizer.lib.vetrast_lift_workspace_bytes(n))
+    want_v, want_c = np.zeros(n, np.float32), np.zeros(n, np.int32)
+    oracle.lift_error(mn, ln, want_v, want_c, view, poses, intr, img, border_pixels=8)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (mn, ln, want_v * 0, want_c * 0, poses, intr, img)]
+    guarded = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    call = lambda ws: rasterizer.lift_error(dev[0], dev[1], dev[2], dev[3], view, dev[4], dev[5], dev[6], border_pixels=8, workspace=ws)
+    with pytest.raises(abi.VetrastError) as e:
+        call(guarded[:need - 1])
+    assert e.value.status == abi.ERR_WORKSPACE_SMALL
+    call(guarded[:need])
+    torch.cuda.synchronize()
+    _assert_parity(dev[2].cpu().numpy(), dev[3].cpu().numpy(), want_v, want_c)
+    assert bool((guarded[need:] == 0x5A).all())
+
+
 def test_argument_checks(rasterizer):
     scene = synthetic.tiny_scene()
     mn, ln = synthetic.cell_grid(scene.position[:, :3], 0.5)

@@ -75,6 +75,15 @@ def test_static_scratch_matches_workspace_twice_in_a_row(rasterizer):
     _assert_same(got_v, got_c, want_v, want_c)
 
 
+def test_static_scratch_takes_larger_images_in_bands(rasterizer):
+    # 3.7 M running sums: one band of rows with a caller's workspace, two in the library's array
+    print("[case] lift_error_static, 2560x1440", flush=True)
+    scene, mn, ln, img = _case(200_000, 0.5, 7, height=1440, width=2560)
+    got_v, got_c, want_v, want_c, c0, _ = _both(rasterizer, scene, mn, ln, img)
+    assert (want_c - c0).sum() > 10_000_000
+    _assert_same(got_v, got_c, want_v, want_c)
+
+
 def test_static_scratch_refuses_grids_beyond_its_maximum(rasterizer):
     n = abi.LIFT_STATIC_MAX_CELLS + 1
     scene = synthetic.tiny_scene()

@@ -205,6 +205,7 @@ SYMBOLS = {
     "vetrast_pack_descriptors": (C.c_int, [C.c_void_p, C.POINTER(PackArgs), C.c_void_p]),
     "vetrast_adam_step": (C.c_int, [C.c_void_p, C.POINTER(AdamArgs), C.c_void_p]),
     "vetrast_lift_workspace_bytes": (C.c_size_t, [C.c_int64]),
+    "vetrast_lift_workspace_bytes_for_image": (C.c_size_t, [C.c_int64, C.c_int32, C.c_int32]),
     "vetrast_lift_error": (C.c_int, [C.c_void_p, C.POINTER(LiftArgs), C.c_void_p]),
     "vetrast_lift_error_static": (C.c_int, [C.c_void_p, C.POINTER(LiftArgs), C.c_void_p]),
     "vetrast_query_device_flags": (C.c_int, [C.c_void_p, C.c_void_p, C.POINTER(WorkspaceLayout), C.c_void_p]),

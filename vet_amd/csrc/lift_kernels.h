@@ -48,8 +48,9 @@ constexpr int kLiftOpenRows     = 128;   // such rows a workgroup keeps (a lane 
 constexpr int kLiftWideRow      = 256;
 constexpr int kLiftWideWork     = 2048;
 constexpr int kLiftWideShare    = 512;
-constexpr size_t kLiftSums      = (size_t)1 << 22;  // running sums that exist at a time (33.5 MB: an image of 4.2 M
-                                                    // pixels); taller images take several bands
+constexpr size_t kLiftSums      = (size_t)1 << 22;  // running sums that exist at a time in a caller's workspace, at most
+                                                    // (33.5 MB: an image of 4.2 M pixels); taller images take several bands
+constexpr size_t kLiftStaticSums = (size_t)1 << 21; // the same in the library's own array (16.8 MB: a 1080p image)
 static_assert(sizeof(DeviceView) <= VETRAST_LIFT_QUEUE_LENGTH_OFFSET && VETRAST_LIFT_QUEUE_LENGTH_OFFSET + 4 <= VETRAST_LIFT_FLAGS_OFFSET,
               "the header's three parts must not overlap");
 

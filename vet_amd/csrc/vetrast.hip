@@ -50,10 +50,17 @@ inline size_t align_up(size_t v, size_t a)
 // the bands so far (images that take several) and what lift_plain_kernel needs of the cells that are left to it (their
 // list, rows and finished shares, counted pixels), the running sums of a band of image rows.
 constexpr size_t align_up_c(size_t v, size_t a) { return (v + a - 1) / a * a; }
-constexpr size_t lift_workspace_bytes_for(size_t num_cells)
+constexpr size_t lift_workspace_bytes_for(size_t num_cells, size_t num_sums)
 {
     return kLiftHeader + align_up_c(num_cells * sizeof(double), kAlign) + 3 * align_up_c(num_cells * sizeof(uint32_t), kAlign) +
-           kLiftSums * sizeof(double);
+           num_sums * sizeof(double);
+}
+
+// Running sums an image can use: whole groups of rows of width + 1 entries.
+inline size_t lift_sums_for(int64_t width, int64_t height)
+{
+    const size_t rows = (size_t)((height + kLiftRows - 1) / kLiftRows * kLiftRows);
+    return std::min(kLiftSums, rows * ((size_t)width + 1));
 }
 
 #define VET_HIP(ctx, expr)                               \
@@ -323,7 +330,7 @@ ViewPass make_view_pass(const vetrast_forward_args* a, const vetrast_workspace_l
 // library's own, sized for VETRAST_LIFT_STATIC_MAX_CELLS cells. Every GPU the library runs on holds a copy of its own
 // until the process ends. In host code this name only stands for the symbol: the device address is looked up once per
 // device (scratch_of_device) and only that pointer is handed to kernels.
-constexpr size_t kLiftStaticBytes = lift_workspace_bytes_for((size_t)VETRAST_LIFT_STATIC_MAX_CELLS);
+constexpr size_t kLiftStaticBytes = lift_workspace_bytes_for((size_t)VETRAST_LIFT_STATIC_MAX_CELLS, kLiftStaticSums);
 static __device__ __align__(256) unsigned char scratch[kLiftStaticBytes];
 
 constexpr int kMaxDevices = 64;
@@ -373,10 +380,10 @@ int validate_lift(const vetrast_lift_args* a, bool* nothing_to_do)
     return VETRAST_OK;
 }
 
-// The launches of the error lifting (three for an image of up to kLiftSums pixels) with their scratch at `ws`
-// (lift_workspace_bytes_for(num_cells) bytes, 256-byte aligned). Every word of the scratch a kernel reads has been written
+// The launches of the error lifting (three for an image of one band of rows) with their scratch at `ws`
+// (lift_workspace_bytes_for(num_cells, num_sums) bytes, 256-byte aligned). Every word of the scratch a kernel reads has been written
 // by an earlier kernel of the same call, so nothing needs clearing between calls that share one scratch.
-void launch_lift(const vetrast_lift_args* a, char* ws, hipStream_t stream)
+void launch_lift(const vetrast_lift_args* a, char* ws, size_t num_sums, hipStream_t stream)
 {
     const vetrast_view& v = a->view;
     LiftPass lp;
@@ -413,7 +420,7 @@ void launch_lift(const vetrast_lift_args* a, char* ws, hipStream_t stream)
 
     // rows a cell can cover, in bands whose running sums fit their room
     const int64_t top = std::min<int64_t>(a->border_pixels, a->height), bottom = std::max<int64_t>(top, (int64_t)a->height - a->border_pixels);
-    int64_t band = (int64_t)(kLiftSums / ((size_t)a->width + 1)) / kLiftRows * kLiftRows;
+    int64_t band = (int64_t)(num_sums / ((size_t)a->width + 1)) / kLiftRows * kLiftRows;
     if (band == 0) lp.sums = nullptr, band = bottom - top;  // a single row is too long: runs are added up pixel by pixel
     band = std::max<int64_t>(band, kLiftRows);
     int64_t y = top;
@@ -1245,7 +1252,13 @@ int vetrast_adam_step(vetrast_ctx* ctx, const vetrast_adam_args* a, void* stream
 size_t vetrast_lift_workspace_bytes(int64_t num_cells)
 {
     if (num_cells < 0) return 0;
-    return lift_workspace_bytes_for((size_t)num_cells);
+    return lift_workspace_bytes_for((size_t)num_cells, kLiftSums);
+}
+
+size_t vetrast_lift_workspace_bytes_for_image(int64_t num_cells, int32_t width, int32_t height)
+{
+    if (num_cells < 0 || width < 1 || height < 1) return 0;
+    return lift_workspace_bytes_for((size_t)num_cells, lift_sums_for(width, height));
 }
 
 int vetrast_lift_error(vetrast_ctx* ctx, const vetrast_lift_args* a, void* stream_)
@@ -1255,10 +1268,11 @@ int vetrast_lift_error(vetrast_ctx* ctx, const vetrast_lift_args* a, void* strea
     const int st       = validate_lift(a, &nothing_to_do);
     if (st != VETRAST_OK || nothing_to_do) return st;
     if (!a->workspace || reinterpret_cast<uintptr_t>(a->workspace) % kAlign) return VETRAST_ERR_INVALID_ARG;
-    if (a->workspace_bytes < vetrast_lift_workspace_bytes(a->num_cells)) return VETRAST_ERR_WORKSPACE_SMALL;
+    const size_t num_sums = lift_sums_for(a->width, a->height);
+    if (a->workspace_bytes < lift_workspace_bytes_for((size_t)a->num_cells, num_sums)) return VETRAST_ERR_WORKSPACE_SMALL;
     hipStream_t stream = (hipStream_t)stream_;
     ScopeTimer tm(ctx, stream, VETRAST_SCOPE_LIFT_ERROR);
-    launch_lift(a, static_cast<char*>(a->workspace), stream);
+    launch_lift(a, static_cast<char*>(a->workspace), num_sums, stream);
     VET_HIP(ctx, hipGetLastError());
     return VETRAST_OK;
 }
@@ -1275,7 +1289,7 @@ int vetrast_lift_error_static(vetrast_ctx* ctx, const vetrast_lift_args* a, void
     VET_HIP(ctx, hipGetDevice(&current));
     if (current != ctx->device || !ctx->lift_scratch) return VETRAST_ERR_INVALID_ARG;
     // No timing scope here: a scope takes HIP events and grows a host vector, and this entry point allocates nothing.
-    launch_lift(a, ctx->lift_scratch, (hipStream_t)stream_);
+    launch_lift(a, ctx->lift_scratch, std::min(kLiftStaticSums, lift_sums_for(a->width, a->height)), (hipStream_t)stream_);
     VET_HIP(ctx, hipGetLastError());
     return VETRAST_OK;
 }

@@ -360,7 +360,7 @@ class Rasterizer:
         if static_scratch:
             abi.check(self.lib.vetrast_lift_error_static(self.ctx, C.byref(a), self._stream()), "lift_error_static")
             return None
-        need = int(self.lib.vetrast_lift_workspace_bytes(a.num_cells))
+        need = int(self.lib.vetrast_lift_workspace_bytes_for_image(a.num_cells, a.width, a.height))
         if workspace is None:
             workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=loss_image.device)
         a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()

@@ -288,7 +288,7 @@ void PointRendererCache::FillSceneGridWithLoss(int batch, const CellTensors& cel
     a.height            = (int32_t)loss_img.size(1);
     a.width             = (int32_t)loss_img.size(2);
     a.border_pixels     = VETRAST_LIFT_BORDER_PIXELS;
-    const int64_t need  = (int64_t)vetrast_lift_workspace_bytes(n);
+    const int64_t need  = (int64_t)vetrast_lift_workspace_bytes_for_image(n, a.width, a.height);
     if (!lift_workspace.defined() || lift_workspace.numel() < need || lift_workspace.device() != loss_img.device())
         lift_workspace = torch::empty({std::max<int64_t>(need, 256)}, torch::dtype(torch::kUInt8).device(loss_img.device()));
     a.workspace       = lift_workspace.data_ptr();
