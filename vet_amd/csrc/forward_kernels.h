@@ -468,11 +468,15 @@ __device__ __forceinline__ void scatter_by_wave(const ViewPass& a, uint32_t* __r
 // point id << 2 | corner.
 // The bins a workgroup's points fall into, per layer: a rectangle of bins, with a counter in LDS for each. Points come in
 // blocks of 256 that are neighbours in space, so the rectangles of all layers together hold a hundred or two bins as a rule.
-// 24 KB of LDS, which still lets 6 workgroups share a compute unit: with 2048 slots the blocks of sparse clouds and small
-// crops, which spread over thousands of small bins, fell back to grouping by wave (60 000 points 28 against 18 us, four
-// 512x512 crops of 2 M points 89 against 72 us).
-constexpr int kScatterSlots   = 6144;
-constexpr int kScatterAtOnce  = 8;  // slots a thread has atomics in flight for
+// As many slots as leave the workgroups their place on a compute unit: with one hit per point 8 of them (their registers
+// allow 8; 6144 slots let 6 in: benchmark frame 47.5 against 45.0 us, four town views 200 against 182), with four hits 6,
+// which is what their registers allow. With 2048 slots the blocks of sparse clouds and small crops, which spread over
+// thousands of small bins, group by wave instead (300 000 points at 801x451 28 against 19 us, four 512x512 crops of 2 M
+// points with the 2x2 splat 89 against 72 us).
+template <int HITS>
+constexpr int kScatterSlots = HITS == 1 ? 5088 : 6144;
+template <int HITS>
+constexpr int kScatterWaves = HITS == 1 ? 8 : 6;  // waves of a SIMD unit to leave room for, in registers and LDS
 struct BinRectangle
 {
     int x0, y0, columns, first;  // first bin column and row, columns, number of the first slot
@@ -504,17 +508,25 @@ __device__ __forceinline__ float wave_min(float v, int lane)
 // This is the part of the pass behind the projection: thread `slot` has point i, which is `visible` at p in this view.
 //
 // The workgroup counts its hits per bin in LDS (the LDS atomic's result is the hit's rank among the workgroup's hits of
-// the bin), issues ONE global atomic per bin it touches, for all layers at once, and every hit's record goes to the
-// bin's room at that atomic's result + rank. Where the rectangles need more slots than there are (points in no spatial
-// order, blocks right in front of the camera) the waves group their hits on their own (scatter_by_wave).
-// Measured against grouping by wave alone (2 M points, 4 layers): 2x2 splat at 1080p 154 -> 109 us, four 512x512 crops
-// 116 -> 72 us, one hit per layer at 1080p 42 -> 41 us (there the position loads and record stores are what is left).
+// the bin), the thread of a bin's first hit issues the ONE global atomic for that bin, all layers' atomics before the first
+// result is looked at, and every hit's record goes to the bin's room at that atomic's result + rank. Where the rectangles
+// need more slots than there are (points in no spatial order, blocks right in front of the camera) the waves group their
+// hits on their own (scatter_by_wave).
+// Measured against grouping by wave alone (this pass, 2 M points and 4 layers unless stated): 2x2 splat at 1080p 154 -> 109
+// us, four 512x512 crops of it 116 -> 72 us; one hit per layer: benchmark frame 47.3 -> 46.4 us, another 1080p frame 45.6
+// -> 40.9, four town views of 5.5 M points 206 -> 182, ten million points 309 -> 287, a 203x155 crop of 60 000 points 11.5
+// -> 9.3, 300 000 points in five layers 28.1 -> 17.4, a shuffled cloud 367 -> 347. A cloud whose last fifth is in no order
+// loses, 115 -> 121: its blocks pay for the rectangles and group by wave after all.
+// (While the threads walked the slots, also the empty ones, and worked a slot's bin out of its number: benchmark frame
+// 51.5, the other 44.2, town 202, the small crop 15.0, 300 000 points 18.9 us, the small crop with the 2x2 splat 19.5 where
+// it is 13.4 now.)
 template <int HITS>
 __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* __restrict__ bin_counts,
                                                   const ScatterTargets& out, const PackJob& pack, int slot, int i, bool visible,
                                                   const Projected& p)
 {
-    __shared__ uint32_t s_count[kScatterSlots];  // hits per slot, then the place of the first one inside the bin
+    // hits per slot, then the place of the first one inside the bin
+    __shared__ __align__(16) uint32_t s_count[kScatterSlots<HITS>];
     __shared__ float s_range[kBlock / kWave][4];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const uint32_t depth_bits = __float_as_uint(p.z);
@@ -575,13 +587,13 @@ __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* _
             const int wl = bin_width_log(a.ly.bin_shift[l]), hl = bin_height_log(a.ly.bin_shift[l]);
             rect[l].x0 = px0 >> wl, rect[l].y0 = py0 >> hl, rect[l].columns = (px1 >> wl) - (px0 >> wl) + 1;
             const long long need = (long long)rect[l].columns * ((py1 >> hl) - (py0 >> hl) + 1) + slots;
-            slots = need > kScatterSlots ? kScatterSlots + 1 : (int)need;
+            slots = need > kScatterSlots<HITS> ? kScatterSlots<HITS> + 1 : (int)need;
         }
-        if (slots > kScatterSlots)
+        if (slots > kScatterSlots<HITS>)
             scatter_by_wave<HITS>(a, bin_counts, out, i, inside, p, lane);
         else
         {
-            for (int k = tid; k < slots; k += kBlock) s_count[k] = 0u;
+            for (int k = tid; 4 * k < slots; k += kBlock) reinterpret_cast<uint4*>(s_count)[k] = make_uint4(0u, 0u, 0u, 0u);
             __syncthreads();
             if (HITS != 1 && inside) a.projected[i] = make_float2(p.ipx, p.ipy);  // see scatter_by_wave
             // per hit: slot | rank << 16, or no hit (a bin takes at most 1024 hits of the workgroup)
@@ -608,36 +620,34 @@ __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* _
                 }
             }
             __syncthreads();
-            // one global atomic per bin that was hit
-            for (int first_slot = tid; first_slot - tid < slots; first_slot += kScatterAtOnce * kBlock)
+            // one global atomic per bin that was hit. With four hits per layer the results of a layer are looked at after
+            // the next layer's atomics have been issued, else all of them at the end.
+            constexpr int kAhead = HITS == 1 ? VETRAST_MAX_LAYERS : 2;
+            uint32_t start[kAhead][HITS];
+            auto first_of_bin = [&](int l, int h) { return place[l][h] < 0x10000u; };
+            auto store_starts = [&](int l) {
+#pragma unroll
+                for (int h = 0; h < HITS; ++h)
+                    if (first_of_bin(l, h)) s_count[place[l][h]] = start[l % kAhead][h];
+            };
+            ipx = inside ? p.ipx : 0.f, ipy = inside ? p.ipy : 0.f;
+#pragma unroll
+            for (int l = 0; l < VETRAST_MAX_LAYERS; ++l, ipx *= 0.5f, ipy *= 0.5f)
             {
-                // (a thread's atomics are on their way before the first result is looked at)
-                uint32_t start[kScatterAtOnce];
+                const float fx = HITS == 1 ? rintf(ipx) : floorf(ipx), fy = HITS == 1 ? rintf(ipy) : floorf(ipy);
 #pragma unroll
-                for (int m = 0; m < kScatterAtOnce; ++m)
+                for (int h = 0; h < HITS; ++h)
                 {
-                    start[m] = 0u;
-                    if (first_slot - tid + m * kBlock >= slots) break;  // the same for every thread
-                    const int k          = first_slot + m * kBlock;
-                    const uint32_t count = k < slots ? s_count[k] : 0u;
-                    if (count == 0u) continue;
-                    int l = 0, x0 = rect[0].x0, y0 = rect[0].y0, columns = rect[0].columns, first = 0;
-#pragma unroll
-                    for (int n = 1; n < VETRAST_MAX_LAYERS; ++n)
-                        if (n < a.ly.L && k >= rect[n].first && rect[n].columns > 0)
-                            l = n, x0 = rect[n].x0, y0 = rect[n].y0, columns = rect[n].columns, first = rect[n].first;
-                    const int by    = (int)(((float)(k - first) + 0.5f) * (1.f / (float)columns)), bx = k - first - by * columns;
-                    const int shift = a.ly.bin_shift[l];
-                    const uint32_t bin = bin_at_pixel(a.ly, l, (uint32_t)(x0 + bx) << bin_width_log(shift), (uint32_t)(y0 + by) << bin_height_log(shift));
-                    start[m] = atomicAdd(&bin_counts[bin], count);
+                    start[l % kAhead][h] = 0u;
+                    if (l >= a.ly.L || !first_of_bin(l, h)) continue;
+                    const uint32_t bin = bin_at_pixel(a.ly, l, (uint32_t)(int)(fx + (float)(h & 1)), (uint32_t)(int)(fy + (float)(h >> 1)));
+                    start[l % kAhead][h] = atomicAdd(&bin_counts[bin], s_count[place[l][h]]);
                 }
-#pragma unroll
-                for (int m = 0; m < kScatterAtOnce; ++m)
-                {
-                    if (first_slot - tid + m * kBlock >= slots) break;
-                    if (first_slot + m * kBlock < slots) s_count[first_slot + m * kBlock] = start[m];
-                }
+                if (l >= kAhead - 1 && l - (kAhead - 1) < a.ly.L) store_starts(l - (kAhead - 1));
             }
+#pragma unroll
+            for (int l = VETRAST_MAX_LAYERS - kAhead + 1; l < VETRAST_MAX_LAYERS; ++l)
+                if (l < a.ly.L) store_starts(l);
             __syncthreads();
             ipx = inside ? p.ipx : 0.f, ipy = inside ? p.ipy : 0.f;
 #pragma unroll
@@ -679,7 +689,7 @@ __device__ __forceinline__ void bin_scatter(const ViewPass& a, uint32_t* __restr
 }
 
 template <int HITS>
-__global__ void __launch_bounds__(kBlock) bin_scatter_kernel(ViewPass a, uint32_t* __restrict__ bin_counts,
+__global__ void __launch_bounds__(kBlock, kScatterWaves<HITS>) bin_scatter_kernel(ViewPass a, uint32_t* __restrict__ bin_counts,
                                                               ScatterTargets out, PackJob pack)
 {
     bin_scatter<HITS>(a, bin_counts, out, pack);
@@ -700,7 +710,7 @@ struct ScatterArgs
 // taking turns, instead of all of one view before those of the next, is slower as well, by a tenth for crops and by
 // half for full frames.)
 template <int HITS>
-__global__ void __launch_bounds__(kBlock) bin_scatter_views_kernel(PerView<ScatterArgs> views)
+__global__ void __launch_bounds__(kBlock, kScatterWaves<HITS>) bin_scatter_views_kernel(PerView<ScatterArgs> views)
 {
     const ScatterArgs& v = views.v[blockIdx.y];
     bin_scatter<HITS>(v.view, v.bin_counts, v.out, v.pack);
