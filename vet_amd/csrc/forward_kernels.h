@@ -333,11 +333,11 @@ __device__ __forceinline__ void store_record(const ScatterTargets& t, const Laye
     }
 }
 
-// The hits of the workgroup's points where no LDS slots stand for their bins: every wave groups its hits by bin with
-// ballots and issues one atomic per bin and layer.
+// The hits of the workgroup's points in the layers (a bit each) where no LDS slots stand for their bins: every wave groups
+// its hits by bin with ballots and issues one atomic per bin and layer.
 template <int HITS>
 __device__ __forceinline__ void scatter_by_wave(const ViewPass& a, uint32_t* __restrict__ bin_counts, const ScatterTargets& out,
-                                                int i, bool inside, const Projected& p, int lane)
+                                                uint32_t layers, int i, bool inside, const Projected& p, int lane)
 {
     const uint32_t depth_bits = __float_as_uint(p.z);
     const bool any_inside     = __ballot(inside) != 0ull;
@@ -354,7 +354,7 @@ __device__ __forceinline__ void scatter_by_wave(const ViewPass& a, uint32_t* __r
         for (int l = 0; l < VETRAST_MAX_LAYERS; ++l, radius *= 0.5f, ipx *= 0.5f, ipy *= 0.5f)
         {
             base[l] = 0, who[l] = 0, bins[l] = 0;
-            if (l >= a.ly.L || !any_inside) continue;
+            if (!(layers >> l & 1u) || !any_inside) continue;
             if (a.drop_by_radius && radius < a.radius_threshold) dropped = true;
             uint32_t tile = 0, in_tile = 0, bin = 0, in_bin = 0;
             const bool has = !dropped && layer_hit<HITS>(a.ly, l, ipx, ipy, 0, tile, in_tile);
@@ -367,7 +367,7 @@ __device__ __forceinline__ void scatter_by_wave(const ViewPass& a, uint32_t* __r
 #pragma unroll
         for (int l = 0; l < VETRAST_MAX_LAYERS; ++l)
         {
-            if (l >= a.ly.L || !any_inside) continue;
+            if (!(layers >> l & 1u) || !any_inside) continue;
             const uint32_t group_base = (uint32_t)__shfl((int)base[l], (int)(who[l] & 0xFF), kWave);
             store_record(out, a.ly, l, (who[l] & 0x80000000u) != 0u, bins[l], group_base + ((who[l] >> 8) & 0xFFu), (uint32_t)i,
                          depth_bits, (who[l] >> 16) & 0xFFu, lane);
@@ -375,87 +375,75 @@ __device__ __forceinline__ void scatter_by_wave(const ViewPass& a, uint32_t* __r
     }
     else
     {
-        // The blend and its backward pass form a fragment's bilinear weight from the point's image position; they
-        // read it from here (8 bytes) instead of projecting the point again for every one of its fragments.
-        if (inside) a.projected[i] = make_float2(p.ipx, p.ipy);
         // The four pixels of a point mostly lie in one bin or two. Per layer the hits of a lane are therefore taken
         // bin by bin: in every turn a lane brings all its remaining hits that share the bin of its first remaining
         // hit, as one entry of that weight, so a layer takes as many grouping turns as the lane with the most
         // distinct bins has (1 or 2 as a rule, never more than 4) instead of 4, and one atomic per bin and turn.
-        // The results of a layer's atomics are looked at after those of the next layer have been issued.
-        // Kept per layer and turn: the atomic's result, the leader lane, the packed ranks and the bin; per layer,
-        // 5 bits per hit: valid | turn << 1 | place among the lane's hits of that turn << 3, and the four pixels in bin.
+        // Kept per turn: the atomic's result, the leader lane, the packed ranks and the bin; 5 bits per hit: valid |
+        // turn << 1 | place among the lane's hits of that turn << 3; and the four pixels in bin.
         constexpr int kTurns = HITS;
-        uint32_t base[VETRAST_MAX_LAYERS][kTurns], leader[VETRAST_MAX_LAYERS][kTurns], ranks[VETRAST_MAX_LAYERS][kTurns],
-            bins[VETRAST_MAX_LAYERS][kTurns], code[VETRAST_MAX_LAYERS], in_bins[VETRAST_MAX_LAYERS];
-        auto store_layer = [&](int l) {
-            uint32_t start[kTurns];  // first slot of the group this lane's hits of every turn belong to
-#pragma unroll
-            for (int t = 0; t < kTurns; ++t) start[t] = (uint32_t)__shfl((int)base[l][t], (int)leader[l][t], kWave);
-#pragma unroll
-            for (int h = 0; h < HITS; ++h)
-            {
-                const uint32_t c = code[l] >> (5 * h);
-                const uint32_t t = (c >> 1) & 3u, place = (c >> 3) & 3u;
-                const uint32_t s = t == 0 ? start[0] : t == 1 ? start[1] : t == 2 ? start[2] : start[3];
-                const uint32_t r = t == 0 ? ranks[l][0] : t == 1 ? ranks[l][1] : t == 2 ? ranks[l][2] : ranks[l][3];
-                const uint32_t b = t == 0 ? bins[l][0] : t == 1 ? bins[l][1] : t == 2 ? bins[l][2] : bins[l][3];
-                store_record(out, a.ly, l, (c & 1u) != 0u, b, s + ((r >> (8u * place)) & 0xFFu), ((uint32_t)i << 2) | (uint32_t)h,
-                             depth_bits, (in_bins[l] >> (8 * h)) & 0xFFu, lane);
-            }
-        };
 #pragma unroll
         for (int l = 0; l < VETRAST_MAX_LAYERS; ++l, radius *= 0.5f, ipx *= 0.5f, ipy *= 0.5f)
         {
-            code[l] = 0, in_bins[l] = 0;
+            if (!(layers >> l & 1u) || !any_inside) continue;
+            uint32_t base[kTurns], leader[kTurns], ranks[kTurns], bins[kTurns], code = 0, in_bins = 0;
 #pragma unroll
-            for (int t = 0; t < kTurns; ++t) base[l][t] = 0, leader[l][t] = 0, ranks[l][t] = 0, bins[l][t] = 0;
-            if (l < a.ly.L && any_inside)
+            for (int t = 0; t < kTurns; ++t) base[t] = 0, leader[t] = 0, ranks[t] = 0, bins[t] = 0;
+            if (a.drop_by_radius && radius < a.radius_threshold) dropped = true;
+            uint32_t bin[HITS];
+            uint32_t left = 0;  // hits not yet counted, one bit each
+#pragma unroll
+            for (int h = 0; h < HITS; ++h)
             {
-                if (a.drop_by_radius && radius < a.radius_threshold) dropped = true;
-                uint32_t bin[HITS];
-                uint32_t left = 0;  // hits not yet counted, one bit each
-#pragma unroll
-                for (int h = 0; h < HITS; ++h)
+                uint32_t tile = 0, in_tile = 0, in_bin = 0;
+                bin[h]         = 0;
+                const bool has = !dropped && layer_hit<HITS>(a.ly, l, ipx, ipy, h, tile, in_tile);
+                if (has)
                 {
-                    uint32_t tile = 0, in_tile = 0, in_bin = 0;
-                    bin[h]         = 0;
-                    const bool has = !dropped && layer_hit<HITS>(a.ly, l, ipx, ipy, h, tile, in_tile);
-                    if (has)
-                    {
-                        bin_of_pixel(a.ly, l, tile, in_tile, bin[h], in_bin);
-                        left |= 1u << h;
-                        in_bins[l] |= in_bin << (8 * h);
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < kTurns; ++t)
-                {
-                    if (__ballot(left != 0u) == 0ull) break;  // the same for the whole wave
-                    uint32_t key = 0;
-#pragma unroll
-                    for (int h = HITS - 1; h >= 0; --h)
-                        if (left & (1u << h)) key = bin[h];  // bin of the first remaining hit
-                    uint32_t weight = 0;
-#pragma unroll
-                    for (int h = 0; h < HITS; ++h)
-                        if ((left & (1u << h)) && bin[h] == key)
-                        {
-                            code[l] |= (1u | ((uint32_t)t << 1) | (weight << 3)) << (5 * h);
-                            ++weight;
-                            left &= ~(1u << h);
-                        }
-                    const bool has        = weight != 0u;
-                    const WeightedGroup g = group_by_bin_weighted(has, key, weight, lane);
-                    leader[l][t]          = (uint32_t)g.leader;
-                    ranks[l][t]           = g.ranks;
-                    bins[l][t]            = key;
-                    if (has && g.leader == lane) base[l][t] = atomicAdd(&bin_counts[key], g.total);
+                    bin_of_pixel(a.ly, l, tile, in_tile, bin[h], in_bin);
+                    left |= 1u << h;
+                    in_bins |= in_bin << (8 * h);
                 }
             }
-            if (l >= 1 && l - 1 < a.ly.L && any_inside) store_layer(l - 1);
+#pragma unroll
+            for (int t = 0; t < kTurns; ++t)
+            {
+                if (__ballot(left != 0u) == 0ull) break;  // the same for the whole wave
+                uint32_t key = 0;
+#pragma unroll
+                for (int h = HITS - 1; h >= 0; --h)
+                    if (left & (1u << h)) key = bin[h];  // bin of the first remaining hit
+                uint32_t weight = 0;
+#pragma unroll
+                for (int h = 0; h < HITS; ++h)
+                    if ((left & (1u << h)) && bin[h] == key)
+                    {
+                        code |= (1u | ((uint32_t)t << 1) | (weight << 3)) << (5 * h);
+                        ++weight;
+                        left &= ~(1u << h);
+                    }
+                const bool has        = weight != 0u;
+                const WeightedGroup g = group_by_bin_weighted(has, key, weight, lane);
+                leader[t]             = (uint32_t)g.leader;
+                ranks[t]              = g.ranks;
+                bins[t]               = key;
+                if (has && g.leader == lane) base[t] = atomicAdd(&bin_counts[key], g.total);
+            }
+            uint32_t start[kTurns];  // first slot of the group this lane's hits of every turn belong to
+#pragma unroll
+            for (int t = 0; t < kTurns; ++t) start[t] = (uint32_t)__shfl((int)base[t], (int)leader[t], kWave);
+#pragma unroll
+            for (int h = 0; h < HITS; ++h)
+            {
+                const uint32_t c = code >> (5 * h);
+                const uint32_t t = (c >> 1) & 3u, place = (c >> 3) & 3u;
+                const uint32_t s = t == 0 ? start[0] : t == 1 ? start[1] : t == 2 ? start[2] : start[3];
+                const uint32_t r = t == 0 ? ranks[0] : t == 1 ? ranks[1] : t == 2 ? ranks[2] : ranks[3];
+                const uint32_t b = t == 0 ? bins[0] : t == 1 ? bins[1] : t == 2 ? bins[2] : bins[3];
+                store_record(out, a.ly, l, (c & 1u) != 0u, b, s + ((r >> (8u * place)) & 0xFFu), ((uint32_t)i << 2) | (uint32_t)h,
+                             depth_bits, (in_bins >> (8 * h)) & 0xFFu, lane);
+            }
         }
-        if (VETRAST_MAX_LAYERS - 1 < a.ly.L && any_inside) store_layer(VETRAST_MAX_LAYERS - 1);
     }
 }
 
@@ -469,10 +457,8 @@ __device__ __forceinline__ void scatter_by_wave(const ViewPass& a, uint32_t* __r
 // The bins a workgroup's points fall into, per layer: a rectangle of bins, with a counter in LDS for each. Points come in
 // blocks of 256 that are neighbours in space, so the rectangles of all layers together hold a hundred or two bins as a rule.
 // As many slots as leave the workgroups their place on a compute unit: with one hit per point 8 of them (their registers
-// allow 8; 6144 slots let 6 in: benchmark frame 47.5 against 45.0 us, four town views 200 against 182), with four hits 6,
-// which is what their registers allow. With 2048 slots the blocks of sparse clouds and small crops, which spread over
-// thousands of small bins, group by wave instead (300 000 points at 801x451 28 against 19 us, four 512x512 crops of 2 M
-// points with the 2x2 splat 89 against 72 us).
+// allow 8; 6144 slots let 6 in: benchmark frame 44.2 against 42.3 us, four town views 196 against 180), with four hits 6,
+// which is what their registers allow (2x2 splat at 1080p 85 us, with 4096 slots 97, with 2048 110).
 template <int HITS>
 constexpr int kScatterSlots = HITS == 1 ? 5088 : 6144;
 template <int HITS>
@@ -509,17 +495,14 @@ __device__ __forceinline__ float wave_min(float v, int lane)
 //
 // The workgroup counts its hits per bin in LDS (the LDS atomic's result is the hit's rank among the workgroup's hits of
 // the bin), the thread of a bin's first hit issues the ONE global atomic for that bin, all layers' atomics before the first
-// result is looked at, and every hit's record goes to the bin's room at that atomic's result + rank. Where the rectangles
-// need more slots than there are (points in no spatial order, blocks right in front of the camera) the waves group their
-// hits on their own (scatter_by_wave).
-// Measured against grouping by wave alone (this pass, 2 M points and 4 layers unless stated): 2x2 splat at 1080p 154 -> 109
-// us, four 512x512 crops of it 116 -> 72 us; one hit per layer: benchmark frame 47.3 -> 46.4 us, another 1080p frame 45.6
-// -> 40.9, four town views of 5.5 M points 206 -> 182, ten million points 309 -> 287, a 203x155 crop of 60 000 points 11.5
-// -> 9.3, 300 000 points in five layers 28.1 -> 17.4, a shuffled cloud 367 -> 347. A cloud whose last fifth is in no order
-// loses, 115 -> 121: its blocks pay for the rectangles and group by wave after all.
-// (While the threads walked the slots, also the empty ones, and worked a slot's bin out of its number: benchmark frame
-// 51.5, the other 44.2, town 202, the small crop 15.0, 300 000 points 18.9 us, the small crop with the 2x2 splat 19.5 where
-// it is 13.4 now.)
+// result is looked at, and every hit's record goes to the bin's room at that atomic's result + rank. In the layers whose
+// rectangles find no room (points in no spatial order, blocks that reach across a jump of the order or stand right in front
+// of the camera) the waves group their hits on their own (scatter_by_wave).
+// Measured against grouping by wave alone (this pass, 2 M points and 4 layers unless stated): 2x2 splat at 1080p 154 -> 85
+// us, four 512x512 crops of it 192 -> 118; one hit per layer: benchmark frame 47.4 -> 42.3 us, another 1080p frame 45.4 ->
+// 41.0, four town views of 5.5 M points 204 -> 180, ten million points 310 -> 290, a 203x155 crop of 60 000 points 11.5 ->
+// 9.4, 300 000 points in five layers 27.9 -> 17.7, a cloud whose last fifth is in no order 116 -> 109, a shuffled one 376 ->
+// 300.
 template <int HITS>
 __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* __restrict__ bin_counts,
                                                   const ScatterTargets& out, const PackJob& pack, int slot, int i, bool visible,
@@ -570,10 +553,14 @@ __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* _
     for (int k = 0; k < 4; ++k) range[k] = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(range[k])));
     if (range[0] < 1e29f)
     {
+        // The blend and its backward pass form a fragment's bilinear weight from the point's image position; they
+        // read it from here (8 bytes) instead of projecting the point again for every one of its fragments.
+        if (HITS != 1 && inside) a.projected[i] = make_float2(p.ipx, p.ipy);
         BinRectangle rect[VETRAST_MAX_LAYERS];
-        int slots = 0;
+        int slots     = 0;
+        uint32_t wide = 0u;  // layers whose rectangle finds no room, one bit each
 #pragma unroll
-        for (int l = 0; l < VETRAST_MAX_LAYERS; ++l)
+        for (int l = VETRAST_MAX_LAYERS - 1; l >= 0; --l)  // the coarse layers first: their bins take the most hits
         {
             rect[l] = {0, 0, 0, slots};
             if (l >= a.ly.L) continue;
@@ -587,15 +574,16 @@ __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* _
             const int wl = bin_width_log(a.ly.bin_shift[l]), hl = bin_height_log(a.ly.bin_shift[l]);
             rect[l].x0 = px0 >> wl, rect[l].y0 = py0 >> hl, rect[l].columns = (px1 >> wl) - (px0 >> wl) + 1;
             const long long need = (long long)rect[l].columns * ((py1 >> hl) - (py0 >> hl) + 1) + slots;
-            slots = need > kScatterSlots<HITS> ? kScatterSlots<HITS> + 1 : (int)need;
+            if (need > kScatterSlots<HITS>)
+                wide |= 1u << l;
+            else
+                slots = (int)need;
         }
-        if (slots > kScatterSlots<HITS>)
-            scatter_by_wave<HITS>(a, bin_counts, out, i, inside, p, lane);
-        else
+        if (wide != 0u) scatter_by_wave<HITS>(a, bin_counts, out, wide, i, inside, p, lane);
+        if (slots > 0)
         {
             for (int k = tid; 4 * k < slots; k += kBlock) reinterpret_cast<uint4*>(s_count)[k] = make_uint4(0u, 0u, 0u, 0u);
             __syncthreads();
-            if (HITS != 1 && inside) a.projected[i] = make_float2(p.ipx, p.ipy);  // see scatter_by_wave
             // per hit: slot | rank << 16, or no hit (a bin takes at most 1024 hits of the workgroup)
             constexpr uint32_t kNone = 0xFFFFFFFFu;
             uint32_t place[VETRAST_MAX_LAYERS][HITS];
@@ -606,7 +594,7 @@ __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* _
             {
 #pragma unroll
                 for (int h = 0; h < HITS; ++h) place[l][h] = kNone;
-                if (l >= a.ly.L) continue;
+                if (l >= a.ly.L || (wide >> l & 1u)) continue;
                 if (a.drop_by_radius && radius < a.radius_threshold) dropped = true;
                 const int wl = bin_width_log(a.ly.bin_shift[l]), hl = bin_height_log(a.ly.bin_shift[l]);
                 const float fx = HITS == 1 ? rintf(ipx) : floorf(ipx), fy = HITS == 1 ? rintf(ipy) : floorf(ipy);
