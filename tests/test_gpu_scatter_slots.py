@@ -1,7 +1,7 @@
 """GPU parity of the scatter pass around the number of bins that a workgroup's 256 points may spread over.
 
 The workgroup counts its hits in LDS, one slot per bin of the rectangle its points span in every layer, up to 5088 slots
-with one hit per layer and 6144 with the 2x2 splat; where the rectangles need more, its waves group their hits themselves.
+with one hit per layer and 6144 with the 2x2 splat; in the layers that find no room its waves group their hits themselves.
 The blocks here span exactly that many bins or a few more, a single bin, half of the image, or nothing that is visible;
 some have hits in the coarser layers only (positions left of pixel 0), and blocks of all kinds are neighbours.
 Counterpart of CountingPrepassMulti and CollectMulti, src/lib/rendering/RenderForward.cu:806-905,1011-1096.
@@ -49,8 +49,10 @@ def _scene(w, h, layers, drop_by_radius, seed=3):
     return scene
 
 
-# tiles of 16x16 pixels are the bins of these layers: 96 x 53 = 5088, 76 x 67 = 5092; 96 x 64 = 6144, 116 x 53 = 6148
-@pytest.mark.parametrize("mode,tiles_x,tiles_y", [(1, 96, 53), (1, 76, 67), (2, 96, 53), (3, 96, 64), (3, 116, 53)])
+# tiles of 16x16 pixels are the bins of these layers: 96 x 53 = 5088, 76 x 67 = 5092; 96 x 64 = 6144, 116 x 53 = 6148; up to
+# 1024 slots the 2x2 splat goes by slots, beyond by first hits: 32 x 32 = 1024, 41 x 25 = 1025
+@pytest.mark.parametrize("mode,tiles_x,tiles_y", [(1, 96, 53), (1, 76, 67), (2, 96, 53), (3, 96, 64), (3, 116, 53), (3, 32, 32),
+                                                  (3, 41, 25)])
 @pytest.mark.parametrize("layers", [1, 2, 4])
 @pytest.mark.parametrize("seed", [2, 3])
 def test_blocks_around_the_number_of_slots(mode, tiles_x, tiles_y, layers, seed, rasterizer, oracle):

@@ -463,6 +463,13 @@ template <int HITS>
 constexpr int kScatterSlots = HITS == 1 ? 5088 : 6144;
 template <int HITS>
 constexpr int kScatterWaves = HITS == 1 ? 8 : 6;  // waves of a SIMD unit to leave room for, in registers and LDS
+// With four hits per layer and this many slots at most (four a thread) the threads go by slots instead of first hits:
+// neighbouring threads then add up neighbouring bins, whose counts share cache lines, where the many bins of a dense block
+// are hit in the points' order (450 000 points that fill a 464x272 view 51 against 41 us, 2.6 M in four crops 287 against
+// 257, 2x2 splat at 1080p 85 against 81). Beyond, most slots are empty as a rule (60 000 points in a 203x155 crop 15 us,
+// going by slots up to 4096 of them 19, six 258x258 crops of a dense cloud 74 and 57). One hit per layer hits a quarter of
+// the bins: benchmark frame 43 us, going by slots 45 to 47.
+constexpr int kScatterWalk = 1024;
 struct BinRectangle
 {
     int x0, y0, columns, first;  // first bin column and row, columns, number of the first slot
@@ -494,12 +501,12 @@ __device__ __forceinline__ float wave_min(float v, int lane)
 // This is the part of the pass behind the projection: thread `slot` has point i, which is `visible` at p in this view.
 //
 // The workgroup counts its hits per bin in LDS (the LDS atomic's result is the hit's rank among the workgroup's hits of
-// the bin), the thread of a bin's first hit issues the ONE global atomic for that bin, all layers' atomics before the first
-// result is looked at, and every hit's record goes to the bin's room at that atomic's result + rank. In the layers whose
+// the bin), one thread issues the ONE global atomic for a bin that was hit (the thread of its first hit, or the thread of
+// the slot, see kScatterWalk), and every hit's record goes to the bin's room at that atomic's result + rank. In the layers whose
 // rectangles find no room (points in no spatial order, blocks that reach across a jump of the order or stand right in front
 // of the camera) the waves group their hits on their own (scatter_by_wave).
-// Measured against grouping by wave alone (this pass, 2 M points and 4 layers unless stated): 2x2 splat at 1080p 154 -> 85
-// us, four 512x512 crops of it 192 -> 118; one hit per layer: benchmark frame 47.4 -> 42.3 us, another 1080p frame 45.4 ->
+// Measured against grouping by wave alone (this pass, 2 M points and 4 layers unless stated): 2x2 splat at 1080p 154 -> 81
+// us, four 512x512 crops of it 192 -> 116; one hit per layer: benchmark frame 47.4 -> 42.3 us, another 1080p frame 45.4 ->
 // 41.0, four town views of 5.5 M points 204 -> 180, ten million points 310 -> 290, a 203x155 crop of 60 000 points 11.5 ->
 // 9.4, 300 000 points in five layers 27.9 -> 17.7, a cloud whose last fifth is in no order 116 -> 109, a shuffled one 376 ->
 // 300.
@@ -608,34 +615,64 @@ __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* _
                 }
             }
             __syncthreads();
-            // one global atomic per bin that was hit. With four hits per layer the results of a layer are looked at after
-            // the next layer's atomics have been issued, else all of them at the end.
-            constexpr int kAhead = HITS == 1 ? VETRAST_MAX_LAYERS : 2;
-            uint32_t start[kAhead][HITS];
-            auto first_of_bin = [&](int l, int h) { return place[l][h] < 0x10000u; };
-            auto store_starts = [&](int l) {
-#pragma unroll
-                for (int h = 0; h < HITS; ++h)
-                    if (first_of_bin(l, h)) s_count[place[l][h]] = start[l % kAhead][h];
-            };
-            ipx = inside ? p.ipx : 0.f, ipy = inside ? p.ipy : 0.f;
-#pragma unroll
-            for (int l = 0; l < VETRAST_MAX_LAYERS; ++l, ipx *= 0.5f, ipy *= 0.5f)
+            // one global atomic per bin that was hit
+            if (HITS != 1 && slots <= kScatterWalk)
             {
-                const float fx = HITS == 1 ? rintf(ipx) : floorf(ipx), fy = HITS == 1 ? rintf(ipy) : floorf(ipy);
+                // a thread for every slot, also those that were not hit
+                constexpr int kAtOnce = kScatterWalk / kBlock;
+                uint32_t start[kAtOnce];
 #pragma unroll
-                for (int h = 0; h < HITS; ++h)
+                for (int m = 0; m < kAtOnce; ++m)
                 {
-                    start[l % kAhead][h] = 0u;
-                    if (l >= a.ly.L || !first_of_bin(l, h)) continue;
-                    const uint32_t bin = bin_at_pixel(a.ly, l, (uint32_t)(int)(fx + (float)(h & 1)), (uint32_t)(int)(fy + (float)(h >> 1)));
-                    start[l % kAhead][h] = atomicAdd(&bin_counts[bin], s_count[place[l][h]]);
-                }
-                if (l >= kAhead - 1 && l - (kAhead - 1) < a.ly.L) store_starts(l - (kAhead - 1));
-            }
+                    const int k          = tid + m * kBlock;
+                    const uint32_t count = k < slots ? s_count[k] : 0u;
+                    start[m]             = 0u;
+                    if (count == 0u) continue;
+                    int l = 0, x0 = 0, y0 = 0, columns = 1, first = 0;
 #pragma unroll
-            for (int l = VETRAST_MAX_LAYERS - kAhead + 1; l < VETRAST_MAX_LAYERS; ++l)
-                if (l < a.ly.L) store_starts(l);
+                    for (int n = VETRAST_MAX_LAYERS - 1; n >= 0; --n)
+                        if (n < a.ly.L && !(wide >> n & 1u) && rect[n].columns > 0 && k >= rect[n].first)
+                            l = n, x0 = rect[n].x0, y0 = rect[n].y0, columns = rect[n].columns, first = rect[n].first;
+                    const int by    = (int)(((float)(k - first) + 0.5f) * (1.f / (float)columns)), bx = k - first - by * columns;
+                    const int shift = a.ly.bin_shift[l];
+                    const uint32_t bin = bin_at_pixel(a.ly, l, (uint32_t)(x0 + bx) << bin_width_log(shift), (uint32_t)(y0 + by) << bin_height_log(shift));
+                    start[m] = atomicAdd(&bin_counts[bin], count);
+                }
+#pragma unroll
+                for (int m = 0; m < kAtOnce; ++m)
+                    if (tid + m * kBlock < slots) s_count[tid + m * kBlock] = start[m];
+            }
+            else
+            {
+                // The thread of a bin's first hit adds the bin up. With four hits per layer the results of a layer are looked
+                // at after the next layer's atomics have been issued, else all of them at the end.
+                constexpr int kAhead = HITS == 1 ? VETRAST_MAX_LAYERS : 2;
+                uint32_t start[kAhead][HITS];
+                auto first_of_bin = [&](int l, int h) { return place[l][h] < 0x10000u; };
+                auto store_starts = [&](int l) {
+#pragma unroll
+                    for (int h = 0; h < HITS; ++h)
+                        if (first_of_bin(l, h)) s_count[place[l][h]] = start[l % kAhead][h];
+                };
+                ipx = inside ? p.ipx : 0.f, ipy = inside ? p.ipy : 0.f;
+#pragma unroll
+                for (int l = 0; l < VETRAST_MAX_LAYERS; ++l, ipx *= 0.5f, ipy *= 0.5f)
+                {
+                    const float fx = HITS == 1 ? rintf(ipx) : floorf(ipx), fy = HITS == 1 ? rintf(ipy) : floorf(ipy);
+#pragma unroll
+                    for (int h = 0; h < HITS; ++h)
+                    {
+                        start[l % kAhead][h] = 0u;
+                        if (l >= a.ly.L || !first_of_bin(l, h)) continue;
+                        const uint32_t bin = bin_at_pixel(a.ly, l, (uint32_t)(int)(fx + (float)(h & 1)), (uint32_t)(int)(fy + (float)(h >> 1)));
+                        start[l % kAhead][h] = atomicAdd(&bin_counts[bin], s_count[place[l][h]]);
+                    }
+                    if (l >= kAhead - 1 && l - (kAhead - 1) < a.ly.L) store_starts(l - (kAhead - 1));
+                }
+#pragma unroll
+                for (int l = VETRAST_MAX_LAYERS - kAhead + 1; l < VETRAST_MAX_LAYERS; ++l)
+                    if (l < a.ly.L) store_starts(l);
+            }
             __syncthreads();
             ipx = inside ? p.ipx : 0.f, ipy = inside ? p.ipy : 0.f;
 #pragma unroll
