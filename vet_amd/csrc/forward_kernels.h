@@ -463,12 +463,12 @@ template <int HITS>
 constexpr int kScatterSlots = HITS == 1 ? 5088 : 6144;
 template <int HITS>
 constexpr int kScatterWaves = HITS == 1 ? 8 : 6;  // waves of a SIMD unit to leave room for, in registers and LDS
-// With four hits per layer and this many slots at most (four a thread) the threads go by slots instead of first hits:
+// With four hits per layer and this many slots at most (four a thread) the threads go by slots instead of by first hits:
 // neighbouring threads then add up neighbouring bins, whose counts share cache lines, where the many bins of a dense block
 // are hit in the points' order (450 000 points that fill a 464x272 view 51 against 41 us, 2.6 M in four crops 287 against
 // 257, 2x2 splat at 1080p 85 against 81). Beyond, most slots are empty as a rule (60 000 points in a 203x155 crop 15 us,
 // going by slots up to 4096 of them 19, six 258x258 crops of a dense cloud 74 and 57). One hit per layer hits a quarter of
-// the bins: benchmark frame 43 us, going by slots 45 to 47.
+// the bins: benchmark frame 43 us, going by slots 45 to 47 (only a cloud in the order of its surfaces, 78 us, gains: 74).
 constexpr int kScatterWalk = 1024;
 struct BinRectangle
 {
@@ -502,14 +502,14 @@ __device__ __forceinline__ float wave_min(float v, int lane)
 //
 // The workgroup counts its hits per bin in LDS (the LDS atomic's result is the hit's rank among the workgroup's hits of
 // the bin), one thread issues the ONE global atomic for a bin that was hit (the thread of its first hit, or the thread of
-// the slot, see kScatterWalk), and every hit's record goes to the bin's room at that atomic's result + rank. In the layers whose
-// rectangles find no room (points in no spatial order, blocks that reach across a jump of the order or stand right in front
-// of the camera) the waves group their hits on their own (scatter_by_wave).
-// Measured against grouping by wave alone (this pass, 2 M points and 4 layers unless stated): 2x2 splat at 1080p 154 -> 81
-// us, four 512x512 crops of it 192 -> 116; one hit per layer: benchmark frame 47.4 -> 42.3 us, another 1080p frame 45.4 ->
-// 41.0, four town views of 5.5 M points 204 -> 180, ten million points 310 -> 290, a 203x155 crop of 60 000 points 11.5 ->
-// 9.4, 300 000 points in five layers 27.9 -> 17.7, a cloud whose last fifth is in no order 116 -> 109, a shuffled one 376 ->
-// 300.
+// the slot, see kScatterWalk), and every hit's record goes to the bin's room at that atomic's result + rank. In the layers
+// whose rectangles find no room (points in no spatial order, blocks that reach across a jump of the order or stand right in
+// front of the camera) the waves group their hits on their own (scatter_by_wave).
+// Measured against grouping by wave alone (HIP events around the pass; 2 M points, 1080p and 4 layers unless stated): 2x2
+// splat 156 -> 81 us, its four 512x512 crops 181 -> 116, 450 000 points that fill a 464x272 view 104 -> 41; one hit per
+// layer: benchmark frame 47.4 -> 43.3 us, another frame 46.2 -> 40.5, four crops 64.3 -> 55.3, four town views of 5.5 M
+// points 203 -> 180, ten million points 307 -> 287, a 203x155 crop of 60 000 points 11.1 -> 9.3, 300 000 points in five
+// layers 27.5 -> 17.5, a cloud whose last fifth is in no order 112 -> 108, a shuffled one 366 -> 299.
 template <int HITS>
 __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* __restrict__ bin_counts,
                                                   const ScatterTargets& out, const PackJob& pack, int slot, int i, bool visible,

@@ -12,7 +12,7 @@
 //      by more than that are left out, and the few in between get the literal test of the reference. The counts are the
 //      literal ones, pixel for pixel.
 // Measured (146 k cells of 0.25 m, 1080p, 121 M covered pixels, the camera inside the grid): 0.87 ms per call with a test per
-// pixel (bound by its ~200 vector instructions per 64 pixels), 0.29 ms by rows (running sums 17 us, rows 211 us, the
+// pixel (bound by its ~200 vector instructions per 64 pixels), 0.29 ms by rows (running sums 17 us, rows 213 us, the
 // cells next to the camera that are tested pixel by pixel 63 us); bound by the ~400 vector instructions per 64 rows and
 // the tests of open pixels.
 #pragma once
@@ -79,7 +79,7 @@ struct LiftPass
 };
 
 // Where the sum of the pixels [0, x) of image row y is, 0 <= x <= width. The entry of x = 0 is zero, with the sign bit set
-// where rounding has swallowed a pixel of the row.
+// where the row has pixels so dim that rounding may have swallowed them.
 __device__ __forceinline__ size_t lift_sum_at(const LiftPass& a, int x, int y)
 {
     const uint32_t r = (uint32_t)(y - a.y0);
@@ -147,8 +147,8 @@ __global__ void __launch_bounds__(kLiftPrefixBlock) lift_prefix_kernel(LiftPass 
             }
         }
     };
-    double carry  = 0.0;
-    bool faithful = true;  // every pixel with an error has raised the sum, none has lowered it
+    double carry     = 0.0;
+    uint32_t dimmest = 0xFFFFFFFFu;  // smallest error of the lane's pixels that have one, as its bits less one
     float g[kLiftPerLane];
     load(kLiftPerLane * lane, g);
     for (int x0 = 0; x0 < a.width; x0 += kLiftStep)
@@ -167,28 +167,28 @@ __global__ void __launch_bounds__(kLiftPrefixBlock) lift_prefix_kernel(LiftPass 
             const double up = __shfl_up(incl, d, kWave);
             if (lane >= d) incl += up;
         }
-        const double in_front = __shfl_up(incl, 1, kWave);
-        const double before   = lane == 0 ? carry : carry + in_front;  // the last entry of the lane in front, to the bit
+        const double before = carry + (incl - own);
+        carry += __shfl(incl, kWave - 1, kWave);
         __syncthreads();  // the block of the step before has been stored
-        double last = before;
 #pragma unroll
         for (int k = 0; k < kLiftPerLane; ++k)
         {
-            const double sum = k == kLiftPerLane - 1 ? carry + incl : before + p[k];
-            faithful &= g[k] > 0.f ? sum > last : sum >= last;
-            last = sum;
-            s_sum[(kLiftPerLane * lane + k) * kLiftRows + wave] = sum;
+            s_sum[(kLiftPerLane * lane + k) * kLiftRows + wave] = before + p[k];
+            dimmest = min(dimmest, __float_as_uint(g[k]) - 1u);  // (no error: the largest number)
         }
-        carry = __shfl(last, kWave - 1, kWave);
         __syncthreads();
         const int columns = min(kLiftStep, a.width - x0);
         for (int k = threadIdx.x; k < columns * kLiftRows; k += kLiftPrefixBlock) group[(size_t)(x0 + 1) * kLiftRows + k] = s_sum[k];
 #pragma unroll
         for (int k = 0; k < kLiftPerLane; ++k) g[k] = next[k];
     }
-    // the empty run; its sign says whether equal entries of the row mean that there is no error between them
-    const bool all_faithful = __ballot(!faithful) == 0ull;
-    if (lane == 0) group[wave] = all_faithful ? 0.0 : -0.0;
+    // The empty run. Neighbouring entries are off by a few units in the last place of the row's sum, so a pixel of at least
+    // 2^-48 of it shows in every difference; where one is dimmer, or the sum is not finite, the sign of the entry says that
+    // it may not.
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) dimmest = min(dimmest, (uint32_t)__shfl_xor((int)dimmest, d, kWave));
+    const bool all_show = dimmest == 0xFFFFFFFFu || (double)__uint_as_float(dimmest + 1u) >= carry * 0x1p-48;
+    if (lane == 0) group[wave] = all_show ? 0.0 : -0.0;
 }
 
 // tris_indices of the reference (src/lib/rendering/RenderForward.cu:665-666): two triangles per face of the box, corner
@@ -317,7 +317,7 @@ __device__ __forceinline__ bool in_any_triangle(const Corners& f, float x, float
 // Sum of the pixels [x0, x1) of row y. The difference of two running sums is taken where it keeps its bits: an entry is
 // off by 2^-50 of itself or so, so a run of at least 2^-12 of what lies in front of it is good to 38 bits, 14 more than the
 // float it ends in. Dimmer runs (also those behind a pixel that is not finite) are added up pixel by pixel; a difference
-// of zero is a run without any error where the row says so.
+// of zero is a run without any error where the row has no pixel that rounding could swallow.
 __device__ __forceinline__ double lift_run_sum(const LiftPass& a, int x0, int x1, int y)
 {
     if (a.sums)
