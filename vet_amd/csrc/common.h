@@ -339,18 +339,28 @@ __device__ __forceinline__ float4 pair_other(float4 v)
     return make_float4(pair_other(v.x), pair_other(v.y), pair_other(v.z), pair_other(v.w));
 }
 
-// Place of the gradient record of the fragment (layer l, corner h, point id) in the record array of the backward pass
-// (hits = 1, or 4 corners in BILINEAR_BLEND). Two layouts, chosen per call on the host. Layer after layer
-// ([layer][corner][point]): the per-point kernel, which walks the points in order, reads every layer's records as one
-// stream; right for views that see most of the cloud. Point after point ([point][layer][corner]): all records of a
+// The gradient records: what the per-pixel backward kernels leave behind for the per-point kernel.
+//   one hit per layer: 32 bytes, (d descriptor 0..3), (d confidence, d image x, d image y, 0)
+//   2x2 splat: 8 bytes for each of the four corners, (descriptor factor, d alpha), 32 bytes for a point and layer. The
+//   gradient with respect to the descriptor is that factor times the upstream gradient of the pixel, which the per-point
+//   kernel reads from a copy that has the channels side by side (BackwardPass::pixel_gradient; the corners share its
+//   cache lines), and what follows from d alpha (confidence and position) it works out itself. With 32 bytes for every
+//   corner the scattered record stores were a third of the per-pixel kernel: 2x2 splat at 1080p 247 -> 166 us.
+// With one hit per layer the same exchange of bytes for a gather does not pay: ten million points 541 -> 491 us in the per-pixel
+// kernel, but 255 -> 289 in the per-point kernel, where the 64 points of a wave find the pixels' upstream gradients in as many
+// cache lines; benchmark frame 115 -> 107 and 47 -> 56, four town views 400 -> 396 and 147 -> 174.
+constexpr int kRecordRoom = 32;  // bytes the workspace keeps for the record of a fragment
+
+// Place of the record(s) of point id in layer l, in units of 32 bytes. Two layouts, chosen per call on the host. Layer after layer
+// ([layer][point]): the per-point kernel, which walks the points in order, reads every layer's records as one
+// stream; right for views that see most of the cloud. Point after point ([point][layer]): all records of a
 // point are neighbours, one burst for the per-point kernel instead of a 64-byte access per record; right for views that
 // see a small part of the cloud (training crops), where the streams of the first layout have turned into scattered
-// reads anyway. Measured at 2 M points: full frame 0.313 against 0.336 ms (FULL_BLEND) in favour of the first, batch of
-// four 512x512 crops 0.631 against 0.556 ms (BILINEAR_BLEND) in favour of the second.
-__device__ __forceinline__ size_t gradient_record(int point_major, int N, int L, int hits, int l, int h, int id)
+// reads anyway. Measured at 2 M points when every record took 32 bytes: full frame 0.313 against 0.336 ms (FULL_BLEND) in favour
+// of the first, batch of four 512x512 crops 0.631 against 0.556 ms (BILINEAR_BLEND) in favour of the second.
+__device__ __forceinline__ size_t gradient_record(int point_major, int N, int L, int l, int id)
 {
-    return point_major ? (size_t)id * (size_t)(L * hits) + (size_t)(l * hits + h)
-                       : (size_t)(l * hits + h) * (size_t)N + (size_t)id;
+    return point_major ? (size_t)id * (size_t)L + (size_t)l : (size_t)l * (size_t)N + (size_t)id;
 }
 
 // Workgroup -> tile mapping of the per-pixel kernels (blend, backward): a workgroup owns a tile, a wave 16x4 pixels of

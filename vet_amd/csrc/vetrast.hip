@@ -278,6 +278,12 @@ size_t camera_rows_bytes(int64_t N)
     return align_up(((size_t)N + kBlock - 1) / kBlock * kCameraRow * sizeof(double), kAlign);
 }
 
+// The upstream gradient with the channels side by side (BackwardPass::pixel_gradient), [P] float4 behind the gradient records.
+size_t pixel_gradient_base(const vetrast_workspace_layout& lay)
+{
+    return align_up(lay.partial_base + (size_t)lay.fragment_capacity * kRecordRoom, kAlign);
+}
+
 TileMap make_tile_map(const LayerTable& ly, const double* list_bound = nullptr, bool split_all = false)
 {
     TileMap m;
@@ -586,7 +592,7 @@ int vetrast_workspace_layout_for_mode(int32_t N, int32_t B, int32_t L, int32_t w
     const size_t forward_block = align_up(at, kAlign) - shared_base;
     at                         = shared_base;
     lay->partial_base          = at;
-    at += align_up(cap * 8 * sizeof(float), kAlign);
+    at = pixel_gradient_base(*lay) + P * sizeof(float4);
     lay->background_partial_base = at;
     // (the FUZZY_BLEND kernel that takes a wave per list keeps rows per replica and kFuzzyFoldRows rows they are folded into)
     at += align_up(((size_t)tile_grid(make_tile_map(t, nullptr, true)) * kFuzzyReplicas + kFuzzyFoldRows) * kBackgroundRow * sizeof(float), kAlign);
@@ -967,6 +973,7 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
                 bp.packed           = packed;
                 bp.background       = ws_ptr<const float>(ws, lay.flags_base) + kPreparedBackgroundOffset;
                 bp.partial          = ws_ptr<float4>(ws, lay.partial_base + lay.lane_scratch_stride * lane);
+                bp.pixel_gradient   = ws_ptr<float4>(ws, pixel_gradient_base(lay) + lay.lane_scratch_stride * lane);
                 bp.point_major_records = point_major_records;
                 bp.background_partial  = ws_ptr<float>(ws, lay.background_partial_base + lay.lane_scratch_stride * lane);
                 bp.ly               = ly;
@@ -1080,6 +1087,7 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             gp.last_key            = ws_ptr<uint64_t>(ws, lay.last_key_base + lay.last_key_stride * first);
             gp.kept                = ws_ptr<uint32_t>(ws, lay.kept_base + lay.kept_stride * first);
             gp.partial             = partial;
+            gp.pixel_gradient      = ws_ptr<float4>(ws, pixel_gradient_base(lay));
             gp.grad_texture        = g->grad_texture;
             gp.grad_confidence     = g->grad_confidence;
             gp.grad_points         = g->grad_points;
@@ -1094,6 +1102,7 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             gp.last_key_stride     = lay.last_key_stride / sizeof(uint64_t);
             gp.kept_stride         = lay.kept_stride / sizeof(uint32_t);
             gp.partial_stride      = lay.lane_scratch_stride / sizeof(float4);
+            gp.pixel_gradient_stride  = lay.lane_scratch_stride / sizeof(float4);
             gp.background_rows_stride = lay.lane_scratch_stride / sizeof(float);
             gp.camera_partial_stride  = camera_rows_bytes(N) / sizeof(double);
             gp.accumulate          = (add_to_rows || first > 0) ? 1 : 0;
