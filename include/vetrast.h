@@ -182,7 +182,7 @@ typedef struct vetrast_workspace_layout
     size_t packed_base;    /* float [N][8]: descriptor (4, zero padded), confidence, 3 pad */
     size_t slots_base;     /* uint32, shaped like the log: rank inside its bin of every logged record (scratch) */
     size_t views_base;     /* prepared per-view camera constants */
-    size_t scan_partials_base;
+    size_t scan_partials_base; /* per lane: partial sums of the scan, behind them the list of the bins that a workgroup builds */
     int64_t num_bins;      /* bins of one view: runs of 256 / 64 / 16 / 4 consecutive pixel numbers, chosen per layer from N */
     size_t bin_counts_base, bin_counts_stride; /* per view, uint32 [2][num_bins+1 padded]: fragments per bin, and their
                                                   exclusive scan (in place of the counts where a view has more than

@@ -12,7 +12,6 @@ constexpr int kWave           = 64;
 constexpr uint64_t kInfKey    = ~0ull;        // sorts behind every real (depth bits, point id) key
 constexpr int kScanPerThread  = 16;
 constexpr int kScanPerBlock   = kBlock * kScanPerThread;  // 4096 counts per workgroup
-constexpr int kBlendChunk     = 4;            // fragments a blend / backward thread prefetches at a time
 constexpr int kBackgroundRow  = 8;            // floats per workgroup row of background-gradient partial sums
 constexpr int kPreparedBackgroundOffset = 16;  // float index inside the flags block: the background as it is blended
 constexpr int kPackedFloats   = 8;            // interleaved record: 4 descriptor floats, confidence, 3 pad
@@ -24,6 +23,9 @@ constexpr int kViewLanes      = 4;            // views of one call that share a 
 // and with sixteen; 2x2 splat at 1080p 17.6, 7.2, under 6 us. An empty log costs 4.5 us with one, 5.9 with sixteen.
 constexpr int kMoveShare      = 8;
 constexpr int kLogSegments    = 256;          // the overflow log is cut into this many segments with a cursor each
+constexpr int kWaveBinCap     = 256;          // fragment records up to which one wave builds a bin's lists
+constexpr int kBuildCap       = 1024;         // ... and up to which a workgroup does at once
+constexpr int kBuildMaxRuns   = 8;            // a bin of more than this many times kBuildCap records is built in memory
 constexpr int kLogCursorStride = 16;          // uint32 between two cursors (64 bytes: one cursor per cache line)
 
 // Camera constants of one view, written by prepare_views_kernel and read (uniformly) by every other kernel.
@@ -124,6 +126,21 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, int /*lane*/
     v += dpp_shifted<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
     v += dpp_shifted<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
     return v;
+}
+
+// Texture row of point `id`, or -1 where id or row are out of range. The row of an index table is waited for inside the branch:
+// a caller without a table (the rule) would otherwise wait at the branch's end for whatever it has under way by then, stores
+// among it.
+__device__ __forceinline__ int texture_row(const int32_t* index, int id, int N)
+{
+    int row = (uint32_t)id < (uint32_t)N ? id : -1;
+    if (index != nullptr)
+    {
+        if (row >= 0) row = index[row];
+        asm volatile("" : "+v"(row));
+        if ((uint32_t)row >= (uint32_t)N) row = -1;
+    }
+    return row;
 }
 
 // Launch descriptor shared by the forward kernels of one view.

@@ -783,6 +783,85 @@ __global__ void __launch_bounds__(kBlock) overflow_move_kernel(ScatterTargets in
     overflow_move(in, bin_offsets, binned, capacity);
 }
 
+// The bins of a view with more records than one wave builds (kWaveBinCap), written down beside the scan for the build pass.
+// Those that do not even fit a workgroup's LDS (kBuildCap) stand at the front of the list, once for every workgroup that is
+// to share them, the others at its back, so that what takes longest starts first. The order inside each half is that in which
+// the workgroups get there; no result depends on it.
+struct CrowdedBins
+{
+    uint2* entries;    // [capacity]: bin, which part of it | number of parts << 16
+    uint32_t* counts;  // [2], 8-byte aligned: entries at the front, at the back; zero before the launch
+    uint32_t capacity;
+};
+// Workgroups that share a bin of n records. The longest bins set the end of the pass where one workgroup takes them alone
+// (4891 records 107 us, with all others done after 73), so a part is sized to fit LDS at once as a rule, with some room for
+// lists that can't be cut. More than kBuildMaxRuns times what fits goes through memory, which one workgroup does.
+__device__ __forceinline__ uint32_t parts_of_bin(uint32_t n)
+{
+    constexpr uint32_t kPart = kBuildCap / 4 * 3;
+    return n > (uint32_t)kBuildCap && n <= (uint32_t)(kBuildMaxRuns * kBuildCap) ? (n + kPart - 1u) / kPart : 1u;
+}
+
+// Writes down the crowded ones of 4 N consecutive bins from `bin` on. All threads of the workgroup must call. Each workgroup
+// draws its places with one atomic; those on one address queue up, 50 ns each, so a workgroup looks at a thousand bins or two.
+template <int N>
+__device__ __forceinline__ void list_crowded(const CrowdedBins& out, const uint4 (&counts)[N], uint32_t bin)
+{
+    __shared__ uint32_t s_wave[2][kBlock / kWave];
+    __shared__ uint32_t s_first[2];
+    uint32_t own[2] = {0u, 0u};
+    auto count = [&](uint32_t n) {
+        if (n > (uint32_t)kBuildCap)
+            own[0] += parts_of_bin(n);
+        else if (n > (uint32_t)kWaveBinCap)
+            ++own[1];
+    };
+#pragma unroll
+    for (int k = 0; k < N; ++k) count(counts[k].x), count(counts[k].y), count(counts[k].z), count(counts[k].w);
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    uint32_t run[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+        const uint32_t incl = wave_inclusive_scan(own[h], lane);
+        if (lane == kWave - 1) s_wave[h][wave] = incl;
+        run[h] = incl - own[h];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        uint32_t entries[2] = {0u, 0u};
+        for (int h = 0; h < 2; ++h)
+            for (int k = 0; k < kBlock / kWave; ++k) entries[h] += s_wave[h][k];
+        unsigned long long first = 0ull;
+        if ((entries[0] | entries[1]) != 0u)
+            first = atomicAdd(reinterpret_cast<unsigned long long*>(out.counts), ((unsigned long long)entries[1] << 32) | entries[0]);
+        s_first[0] = (uint32_t)first, s_first[1] = (uint32_t)(first >> 32);
+    }
+    __syncthreads();
+    if ((own[0] | own[1]) == 0u) return;
+    for (int h = 0; h < 2; ++h)
+    {
+        run[h] += s_first[h];
+        for (int k = 0; k < wave; ++k) run[h] += s_wave[h][k];
+    }
+    auto put = [&](uint32_t n, uint32_t b) {
+        if (n <= (uint32_t)kWaveBinCap) return;
+        const uint32_t parts = parts_of_bin(n);
+        for (uint32_t part = 0; part < parts; ++part)
+        {
+            const uint32_t at = n > (uint32_t)kBuildCap ? run[0]++ : out.capacity - 1u - run[1]++;
+            if (at < out.capacity) out.entries[at] = make_uint2(b, part | (parts << 16));  // guard: never false
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+    {
+        put(counts[k].x, bin + 4 * k), put(counts[k].y, bin + 4 * k + 1);
+        put(counts[k].z, bin + 4 * k + 2), put(counts[k].w, bin + 4 * k + 3);
+    }
+}
+
 // What the scan and move kernels of one view work on.
 struct ScanArgs
 {
@@ -793,6 +872,7 @@ struct ScanArgs
     ScatterTargets in;
     uint4* binned;
     uint32_t capacity;
+    CrowdedBins crowded;
 };
 
 __global__ void __launch_bounds__(kBlock) overflow_move_views_kernel(PerView<ScanArgs> views)
@@ -818,9 +898,21 @@ __device__ __forceinline__ uint32_t block_reduce_sum(uint32_t v, uint32_t* lds4)
     return total;
 }
 
-__device__ __forceinline__ void scan_partials(const uint4* __restrict__ counts4, uint32_t* __restrict__ partials)
+// Workgroups of the first launch beyond those that add up look for crowded bins, kListPerBlock counts each.
+constexpr int kListPerBlock = 2 * 4 * kBlock;
+static_assert(kScanPerBlock % kListPerBlock == 0, "the padded counts are a whole number of stretches");
+__device__ __forceinline__ void scan_partials(const uint4* __restrict__ counts4, uint32_t* __restrict__ partials,
+                                              const CrowdedBins& crowded)
 {
     __shared__ uint32_t lds4[4];
+    const uint32_t adding = gridDim.x / (1u + kScanPerBlock / kListPerBlock);
+    if (blockIdx.x >= adding)
+    {
+        const uint32_t first = (blockIdx.x - adding) * (uint32_t)kListPerBlock + threadIdx.x * 8u;
+        const uint4 c[2]     = {counts4[first / 4u], counts4[first / 4u + 1u]};
+        list_crowded(crowded, c, first);
+        return;
+    }
     const uint4* src = counts4 + (size_t)blockIdx.x * (kScanPerBlock / 4);
     uint32_t sum     = 0;
 #pragma unroll
@@ -834,15 +926,15 @@ __device__ __forceinline__ void scan_partials(const uint4* __restrict__ counts4,
 }
 
 __global__ void __launch_bounds__(kBlock) scan_partials_kernel(const uint4* __restrict__ counts4,
-                                                                uint32_t* __restrict__ partials)
+                                                                uint32_t* __restrict__ partials, CrowdedBins crowded)
 {
-    scan_partials(counts4, partials);
+    scan_partials(counts4, partials, crowded);
 }
 
 __global__ void __launch_bounds__(kBlock) scan_partials_views_kernel(PerView<ScanArgs> views)
 {
     const ScanArgs& v = views.v[blockIdx.y];
-    scan_partials(reinterpret_cast<const uint4*>(v.bin_counts), v.partials);
+    scan_partials(reinterpret_cast<const uint4*>(v.bin_counts), v.partials, v.crowded);
 }
 
 __device__ __forceinline__ void scan_apply(uint4* __restrict__ counts4, const uint32_t* __restrict__ partials)
@@ -905,13 +997,22 @@ __global__ void __launch_bounds__(kBlock) scan_apply_views_kernel(PerView<ScanAr
 constexpr int kScanMoveMax = 60 * kBlock;  // 61 440 bytes of LDS
 
 __device__ __forceinline__ void scan_move(const uint4* __restrict__ counts4, uint32_t n, uint4* __restrict__ offsets4,
-                                          const ScatterTargets& in, uint4* __restrict__ binned, uint32_t capacity)
+                                          const ScatterTargets& in, uint4* __restrict__ binned, uint32_t capacity,
+                                          const CrowdedBins& crowded)
 {
     __shared__ uint32_t s_off[kScanMoveMax];
     __shared__ uint32_t wave_tot[kBlock / kWave];
     const uint32_t segment = blockIdx.x;
     // (workgroup 0 scans whatever its segment holds: it asks for its cursor and for the counts at once)
     const uint32_t entries = min(in.log_cursor[segment * kLogCursorStride], in.segment_capacity);
+    // workgroup k > 0 also looks for crowded bins in a stretch of the counts
+    const uint32_t stretch = (segment - 1u) * (4u * kBlock);
+    if (segment != 0u && stretch < n)
+    {
+        uint4 c[1];
+        c[0] = stretch + 4u * threadIdx.x < n ? counts4[stretch / 4u + threadIdx.x] : make_uint4(0u, 0u, 0u, 0u);
+        list_crowded(crowded, c, stretch + 4u * threadIdx.x);
+    }
     if (segment != 0u && entries == 0u) return;
     constexpr int kPer = kScanMoveMax / kBlock;  // 60 consecutive counts per thread, as 15 16-byte loads
     const uint4* src   = counts4 + threadIdx.x * (kPer / 4);
@@ -963,68 +1064,17 @@ __device__ __forceinline__ void scan_move(const uint4* __restrict__ counts4, uin
 
 __global__ void __launch_bounds__(kBlock) scan_move_kernel(const uint4* __restrict__ counts4, uint32_t n,
                                                             uint4* __restrict__ offsets4, ScatterTargets in,
-                                                            uint4* __restrict__ binned, uint32_t capacity)
+                                                            uint4* __restrict__ binned, uint32_t capacity, CrowdedBins crowded)
 {
-    scan_move(counts4, n, offsets4, in, binned, capacity);
+    scan_move(counts4, n, offsets4, in, binned, capacity, crowded);
 }
 
 __global__ void __launch_bounds__(kBlock) scan_move_views_kernel(PerView<ScanArgs> views)
 {
     const ScanArgs& v = views.v[blockIdx.y];
     scan_move(reinterpret_cast<const uint4*>(v.bin_counts), v.n,
-              reinterpret_cast<uint4*>(v.bin_counts + v.scanned_behind), v.in, v.binned, v.capacity);
-}
-
-// Front-to-back blend of one pixel's sorted list read from memory: out += (T*c)*t, T = (1-c)*T, in exactly this order
-// (BlendMulti, src/lib/rendering/RenderForward.cu:1303-1357). The list is walked in chunks of kBlendChunk fragments: all
-// keys of a chunk are loaded first, then all descriptor records, and only then the (strictly sequential) arithmetic
-// runs, so a thread keeps several gathers in flight instead of one dependent load chain per fragment.
-template <int C>
-__device__ __forceinline__ void blend_list_from_memory(const uint64_t* list, uint32_t n, const int32_t* index,
-                                                       const float4* packed, int N, float* transmittance, float& T,
-                                                       float (&color)[C])
-{
-    for (uint32_t base = 0; base < n; base += kBlendChunk)
-    {
-        int ti[kBlendChunk];
-        float4 t4[kBlendChunk];
-        float c[kBlendChunk];
-#pragma unroll
-        for (int u = 0; u < kBlendChunk; ++u)
-        {
-            ti[u] = -1;
-            if (base + u < n)
-            {
-                const int id = (int)(uint32_t)list[base + u];
-                // an id or texture index out of range cannot come from a list the scatter pass wrote; such a fragment is
-                // skipped instead of gathered (the reference asserts on the texture index, RenderForward.cu:1335-1336)
-                if ((uint32_t)id < (uint32_t)N) ti[u] = index ? index[id] : id;
-                if ((uint32_t)ti[u] >= (uint32_t)N) ti[u] = -1;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kBlendChunk; ++u)
-        {
-            if (ti[u] >= 0)
-            {
-                t4[u] = packed[2 * (size_t)ti[u]];
-                c[u]  = packed[2 * (size_t)ti[u] + 1].x;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kBlendChunk; ++u)
-        {
-            if (ti[u] >= 0)
-            {
-                if (transmittance) transmittance[base + u] = T;
-                const float t[4] = {t4[u].x, t4[u].y, t4[u].z, t4[u].w};
-                const float Tc   = T * c[u];
-#pragma unroll
-                for (int ci = 0; ci < C; ++ci) color[ci] = Tc * t[ci] + color[ci];
-                T = (1.f - c[u]) * T;
-            }
-        }
-    }
+              reinterpret_cast<uint4*>(v.bin_counts + v.scanned_behind), v.in, v.binned, v.capacity,
+              v.crowded);
 }
 
 }  // namespace vetrast

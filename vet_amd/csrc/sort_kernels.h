@@ -113,23 +113,51 @@ __device__ __forceinline__ void sort_class(uint64_t* fragments, const uint8_t* s
     }
 }
 
-// K smallest keys (K <= 64) of a list longer than 64, sorted, written to its first K places. The wave keeps the 64
-// smallest keys seen so far in sorted order; a chunk of 64 further keys is looked at only if one of them beats the
-// current K-th smallest.
+// K smallest keys (K <= 64) of a list longer than 64, sorted, written to its first K places. The wave keeps the K smallest
+// keys seen so far, sorted, in its first lanes. Of every further 64 keys those that beat the K-th gather in the lanes behind,
+// in no order; only when they do not fit there any more all 64 lanes are sorted (115 vector instructions), which leaves the K
+// smallest in front. Most of a long list never beats the K-th, so that is two or three times where sorting every 64 keys in
+// turn and merging them took one of each (ten million points, lists of up to a thousand cut to 16: the list-building pass went
+// from 239 to 215 million vector instructions and 540 to 525 us).
 __device__ __forceinline__ void select_smallest(uint64_t* list, uint32_t n, int lane, int K)
 {
-    uint64_t best = list[lane];  // n > 64
-    best          = bitonic_sort_groups<6>(best, lane);
+    uint64_t best = bitonic_sort_groups<6>(list[lane], lane);  // n > 64
+    uint64_t kth  = shfl_u64(best, K - 1);
+    int filled    = K;  // lanes in use
+    if (lane >= K) best = kInfKey;
     for (uint32_t base = kWave; base < n; base += kWave)
     {
-        const uint64_t v   = (base + lane < n) ? list[base + lane] : kInfKey;
-        const uint64_t thr = shfl_u64(best, K - 1);
-        if (__ballot(v < thr) == 0ull) continue;
-        const uint64_t sorted = bitonic_sort_groups<6>(v, lane);
-        const uint64_t mirror = shfl_u64(sorted, kWave - 1 - lane);
-        best                  = (mirror < best) ? mirror : best;  // 64 smallest of the 128, a bitonic sequence
-        best                  = bitonic_merge64(best, lane);
+        const uint64_t v = (base + lane < n) ? list[base + lane] : kInfKey;
+        uint64_t m       = __ballot(v < kth);
+        if (m == 0ull) continue;
+        if (filled + __popcll(m) > kWave && filled > K)
+        {
+            best   = bitonic_sort_groups<6>(best, lane);
+            kth    = shfl_u64(best, K - 1);
+            filled = K;
+            if (lane >= K) best = kInfKey;
+            m = __ballot(v < kth);
+        }
+        const int more = __popcll(m);
+        if (filled + more > kWave)
+        {
+            // too many at once: 64 smallest of them and of what there is, a bitonic sequence
+            const uint64_t sorted = bitonic_sort_groups<6>(v, lane);
+            const uint64_t mirror = shfl_u64(sorted, kWave - 1 - lane);
+            best                  = bitonic_merge64((mirror < best) ? mirror : best, lane);
+            kth                   = shfl_u64(best, K - 1);
+            if (lane >= K) best = kInfKey;
+            continue;
+        }
+        // the keys that count go to the lanes from `filled` on; the others to lane 0, which does not look at what it gets
+        const int below    = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        const int to       = (m >> lane) & 1ull ? (filled + below) << 2 : 0;
+        const uint32_t lo  = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)(uint32_t)v);
+        const uint32_t hi  = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)(uint32_t)(v >> 32));
+        if (lane >= filled && lane < filled + more) best = ((uint64_t)hi << 32) | lo;
+        filled += more;
     }
+    if (filled > K) best = bitonic_sort_groups<6>(best, lane);
     if (lane < K) list[lane] = best;
 }
 
@@ -233,12 +261,10 @@ __device__ __forceinline__ void sort_in_registers(uint64_t* list, uint32_t n, in
     }
 }
 
-constexpr uint32_t kRegisterSortKeys = 256;  // longest list sort_wave_lists sorts in registers
-
 // Sorts the lists of one wave: lane i holds the start `off` (an index into `fragments`) and the length `n` of its list
 // (n = 0 for lanes without a list). `fragments` may point to global memory or to LDS. Lists that have to be sorted in
-// full and hold more than kRegisterSortKeys and up to `skip_longer` keys are left alone: the caller sorts them by other
-// means.
+// full and hold more than 64 CHUNKS and up to `skip_longer` keys are left alone: the caller sorts them by other means.
+template <int CHUNKS = 4>
 __device__ __forceinline__ void sort_wave_lists(uint64_t* fragments, uint8_t* src_lane, uint32_t off, uint32_t n,
                                                 int lane, int K, uint32_t skip_longer = 0)
 {
@@ -285,8 +311,8 @@ __device__ __forceinline__ void sort_wave_lists(uint64_t* fragments, uint8_t* sr
             select_smallest(fragments + o, nn, lane, K);
         else if (nn <= 2 * kWave)
             sort_in_registers<2>(fragments + o, nn, lane);
-        else if (nn <= kRegisterSortKeys)
-            sort_in_registers<4>(fragments + o, nn, lane);
+        else if (CHUNKS > 2 && nn <= (uint32_t)(CHUNKS * kWave))
+            sort_in_registers<CHUNKS>(fragments + o, nn, lane);
         else if (nn <= skip_longer)
             continue;  // the caller sorts lists of this length with the whole workgroup
         else

@@ -270,6 +270,9 @@ uint32_t log_segment_records(int64_t N, int L, int hits)
     return (uint32_t)((groups + kLogSegments - 1) / kLogSegments * kBlock * L * hits);
 }
 size_t log_records(int64_t N, int L, int hits) { return (size_t)log_segment_records(N, L, hits) * kLogSegments; }
+// The list of crowded bins (CrowdedBins), behind the scan's partial sums: every bin, and once more for every further
+// workgroup that shares one. Its two counts are in unused words of the first log cursor's cache line, which every call clears.
+size_t crowded_list_entries(size_t bins, size_t fragments) { return bins + fragments / (kBuildCap / 4 * 3) + 1; }
 size_t log_cursor_bytes(int B) { return (size_t)B * kLogSegments * kLogCursorStride * sizeof(uint32_t); }
 
 // Per-workgroup pose / intrinsics rows one view's per-point backward pass leaves.
@@ -544,7 +547,7 @@ int vetrast_workspace_layout_for_mode(int32_t N, int32_t B, int32_t L, int32_t w
     const int lanes            = std::min(B, kViewLanes);
     lay->view_lanes            = lanes;
     lay->scan_partials_base    = at;
-    lay->scan_partials_stride  = align_up((Tpad / kScanPerBlock) * sizeof(uint32_t), kAlign);
+    lay->scan_partials_stride  = align_up((Tpad / kScanPerBlock) * sizeof(uint32_t), kAlign) + align_up(crowded_list_entries(bins, cap) * sizeof(uint2), kAlign);
     at += lay->scan_partials_stride * lanes;
     lay->offsets_base   = at;
     lay->offsets_stride = align_up((P + 1) * sizeof(uint32_t), kAlign);
@@ -687,6 +690,7 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
     // bytes): with one view, and with several where the caller expects each to see little of the cloud.
     const bool rows_of_visible_points =
         a->index == nullptr && a->point_order == nullptr && (B == 1 || views_see_little(p, N, hits));
+    const uint32_t crowded_blocks = std::min<uint32_t>((bins + 3) / 4, kCrowdedBlocks);
     for (int first = 0; first < B; first += lanes)
     {
         const int last = std::min(B, first + lanes), count = last - first;
@@ -729,6 +733,10 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
             sa.in             = targets;
             sa.binned         = ws_ptr<uint4>(ws, lay.binned_base + lay.binned_stride * lane);
             sa.capacity       = (uint32_t)lay.fragment_capacity;
+            sa.crowded.entries  = ws_ptr<uint2>(ws, lay.scan_partials_base + lay.scan_partials_stride * lane +
+                                                       align_up((lay.bin_counts_stride / 2 / sizeof(uint32_t) / kScanPerBlock) * sizeof(uint32_t), kAlign));
+            sa.crowded.counts   = targets.log_cursor + 2;
+            sa.crowded.capacity = (uint32_t)crowded_list_entries(bins, (size_t)lay.fragment_capacity);
 
             BuildPass& bp          = build.v[lane];
             bp.bin_offsets         = scan_and_move ? sc.bin_counts + Tpad : sc.bin_counts;
@@ -747,6 +755,10 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
             bp.transmittance       = a->save_for_backward ? ws_ptr<float>(ws, lay.transmittance_base + lay.transmittance_stride * b) : nullptr;
             bp.weight              = ws_ptr<float>(ws, lay.weight_base + lay.weight_stride * b);
             bp.ly                  = ly;
+            bp.crowded             = sa.crowded.entries;
+            bp.crowded_counts      = sa.crowded.counts;
+            bp.crowded_capacity    = sa.crowded.capacity;
+            bp.crowded_blocks      = crowded_blocks;
             bp.num_bins            = bins;
             bp.N                   = N;
             bp.K                   = p.debug_max_list_length;
@@ -787,23 +799,23 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
                 if (one)
                     hipLaunchKernelGGL(scan_move_kernel, dim3(kLogSegments), blk, 0, stream,
                                        reinterpret_cast<const uint4*>(sa.bin_counts), sa.n,
-                                       reinterpret_cast<uint4*>(sa.bin_counts + Tpad), sa.in, sa.binned, sa.capacity);
+                                       reinterpret_cast<uint4*>(sa.bin_counts + Tpad), sa.in, sa.binned, sa.capacity, sa.crowded);
                 else
                     hipLaunchKernelGGL(scan_move_views_kernel, dim3(kLogSegments, views_y), blk, 0, stream, scan);
             }
             else
             {
-                const unsigned blocks = (unsigned)(Tpad / kScanPerBlock);
+                const unsigned blocks = (unsigned)(Tpad / kScanPerBlock), with_list = blocks * (1 + kScanPerBlock / kListPerBlock);
                 if (one)
                 {
-                    hipLaunchKernelGGL(scan_partials_kernel, dim3(blocks), blk, 0, stream,
-                                       reinterpret_cast<const uint4*>(sa.bin_counts), sa.partials);
+                    hipLaunchKernelGGL(scan_partials_kernel, dim3(with_list), blk, 0, stream,
+                                       reinterpret_cast<const uint4*>(sa.bin_counts), sa.partials, sa.crowded);
                     hipLaunchKernelGGL(scan_apply_kernel, dim3(blocks), blk, 0, stream,
                                        reinterpret_cast<uint4*>(sa.bin_counts), sa.partials);
                 }
                 else
                 {
-                    hipLaunchKernelGGL(scan_partials_views_kernel, dim3(blocks, views_y), blk, 0, stream, scan);
+                    hipLaunchKernelGGL(scan_partials_views_kernel, dim3(with_list, views_y), blk, 0, stream, scan);
                     hipLaunchKernelGGL(scan_apply_views_kernel, dim3(blocks, views_y), blk, 0, stream, scan);
                 }
             }
@@ -821,7 +833,8 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
         {
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BUILD);
             const BuildPass& bp = build.v[0];
-            const dim3 g(bins), gv(bins, views_y);
+            const unsigned blocks = crowded_blocks + (bins + kBlock / kWave - 1) / (kBlock / kWave);
+            const dim3 g(blocks), gv(blocks, views_y);
             auto launch = [&](auto channels, auto bilinear, auto fuzzy) {
                 constexpr int kC         = decltype(channels)::value;
                 constexpr bool kBilinear = decltype(bilinear)::value, kFuzzy = decltype(fuzzy)::value;
