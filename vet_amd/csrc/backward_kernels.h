@@ -95,6 +95,12 @@ __device__ __forceinline__ bool interior_pixel(int x, int y, int w, int h)
 // 64 pixels out as one dense item list (in windows of 16 fragments per pixel), and every lane processes one FRAGMENT:
 // per-pixel data (upstream gradient, neighbour samples) is staged in LDS, the suffix sum is a segmented scan over the
 // lanes of a pixel plus a per-pixel carry, rounds run from the deepest fragments to the nearest.
+//
+// What bounds it: chains of memory round trips (list, keys, descriptor records, gradient records) and the traffic behind
+// them, 340 MB of a benchmark frame at three quarters of the rate of a copy; vector instructions are half of its cycles.
+// More pixels to a wave where tiles hold little cost 40 % fewer instructions and a third more time. Against a table of items
+// filled by their pixels, sums through the LDS permute and waits behind branches: benchmark frame 101 -> 94 us, four town
+// views 373 -> 344, four crops with the 2x2 splat 67 -> 59, 2x2 splat at 1080p 140 -> 136 (busy cycles at 2.4 GHz).
 constexpr int kWindow     = 16;                 // fragments per pixel in one window
 constexpr int kWaveItems  = kWave * kWindow;    // item table of a wave
 
@@ -107,53 +113,67 @@ template <int C, bool BILINEAR>
 __device__ __forceinline__ void blend_backward(const BackwardPass& a)
 {
     constexpr int kWaves = kBlock / kWave;
-    __shared__ uint32_t s_off[kWaves][kWave];
-    __shared__ uint32_t s_base[kWaves][kWave];
+    // per pixel: place of its deepest fragment of the window in the list buffer + place of that one among the items, and the
+    // latter | whether the pixel gives a position gradient << 31
+    __shared__ uint2 s_place[kWaves][kWave];
     __shared__ float s_carry[kWaves][kWave];
     __shared__ float4 s_g[kWaves][kWave];
     // position heuristic of a pixel as coefficients: d image x = (t . ax + bx) / C, d image y = (t . ay + by) / C
     __shared__ float4 s_ax[kWaves][kWave];
     __shared__ float4 s_ay[kWaves][kWave];
     __shared__ float2 s_bxy[kWaves][kWave];
-    __shared__ uint8_t s_point[kWaves][kWave];
-    __shared__ uint8_t s_item[kWaves][kWaveItems];
+    __shared__ uint32_t s_starts[kWaves][kWaveItems / 32];  // a bit per item: a pixel's items start here
+    __shared__ uint8_t s_order[kWaves][kWave];              // lanes of the pixels that have items, in their order
     __shared__ float red[kWaves][C + 1];
 
     clear_small_accumulators(a.clear);
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const TilePixel px = tile_pixel(a.tiles, a.ly);
     const int l        = px.l;
+    const int lw = a.ly.w[l], lh = a.ly.h[l];
+    const size_t plane = (size_t)lw * lh;
+    const float* G     = a.grad_out[l];
+    auto sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     float bg_grad[C];
 #pragma unroll
     for (int ci = 0; ci < C; ++ci) bg_grad[ci] = 0.f;
     float leak = 0.f;
     uint32_t off = 0, n = 0;
-
+    float g[4] = {0.f, 0.f, 0.f, 0.f}, Tn = 0.f;
     if (px.active)
     {
-        const int lw = a.ly.w[l], lh = a.ly.h[l];
-        const size_t plane   = (size_t)lw * lh;
-        const uint32_t local = px.local;
-        const float* G       = a.grad_out[l];
-        float g[4]           = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ci = 0; ci < C; ++ci) g[ci] = G[ci * plane + local];
+        // the list first: the fragments' keys are asked for while what else the pixel needs is under way
         off = a.offsets[px.q];
         if constexpr (BILINEAR)
             n = a.kept[px.q];
         else
+            n = a.offsets[px.q + 1];
+#pragma unroll
+        for (int ci = 0; ci < C; ++ci) g[ci] = G[ci * plane + px.local];
+        Tn = a.weight[px.q];
+        if constexpr (!BILINEAR)
         {
-            n = a.offsets[px.q + 1] - off;
+            n -= off;
             if (a.K > 0) n = min(n, (uint32_t)a.K);
         }
+    }
+    const bool do_point = !BILINEAR && a.need_point_gradient && n > 0 && interior_pixel(px.x, px.y, lw, lh);
 
+    // What a pixel needs besides its fragments; with the 2x2 splat while the first fragments' keys are under way.
+    auto prepare_pixel = [&] {
+        if (!px.active) return;
+        const uint32_t local = px.local;
         float S = 0.f;
-        const float Tn = a.use_environment_map ? 0.f : a.weight[px.q];
         // BILINEAR_BLEND leaves the background out once the transmittance is below 0.001 (RenderBackward.cu:3014-3019:
-        // the loop stops before the background element)
-        if (!a.use_environment_map && !(BILINEAR && (double)Tn < 0.001))
+        // the loop stops before the background element; compared in double there, which comes out the same for every T, see
+        // blend_is_saturated)
+        if (!a.use_environment_map && !(BILINEAR && Tn < 0.001f))
         {
-            float dot      = 0.f;
+            float dot = 0.f;
 #pragma unroll
             for (int ci = 0; ci < C; ++ci)
             {
@@ -164,11 +184,8 @@ __device__ __forceinline__ void blend_backward(const BackwardPass& a)
             }
             if (!BILINEAR && a.quirk_background_confidence_leak) leak = dot * Tn;
         }
-        const bool do_point = !BILINEAR && a.need_point_gradient && n > 0 && interior_pixel(px.x, px.y, lw, lh);
-        s_off[wave][lane]   = off;
         s_carry[wave][lane] = S;
         s_g[wave][lane]     = make_float4(g[0], g[1], g[2], g[3]);
-        s_point[wave][lane] = do_point ? 1 : 0;
         if (do_point)
         {
             // The reference evaluates, per fragment with descriptor t and per channel,
@@ -194,20 +211,20 @@ __device__ __forceinline__ void blend_backward(const BackwardPass& a)
             s_ay[wave][lane]  = make_float4(ay[0], ay[1], ay[2], ay[3]);
             s_bxy[wave][lane] = make_float2(bx, by);
         }
-    }
+    };
 
     // ---- fragments: windows of kWindow per pixel, deepest window first ------------------------------------------
-    uint32_t max_n = n;
-#pragma unroll
-    for (int d = kWave / 2; d >= 1; d >>= 1) max_n = max(max_n, (uint32_t)__shfl_xor((int)max_n, d, kWave));
-    float4* partial_l = a.partial;  // (records are addressed by gradient_record)
-    // (all pixels of the wave: whole cache lines)
-    if (BILINEAR && max_n > 0u && px.active) a.pixel_gradient[px.q] = s_g[wave][lane];
+    const uint32_t max_n = wave_max(n);
+    float4* partial_l    = a.partial;  // (records are addressed by gradient_record)
+    // (With one hit per layer the pixel first: its 32 neighbour samples beside the fragments' keys take 116 registers, and two
+    // thirds of the waves are gone: benchmark frame 103 us against 94.)
+    bool prepared = !BILINEAR;
+    if constexpr (!BILINEAR) prepare_pixel();
     // Windows run from the deepest list places to the nearest. Where only a few pixels of the wave still have fragments
     // that deep (uncut lists of hundreds of fragments at a handful of pixels), a window of 16 places would fill a
     // quarter of the lanes or less and every window costs a dependent chain of memory round trips, so the window is
-    // widened to 64 places (at most 16 pixels reach into it) or 256 places (at most 4): the item table never holds
-    // more than kWaveItems entries.
+    // widened to 64 places (at most 16 pixels reach into it) or 256 places (at most 4): there are never
+    // more than kWaveItems items.
     for (uint32_t top = (max_n + kWindow - 1) / kWindow * kWindow; top > 0;)
     {
         uint32_t width = kWindow;
@@ -217,101 +234,116 @@ __device__ __forceinline__ void blend_backward(const BackwardPass& a)
             if (top >= 16u * kWindow && __popcll(__ballot(n + 16u * kWindow > top)) <= kWave / 16) width = 16u * kWindow;
         }
         top -= width;
+        // The items of a window: its fragments, pixel after pixel from the wave's last lane to its first, each pixel's from the
+        // deepest on, so that the sum over the deeper ones is a sum over the lanes below. A bit marks where a pixel's items
+        // start, and an item finds its pixel by counting the bits up to it: a bit per pixel and two instructions per step,
+        // where a table of the items took a store for every one of them, one lane's after the other.
         const uint32_t jw = top;
         const uint32_t nw = (n > jw) ? min(n - jw, width) : 0u;
-        const uint32_t incl = wave_inclusive_scan(nw, lane);
-        const uint32_t base  = incl - nw;
-        const uint32_t total = __shfl(incl, kWave - 1, kWave);
-        s_base[wave][lane]   = base;
-        for (uint32_t j = 0; j < nw; ++j) s_item[wave][base + j] = (uint8_t)lane;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-        // BILINEAR_BLEND asks for the key and the transmittance of a step's fragments one step ahead: they only depend
-        // on the item table, and the step's own chain (key -> descriptor record and position -> arithmetic -> store)
-        // is then one memory round trip shorter (per-pixel backward kernel of a 1080p frame 247 -> 237 us). With one
-        // fragment per point and layer it gains nothing at one view and costs 4 % at four (measured), so there the
-        // step asks for its own.
-        int p_next = -1;
-        uint32_t low_next = 0;
-        float T_next      = 0.f;
-        auto fetch = [&](int k0) {
-            const uint32_t k = (uint32_t)k0 + lane;
-            p_next           = k < total ? (int)s_item[wave][k] : -1;  // lane of the pixel this fragment belongs to
-            if (p_next >= 0)
-            {
-                const uint32_t pos = s_off[wave][p_next] + jw + (k - s_base[wave][p_next]);
-                low_next           = (uint32_t)a.fragments[pos];
-                T_next             = a.transmittance[pos];
-            }
-        };
-        const int k_first = total > 0 ? (int)((total - 1) / kWave) * kWave : -1;
-        if (BILINEAR && k_first >= 0) fetch(k_first);
-        for (int k0 = k_first; k0 >= 0; k0 -= kWave)
+        const uint32_t incl  = wave_inclusive_scan(nw, lane);
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        const uint32_t first = total - incl;
+        const uint64_t some  = __ballot(nw > 0u);
+        sync();
+        if (lane < kWaveItems / 32) s_starts[wave][lane] = 0u;
+        s_place[wave][lane] = make_uint2(off + jw + nw - 1u + first, first | (do_point ? 0x80000000u : 0u));
+        sync();
+        if (nw > 0u)
         {
-            if constexpr (!BILINEAR) fetch(k0);
-            const int p        = p_next;
-            const bool valid   = p >= 0;
-            const uint32_t low = low_next;
-            float x = 0.f, T = T_next, c = 0.f, dot = 0.f;
-            if (BILINEAR && k0 >= kWave) fetch(k0 - kWave);
-            float t[4] = {0.f, 0.f, 0.f, 0.f};
-            float4 g4  = make_float4(0.f, 0.f, 0.f, 0.f);
-            int id = -1, ti = -1, corner = 0;
-            if (valid)
-            {
-                id                 = BILINEAR ? (int)(low >> 2) : (int)low;
-                corner             = BILINEAR ? (int)(low & 3u) : 0;
-                // guards the gathers; never false for a workspace the forward pass wrote
-                if ((uint32_t)id < (uint32_t)a.N) ti = a.index ? a.index[id] : id;
-                if ((uint32_t)ti >= (uint32_t)a.N) ti = -1;
-                g4 = s_g[wave][p];
-            }
-            if (ti >= 0)
-            {
-                const float4 t4 = a.packed[2 * (size_t)ti];
-                c               = a.packed[2 * (size_t)ti + 1].x;
-                if constexpr (BILINEAR)
-                {
-                    // alpha = bilinear weight of this pixel's corner at the point's position in this layer x confidence;
-                    // the position is the one the scatter pass stored for the forward blend
-                    const float2 ip = a.projected[id];
-                    float u = ip.x, v = ip.y;
-                    for (int h = 0; h < l; ++h) u *= 0.5f, v *= 0.5f;
-                    c = bilinear_weight(u, v, corner) * c;
-                }
-                t[0] = t4.x, t[1] = t4.y, t[2] = t4.z, t[3] = t4.w;
-                const float g[4] = {g4.x, g4.y, g4.z, g4.w};
-#pragma unroll
-                for (int ci = 0; ci < C; ++ci)
-                {
-                    dot += t[ci] * g[ci];
-                    x += ((g[ci] * t[ci]) * T) * c;
-                }
-            }
-            // suffix sum over the fragments of the same pixel that sit in higher lanes of this step. The fragments of a
-            // pixel are neighbouring lanes: `last` is the end of this lane's run, found from the mask of run starts, so
-            // that the scan steps only have to move the sums.
-            const int pp         = __shfl_up(p, 1, kWave);
-            const bool head      = lane == 0 || pp != p;
-            const uint64_t heads = __ballot(head);
-            const uint64_t above = lane == kWave - 1 ? 0ull : heads >> (lane + 1);
-            const int last       = above != 0ull ? lane + __ffsll((unsigned long long)above) - 1 : kWave - 1;
-            float v = x;
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1)
-            {
-                const float o = __shfl_down(v, d, kWave);
-                if (lane + d <= last) v += o;
-            }
-            const float vn = __shfl_down(v, 1, kWave);
-            float S        = lane < last ? vn : 0.f;                     // deeper fragments of this step
-            if (valid) S += s_carry[wave][p];                            // and of the steps / windows before
-            if (valid && head) s_carry[wave][p] += v;                    // one lane per pixel moves the carry on
+            const uint32_t before = __builtin_amdgcn_mbcnt_hi((uint32_t)(some >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some, 0u));
+            s_order[wave][__popcll(some) - 1 - (int)before] = (uint8_t)lane;
+            atomicOr(&s_starts[wave][first / 32u], 1u << (first % 32u));
+        }
+        sync();
+
+        // A step asks for the keys and the transmittances of the next step's fragments before it asks for its own descriptor
+        // records: they depend on the item order only, so that a step waits for one memory round trip. Loads are not put under
+        // conditions (lanes without an item read place 0 of the lists), since behind a branch the compiler no longer knows how
+        // many are under way and waits for all of them, stores too.
+        uint32_t pixels_before = 0;  // pixels whose items started in front of the step
+        uint32_t next_low = 0;
+        int next_p        = 0;
+        uint2 next_place  = make_uint2(0u, 0u);
+        uint64_t next_starts = 0ull;
+        float next_T         = 0.f;
+        auto fetch = [&](uint32_t r0) {
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_starts[wave][r0 / 32u]);
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_starts[wave][r0 / 32u + 1u]);
+            next_starts       = ((uint64_t)hi << 32) | lo;
+            const uint64_t above = next_starts >> 1;  // (a lane's own bit counts too)
+            const uint32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)(above >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)above, pixels_before + (lo & 1u) - 1u));
+            pixels_before += (uint32_t)__popcll(next_starts);
+            next_p             = s_order[wave][k];
+            next_place         = s_place[wave][next_p];
+            const uint32_t r   = r0 + (uint32_t)lane;
+            const uint32_t pos = r < total ? next_place.x - r : 0u;
+            next_low           = (uint32_t)a.fragments[pos];
+            next_T             = a.transmittance[pos];
+        };
+        fetch(0u);  // (a window has items)
+        if (!prepared)
+        {
+            prepare_pixel();
+            prepared = true;
+            sync();
+            // (all pixels of the wave: whole cache lines)
+            if (BILINEAR && px.active) a.pixel_gradient[px.q] = make_float4(g[0], g[1], g[2], g[3]);
+        }
+        for (uint32_t r0 = 0; r0 < total; r0 += kWave)
+        {
+            const uint32_t low = next_low, r = r0 + (uint32_t)lane;
+            const uint2 place  = next_place;
+            const float T      = next_T;
+            const int p        = next_p;  // lane of the pixel this fragment belongs to
+            const bool valid   = r < total;
+            // lanes that hold a pixel's last item of this step
+            const uint64_t ends = (next_starts >> 1) | (1ull << 63) | (total - r0 <= (uint32_t)kWave ? 1ull << (total - r0 - 1u) : 0ull);
+            if (r0 + kWave < total) fetch(r0 + kWave);
+            const int id     = BILINEAR ? (int)(low >> 2) : (int)low;
+            const int corner = BILINEAR ? (int)(low & 3u) : 0;
+            // guards the gathers; never below 0 for a workspace the forward pass wrote
+            const int ti     = texture_row(a.index, id, a.N);
+            const bool there = valid && ti >= 0;
+            const size_t row = (size_t)max(ti, 0);
+            const float4 t4  = a.packed[2 * row];
+            float c          = a.packed[2 * row + 1].x;
             if constexpr (BILINEAR)
             {
-                if (ti >= 0)
+                // alpha = bilinear weight of this pixel's corner at the point's position in this layer x confidence;
+                // the position is the one the scatter pass stored for the forward blend
+                const float2 ip = a.projected[ti >= 0 ? id : 0];
+                float u = ip.x, v = ip.y;
+                for (int h = 0; h < l; ++h) u *= 0.5f, v *= 0.5f;
+                c = bilinear_weight(u, v, corner) * c;
+            }
+            const float4 g4   = s_g[wave][p];
+            const float t[4]  = {t4.x, t4.y, t4.z, t4.w};
+            const float gp[4] = {g4.x, g4.y, g4.z, g4.w};
+            const float carry = s_carry[wave][p];
+            float x = 0.f, dot = 0.f;
+#pragma unroll
+            for (int ci = 0; ci < C; ++ci)
+            {
+                dot += t[ci] * gp[ci];
+                x += ((gp[ci] * t[ci]) * T) * c;
+            }
+            // sum over the fragments of the same pixel in the lanes up to this one, in moves between registers: inside a row of
+            // 16 lanes, then from the last lane of a row to the next one, then from the lower half to the upper one
+            const uint32_t back = min(r - (place.y & 0x7FFFFFFFu), (uint32_t)lane);  // lanes below that belong to the pixel
+            float v = there ? x : 0.f;
+            auto add = [&](uint32_t from, bool same) { v += same ? __uint_as_float(from) : 0.f; };
+            add(dpp_shifted<0x111, 0xF>(__float_as_uint(v)), back >= 1u);
+            add(dpp_shifted<0x112, 0xF>(__float_as_uint(v)), back >= 2u);
+            add(dpp_shifted<0x114, 0xF>(__float_as_uint(v)), back >= 4u);
+            add(dpp_shifted<0x118, 0xF>(__float_as_uint(v)), back >= 8u);
+            add(dpp_shifted<0x142, 0xA>(__float_as_uint(v)), back > (uint32_t)(lane & 15));
+            add(dpp_shifted<0x143, 0xC>(__float_as_uint(v)), back > (uint32_t)(lane & 31));
+            const float below = lane_below(v);
+            const float S     = carry + (back > 0u ? below : 0.f);  // the deeper fragments of this step, and of those before
+            if (valid && (ends >> lane & 1ull) != 0ull) s_carry[wave][p] = carry + v;  // one lane per pixel moves the carry on
+            if constexpr (BILINEAR)
+            {
+                if (there)
                 {
                     const float galpha = dot * T - S / ((1.f - c) + 1e-9f);
                     reinterpret_cast<float2*>(partial_l)[4 * gradient_record(a.point_major_records, a.N, a.ly.L, l, id) + corner] = make_float2(T * c, galpha);
@@ -319,56 +351,48 @@ __device__ __forceinline__ void blend_backward(const BackwardPass& a)
             }
             else
             {
-                float4 rec_lo = make_float4(0.f, 0.f, 0.f, 0.f), rec_hi = rec_lo;
-                if (ti >= 0)
+                const float Tc     = T * c;
+                const float galpha = dot * T - S / ((1.f - c) + 1e-9f);
+                float gp0 = 0.f, gp1 = 0.f;
+                if (place.y & 0x80000000u)
                 {
-                    const float g[4]  = {g4.x, g4.y, g4.z, g4.w};
-                    const float Tc     = T * c;
-                    const float galpha = dot * T - S / ((1.f - c) + 1e-9f);
-                    float gp0 = 0.f, gp1 = 0.f;
-                    if (s_point[wave][p])
+                    const float4 ax4 = s_ax[wave][p], ay4 = s_ay[wave][p];
+                    const float2 b2  = s_bxy[wave][p];
+                    const float ax[4] = {ax4.x, ax4.y, ax4.z, ax4.w}, ay[4] = {ay4.x, ay4.y, ay4.z, ay4.w};
+                    float dR_dpx = b2.x, dR_dpy = b2.y;
+#pragma unroll
+                    for (int ci = 0; ci < C; ++ci)
                     {
-                        const float4 ax4 = s_ax[wave][p], ay4 = s_ay[wave][p];
-                        const float2 b2  = s_bxy[wave][p];
-                        const float ax[4] = {ax4.x, ax4.y, ax4.z, ax4.w}, ay[4] = {ay4.x, ay4.y, ay4.z, ay4.w};
-                        float dR_dpx = b2.x, dR_dpy = b2.y;
-#pragma unroll
-                        for (int ci = 0; ci < C; ++ci)
-                        {
-                            dR_dpx += t[ci] * ax[ci];
-                            dR_dpy += t[ci] * ay[ci];
-                        }
-                        gp0 = dR_dpx / (float)C;  // image-space gradient of this fragment at the layer's resolution;
-                        gp1 = dR_dpy / (float)C;  // the per-point kernel pushes it through the projection Jacobian
+                        dR_dpx += t[ci] * ax[ci];
+                        dR_dpy += t[ci] * ay[ci];
                     }
-                    float gt[4] = {0.f, 0.f, 0.f, 0.f};
+                    gp0 = dR_dpx / (float)C;  // image-space gradient of this fragment at the layer's resolution;
+                    gp1 = dR_dpy / (float)C;  // the per-point kernel pushes it through the projection Jacobian
+                }
+                float gt[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int ci = 0; ci < C; ++ci) gt[ci] = Tc * g[ci];
-                    rec_lo = make_float4(gt[0], gt[1], gt[2], gt[3]);
-                    rec_hi = make_float4(galpha, gp0, gp1, 0.f);
-                }
-                {
-                    // Record stores, two lanes per record: first the even lane's record (even lane its low half, odd lane
-                    // the high half), then the odd lane's, so that each instruction issues one 32-byte request per record.
-                    const int odd        = lane & 1;
-                    const int own        = ti >= 0 ? (int)gradient_record(a.point_major_records, a.N, a.ly.L, l, id) : -1;
-                    const int other      = pair_other(own);
-                    const float4 o_lo    = pair_other(rec_lo);
-                    const float4 o_hi    = pair_other(rec_hi);
-                    const int id_first   = odd ? other : own;
-                    const int id_second  = odd ? own : other;
-                    const float4 v_first = odd ? o_hi : rec_lo;
-                    const float4 v_second = odd ? rec_hi : o_lo;
-                    // own/other are record numbers
-                    if (id_first >= 0) partial_l[2 * (size_t)id_first + odd] = v_first;
-                    if (id_second >= 0) partial_l[2 * (size_t)id_second + odd] = v_second;
-                }
+                for (int ci = 0; ci < C; ++ci) gt[ci] = Tc * gp[ci];
+                const float4 rec_lo = make_float4(gt[0], gt[1], gt[2], gt[3]);
+                const float4 rec_hi = make_float4(galpha, gp0, gp1, 0.f);
+                // Record stores, two lanes per record: first the even lane's record (even lane its low half, odd lane
+                // the high half), then the odd lane's, so that each instruction issues one 32-byte request per record.
+                const int odd        = lane & 1;
+                const int own        = there ? (int)gradient_record(a.point_major_records, a.N, a.ly.L, l, id) : -1;
+                const int other      = pair_other(own);
+                const float4 o_lo    = pair_other(rec_lo);
+                const float4 o_hi    = pair_other(rec_hi);
+                const int id_first   = odd ? other : own;
+                const int id_second  = odd ? own : other;
+                const float4 v_first = odd ? o_hi : rec_lo;
+                const float4 v_second = odd ? rec_hi : o_lo;
+                // own/other are record numbers
+                if (id_first >= 0) partial_l[2 * (size_t)id_first + odd] = v_first;
+                if (id_second >= 0) partial_l[2 * (size_t)id_second + odd] = v_second;
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            sync();
         }
     }
+    if (!prepared) prepare_pixel();  // (no list at all: only the background is left)
 
     // Every pixel adds to the same C background values. Atomics on one address serialise (the reference issues one per
     // pixel and channel, src/lib/rendering/RenderBackward.cu:1150-1152), so each workgroup reduces its 256 pixels and

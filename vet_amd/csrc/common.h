@@ -143,6 +143,21 @@ __device__ __forceinline__ int texture_row(const int32_t* index, int id, int N)
     return row;
 }
 
+// Value of the lane below, 0 where there is none. Every lane of the wave must be active.
+__device__ __forceinline__ float lane_below(float v)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x138, 0xF, 0xF, false));  // wave_shr:1
+}
+
+// Largest value over the lanes, the same in all of them.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v)
+{
+    v = max(v, dpp_shifted<0x111, 0xF>(v)), v = max(v, dpp_shifted<0x112, 0xF>(v));
+    v = max(v, dpp_shifted<0x114, 0xF>(v)), v = max(v, dpp_shifted<0x118, 0xF>(v));
+    v = max(v, dpp_shifted<0x142, 0xA>(v)), v = max(v, dpp_shifted<0x143, 0xC>(v));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, kWave - 1);
+}
+
 // Launch descriptor shared by the forward kernels of one view.
 // Several views of a call in one launch: the arguments of every view travel side by side as the kernel argument and
 // blockIdx.y (blockIdx.z where a kernel uses y itself) picks the view. Small views (training crops) leave most of the
