@@ -13,20 +13,29 @@
 
 namespace vetrast
 {
-// Small accumulators of the call (pose and intrinsics gradients and their counts) that have to start at zero: the first
-// workgroup of the first view's per-pixel kernel clears them, which is in front of every kernel that adds to them in
-// stream order and saves the launches of a fill kernel each.
+// Accumulators of the call that have to start at zero: the pose and intrinsics gradients and their counts, and with a texture
+// index the rows that points add to. The first view's per-pixel kernel, which is in front of every kernel that adds to them
+// in stream order, clears them in passing: its first workgroup the small ones, all of them the others. (A fill launch
+// takes 4.5 us and more each: two FUZZY_BLEND views with an index 21 us for four.)
+constexpr int kClearJobs          = 6;
+constexpr uint32_t kClearByOne    = 16384;  // words one workgroup clears
 struct ClearJob
 {
-    uint32_t* ptr[4];
-    uint32_t count[4];  // 32-bit words; 0 = nothing to clear
+    uint32_t* ptr[kClearJobs];
+    uint32_t count[kClearJobs];  // 32-bit words; 0 = nothing to clear
 };
-__device__ __forceinline__ void clear_small_accumulators(const ClearJob& job)
+__device__ __forceinline__ void clear_accumulators(const ClearJob& job)
 {
-    if (blockIdx.x != 0 || blockIdx.y != 0) return;
+    if (blockIdx.y != 0) return;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-        for (uint32_t i = threadIdx.x; i < job.count[k]; i += blockDim.x) job.ptr[k][i] = 0u;
+    for (int k = 0; k < kClearJobs; ++k)
+    {
+        if (job.count[k] == 0u) continue;
+        const bool shared = job.count[k] > kClearByOne;
+        if (!shared && blockIdx.x != 0) continue;
+        const size_t step = shared ? (size_t)gridDim.x * kBlock : (size_t)kBlock;
+        for (size_t i = (shared ? (size_t)blockIdx.x * kBlock : 0) + threadIdx.x; i < job.count[k]; i += step) job.ptr[k][i] = 0u;
+    }
 }
 
 struct BackwardPass
@@ -126,7 +135,7 @@ __device__ __forceinline__ void blend_backward(const BackwardPass& a)
     __shared__ uint8_t s_order[kWaves][kWave];              // lanes of the pixels that have items, in their order
     __shared__ float red[kWaves][C + 1];
 
-    clear_small_accumulators(a.clear);
+    clear_accumulators(a.clear);
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const TilePixel px = tile_pixel(a.tiles, a.ly);
     const int l        = px.l;
@@ -541,7 +550,7 @@ __device__ __forceinline__ void blend_backward_fuzzy(const BackwardPass& a, floa
     __shared__ float2 s_bxy[kWaves][kWave];
     __shared__ uint8_t s_item[kWaves][kWaveItems];
     __shared__ float red[kWaves][C + 3];
-    clear_small_accumulators(a.clear);
+    clear_accumulators(a.clear);
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const TilePixel px = tile_pixel(a.tiles, a.ly);
     float4* partial_l  = a.partial;  // (records are addressed by gradient_record)
@@ -1517,7 +1526,8 @@ struct GatherPass
     int view_count;
     size_t dropout_stride, flags_stride, last_key_stride, kept_stride;  // elements of the respective arrays
     size_t partial_stride, pixel_gradient_stride, background_rows_stride, camera_partial_stride;
-    int accumulate;  // 0: overwrite the gradient rows (the call's first round), 1: add to them (further rounds)
+    int accumulate;  // 0: overwrite the gradient rows (the call's first round), 1: add to them (further rounds); texture and
+                     // confidence rows behind an index are always added to
     // background gradient: workgroup 0 also sums the rows the per-pixel kernel left (hidden behind the other workgroups)
     const float* background_rows;
     int num_background_rows;
@@ -1609,9 +1619,13 @@ __device__ __forceinline__ double wave_sum_terms(const double (&term_values)[kCa
 // the hits of several layers (the four corners of one layer) go through these steps side by side. One hit per layer, two
 // layers at a time against one after the other: ten million points 255 -> 233 us, four town views 147 -> 135, benchmark frame 47 -> 44;
 // four at a time needs 85 registers and gives 243, 150 and 45. 2x2 splat at 1080p (with 8-byte records in both cases) 127 -> 96 us.
+// Further it does not go: all flags first and every hit's record without waiting for its key, one round trip for a layer, took
+// 97 instead of 87 thousand cycles for the benchmark frame, 828 instead of 528 for ten million points (16 of 39 million
+// records are wanted there), 368 instead of 291 for four town views, where nearly all are.
+// Registers for five waves of a SIMD unit: several views with the 2x2 splat would take 104 and four waves, 100 against 95 us.
 constexpr int kGatherLayers = 2;
 template <int C, int HITS, bool DISTORT = false, bool MANY = false>
-__global__ void __launch_bounds__(kBlock) gather_point_gradients_kernel(GatherPass a)
+__global__ void __launch_bounds__(kBlock, 5) gather_point_gradients_kernel(GatherPass a)
 {
     constexpr int kLayers = HITS == 1 ? kGatherLayers : 1, kSlots = kLayers * HITS;
     const int view_count = MANY ? a.view_count : 1;

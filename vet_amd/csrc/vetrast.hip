@@ -897,54 +897,36 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
 
     // The per-point kernel overwrites every gradient row in the first view, so the zeros_like fills of
     // PointRenderer.cu:267-277 are only needed where rows are added to with atomics: with a texture index
-    // indirection, where several points may share a row.
-    const bool add_to_rows = a->index != nullptr;
-    ClearJob clear          = {};
-    constexpr size_t kClearByKernel = 16384;  // words one workgroup clears in passing
+    // indirection, where several points may share a row. They and the pose and intrinsics accumulators are cleared by the
+    // first view's per-pixel kernel (ClearJob).
+    ClearJob clear = {};
     {
         ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_PREPARE);
-        auto zero = [&](float* ptr, size_t n) {
-            if (!ptr || n == 0) return;
-            hipLaunchKernelGGL(fill_u32_kernel, dim3(std::min(grid_for(n), 8192)), dim3(kBlock), 0, stream,
-                               reinterpret_cast<uint32_t*>(ptr), n, 0u);
-        };
-        // the pose and intrinsics accumulators: by the first view's per-pixel kernel where they are small (ClearJob)
-        const size_t pose_words = (size_t)12 * a->num_poses, camera_words = (size_t)13 * a->num_cameras;
-        if (g->grad_pose)
-        {
-            if (pose_words <= kClearByKernel)
+        int jobs  = 0;
+        auto zero = [&](void* ptr, size_t words) {
+            if (!ptr || words == 0) return;
+            if (words <= 0xFFFFFFFFull)
             {
-                clear.ptr[0] = reinterpret_cast<uint32_t*>(g->grad_pose), clear.count[0] = (uint32_t)pose_words;
-                clear.ptr[1] = reinterpret_cast<uint32_t*>(g->grad_pose_count), clear.count[1] = (uint32_t)a->num_poses;
+                clear.ptr[jobs]     = reinterpret_cast<uint32_t*>(ptr);
+                clear.count[jobs++] = (uint32_t)words;
             }
             else
-            {
-                zero(reinterpret_cast<float*>(g->grad_pose), pose_words);
-                zero(g->grad_pose_count, (size_t)a->num_poses);
-            }
+                hipLaunchKernelGGL(fill_u32_kernel, dim3(8192), dim3(kBlock), 0, stream, reinterpret_cast<uint32_t*>(ptr), words, 0u);
+        };
+        if (g->grad_pose)
+        {
+            zero(g->grad_pose, (size_t)12 * a->num_poses);
+            zero(g->grad_pose_count, (size_t)a->num_poses);
         }
         if (g->grad_intrinsics)
         {
-            if (camera_words <= kClearByKernel)
-            {
-                clear.ptr[2] = reinterpret_cast<uint32_t*>(g->grad_intrinsics), clear.count[2] = (uint32_t)camera_words;
-                clear.ptr[3] = reinterpret_cast<uint32_t*>(g->grad_intrinsics_count), clear.count[3] = (uint32_t)a->num_cameras;
-            }
-            else
-            {
-                zero(g->grad_intrinsics, camera_words);
-                zero(g->grad_intrinsics_count, (size_t)a->num_cameras);
-            }
+            zero(g->grad_intrinsics, (size_t)13 * a->num_cameras);
+            zero(g->grad_intrinsics_count, (size_t)a->num_cameras);
         }
-        if (add_to_rows)
+        if (a->index != nullptr)
         {
             zero(g->grad_texture, (size_t)C * N);
             zero(g->grad_confidence, (size_t)N);
-            if (g->grad_points)
-            {
-                zero(g->grad_points, (size_t)4 * N);
-                zero(g->grad_point_count, (size_t)N);
-            }
         }
     }
     // position, pose and intrinsics gradients all hang off the per-fragment image-space gradient
@@ -1118,7 +1100,7 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             gp.pixel_gradient_stride  = lay.lane_scratch_stride / sizeof(float4);
             gp.background_rows_stride = lay.lane_scratch_stride / sizeof(float);
             gp.camera_partial_stride  = camera_rows_bytes(N) / sizeof(double);
-            gp.accumulate          = (add_to_rows || first > 0) ? 1 : 0;
+            gp.accumulate          = first > 0 ? 1 : 0;
             gp.background_rows       = background_rows;
             // (with the folded rows of the FUZZY_BLEND kernel that takes a wave per list, where it ran)
             gp.num_background_rows   = background_rows_count;
