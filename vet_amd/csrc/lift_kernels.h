@@ -13,8 +13,11 @@
 //      literal ones, pixel for pixel.
 // Measured (146 k cells of 0.25 m, 1080p, 121 M covered pixels, the camera inside the grid): 0.87 ms per call with a test per
 // pixel (bound by its ~200 vector instructions per 64 pixels), 0.29 ms by rows (running sums 17 us, rows 213 us, the
-// cells next to the camera that are tested pixel by pixel 63 us); bound by the ~400 vector instructions per 64 rows and
-// the tests of open pixels.
+// cells next to the camera that are tested pixel by pixel 63 us). The rows need 37 M wave instructions a view of three 1080p
+// views of 176 k cells, 61 us, and took 138 us: 62 % of a wave's life was waiting, with 12 waves to a compute unit, as many as the
+// cells' bounds in LDS leave with 128 threads to 32 cells. Hence 256 threads, triangles
+// and outlines set up side by side, and waves that go through their rows without waiting for each other: 99 us. (16 cells with
+// 128 or 256 threads, 32 with 384 or 512: a fifth slower; 64 with 512: the same.)
 #pragma once
 #include "common.h"
 #include "forward_kernels.h"
@@ -23,9 +26,11 @@ namespace vetrast
 {
 constexpr int kLiftLargeCell    = 4096;  // boxes of more pixels are counted in the header (a diagnostic of the interface)
 constexpr int kLiftHeader       = 256;   // bytes: DeviceView (160), the count of large cells at 176, flag word at 192
-constexpr int kLiftBlock        = 128;   // threads of a workgroup of the cells kernel
-constexpr int kLiftCells        = 32;    // its cells, kLiftBlock / kLiftCells threads each in the set-up
-constexpr int kLiftSetup        = kLiftBlock / kLiftCells;
+constexpr int kLiftBlock        = 256;   // threads of a workgroup of the cells kernel
+constexpr int kLiftCells        = 32;    // its cells
+constexpr int kLiftSetup        = 4;     // threads that set a cell's triangles up, and as many its outline
+constexpr int kLiftSetupAll     = kLiftCells * kLiftSetup;
+static_assert(kLiftSetupAll % kWave == 0 && kLiftBlock >= 2 * kLiftSetupAll, "triangles and outlines are set up by different waves");
 constexpr int kLiftTriangleMax  = 8;     // triangles that wind one way: three faces of a box, and one seen edge-on
 constexpr int kLiftOutlineMax   = 8;     // edges of the outline that are kept: a box shows 6 at most
 constexpr int kLiftSliverMax    = 8;     // thin triangles whose lines are looked at (the four side faces of a frontal box)
@@ -36,7 +41,7 @@ constexpr int kLiftPlainShare   = 128;   // workgroups that share such a cell
 constexpr int kLiftPlainAtOnce  = 8;     // cells in work at a time
 constexpr float kLiftThin       = 0.05f; // smallest angle (about) of a triangle that is not a sliver
 constexpr int kLiftOpen         = 8;     // open pixels of a row that go to the list; a row with more is left to a wave
-constexpr int kLiftOpenPixels   = 256;   // the list; it is worked off when half full (a lane tests what does not fit)
+constexpr int kLiftOpenPixels   = 128;   // the list of a wave; it is worked off when half full (a lane tests what does not fit)
 constexpr int kLiftOpenRows     = 128;   // such rows a workgroup keeps (a lane finishes what does not fit)
 // A cell whose open rows of more than kLiftWideRow columns add up to more than kLiftWideWork and more than one in
 // kLiftWideShare of its box's pixels is tested pixel by pixel by lift_plain_kernel: next to the camera the lines of slivers
@@ -95,16 +100,18 @@ __device__ __forceinline__ float lift_pixel_error(const LiftPass& a, int x, int 
     return grad;
 }
 
-// One workgroup of kLiftRows waves per group of kLiftRows rows: a wave scans its row 512 pixels at a time (8 per lane),
-// the 512 x 4 block goes through LDS so that the stores are whole 32-byte groups. The first workgroup of a call also
-// writes the camera constants of the view. Bound by the chain of steps along a row (1080p: 254 workgroups of 4 steps).
+// One workgroup of kLiftRows waves per group of kLiftRows rows: a wave scans its row 1024 pixels at a time (16 per lane),
+// the 1024 x 4 block goes through LDS so that the stores are whole 32-byte groups. The first workgroup of a call also
+// writes the camera constants of the view. Bound by the chain of steps along a row (1080p: 254 workgroups of 2
+// steps; of 4 steps of 512 pixels three views take 6 us more).
 constexpr int kLiftPrefixBlock = kLiftRows * kWave;
-constexpr int kLiftPerLane     = 8;
+constexpr int kLiftPerLane     = 16;
 constexpr int kLiftStep        = kLiftPerLane * kWave;
 __global__ void __launch_bounds__(kLiftPrefixBlock) lift_prefix_kernel(LiftPass a, ViewSource src, const double* __restrict__ poses_se3,
                                                                        const float* __restrict__ intrinsics)
 {
-    __shared__ double s_sum[kLiftStep * kLiftRows];
+    // (a place is left free behind a lane's, or all lanes would store to one bank)
+    __shared__ double s_sum[kLiftStep * kLiftRows + kWave];
     if (a.first && blockIdx.x == gridDim.x - 1 && threadIdx.x == kLiftPrefixBlock - 1)
     {
         bool distorted = false;
@@ -173,12 +180,12 @@ __global__ void __launch_bounds__(kLiftPrefixBlock) lift_prefix_kernel(LiftPass 
 #pragma unroll
         for (int k = 0; k < kLiftPerLane; ++k)
         {
-            s_sum[(kLiftPerLane * lane + k) * kLiftRows + wave] = before + p[k];
+            s_sum[(kLiftPerLane * lane + k) * kLiftRows + wave + lane] = before + p[k];
             dimmest = min(dimmest, __float_as_uint(g[k]) - 1u);  // (no error: the largest number)
         }
         __syncthreads();
         const int columns = min(kLiftStep, a.width - x0);
-        for (int k = threadIdx.x; k < columns * kLiftRows; k += kLiftPrefixBlock) group[(size_t)(x0 + 1) * kLiftRows + k] = s_sum[k];
+        for (int k = threadIdx.x; k < columns * kLiftRows; k += kLiftPrefixBlock) group[(size_t)(x0 + 1) * kLiftRows + k] = s_sum[k + k / (kLiftPerLane * kLiftRows)];
 #pragma unroll
         for (int k = 0; k < kLiftPerLane; ++k) g[k] = next[k];
     }
@@ -346,17 +353,23 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     __shared__ LiftCell s_cell[kLiftCells];
     __shared__ int s_start[kLiftCells + 1];  // rows of the cells in front
     __shared__ int4 s_open[kLiftOpenRows];   // slot, y, columns [z, w)
-    __shared__ uint2 s_pixel[kLiftOpenPixels];  // open pixels: x | slot << 24, y
-    __shared__ int s_num_open, s_num_pixels;
+    __shared__ uint2 s_pixel[kLiftBlock / kWave][kLiftOpenPixels];  // open pixels of a wave: x | slot << 24, y
+    __shared__ int s_num_open, s_num_pixels[kLiftBlock / kWave];
     __shared__ uint32_t s_large;
     __shared__ bool s_left[kLiftCells];  // the cell is lift_plain_kernel's
-    if (threadIdx.x == 0) s_num_open = s_num_pixels = 0, s_large = 0u;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    if (lane == 0) s_num_pixels[wave] = 0;
+    if (tid == 0) s_num_open = 0, s_large = 0u;
     __syncthreads();
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    // ---- set-up: kLiftSetup threads per cell. The workgroup's cells lie far apart in the grid (cells next to the camera
-    // cover hundreds of rows and are neighbours in it), so every workgroup gets about the same number of rows.
+    // ---- set-up: kLiftSetup threads per cell for its triangles, as many in other waves for its outline; both look at the box
+    // first. The workgroup's cells lie far apart in the grid (cells next to the camera cover hundreds of rows and are
+    // neighbours in it), so every workgroup gets about the same number of rows.
+    const bool outlines = tid >= kLiftSetupAll;  // the same in a wave
+    const int slot = tid / kLiftSetup % kLiftCells, part = tid % kLiftSetup;
+    bool seen      = false;
+    float raw_x0 = 0.f, raw_x1 = 0.f, raw_y0 = 0.f, raw_y1 = 0.f, bottom_y = 0.f, first_x = 0.f, last_x = 0.f;  // of the box
+    if (tid < 2 * kLiftSetupAll)
     {
-        const int slot = tid / kLiftSetup, part = tid % kLiftSetup;
         LiftCell& f        = s_cell[slot];
         const int64_t cell = (int64_t)slot * gridDim.x + blockIdx.x;
         const bool left    = !a.first && cell < a.num_cells && a.plain_state[cell] != 0u;  // by an earlier band
@@ -385,8 +398,7 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
                     behind = true;
                     continue;
                 }
-                f.px[i] = o.ipx;
-                f.py[i] = o.ipy;
+                if (!outlines) f.px[i] = o.ipx, f.py[i] = o.ipy;
                 max_x   = fmaxf(o.ipx, max_x);
                 max_y   = fmaxf(o.ipy, max_y);
                 min_x   = fminf(o.ipx, min_x);
@@ -409,18 +421,20 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         const float border = (float)a.border;
         const float right  = (float)(a.width - a.border);
         const float bottom = (float)(a.height - a.border);
-        const float raw_x0 = min_x, raw_x1 = max_x, raw_y0 = min_y, raw_y1 = max_y;
-        bool seen = !gone && !(max_x < border || min_x >= right || max_y < border || min_y >= bottom);
+        raw_x0 = min_x, raw_x1 = max_x, raw_y0 = min_y, raw_y1 = max_y;
+        seen      = !gone && !(max_x < border || min_x >= right || max_y < border || min_y >= bottom);
         min_x     = fmaxf(min_x, border);
         min_y     = fmaxf(min_y, border);
         max_x     = fminf(max_x, right);
         max_y     = fminf(max_y, bottom);
         const int x_size = seen ? (int)(max_x - min_x) : 0, y_size = seen ? (int)(max_y - min_y) : 0;
         seen             = x_size > 0 && y_size > 0;
-        const bool large = part == 0 && seen && x_size * y_size > kLiftLargeCell;
+        const bool large = !outlines && part == 0 && seen && x_size * y_size > kLiftLargeCell;
         const bool leaves = seen && plain;  // (in the first band: the corners say so)
         if (leaves) seen = false;
-        if (part == 0)
+        bottom_y = max_y;
+        if (seen) first_x = (float)(int)min_x, last_x = (float)(int)((float)(x_size - 1) + min_x);
+        if (!outlines && part == 0)
         {
             if (leaves) leave_to_plain_kernel(a, cell, 0.0);
             s_left[slot]  = leaves || left;
@@ -456,17 +470,18 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         }
         const uint64_t large_here = __ballot(large);
         if (a.first && large_here != 0ull && lane == 0) atomicAdd(&s_large, (uint32_t)__popcll(large_here));
-        // what the four threads of a cell wrote is read by each other below
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    __syncthreads();
+    {
+        LiftCell& f = s_cell[slot];
         if (seen)
         {
             // Rounding error of edge_sign at any pixel of the box: four roundings of two products, each bounded by the
             // extents; twice that.
-            const float xs = (float)f.xs, xe = (float)f.xe, ys = border > raw_y0 ? border : raw_y0;
+            const float border = (float)a.border;
+            const float xs = first_x, xe = last_x, ys = border > raw_y0 ? border : raw_y0;
             const float reach_x = fmaxf(fmaxf(raw_x1, xe) - fminf(raw_x0, xs), 1.f);
-            const float reach_y = fmaxf(fmaxf(raw_y1, max_y) - fminf(raw_y0, ys), 1.f) + 1.f;
+            const float reach_y = fmaxf(fmaxf(raw_y1, bottom_y) - fminf(raw_y0, ys), 1.f) + 1.f;
             const float err     = 16.f * 5.9604645e-8f * (2.f * reach_x * reach_y);
             // The same as a distance, and how far beyond a corner rounding can still see a triangle: the test accepts the
             // triangle with its edges moved out by `moved` at most, whose corners lie 2 / angle times as far out. That
@@ -480,6 +495,7 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
             {
                 const int t = part * (12 / kLiftSetup) + u;
                 // a triangle that winds one way, by enough: rows of pixels that are inside it whatever the rounding
+                if (!outlines)
                 {
                     const int swap = (kLiftInward >> t) & 1;
                     const int v[3] = {nibble(kLiftFirst, t), nibble(swap ? kLiftThird : kLiftSecond, t), nibble(swap ? kLiftSecond : kLiftThird, t)};
@@ -559,6 +575,7 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
                     }
                 }
                 // a box edge with all corners on one side of it: part of the outline, moved out past every corner
+                else
                 {
                     const int i = nibble(kLiftEdgeFrom, t), j = nibble(kLiftEdgeTo, t);
                     const float bx = f.px[j], by = f.py[j], c1 = f.py[i] - by, dx = f.px[i] - bx;
@@ -723,13 +740,13 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         }
         if (open > 0)
         {
-            const int at = atomicAdd(&s_num_pixels, open);
+            const int at = atomicAdd(&s_num_pixels[wave], open);
 #pragma unroll
             for (int k = 0; k < kLiftOpen; ++k)
                 if (k < open)
                 {
                     if (at + k < kLiftOpenPixels)
-                        s_pixel[at + k] = make_uint2(open_x[k] | ((uint32_t)slot << 24), (uint32_t)y);
+                        s_pixel[wave][at + k] = make_uint2(open_x[k] | ((uint32_t)slot << 24), (uint32_t)y);
                     else
                         test_pixel(f, (int)open_x[k], y);
                 }
@@ -740,25 +757,31 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
             atomicAdd(&f.sum, sum);
         }
     };
-    for (int r0 = 0; r0 < total; r0 += kLiftBlock)
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    for (int r0 = wave * kWave; r0 < total; r0 += kLiftBlock)
     {
-        if (r0 + tid < total) do_row(r0 + tid);
-        __syncthreads();
-        const int pixels = s_num_pixels;
+        if (r0 + lane < total) do_row(r0 + lane);
+        wave_sync();
+        const int pixels = s_num_pixels[wave];
         if (pixels >= kLiftOpenPixels / 2 || (r0 + kLiftBlock >= total && pixels > 0))
         {
-            for (int k = tid; k < min(pixels, kLiftOpenPixels); k += kLiftBlock)
+            for (int k = lane; k < min(pixels, kLiftOpenPixels); k += kWave)
             {
-                const uint2 v = s_pixel[k];
+                const uint2 v = s_pixel[wave][k];
                 test_pixel(s_cell[v.x >> 24], (int)(v.x & 0xFFFFFFu), (int)v.y);
             }
-            __syncthreads();
-            if (tid == 0) s_num_pixels = 0;
+            wave_sync();
+            if (lane == 0) s_num_pixels[wave] = 0;
         }
-        __syncthreads();
+        wave_sync();
     }
+    __syncthreads();
     // ---- rows with many open pixels (next to the line of a face seen edge-on, in cells that touch the camera plane)
-    for (int k = tid / kWave; k < min(s_num_open, kLiftOpenRows); k += kLiftBlock / kWave)
+    for (int k = wave; k < min(s_num_open, kLiftOpenRows); k += kLiftBlock / kWave)
     {
         const int4 row = s_open[k];
         LiftCell& f    = s_cell[row.x];
