@@ -40,11 +40,7 @@ struct vetrast_ctx
 namespace
 {
 constexpr size_t kAlign = 256;
-// Layers that blend at least this many fragments per pixel (a bound: all points inside the view) are split. From 4 on: the finest
-// layer of ten million points (4.8) gains, 1730 -> 1695 us the step; from 2 on the 2x2 splat at 1080p (3.9, nearly half of it
-// outside the view) loses 592 -> 604 and four town views (2.7, a tenth of it seen) 947 -> 1229. Sixteen parts instead of four
-// where the bound is 16: benchmark frame 292 -> 286, four 512x512 crops 411 -> 526.
-constexpr double kSplitListLength = 4.0;
+constexpr double kSplitListLength = 8.0;  // layers that blend at least this many fragments per pixel are split
 inline size_t align_up(size_t v, size_t a)
 {
     return (v + a - 1) / a * a;
