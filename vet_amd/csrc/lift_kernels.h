@@ -12,12 +12,12 @@
 //      by more than that are left out, and the few in between get the literal test of the reference. The counts are the
 //      literal ones, pixel for pixel.
 // Measured (146 k cells of 0.25 m, 1080p, 121 M covered pixels, the camera inside the grid): 0.87 ms per call with a test per
-// pixel (bound by its ~200 vector instructions per 64 pixels), 0.29 ms by rows (running sums 17 us, rows 213 us, the
-// cells next to the camera that are tested pixel by pixel 63 us). The rows need 37 M wave instructions a view of three 1080p
-// views of 176 k cells, 61 us, and took 138 us: 62 % of a wave's life was waiting, with 12 waves to a compute unit, as many as the
-// cells' bounds in LDS leave with 128 threads to 32 cells. Hence 256 threads, triangles
-// and outlines set up side by side, and waves that go through their rows without waiting for each other: 99 us. (16 cells with
-// 128 or 256 threads, 32 with 384 or 512: a fifth slower; 64 with 512: the same.)
+// pixel (bound by its ~200 vector instructions per 64 pixels), 0.22 ms by rows (running sums 13 us, rows 143 us, the
+// cells next to the camera that are tested pixel by pixel 63 us). The rows take 37 M wave instructions a view of three 1080p
+// views of 176 k cells, 61 us of them, and took 138 us: a wave waited 62 % of its life, with 12 waves on a compute unit, as
+// many as the cells' bounds in LDS leave with 128 threads to 32 cells. Hence 256 threads, triangles and outlines set up
+// side by side, and waves that go through their rows without waiting for each other: 99 us. (16 cells with 128 or 256
+// threads, 32 with 384 or 512: a fifth slower; 64 with 512: the same.)
 #pragma once
 #include "common.h"
 #include "forward_kernels.h"
