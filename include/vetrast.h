@@ -193,8 +193,8 @@ typedef struct vetrast_workspace_layout
     size_t flags_base;     /* uint32 [4] device status flags, then at +64 bytes float [4]: the background as it is blended */
     size_t forward_only_bytes; /* a forward call with save_for_backward = 0 needs only this much */
     size_t partial_base;   /* float [L][N][8]: backward scratch, gradient record of the fragment of point i in layer l (with
-                              the 2x2 splat float [L][N][4][2]); behind room for 32 bytes per fragment follows
-                              float [P][4], the upstream gradient with its channels side by side */
+                              the 2x2 splat float [L][N][4][2], behind which follows float [P][4], the upstream gradient
+                              with its channels side by side) */
     size_t background_partial_base; /* float [workgroups][8]: backward scratch, per-workgroup background-gradient sums */
     size_t camera_partial_base;     /* double [ceil(N/256)][12]: backward scratch, per-workgroup pose / intrinsics sums */
     /* scratch shared by all views: the scatter pass writes the records of a bin to the bin's own room while their rank

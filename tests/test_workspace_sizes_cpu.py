@@ -1,0 +1,29 @@
+"""The backward scratch of the workspace: 32 bytes for a point and layer in every mode (the four corners of the 2x2 splat share
+them) and, with the 2x2 splat only, a float4 for every pixel behind them; there the block is no smaller than 32 bytes for each
+corner, and no larger unless the pixels do not fit into what the corners leave."""
+import ctypes as C
+
+import pytest
+
+from vet_amd import abi
+
+
+def _align(n):
+    return (n + 255) // 256 * 256
+
+
+@pytest.mark.parametrize("mode", [abi.RENDER_FULL_BLEND, abi.RENDER_FUZZY_BLEND, abi.RENDER_BILINEAR_BLEND])
+@pytest.mark.parametrize("points,views,layers,w,h", [(0, 1, 1, 16, 16), (1, 1, 4, 17, 33), (60_007, 1, 4, 203, 155), (2_000_000, 4, 4, 512, 512),
+                                                     (5_000_001, 2, 5, 1920, 1080)])
+def test_backward_scratch(mode, points, views, layers, w, h):
+    lay = abi.WorkspaceLayout()
+    assert abi.load_library().vetrast_workspace_layout_for_mode(points, views, layers, w, h, mode, C.byref(lay)) == 0
+    pixels = 256 * lay.layer_tile_base[layers]
+    want = _align(points * layers * 32)
+    if mode == abi.RENDER_BILINEAR_BLEND:
+        want = max(want + pixels * 16, _align(4 * points * layers * 32))
+    assert lay.background_partial_base - lay.partial_base == want
+    # what is folded into the records' place behind the per-point kernel: 64 rows of 160 bytes for each view of a round, where there
+    # are more than 256 workgroups of points
+    if points > 256 * 256:
+        assert points * layers * 32 >= lay.view_lanes * 64 * 160

@@ -381,7 +381,7 @@ __device__ __forceinline__ float4 pair_other(float4 v)
 // With one hit per layer the same exchange of bytes for a gather does not pay: ten million points 541 -> 491 us in the per-pixel
 // kernel, but 255 -> 289 in the per-point kernel, where the 64 points of a wave find the pixels' upstream gradients in as many
 // cache lines; benchmark frame 115 -> 107 and 47 -> 56, four town views 400 -> 396 and 147 -> 174.
-constexpr int kRecordRoom = 32;  // bytes the workspace keeps for the record of a fragment
+constexpr int kRecordRoom = 32;  // bytes the workspace keeps for the record(s) of a point in a layer
 
 // Place of the record(s) of point id in layer l, in units of 32 bytes. Two layouts, chosen per call on the host. Layer after layer
 // ([layer][point]): the per-point kernel, which walks the points in order, reads every layer's records as one

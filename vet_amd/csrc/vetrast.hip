@@ -281,10 +281,11 @@ size_t camera_rows_bytes(int64_t N)
     return align_up(((size_t)N + kBlock - 1) / kBlock * kCameraRow * sizeof(double), kAlign);
 }
 
-// The upstream gradient with the channels side by side (BackwardPass::pixel_gradient), [P] float4 behind the gradient records.
+// With the 2x2 splat the upstream gradient with the channels side by side (BackwardPass::pixel_gradient), [P] float4, lies
+// behind the gradient records, which take kRecordRoom bytes for a point and layer whatever the number of hits.
 size_t pixel_gradient_base(const vetrast_workspace_layout& lay)
 {
-    return align_up(lay.partial_base + (size_t)lay.fragment_capacity * kRecordRoom, kAlign);
+    return align_up(lay.partial_base + (size_t)lay.fragment_capacity / (size_t)lay.hits_per_layer * kRecordRoom, kAlign);
 }
 
 TileMap make_tile_map(const LayerTable& ly, const double* list_bound = nullptr, bool split_all = false)
@@ -595,7 +596,9 @@ int vetrast_workspace_layout_for_mode(int32_t N, int32_t B, int32_t L, int32_t w
     const size_t forward_block = align_up(at, kAlign) - shared_base;
     at                         = shared_base;
     lay->partial_base          = at;
-    at = pixel_gradient_base(*lay) + P * sizeof(float4);
+    at = pixel_gradient_base(*lay) + (hits == 4 ? P * sizeof(float4) : 0);
+    // (the 2x2 splat's block is no smaller than a record for each corner would make it, which is what callers have reserved)
+    at = std::max(at, shared_base + align_up(cap * kRecordRoom, kAlign));
     lay->background_partial_base = at;
     // (the FUZZY_BLEND kernel that takes a wave per list keeps rows per replica and kFuzzyFoldRows rows they are folded into)
     at += align_up(((size_t)tile_grid(make_tile_map(t, nullptr, true)) * kFuzzyReplicas + kFuzzyFoldRows) * kBackgroundRow * sizeof(float), kAlign);
