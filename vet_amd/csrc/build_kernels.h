@@ -32,8 +32,10 @@ static_assert(kPrimaryCapSmall >= kBuildCap, "a bin built in LDS must find all i
 constexpr uint32_t kBuildLongest = kBuildCap;  // a bin of more than kBuildCap records with a longer list goes through memory
 
 // Workgroups of a launch that go through the crowded bins, several each where there are more. One that finds no bin costs
-// a load, so there are no more of them than of the others; and at most twice what the compute units hold at a time, so that
-// one that is done early makes room for another.
+// a load, so there are no more of them than of the others, or than bins can be crowded at all; but where there are few bins,
+// as many as the compute units hold at a time, since all may be crowded (a hundred points a pixel in 64x64: with a workgroup to four
+// bins 84 us, with 1024 workgroups 44, with 2048 42). And at most twice that, so that one that is done early makes room for another.
+constexpr uint32_t kCrowdedAtOnce = 2048;
 constexpr uint32_t kCrowdedBlocks = 4096;
 
 struct BuildPass

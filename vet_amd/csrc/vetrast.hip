@@ -4,6 +4,7 @@
 // device->host reads, per-frame allocations and __constant__ uploads.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -273,6 +274,8 @@ size_t log_records(int64_t N, int L, int hits) { return (size_t)log_segment_reco
 // The list of crowded bins (CrowdedBins), behind the scan's partial sums: every bin, and once more for every further
 // workgroup that shares one. Its two counts are in unused words of the first log cursor's cache line, which every call clears.
 size_t crowded_list_entries(size_t bins, size_t fragments) { return bins + fragments / (kBuildCap / 4 * 3) + 1; }
+// Entries there can be at most: a bin with one has more than kWaveBinCap records, a part of a shared one more than 500.
+uint32_t crowded_entries_most(size_t fragments) { return (uint32_t)(fragments / (kWaveBinCap + 1)); }
 size_t log_cursor_bytes(int B) { return (size_t)B * kLogSegments * kLogCursorStride * sizeof(uint32_t); }
 
 // Per-workgroup pose / intrinsics rows one view's per-point backward pass leaves.
@@ -693,7 +696,7 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
     // bytes): with one view, and with several where the caller expects each to see little of the cloud.
     const bool rows_of_visible_points =
         a->index == nullptr && a->point_order == nullptr && (B == 1 || views_see_little(p, N, hits));
-    const uint32_t crowded_blocks = std::min<uint32_t>((bins + 3) / 4, kCrowdedBlocks);
+    const uint32_t crowded_blocks = std::min({kCrowdedBlocks, crowded_entries_most((size_t)lay.fragment_capacity), std::max((bins + 3) / 4, kCrowdedAtOnce)});
     for (int first = 0; first < B; first += lanes)
     {
         const int last = std::min(B, first + lanes), count = last - first;
