@@ -325,12 +325,16 @@ __device__ __forceinline__ void store_pixel(BuildArgs& args, const BinPlace& bin
     {
         const size_t plane   = (size_t)a.ly.w[l] * a.ly.h[l];
         const uint32_t local = (uint32_t)y * (uint32_t)a.ly.w[l] + (uint32_t)x;
-#pragma unroll
-        for (int ci = 0; ci < C; ++ci)
+        // The background comes from the scalar cache, the same for every pixel: as a vector load it was waited for together with all
+        // stores in front of it, for every channel of every 64 pixels.
+        if (!a.use_environment_map && !saturated)
         {
-            if (!a.use_environment_map && !saturated) color[ci] = (T * 1.f) * a.background[ci] + color[ci];
-            a.out[l][ci * plane + local] = color[ci];
+            const __attribute__((address_space(4))) float* background = (const __attribute__((address_space(4))) float*)a.background;
+#pragma unroll
+            for (int ci = 0; ci < C; ++ci) color[ci] = (T * 1.f) * background[ci] + color[ci];
         }
+#pragma unroll
+        for (int ci = 0; ci < C; ++ci) a.out[l][ci * plane + local] = color[ci];
         a.weight[q] = T;
         if (a.out_mask[l]) a.out_mask[l][local] = (T == 0.f) ? a.mask_value : 1.f;
         if (a.out_weight[l]) a.out_weight[l][local] = T;
