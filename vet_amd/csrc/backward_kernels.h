@@ -1612,8 +1612,8 @@ __device__ __forceinline__ double wave_sum_terms(const double (&term_values)[kCa
 // descriptor and confidence sums are added with atomics (onto rows the host zero-filled).
 // HITS = 4 (BILINEAR_BLEND): a point has up to four fragments per layer, one per corner of its 2x2 pixels.
 // MANY: the launch takes a round of several views (a.view_count of them); otherwise one view, and the loop over the
-// views and its address arithmetic fold away (the kernel then needs 58 registers instead of 71 to 77, and it lives
-// off the number of waves in flight).
+// views and its address arithmetic fold away (the kernel lives off the number of waves in flight: with four channels one
+// view needs 63 registers with one hit per layer and 86 with four, several 79 and 96).
 //
 // The kernel waits for memory, not for its bytes: a hit is a chain of a flag, a key where the flag says so, and a record, so
 // the hits of several layers (the four corners of one layer) go through these steps side by side. One hit per layer, two
@@ -1622,12 +1622,19 @@ __device__ __forceinline__ double wave_sum_terms(const double (&term_values)[kCa
 // Further it does not go: all flags first and every hit's record without waiting for its key, one round trip for a layer, took
 // 97 instead of 87 thousand cycles for the benchmark frame, 828 instead of 528 for ten million points (16 of 39 million
 // records are wanted there), 368 instead of 291 for four town views, where nearly all are.
-// Registers for five waves of a SIMD unit: several views with the 2x2 splat would take 104 and four waves, 100 against 95 us.
+// Registers: those of five waves of a SIMD unit. Several views with the 2x2 splat need two corners' upstream gradients at a time for
+// that: four crops 116 us; with all four at once 117 and 32 bytes a lane put off to memory, or 104 registers, four waves and 125.
+// Distortion's 16 more sums and the 2x2 splat together have the registers of four waves: with five, 60 bytes a lane went to memory
+// and came back in every layer for one view and 116 for several, 1080p 225 against 126 us, four crops 243 against 153. With
+// one hit per layer, distortion and several views five waves and 28 bytes are the better: four views of 960x540 182 against 195 us.
+constexpr int gather_waves(int hits, bool distort) { return hits == 4 && distort ? 4 : 5; }
 constexpr int kGatherLayers = 2;
 template <int C, int HITS, bool DISTORT = false, bool MANY = false>
-__global__ void __launch_bounds__(kBlock, 5) gather_point_gradients_kernel(GatherPass a)
+__global__ void __launch_bounds__(kBlock, gather_waves(HITS, DISTORT)) gather_point_gradients_kernel(GatherPass a)
 {
     constexpr int kLayers = HITS == 1 ? kGatherLayers : 1, kSlots = kLayers * HITS;
+    // corners whose pixels' upstream gradients are asked for together: all of them, or two where several views leave no registers
+    constexpr int kTogether = HITS == 1 ? 1 : (MANY && !DISTORT ? 2 : HITS);
     const int view_count = MANY ? a.view_count : 1;
     const int i      = blockIdx.x * blockDim.x + threadIdx.x;
     const bool alive = i < a.vp.N;
@@ -1717,7 +1724,7 @@ __global__ void __launch_bounds__(kBlock, 5) gather_point_gradients_kernel(Gathe
                 last[n] = kInfKey;
                 if (kept[n] && cut[n] && (HITS != 1 || a.K > 0)) last[n] = last_key[q[n]];
             }
-            float4 record[2 * kLayers], g4[HITS == 1 ? 1 : kSlots];
+            float4 record[2 * kLayers];
 #pragma unroll
             for (int k = 0; k < kLayers; ++k)
             {
@@ -1729,7 +1736,6 @@ __global__ void __launch_bounds__(kBlock, 5) gather_point_gradients_kernel(Gathe
                     const uint64_t key = depth_key | (HITS == 1 ? (uint32_t)i : (((uint32_t)i << 2) | (uint32_t)h));
                     kept[n]            = kept[n] && key <= last[n];  // (0 where no fragment was blended: every key is beyond it)
                     any |= kept[n];
-                    if (HITS != 1 && kept[n]) g4[HITS == 1 ? 0 : n] = pixel_gradient[q[n]];
                 }
                 if (any)
                 {
@@ -1738,9 +1744,16 @@ __global__ void __launch_bounds__(kBlock, 5) gather_point_gradients_kernel(Gathe
                     record[2 * k + 1] = partial[2 * rec + 1];
                 }
             }
+            float4 g4[kTogether];
 #pragma unroll
             for (int n = 0; n < kSlots; ++n)
             {
+            if (HITS != 1 && n % kTogether == 0)
+            {
+#pragma unroll
+                for (int k = 0; k < kTogether; ++k)
+                    if (kept[n + k]) g4[k] = pixel_gradient[q[n + k]];
+            }
             if (!kept[n]) continue;
             const int h = n % HITS, k = n / HITS, l = l0 + k;
             const float fx = HITS == 1 ? rintf(px[k]) : floorf(px[k]) + (float)(h & 1);
@@ -1763,7 +1776,8 @@ __global__ void __launch_bounds__(kBlock, 5) gather_point_gradients_kernel(Gathe
                 // d alpha / d weight = confidence (:3075-3088)
                 const float4 r      = h < 2 ? r0 : r1;
                 const float factor  = (h & 1) ? r.z : r.x, d_alpha = (h & 1) ? r.w : r.y;
-                const float g[4]    = {g4[n].x, g4[n].y, g4[n].z, g4[n].w};
+                const float4 up     = g4[n % kTogether];
+                const float g[4]    = {up.x, up.y, up.z, up.w};
                 float du, dv;
                 const float weight = bilinear_weight(px[k], py[k], h, &du, &dv);
                 const float single = conf * d_alpha;
