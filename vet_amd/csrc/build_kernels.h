@@ -141,30 +141,36 @@ struct FuzzyBucket
     }
 };
 
-// Sorts list[0, n), n <= kBuildCap, by the whole workgroup through the LDS room `room` (kBuildCap keys). Copy in (padded
-// with +infinity to a power of two), every wave sorts 64-key chunks in registers, then the chunks are merged pairwise,
-// level by level, in the all-ascending form of the bitonic network: a mirror step and the halving steps over 64 or more
-// places run on LDS with a barrier each, the last six halving steps of every level again in registers. A list of 512
-// keys takes 13 barriers instead of the 45 of the plain network. Every thread of the workgroup must call.
-__device__ __forceinline__ void block_sort_in_lds(uint64_t* list, uint32_t n, uint64_t* room, int tid)
+// Sorts list[0, n) in LDS, n <= kBuildCap, by the whole workgroup; places beyond n act as +infinity and are never touched. Every
+// wave sorts 64-key chunks in registers, then the chunks are merged pairwise, level by level, in the all-ascending form of the
+// bitonic network: a mirror step and the halving steps over 64 or more places run on LDS with a barrier each, the last six halving
+// steps of every level again in registers. A list of 512 keys takes 13 barriers instead of the 45 of the plain network. Every
+// thread of the workgroup must call.
+__device__ __forceinline__ void block_sort(uint64_t* list, uint32_t n, int tid)
 {
     const int lane = tid & (kWave - 1), wave = tid / kWave;
     uint32_t m = kWave;
     while (m < n) m <<= 1;  // <= kBuildCap
-    for (uint32_t k = tid; k < m; k += kBlock) room[k] = k < n ? list[k] : kInfKey;
-    __syncthreads();
-    const uint32_t chunks = m / kWave;
-    for (uint32_t c = wave; c < chunks; c += kBlock / kWave)
-        room[c * kWave + lane] = bitonic_sort_groups<6>(room[c * kWave + lane], lane);
-    __syncthreads();
+    auto in_chunks = [&](auto sorted) {
+        for (uint32_t c = wave; c * kWave < n; c += kBlock / kWave)
+        {
+            const uint32_t at  = c * kWave + lane;
+            const uint64_t key = sorted(at < n ? list[at] : kInfKey);
+            if (at < n) list[at] = key;
+        }
+        __syncthreads();
+    };
     auto order = [&](uint32_t i, uint32_t j) {  // i < j: the smaller key to place i
-        const uint64_t x = room[i], y = room[j];
+        if (j >= n) return;
+        const uint64_t x = list[i], y = list[j];
         if (y < x)
         {
-            room[i] = y;
-            room[j] = x;
+            list[i] = y;
+            list[j] = x;
         }
     };
+    __syncthreads();
+    in_chunks([&](uint64_t key) { return bitonic_sort_groups<6>(key, lane); });
     for (uint32_t k = 2 * kWave; k <= m; k <<= 1)
     {
         const uint32_t hk = k >> 1;
@@ -183,10 +189,15 @@ __device__ __forceinline__ void block_sort_in_lds(uint64_t* list, uint32_t n, ui
             }
             __syncthreads();
         }
-        for (uint32_t c = wave; c < chunks; c += kBlock / kWave)
-            room[c * kWave + lane] = bitonic_merge64(room[c * kWave + lane], lane);
-        __syncthreads();
+        in_chunks([&](uint64_t key) { return bitonic_merge64(key, lane); });
     }
+}
+
+// The same for a list in memory, through the LDS room `room` (kBuildCap keys).
+__device__ __forceinline__ void block_sort_through_lds(uint64_t* list, uint32_t n, uint64_t* room, int tid)
+{
+    for (uint32_t k = tid; k < n; k += kBlock) room[k] = list[k];
+    block_sort(room, n, tid);
     for (uint32_t k = tid; k < n; k += kBlock) list[k] = room[k];
     __syncthreads();
 }
@@ -629,7 +640,7 @@ __device__ __forceinline__ void build_in_memory(BuildArgs& args, const BinPlace&
         const uint32_t c = (uint32_t)tid < pixels ? cursors[tid] : 0u;
         const bool mine  = c > (uint32_t)(kChunks * kWave) && c <= (uint32_t)kBuildCap;  // pixel tid
         const uint64_t wave_mask = __ballot(mine);
-        if (lane == 0) lists_by_block[wave] = wave_mask;
+        if (lane == 0) lists_by_block[opaque(threadIdx.x) / kWave] = wave_mask;
         __syncthreads();
         for (int w = 0; w < kBlock / kWave; ++w)  // the same trips for every thread
         {
@@ -638,7 +649,7 @@ __device__ __forceinline__ void build_in_memory(BuildArgs& args, const BinPlace&
             {
                 const uint32_t px = w * kWave + (__ffsll((unsigned long long)todo) - 1);
                 todo &= todo - 1ull;
-                block_sort_in_lds(a.fragments + begin + starts[px], cursors[px], room.keys, tid);
+                block_sort_through_lds(a.fragments + begin + starts[px], cursors[px], room.keys, opaque(threadIdx.x));
             }
         }
     }
@@ -869,7 +880,28 @@ __device__ __forceinline__ void build_by_workgroup(BuildArgs& args, uint32_t bin
             off    = room.places[p0 + lane];
             length = (room.places[p0 + lane + 1] - off) & 0xFFFFu;
         }
-        sort_wave_lists(room.keys, reinterpret_cast<uint8_t*>(mine.t), off & 0xFFFFu, length, lane, a.K);
+        sort_wave_lists(room.keys, reinterpret_cast<uint8_t*>(mine.t), off & 0xFFFFu, length, lane, a.K, /*skip_longer=*/(uint32_t)kBuildCap);
+        if (!(a.K > 0 && a.K <= kWave))
+        {
+            // Lists that have to be sorted in full and are too long for a wave's registers: by the whole workgroup, one after the
+            // other. (By the wave that has them, every step of the network in LDS, 300 to 800 fragments a pixel: 201 against 129 us,
+            // with the 2x2 splat 113 against 49. From 128 on instead of 256: 134 and 48.)
+            const uint64_t longer = __ballot(length > (uint32_t)(4 * kWave));
+            if (lane == 0) lists_by_block[wave] = longer;
+            __syncthreads();
+            for (int w = 0; w < kBlock / kWave; ++w)  // the same trips for every thread
+            {
+                uint64_t todo = lists_by_block[w];
+                while (todo != 0ull)
+                {
+                    const uint32_t px = g0 + (uint32_t)w * per_wave + (uint32_t)(__ffsll((unsigned long long)todo) - 1);
+                    todo &= todo - 1ull;
+                    const uint32_t at = room.places[px] & 0xFFFFu, behind = room.places[px + 1] & 0xFFFFu;
+                    block_sort(room.keys + at, behind - at, opaque(threadIdx.x));
+                }
+            }
+            __syncthreads();  // (the next run writes these masks)
+        }
         if (g1 - g0 > (uint32_t)kWave)
         {
             wave_sync();
