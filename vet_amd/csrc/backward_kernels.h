@@ -16,7 +16,9 @@ namespace vetrast
 // Accumulators of the call that have to start at zero: the pose and intrinsics gradients and their counts, and with a texture
 // index the rows that points add to. The first view's per-pixel kernel, which is in front of every kernel that adds to them
 // in stream order, clears them in passing: its first workgroup the small ones, all of them the others. (A fill launch
-// takes 4.5 us and more each: two FUZZY_BLEND views with an index 21 us for four.)
+// takes 4.5 us and more each: two FUZZY_BLEND views with an index 21 us for four.) Rows beyond kClearByOne words for each of its
+// workgroups are left to a fill launch: a 64x64 crop has 16 of them, which took 40 us longer than the launches for ten million
+// points.
 constexpr int kClearJobs          = 6;
 constexpr uint32_t kClearByOne    = 16384;  // words one workgroup clears
 struct ClearJob

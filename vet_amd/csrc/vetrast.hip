@@ -904,20 +904,20 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
     // The per-point kernel overwrites every gradient row in the first view, so the zeros_like fills of
     // PointRenderer.cu:267-277 are only needed where rows are added to with atomics: with a texture index
     // indirection, where several points may share a row. They and the pose and intrinsics accumulators are cleared by the
-    // first view's per-pixel kernel (ClearJob).
+    // first view's per-pixel kernel (ClearJob), unless that has too few workgroups for so many rows.
     ClearJob clear = {};
     {
         ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_PREPARE);
         int jobs  = 0;
         auto zero = [&](void* ptr, size_t words) {
             if (!ptr || words == 0) return;
-            if (words <= 0xFFFFFFFFull)
+            if (words <= std::min<size_t>((size_t)tile_grid(tiles) * kClearByOne, 0xFFFFFFFFull))
             {
                 clear.ptr[jobs]     = reinterpret_cast<uint32_t*>(ptr);
                 clear.count[jobs++] = (uint32_t)words;
             }
             else
-                hipLaunchKernelGGL(fill_u32_kernel, dim3(8192), dim3(kBlock), 0, stream, reinterpret_cast<uint32_t*>(ptr), words, 0u);
+                hipLaunchKernelGGL(fill_u32_kernel, dim3(std::min(grid_for(words), 8192)), dim3(kBlock), 0, stream, reinterpret_cast<uint32_t*>(ptr), words, 0u);
         };
         if (g->grad_pose)
         {
