@@ -17,24 +17,32 @@ from vet_amd.rasterizer import make_params
 pytestmark = pytest.mark.gpu
 
 SIDE, TILE = 512, 16
-SPREAD = [1, 2, 63, 64, 65, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 1537, 2048, 3100, 8191, 8193]
+LIMITS = [64, 256, 512, 1024, 8192]
+SPREAD = [4, 8, 1540, 2048, 3100, 5000, 7300] + [n + d for n in LIMITS for d in (-1, 0, 1)]
 IN_A_PIXEL = [64, 65, 128, 129, 256, 257, 1024, 1025]
 
 
+def _spots(hits):
+    """Points of every spot that is spread over a tile. With four hits per layer a point is four records (a pixel away from the
+    tile's border all of them lie in the tile): next to a limit the nearest multiples of four."""
+    return [n if hits == 1 else (n // 4 if n not in [m + 1 for m in LIMITS] else n // 4 + 1) for n in SPREAD]
+
+
 def _scene(K, hits, seed=5):
-    """With four hits per layer a spot of n points is a bin of 4 n records in layer 0: the same numbers, a quarter of the points
-    each (a point a pixel away from the tile's border has all of its hits in the tile)."""
     rng = np.random.default_rng(seed)
     uv, tiles = [], rng.permutation((SIDE // TILE) ** 2)
-    for k, n in enumerate(SPREAD + IN_A_PIXEL):
+    for k, n in enumerate(_spots(hits) + [max(1, n // hits) for n in IN_A_PIXEL]):
         corner = np.array([tiles[k] % (SIDE // TILE), tiles[k] // (SIDE // TILE)]) * TILE
-        n = max(1, n // hits)
         if k < len(SPREAD):
             spot = corner + rng.uniform(1.0, TILE - 2.0, (n, 2))
         else:  # in one pixel and, for a bin of more than that list, the tile
             spot = np.concatenate([corner + 5 + rng.uniform(0.0, 0.4, (n, 2)), corner + rng.uniform(1.0, TILE - 2.0, (200, 2))])
         uv.append(spot)
-    uv.append(rng.uniform(0, SIDE - 1, (3000, 2)))  # and a few everywhere
+    everywhere = rng.uniform(0, SIDE - 1, (3000, 2))  # and a few in the other tiles
+    own = np.zeros((SIDE // TILE, SIDE // TILE), bool)
+    own[tiles[:len(SPREAD)] // (SIDE // TILE), tiles[:len(SPREAD)] % (SIDE // TILE)] = True
+    near = np.floor((everywhere[:, None] + [[-1, -1], [-1, 1.5], [1.5, -1], [1.5, 1.5]]) / TILE).astype(int).clip(0, SIDE // TILE - 1)
+    uv.append(everywhere[~own[near[..., 1], near[..., 0]].any(axis=1)])
     uv = np.concatenate(uv)
     uv = uv[rng.permutation(len(uv))]
     n = len(uv)
@@ -46,10 +54,21 @@ def _scene(K, hits, seed=5):
                            max_list_length=K, seed=seed)
 
 
+def _has_its_sizes(ref, hits):
+    """Layer 0 is built in tiles: there is one with each of the numbers of records."""
+    counts = np.diff(ref.offsets[0, :SIDE * SIDE + 1].astype(np.int64)).reshape(SIDE // TILE, TILE, SIDE // TILE, TILE).sum(axis=(1, 3))
+    want = {n * hits for n in _spots(hits)}
+    assert want <= set(counts.ravel().tolist()), sorted(want - set(counts.ravel().tolist()))
+    for n in LIMITS:
+        assert {n - hits if hits == 4 else n - 1, n, n + hits if hits == 4 else n + 1} <= want, n
+
+
 @pytest.mark.parametrize("mode", [1, 2, 3])
 @pytest.mark.parametrize("K", [-1, 1, 16, 64, 100])
 def test_bins_around_the_sizes_of_their_ways(mode, K, rasterizer, oracle):
     print(f"[case] bin sizes: mode {mode}, K {K}", flush=True)
-    scene = _scene(K, 4 if mode == 3 else 1)
-    _compare(scene, make_params(scene, render_mode=mode, need_point_gradient=1), rasterizer, oracle,
-             bilinear=mode == abi.RENDER_BILINEAR_BLEND)
+    hits = 4 if mode == 3 else 1
+    scene = _scene(K, hits)
+    _, ref = _compare(scene, make_params(scene, render_mode=mode, need_point_gradient=1), rasterizer, oracle,
+                      bilinear=mode == abi.RENDER_BILINEAR_BLEND)
+    _has_its_sizes(ref, hits)

@@ -14,6 +14,36 @@ from vet_amd.rasterizer import DeviceScene, make_params
 pytestmark = pytest.mark.gpu
 
 GRAD_TOL = 1e-4  # 32-bit sums in another order, against the largest entry of the tensor
+# The background's gradient is one sum over all pixels of transmittance x upstream gradient, in 32 bits: each term goes through
+# eight additions inside its workgroup and fewer than a hundred behind it; FUZZY_BLEND works its transmittance out anew, with two
+# roundings for each of the fragments in front (beyond some 40 nothing to speak of is left). 180 x 2^-24 = 1.1e-5 of the terms'
+# absolute sum if all of them erred one way.
+BACKGROUND_TOL = 1.1e-5
+
+
+def _transmittance(ref, mode):
+    """What is left for the background, per layer [B,h,w] in float64. FULL_BLEND and BILINEAR_BLEND: what the forward pass left,
+    and nothing where the 2x2 splat stopped early. FUZZY_BLEND: the backward pass forms buckets all along a list
+    (src/lib/rendering/RenderBackward.cu:628-720)."""
+    scene, left = ref.scene, []
+    for l, (w, h) in enumerate(ref.sizes):
+        base = ref.layer_base(l)
+        T = ref.weight[:, base:base + w * h].astype(np.float64).reshape(-1, h, w)
+        if mode == 3:
+            T = np.where(T < 0.001, 0.0, T)
+        if mode == 2:
+            K = ref.params.debug_max_list_length
+            for b, y, x in np.argwhere(np.diff(ref.offsets[:, base:base + w * h + 1].astype(np.int64)).reshape(-1, h, w) > 1):
+                keys = ref.pixel_list(b, l, x, y)[:K if K > 0 else None]
+                depth = (keys >> np.uint64(32)).astype(np.uint32).view(np.float32)
+                conf = scene.confidence[scene.index[(keys & np.uint64(0xFFFFFFFF)).astype(np.int64)]].astype(np.float64)
+                T[b, y, x], j = 1.0, 0
+                while j < len(keys):
+                    e = j + int(np.argmin(np.append(depth[j:] - depth[j] < np.float32(ref.params.depth_accept_blend), False)))
+                    T[b, y, x] *= 1.0 - conf[j:e].mean()
+                    j = e
+        left.append(T)
+    return left
 
 
 @pytest.mark.parametrize("mode", [1, 2, 3])
@@ -43,8 +73,9 @@ def test_gradients_for_every_record_layout(mode, points, size, layers, channels,
     torch.cuda.synchronize()
     for l in range(layers):
         np.testing.assert_array_equal(res.out[l].cpu().numpy(), ref.out[l])
-    # (the background's gradient is one sum over all pixels that no record takes part in; in the oracle's float32 the order of
-    # its some 6000 terms of both signs alone moves it by up to 6000 x 2^-24 = 3.6e-4 of their size)
     for key in ("texture", "confidence", "points", "pose", "intrinsics"):
         err = max_rel_err(got[key].cpu().numpy(), want[key])
         assert err <= (1e-3 if key == "intrinsics" else GRAD_TOL), (key, err)  # (intrinsics: the oracle's sums are in float32)
+    terms = [(T[:, None] * g.astype(np.float64)) for T, g in zip(_transmittance(ref, mode), grad_out)]
+    off = got["background"].cpu().numpy() - sum(t.sum(axis=(0, 2, 3)) for t in terms)
+    assert (np.abs(off) <= BACKGROUND_TOL * sum(np.abs(t).sum(axis=(0, 2, 3)) for t in terms)).all(), off
