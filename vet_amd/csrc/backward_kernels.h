@@ -1506,11 +1506,8 @@ __global__ void __launch_bounds__(kReduceBlock) reduce_background_kernel(const f
 struct GatherPass
 {
     ViewPass vp;
-    const uint32_t* offsets;
-    const uint64_t* fragments;
     const uint8_t* list_is_cut;  // per pixel, written by the build pass
     const uint64_t* last_key;    // per pixel with list_is_cut: key of the last fragment that took part in the blend
-    const uint32_t* kept;        // per pixel, BILINEAR_BLEND: fragments of its list that took part in the blend
     const float4* partial;
     const float4* pixel_gradient;  // BILINEAR_BLEND: [P], see BackwardPass
     float* grad_texture;      // [C,N]
@@ -1526,7 +1523,7 @@ struct GatherPass
     // gradient rows are written once.
     int point_major_records;  // layout of the record array, see gradient_record
     int view_count;
-    size_t dropout_stride, flags_stride, last_key_stride, kept_stride;  // elements of the respective arrays
+    size_t dropout_stride, flags_stride, last_key_stride;  // elements of the respective arrays
     size_t partial_stride, pixel_gradient_stride, background_rows_stride, camera_partial_stride;
     int accumulate;  // 0: overwrite the gradient rows (the call's first round), 1: add to them (further rounds); texture and
                      // confidence rows behind an index are always added to

@@ -1082,11 +1082,8 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_GATHER);
             GatherPass gp;
             gp.vp                  = make_view_pass(a, lay, ly, first);
-            gp.offsets             = ws_ptr<uint32_t>(ws, lay.offsets_base + lay.offsets_stride * first);
-            gp.fragments           = ws_ptr<uint64_t>(ws, lay.fragments_base + lay.fragments_stride * first);
             gp.list_is_cut         = ws_ptr<uint8_t>(ws, lay.cut_flags_base + lay.cut_flags_stride * first);
             gp.last_key            = ws_ptr<uint64_t>(ws, lay.last_key_base + lay.last_key_stride * first);
-            gp.kept                = ws_ptr<uint32_t>(ws, lay.kept_base + lay.kept_stride * first);
             gp.partial             = partial;
             gp.pixel_gradient      = ws_ptr<float4>(ws, pixel_gradient_base(lay));
             gp.grad_texture        = g->grad_texture;
@@ -1101,7 +1098,6 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             gp.dropout_stride      = (size_t)N;
             gp.flags_stride        = lay.cut_flags_stride;
             gp.last_key_stride     = lay.last_key_stride / sizeof(uint64_t);
-            gp.kept_stride         = lay.kept_stride / sizeof(uint32_t);
             gp.partial_stride      = lay.lane_scratch_stride / sizeof(float4);
             gp.pixel_gradient_stride  = lay.lane_scratch_stride / sizeof(float4);
             gp.background_rows_stride = lay.lane_scratch_stride / sizeof(float);
