@@ -66,6 +66,7 @@ struct BuildPass
     uint32_t crowded_capacity;
     uint32_t crowded_blocks;         // workgroups at the front of the grid that go through them
     uint32_t num_bins;
+    uint32_t shared_end;             // see CrowdedBins
     int N;
     int K;
     int use_environment_map;
@@ -821,7 +822,7 @@ __device__ __forceinline__ void build_by_workgroup(BuildArgs& args, uint32_t bin
     if (!one_run)
     {
         const bool long_lists = (wave_words[8] | wave_words[9] | wave_words[10] | wave_words[11]) != 0u;
-        if (long_lists || n > (uint32_t)(kBuildMaxRuns * kBuildCap))
+        if (long_lists || bin >= a.shared_end || n > (uint32_t)(kBuildMaxRuns * kBuildCap))
         {
             if (part != 0u) return;
             if ((uint32_t)tid < pixels) a.offsets[place.q0 + tid] = begin + start;

@@ -26,6 +26,7 @@ constexpr int kLogSegments    = 256;          // the overflow log is cut into th
 constexpr int kWaveBinCap     = 256;          // fragment records up to which one wave builds a bin's lists
 constexpr int kBuildCap       = 1024;         // ... and up to which a workgroup does at once
 constexpr int kBuildMaxRuns   = 8;            // a bin of more than this many times kBuildCap records is built in memory
+constexpr int kSmallBinShift  = 4;            // ... and one of up to 16 pixels whose lists are cut, of more than kBuildCap
 constexpr int kLogCursorStride = 16;          // uint32 between two cursors (64 bytes: one cursor per cache line)
 
 // Camera constants of one view, written by prepare_views_kernel and read (uniformly) by every other kernel.

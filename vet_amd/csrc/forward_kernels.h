@@ -792,14 +792,16 @@ struct CrowdedBins
     uint2* entries;    // [capacity]: bin, which part of it | number of parts << 16
     uint32_t* counts;  // [2], 8-byte aligned: entries at the front, at the back; zero before the launch
     uint32_t capacity;
+    uint32_t shared_end;  // bins from this one on are not shared
 };
 // Workgroups that share a bin of n records. The longest bins set the end of the pass where one workgroup takes them alone
 // (4891 records 107 us, with all others done after 73), so a part is sized to fit LDS at once as a rule, with some room for
-// lists that can't be cut. More than kBuildMaxRuns times what fits goes through memory, which one workgroup does.
-__device__ __forceinline__ uint32_t parts_of_bin(uint32_t n)
+// lists that can't be cut. More than kBuildMaxRuns times what fits goes through memory, which one workgroup does; and so do
+// from kBuildCap on the small bins whose lists are cut (shared_end, on the host).
+__device__ __forceinline__ uint32_t parts_of_bin(uint32_t n, bool shared)
 {
     constexpr uint32_t kPart = kBuildCap / 4 * 3;
-    return n > (uint32_t)kBuildCap && n <= (uint32_t)(kBuildMaxRuns * kBuildCap) ? (n + kPart - 1u) / kPart : 1u;
+    return shared && n > (uint32_t)kBuildCap && n <= (uint32_t)(kBuildMaxRuns * kBuildCap) ? (n + kPart - 1u) / kPart : 1u;
 }
 
 // Writes down the crowded ones of 4 N consecutive bins from `bin` on. All threads of the workgroup must call. Each workgroup
@@ -810,14 +812,18 @@ __device__ __forceinline__ void list_crowded(const CrowdedBins& out, const uint4
     __shared__ uint32_t s_wave[2][kBlock / kWave];
     __shared__ uint32_t s_first[2];
     uint32_t own[2] = {0u, 0u};
-    auto count = [&](uint32_t n) {
+    auto count = [&](uint32_t n, uint32_t b) {
         if (n > (uint32_t)kBuildCap)
-            own[0] += parts_of_bin(n);
+            own[0] += parts_of_bin(n, b < out.shared_end);
         else if (n > (uint32_t)kWaveBinCap)
             ++own[1];
     };
 #pragma unroll
-    for (int k = 0; k < N; ++k) count(counts[k].x), count(counts[k].y), count(counts[k].z), count(counts[k].w);
+    for (int k = 0; k < N; ++k)
+    {
+        count(counts[k].x, bin + 4 * k), count(counts[k].y, bin + 4 * k + 1);
+        count(counts[k].z, bin + 4 * k + 2), count(counts[k].w, bin + 4 * k + 3);
+    }
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     uint32_t run[2];
 #pragma unroll
@@ -847,7 +853,7 @@ __device__ __forceinline__ void list_crowded(const CrowdedBins& out, const uint4
     }
     auto put = [&](uint32_t n, uint32_t b) {
         if (n <= (uint32_t)kWaveBinCap) return;
-        const uint32_t parts = parts_of_bin(n);
+        const uint32_t parts = parts_of_bin(n, b < out.shared_end);
         for (uint32_t part = 0; part < parts; ++part)
         {
             const uint32_t at = n > (uint32_t)kBuildCap ? run[0]++ : out.capacity - 1u - run[1]++;
