@@ -108,10 +108,10 @@ __device__ __forceinline__ bool interior_pixel(int x, int y, int w, int h)
 // lanes of a pixel plus a per-pixel carry, rounds run from the deepest fragments to the nearest.
 //
 // What bounds it: chains of memory round trips (list, keys, descriptor records, gradient records) and the traffic behind
-// them, 340 MB of a benchmark frame at three quarters of the rate of a copy; vector instructions are half of its cycles.
+// them, 340 MB of a benchmark frame; vector instructions alone would take 47 of its 102 us.
 // More pixels to a wave where tiles hold little cost 40 % fewer instructions and a third more time. Against a table of items
-// filled by their pixels, sums through the LDS permute and waits behind branches: benchmark frame 101 -> 94 us, four town
-// views 373 -> 344, four crops with the 2x2 splat 67 -> 59, 2x2 splat at 1080p 140 -> 136 (busy cycles at 2.4 GHz).
+// filled by their pixels, sums through the LDS permute and waits behind branches (us, kernel traces on one card): benchmark frame
+// 109 -> 102, four town views 389 -> 365, four crops with the 2x2 splat 88 -> 78, 2x2 splat at 1080p 155 -> 145.
 constexpr int kWindow     = 16;                 // fragments per pixel in one window
 constexpr int kWaveItems  = kWave * kWindow;    // item table of a wave
 

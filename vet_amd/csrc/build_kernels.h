@@ -19,13 +19,18 @@ namespace vetrast
 //  * up to kBuildCap a workgroup, 8 to a compute unit, whose waves part where every wave has its pixels' keys (bins of
 //    few pixels stay together: the walk wants their pixels side by side in one wave);
 //  * up to kBuildMaxRuns times that several workgroups, each a stretch of the bin's pixels (parts_of_bin), in runs that fit;
-//  * beyond, or with a list that does not fit by itself, one workgroup in the fragment buffer.
+//  * beyond, or with a list that does not fit by itself, or in small bins with cut lists (shared_end) beyond kBuildCap, one workgroup
+//    in the fragment buffer.
+// Lists that have to be sorted in full are sorted in a wave's registers up to 256 keys (128 in the fragment buffer), by the workgroup
+// up to 1024, and by a wave in the fragment buffer beyond.
 // The scan of the bin counts writes down the bins with more than kWaveBinCap records; the first crowded_blocks workgroups go
 // through that list, the others take four neighbouring bins each. With a workgroup for every bin and everything beyond
-// kBuildCap in the fragment buffer, against now, us of the pass: benchmark frame 100 and 81, the same with the
-// 2x2 splat 320 and 250, four of its 512x512 crops 102 and 76, four town views of 39 records a bin 444 and 264 (of which the
-// stores of the results are 75), a million points in 1279x719 82 and 58, two FUZZY_BLEND views 113 and 92, ten million
-// points 666 and 550.
+// kBuildCap in the fragment buffer, against now (us, kernel traces on one card): benchmark frame 89 and 71, the same with the
+// 2x2 splat 288 and 196, four of its 512x512 crops 255 and 87, four town views of 39 records a bin 457 and 236 (of which the
+// stores of the results are 75), a million points in 1279x719 with the 2x2 splat 86 and 74, two FUZZY_BLEND views 151 and 111, ten
+// million points 667 and 447. A view in which only a few hundred bins hold anything, and those up to 256 records, is the slower for a
+// wave's longer chain: 230 thousand points in 1418x834 19 and 22, 120 thousand FUZZY_BLEND in 1471x814 21 and 25. Neither a workgroup
+// for each bin there (25 and 31) nor four waves, each a quarter of the pixels (26 and 28), makes up for it.
 constexpr int kBuildPerThread = kBuildCap / kBlock;
 constexpr int kWavePerLane    = kWaveBinCap / kWave;
 static_assert(kPrimaryCapSmall >= kBuildCap, "a bin built in LDS must find all its records in its own room");

@@ -171,8 +171,8 @@ __device__ __forceinline__ bool point_is_skipped(const ViewPass& a, int i)
 //      straight to place `rank` of the room the bin owns (no second projection pass).
 //   2. exclusive scan over the bin counts; the few records that did not fit a bin's room are filed behind it (the same
 //      launch, scan_move_kernel, where a view has at most kScanMoveMax bins; overflow_move_kernel otherwise).
-//   3. bin_build_kernel: one workgroup per bin counts the pixels, scans them, scatters the keys and sorts the lists, all
-//      in LDS. Pixels are numbered tile by tile, so the scan of the bin counts IS the start of every bin's lists and no
+//   3. bin_build_kernel: a wave, a workgroup or several, by the number of its records, count a bin's pixels, scan them, scatter the
+//      keys and sort the lists, in LDS as a rule. Pixels are numbered tile by tile, so the scan of the bin counts IS the start of every bin's lists and no
 //      scan over the pixels is needed.
 
 // Per-lane grouping of equal bin numbers inside a wave: leader = lowest lane with the same bin, rank = number of

@@ -143,8 +143,8 @@ LayerTable make_layer_table(int w, int h, int L, int64_t N, const float* expecte
         const double mean_len = in_layer / ((double)w * (double)h);
         int shift             = 8;
         while (shift > 2 && mean_len * (double)(1 << shift) > 1024.0) shift -= 2;
-        // ... and small enough for the layer to have a thousand bins where it has the pixels for them: every bin is one
-        // workgroup's chain of dependent steps, and a layer of a few dozen big bins (a coarse layer of a 512x512
+        // ... and small enough for the layer to have a thousand bins where it has the pixels for them: a bin is a chain of dependent
+        // steps, whether of a wave or of a workgroup, and a layer of a few dozen big bins (a coarse layer of a 512x512
         // training crop) runs them on a few dozen compute units while the others wait
         while (shift > 2 && (tiles << (8 - shift)) < 1024u) shift -= 2;
         t.bin_shift[l] = shift;
