@@ -108,10 +108,10 @@ __device__ __forceinline__ bool interior_pixel(int x, int y, int w, int h)
 // lanes of a pixel plus a per-pixel carry, rounds run from the deepest fragments to the nearest.
 //
 // What bounds it: chains of memory round trips (list, keys, descriptor records, gradient records) and the traffic behind
-// them, 340 MB of a benchmark frame; vector instructions alone would take 47 of its 102 us.
+// them, 350 MB of a benchmark frame; vector instructions alone would take 47 of its 111 us.
 // More pixels to a wave where tiles hold little cost 40 % fewer instructions and a third more time. Against a table of items
-// filled by their pixels, sums through the LDS permute and waits behind branches (us, kernel traces on one card): benchmark frame
-// 109 -> 102, four town views 389 -> 365, four crops with the 2x2 splat 88 -> 78, 2x2 splat at 1080p 155 -> 145.
+// filled by their pixels, sums through the LDS permute and waits behind branches (us, kernel traces on one card): two million points
+// at 1080p 109 -> 102, with the 2x2 splat 155 -> 145, four 512x512 crops of them 88 -> 78, four town views 389 -> 365.
 constexpr int kWindow     = 16;                 // fragments per pixel in one window
 constexpr int kWaveItems  = kWave * kWindow;    // item table of a wave
 

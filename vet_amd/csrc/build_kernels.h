@@ -25,7 +25,7 @@ namespace vetrast
 // up to 1024, and by a wave in the fragment buffer beyond.
 // The scan of the bin counts writes down the bins with more than kWaveBinCap records; the first crowded_blocks workgroups go
 // through that list, the others take four neighbouring bins each. With a workgroup for every bin and everything beyond
-// kBuildCap in the fragment buffer, against now (us, kernel traces on one card): benchmark frame 89 and 71, the same with the
+// kBuildCap in the fragment buffer, against now (us, kernel traces on one card): two million points at 1080p 89 and 71, with the
 // 2x2 splat 288 and 196, four of its 512x512 crops 255 and 87, four town views of 39 records a bin 457 and 236 (of which the
 // stores of the results are 75), a million points in 1279x719 with the 2x2 splat 86 and 74, two FUZZY_BLEND views 151 and 111, ten
 // million points 667 and 447. A view in which only a few hundred bins hold anything, and those up to 256 records, is the slower for a
