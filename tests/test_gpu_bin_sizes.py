@@ -1,7 +1,8 @@
 """GPU parity of the list-building pass around the sizes at which a bin changes hands.
 
 A bin of up to 256 records is built by a wave, of up to 1024 by a workgroup at once, of up to 8192 by several workgroups that
-take a run of its pixels each, beyond that, or where a list does not fit by itself, in memory. The spots here hold a number of
+take a run of its pixels each, beyond that, or where a list does not fit by itself, in memory; with a cut of up to 64 also from 1024
+on where it has 4 or 16 pixels. The spots here hold a number of
 points next to these sizes, spread over a 16x16 pixel tile of layer 0 (or within a pixel: lists as long as the bin), and fall
 into bins of 64, 16 and 4 pixels in the layers behind it. The cut of the longest lists takes the K smallest keys as they pass
 (K <= 64) or sorts lists in full. Counterpart of SegmentedSortBitonicHelper2 and BlendMulti,
