@@ -420,7 +420,7 @@ __device__ __forceinline__ void blend_backward(const BackwardPass& a)
     }
     __syncthreads();
     if (threadIdx.x <= C)
-        a.background_partial[(size_t)blockIdx.x * kBackgroundRow + threadIdx.x] =
+        a.background_partial[(size_t)px.home * kBackgroundRow + threadIdx.x] =
             (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
@@ -521,14 +521,16 @@ __device__ __forceinline__ FuzzyPixel fuzzy_pixel(const BackwardPass& a, const T
 // slot's depths. Sums and products are combined pairwise instead of front to back, which moves the results by
 // rounding only. The table that says which pixel a lane's fragment belongs to holds kWaveItems slots; a wave whose
 // pixels need more goes through it in batches. Longer lists are left to blend_backward_fuzzy_long_kernel; the
-// workgroup says in column kFuzzyLongColumn of its background row whether it has any.
+// workgroup says in column kFuzzyLongColumn of the row of its own number whether it has any, beside the row its sums go to
+// (2 home + 1, see TilePixel::home), so that the workgroups of the second kernel that have nothing to do leave after one load (with
+// the place of their tile worked out first that kernel took 117 us instead of 87).
 constexpr int kFuzzyDense      = 32;  // longest list of the dense layout
 constexpr int kFuzzyNarrow     = 16;  // longest slot that lies inside a row of 16 lanes
 // The kernel is compiled for DENSE = kFuzzyNarrow (no slot spans rows: fewer registers, more waves per SIMD) and for
 // DENSE = kFuzzyDense; the host takes the narrow one where the cut keeps every list that short, and also where lists
 // beyond kFuzzyDense may exist: those go to blend_backward_fuzzy_long_kernel, which then is the faster one for the lists
 // of 17 to 32 fragments as well (measured; slots of 64 lanes lost against it too).
-constexpr int kFuzzyLongColumn = 6;   // background row, column 6: the workgroup has a list for the wave-per-list kernel
+constexpr int kFuzzyLongColumn = 6;   // background row, column 6, as bits: 2 home + whether the workgroup has a list for the wave-per-list kernel
 // The wave-per-list kernel is launched kFuzzyReplicas times over (grid.y): replica r takes every kFuzzyReplicas-th long
 // list of a wave's pixels. Long lists cluster (where a surface is seen edge-on a whole strip of pixels holds hundreds
 // of fragments each), and a wave takes its lists one after the other. Replica 0 adds its background sums to the row
@@ -1007,10 +1009,13 @@ __device__ __forceinline__ void blend_backward_fuzzy(const BackwardPass& a, floa
         if (lane == 0) red[wave][C + 1] = longest ? 1.f : 0.f;
     }
     __syncthreads();
-    float* row = a.background_partial + (size_t)blockIdx.x * kBackgroundRow;
+    float* row = a.background_partial + (size_t)px.home * kBackgroundRow;
     if (threadIdx.x <= C) row[threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
     if (threadIdx.x == C + 1)
-        row[kFuzzyLongColumn] = (red[0][C + 1] + red[1][C + 1]) + (red[2][C + 1] + red[3][C + 1]);
+    {
+        const float any = (red[0][C + 1] + red[1][C + 1]) + (red[2][C + 1] + red[3][C + 1]);
+        a.background_partial[(size_t)blockIdx.x * kBackgroundRow + kFuzzyLongColumn] = __uint_as_float((px.home << 1) | (any != 0.f ? 1u : 0u));
+    }
 }
 
 template <int C, int DENSE>
@@ -1043,10 +1048,10 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
     constexpr int kWaves = kBlock / kWave;
     __shared__ float red[kWaves][C];
     const uint32_t replica = blockIdx.y;
-    float* row      = a.background_partial + (size_t)blockIdx.x * kBackgroundRow;
-    float* row_mine = replica == 0u ? row
-                                    : a.background_partial + ((size_t)kFuzzyFoldRows + (size_t)replica * gridDim.x + blockIdx.x) * kBackgroundRow;
-    if (row[kFuzzyLongColumn] == 0.f)
+    const uint32_t state = __float_as_uint(a.background_partial[(size_t)blockIdx.x * kBackgroundRow + kFuzzyLongColumn]);
+    float* row      = a.background_partial + (size_t)(state >> 1) * kBackgroundRow;
+    float* row_mine = replica == 0u ? row : row + ((size_t)kFuzzyFoldRows + (size_t)replica * gridDim.x) * kBackgroundRow;
+    if ((state & 1u) == 0u)
     {
         if (replica != 0u && threadIdx.x < (uint32_t)kBackgroundRow) row_mine[threadIdx.x] = 0.f;
         return;

@@ -404,7 +404,19 @@ __device__ __forceinline__ size_t gradient_record(int point_major, int N, int L,
 // round-robin to the 8 XCDs (each with its own L2), so workgroup b belongs to XCD b % 8 and takes slot b / 8 of that
 // XCD's run of regions (region r goes to XCD r % 8): what one layer's tiles pulled into the XCD's L2 is still there
 // when the next layer's tiles of the region ask for the same points.
+// Where a launch has few regions, or its lists may be long, an XCD's regions hold a multiple of another's fragments (up to
+// 8 times, for one region), and the kernel lasts as long as the fullest XCD. There a region is cut into parts
+// (parts_log: 4^parts_log of them) and its part (x, y) is given to the XCD x + 3 y further on; on row by row of eight regions
+// every XCD then has each part of one of them. Per-pixel kernel, whole regions against 16 parts (us, kernel traces on one card):
+// six 228x228 crops of 5 layers 59 -> 40, 9.5 million points in 813x436 167 -> 139, two 602x267 crops of 3 million points 81 -> 52,
+// four 512x512 crops with the 2x2 splat 92 -> 84, ten million points at 1080p 545 -> 521. Everywhere it would cost
+// more than it gives, since a cache line of an image then belongs to several XCDs: four town views 387 -> 402, benchmark frame 107 ->
+// 111, two FUZZY_BLEND views of 1237x701 91 -> 94 (64 parts: 417, 114, 96; 4 parts: 392, 108, 92). Hence kPartsRegions, between the
+// four crops' 64 regions and those views' 120, and kPartsListLength, between the 2x2 splat's 3.9 fragments a pixel at
+// 1080p (152 either way) and the ten million points' 4.8.
 constexpr int kXcds = 8;
+constexpr uint32_t kPartsRegions  = 64;   // regions of all views of a launch
+constexpr double kPartsListLength = 4.0;  // fragments a pixel of layer 0 may blend
 // A layer whose pixels hold long lists is split: a workgroup then owns one 16x4 strip of a tile and each of its waves
 // one row of 16 pixels (lanes 16..63 carry no pixel, only fragments), so that such a layer (few pixels, many fragments)
 // is spread over four times as many waves, each with a quarter of the rounds to run one after the other.
@@ -415,6 +427,7 @@ struct TileMap
     uint32_t tiles_per_region;       // (4^L - 1) / 3
     uint32_t regions_per_xcd;        // ceil(regions / 8)
     uint32_t split[VETRAST_MAX_LAYERS];  // workgroups per tile of the layer: 1, or 4 (one per 16x4 strip)
+    uint32_t parts_log;              // parts of a region's side: 1 << parts_log
     uint32_t groups_per_region;      // sum over the layers of (tiles of the layer in a region) x split
 };
 
@@ -424,6 +437,8 @@ struct TilePixel
     int l, x, y;
     uint32_t q;      // pixel number over all layers
     uint32_t local;  // y * w + x inside the layer: index into the image planes
+    uint32_t home;   // workgroup that would have the tile if regions were whole: its row of partial sums, so that those are
+                     // added up in the same order either way
 };
 
 __device__ __forceinline__ TilePixel tile_pixel(const TileMap& tm, const LayerTable& ly)
@@ -432,14 +447,12 @@ __device__ __forceinline__ TilePixel tile_pixel(const TileMap& tm, const LayerTa
     r.active = false;
     r.l = r.x = r.y = 0;
     r.q = r.local = 0;
-    const uint32_t b      = blockIdx.x;
-    const uint32_t xcd    = b % kXcds;
-    const uint32_t slot   = b / kXcds;
-    const uint32_t region = (slot / tm.groups_per_region) * kXcds + xcd;
-    uint32_t t            = slot % tm.groups_per_region;  // workgroup inside the region, coarsest layer first
-    if (region >= tm.regions) return r;
+    const uint32_t xcd  = blockIdx.x % kXcds;
+    const uint32_t slot = blockIdx.x / kXcds;
+    const uint32_t row  = slot / tm.groups_per_region;  // of kXcds regions
+    uint32_t t          = slot - row * tm.groups_per_region;  // workgroup inside the region, coarsest layer first
     // layer L-1 has 1 tile per region, L-2 has 4, L-3 has 16, ...; split[l] workgroups per tile
-    int l            = tm.L - 1;
+    int l             = tm.L - 1;
     uint32_t side_log = 0;  // tiles per region side in layer l: 1 << side_log
     while (t >= tm.split[l] << (2 * side_log))
     {
@@ -451,8 +464,15 @@ __device__ __forceinline__ TilePixel tile_pixel(const TileMap& tm, const LayerTa
     const uint32_t split_log = tm.split[l] == 1 ? 0u : 2u;
     const uint32_t strip     = t & (tm.split[l] - 1u);  // 16x4 strip of the tile, if the layer is split
     t >>= split_log;
+    const uint32_t y_in = t >> side_log, x_in = t & ((1u << side_log) - 1u);
+    // the part of the region it lies in, or the strip where its tile is larger than a part
+    const uint32_t down   = side_log > tm.parts_log ? side_log - tm.parts_log : 0u;
+    const uint32_t turn   = (x_in >> down) + 3u * (y_in >> down) + (side_log < tm.parts_log ? 2u * strip : 0u);
+    const uint32_t region = row * kXcds + (xcd + turn) % kXcds;
+    r.home                = slot * kXcds + region % kXcds;
+    if (region >= tm.regions) return r;
     const uint32_t ry = region / tm.regions_x, rx = region - ry * tm.regions_x;
-    const uint32_t ty = (ry << side_log) + (t >> side_log), tx = (rx << side_log) + (t & ((1u << side_log) - 1u));
+    const uint32_t ty = (ry << side_log) + y_in, tx = (rx << side_log) + x_in;
     r.l = l;
     if (tx >= (uint32_t)ly.tiles_x[l] || ty >= (uint32_t)ly.tiles_y[l]) return r;
     uint32_t in_tile = threadIdx.x;  // 16 * (row of the tile) + column
