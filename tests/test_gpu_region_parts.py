@@ -1,6 +1,6 @@
 """GPU parity of the per-pixel backward kernels where the regions of the screen are cut into parts that different XCDs take: up to
 64 regions in a launch, or a layer 0 that may blend four fragments a pixel; one more region, and one fragment less, on the other
-side. Every pixel's records must be there, and the sums over pixels must come out whichever workgroup added them up."""
+side. The FUZZY_BLEND kernel for long lists looks at every eighth workgroup or so of these grids. Every pixel's records must be there, and the sums over pixels must come out whichever workgroup added them up."""
 import numpy as np
 import pytest
 import torch

@@ -139,7 +139,7 @@ __device__ __forceinline__ void blend_backward(const BackwardPass& a)
 
     clear_accumulators(a.clear);
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const TilePixel px = tile_pixel(a.tiles, a.ly);
+    const TilePixel px = tile_pixel(a.tiles, a.ly, blockIdx.x);
     const int l        = px.l;
     const int lw = a.ly.w[l], lh = a.ly.h[l];
     const size_t plane = (size_t)lw * lh;
@@ -537,8 +537,13 @@ constexpr int kFuzzyLongColumn = 6;   // background row, column 6, as bits: 2 ho
 // the dense kernel left for the workgroup; the others write rows of their own, which fold_background_rows_kernel adds up
 // into kFuzzyFoldRows rows right behind the per-workgroup ones, so that the sum over the rows stays short:
 // [workgroups] [kFuzzyFoldRows] [replica 1: workgroups] [replica 2: workgroups] ...
-constexpr int kFuzzyReplicas   = 4;
+// Most workgroups have no such list, so one of this kernel looks at kFuzzyStride of the dense kernel's, whose lists it takes one
+// workgroup after the other. Two views of 1237x701 without a cut: 88 us with 4 replicas and a workgroup for each, 88 with 4 or 8
+// looked at (what lasts is the waves with the most lists), 80 with 8 replicas and 8 looked at, 90 with 16 replicas.
+constexpr int kFuzzyReplicas   = 8;
 constexpr int kFuzzyFoldRows   = 256;
+constexpr int kFuzzyStride     = 8;  // tiles' workgroups of the dense kernel that one of the second kernel looks at
+static_assert(kFuzzyStride * kBackgroundRow <= kWave, "a wave looks at them, and clears their rows, at once");
 
 template <int C, int DENSE>
 __device__ __forceinline__ void blend_backward_fuzzy(const BackwardPass& a, float depth_accept)
@@ -556,7 +561,7 @@ __device__ __forceinline__ void blend_backward_fuzzy(const BackwardPass& a, floa
     __shared__ float red[kWaves][C + 3];
     clear_accumulators(a.clear);
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const TilePixel px = tile_pixel(a.tiles, a.ly);
+    const TilePixel px = tile_pixel(a.tiles, a.ly, blockIdx.x);
     float4* partial_l  = a.partial;  // (records are addressed by gradient_record)
     const bool with_background = !a.use_environment_map;  // every list ends with the background element
     float bg_grad[C];
@@ -1041,23 +1046,29 @@ __global__ void __launch_bounds__(kBlock) blend_backward_fuzzy_views_kernel(PerV
 // twice: the first pass only adds up the terms, the second has the total and writes (a list of up to 64 fragments has
 // its total inside its one step and is processed once). The elements of a bucket that was
 // still open at the end of their step get the position part of their record there and the bucket's part when it
-// closes, from a loop over their keys. Same grid as the dense kernel; a workgroup without such a list leaves at once.
+// closes, from a loop over their keys. Grid: fuzzy_long_grid x kFuzzyReplicas.
 template <int C>
 __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a, float depth_accept, uint32_t dense_max)
 {
     constexpr int kWaves = kBlock / kWave;
     __shared__ float red[kWaves][C];
     const uint32_t replica = blockIdx.y;
-    const uint32_t state = __float_as_uint(a.background_partial[(size_t)blockIdx.x * kBackgroundRow + kFuzzyLongColumn]);
-    float* row      = a.background_partial + (size_t)(state >> 1) * kBackgroundRow;
-    float* row_mine = replica == 0u ? row : row + ((size_t)kFuzzyFoldRows + (size_t)replica * gridDim.x) * kBackgroundRow;
-    if ((state & 1u) == 0u)
-    {
-        if (replica != 0u && threadIdx.x < (uint32_t)kBackgroundRow) row_mine[threadIdx.x] = 0.f;
-        return;
-    }
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const TilePixel px = tile_pixel(a.tiles, a.ly);
+    // kFuzzyStride of the dense kernel's workgroups: lanes 8 k .. 8 k + 7 stand for the k-th of them, this grid's size apart
+    const uint32_t all      = a.tiles.regions_per_xcd * a.tiles.groups_per_region * kXcds;
+    const uint32_t own      = blockIdx.x + (uint32_t)(lane / kBackgroundRow) * gridDim.x;
+    const bool there        = lane < kFuzzyStride * kBackgroundRow && own < all;
+    const uint32_t own_state = there ? __float_as_uint(a.background_partial[(size_t)own * kBackgroundRow + kFuzzyLongColumn]) : 0u;
+    const size_t replica_rows = replica == 0u ? 0 : (size_t)kFuzzyFoldRows + (size_t)replica * all;
+    if (wave == 0 && there && replica != 0u && (own_state & 1u) == 0u)
+        a.background_partial[(replica_rows + (own_state >> 1)) * kBackgroundRow + lane % kBackgroundRow] = 0.f;
+    uint64_t with_list = __ballot((own_state & 1u) != 0u && lane % kBackgroundRow == 0);  // the same in all waves
+  for (; with_list != 0ull; with_list &= with_list - 1ull)
+  {
+    const int from       = __ffsll((unsigned long long)with_list) - 1;
+    const uint32_t home  = (uint32_t)__builtin_amdgcn_readlane((int)own_state, from) >> 1;
+    float* row_mine      = a.background_partial + (replica_rows + home) * kBackgroundRow;
+    const TilePixel px   = tile_pixel(a.tiles, a.ly, blockIdx.x + (uint32_t)(from / kBackgroundRow) * gridDim.x);
     const FuzzyPixel f = fuzzy_pixel<C>(a, px);
     float4* partial_l  = a.partial;  // (records are addressed by gradient_record)
     const bool with_background = !a.use_environment_map;
@@ -1361,11 +1372,13 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
         const float sum = threadIdx.x < C ? (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]) : 0.f;
         if (replica == 0u)
         {
-            if (threadIdx.x < C) row[threadIdx.x] += sum;
+            if (threadIdx.x < C) row_mine[threadIdx.x] += sum;
         }
         else
             row_mine[threadIdx.x] = sum;
     }
+    __syncthreads();  // (the next one uses the array again)
+  }
 }
 
 template <int C>

@@ -441,14 +441,14 @@ struct TilePixel
                      // added up in the same order either way
 };
 
-__device__ __forceinline__ TilePixel tile_pixel(const TileMap& tm, const LayerTable& ly)
+__device__ __forceinline__ TilePixel tile_pixel(const TileMap& tm, const LayerTable& ly, uint32_t block)
 {
     TilePixel r;
     r.active = false;
     r.l = r.x = r.y = 0;
     r.q = r.local = 0;
-    const uint32_t xcd  = blockIdx.x % kXcds;
-    const uint32_t slot = blockIdx.x / kXcds;
+    const uint32_t xcd  = block % kXcds;
+    const uint32_t slot = block / kXcds;
     const uint32_t row  = slot / tm.groups_per_region;  // of kXcds regions
     uint32_t t          = slot - row * tm.groups_per_region;  // workgroup inside the region, coarsest layer first
     // layer L-1 has 1 tile per region, L-2 has 4, L-3 has 16, ...; split[l] workgroups per tile

@@ -314,6 +314,17 @@ TileMap make_tile_map(const LayerTable& ly, const double* list_bound = nullptr, 
     return m;
 }
 
+// Workgroups of the FUZZY_BLEND kernel that takes a wave per list: as many as look at all of the dense kernel's, kFuzzyStride
+// each. Those one looks at lie a region and an eighth apart or so (in slots of an XCD), or the coarse layers of all
+// regions, which hold most of the long lists, would be the same workgroups'.
+uint32_t fuzzy_long_grid(const TileMap& m)
+{
+    const uint32_t slots = m.regions_per_xcd * m.groups_per_region, region = m.groups_per_region, apart = (region + 7) / 8;
+    uint32_t n = (slots + kFuzzyStride - 1) / kFuzzyStride;
+    n += (region + apart - n % region) % region;
+    return std::min(n, slots) * kXcds;
+}
+
 uint32_t tile_grid(const TileMap& m)
 {
     return m.regions_per_xcd * m.groups_per_region * kXcds;
@@ -1040,14 +1051,14 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
                         }
                         if (one)
                         {
-                            hipLaunchKernelGGL(blend_backward_fuzzy_long_kernel<kC>, dim3(tiles_x, kFuzzyReplicas), blk, 0, stream, bp,
+                            hipLaunchKernelGGL(blend_backward_fuzzy_long_kernel<kC>, dim3(fuzzy_long_grid(tiles), kFuzzyReplicas), blk, 0, stream, bp,
                                                accept, dense_max);
                             hipLaunchKernelGGL(fold_background_rows_kernel, dim3(kFuzzyFoldRows), blk, 0, stream, folds.v[0].rows,
                                                folds.v[0].num_rows, folds.v[0].folded);
                         }
                         else
                         {
-                            hipLaunchKernelGGL(blend_backward_fuzzy_long_views_kernel<kC>, dim3(tiles_x, kFuzzyReplicas, (unsigned)count),
+                            hipLaunchKernelGGL(blend_backward_fuzzy_long_views_kernel<kC>, dim3(fuzzy_long_grid(tiles), kFuzzyReplicas, (unsigned)count),
                                                blk, 0, stream, views, accept, dense_max);
                             hipLaunchKernelGGL(fold_background_rows_views_kernel, dim3(kFuzzyFoldRows, (unsigned)count), blk, 0,
                                                stream, folds);
