@@ -291,6 +291,7 @@ size_t pixel_gradient_base(const vetrast_workspace_layout& lay)
     return align_up(lay.partial_base + (size_t)lay.fragment_capacity / (size_t)lay.hits_per_layer * kRecordRoom, kAlign);
 }
 
+// `views`: of a launch, see kPartsRegions.
 TileMap make_tile_map(const LayerTable& ly, const double* list_bound = nullptr, bool split_all = false, int views = 1)
 {
     TileMap m;
