@@ -27,3 +27,19 @@ def test_backward_scratch(mode, points, views, layers, w, h):
     # are more than 256 workgroups of points
     if points > 256 * 256:
         assert points * layers * 32 >= lay.view_lanes * 64 * 160
+
+
+@pytest.mark.parametrize("mode", [abi.RENDER_FULL_BLEND, abi.RENDER_FUZZY_BLEND, abi.RENDER_BILINEAR_BLEND])
+@pytest.mark.parametrize("points,views,layers,w,h", [(0, 1, 1, 16, 16), (1, 1, 4, 17, 33), (777_777, 2, 4, 1237, 701), (60_007, 1, 4, 203, 155),
+                                                     (100_000, 3, 5, 1000, 700), (2_000_000, 4, 4, 1920, 1080)])
+def test_background_rows_take_what_callers_have_reserved(mode, points, views, layers, w, h):
+    """The rows of background-gradient sums have 128 bytes for each workgroup there can be (a tile of each layer in regions of one
+    coarsest tile, eight regions at a time, four workgroups to a tile), and 8 KiB: buffers of that size have to stay large enough."""
+    lay = abi.WorkspaceLayout()
+    assert abi.load_library().vetrast_workspace_layout_for_mode(points, views, layers, w, h, mode, C.byref(lay)) == 0
+    span = 16 << (layers - 1)
+    regions = ((w + span - 1) // span) * ((h + span - 1) // span)
+    groups = (regions + 7) // 8 * 8 * 4 * sum(4**l for l in range(layers))
+    backward_block = lay.background_partial_base - lay.partial_base + _align(groups * 128 + 256 * 32)
+    forward_block = lay.forward_only_bytes - lay.log_base - lay.lane_scratch_stride * (lay.view_lanes - 1)
+    assert lay.lane_scratch_stride == max(forward_block, backward_block)

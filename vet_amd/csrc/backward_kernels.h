@@ -521,29 +521,33 @@ __device__ __forceinline__ FuzzyPixel fuzzy_pixel(const BackwardPass& a, const T
 // slot's depths. Sums and products are combined pairwise instead of front to back, which moves the results by
 // rounding only. The table that says which pixel a lane's fragment belongs to holds kWaveItems slots; a wave whose
 // pixels need more goes through it in batches. Longer lists are left to blend_backward_fuzzy_long_kernel; the
-// workgroup says in column kFuzzyLongColumn of the row of its own number whether it has any, beside the row its sums go to
-// (2 home + 1, see TilePixel::home), so that the workgroups of the second kernel that have nothing to do leave after one load (with
-// the place of their tile worked out first that kernel took 117 us instead of 87).
+// workgroup says in column kFuzzyLongColumn of the row of its own number whether it has any, so that the workgroups of the second
+// kernel that have nothing to do leave after one load (with the place of their tile worked out first that kernel took 117 us
+// instead of 87).
 constexpr int kFuzzyDense      = 32;  // longest list of the dense layout
 constexpr int kFuzzyNarrow     = 16;  // longest slot that lies inside a row of 16 lanes
 // The kernel is compiled for DENSE = kFuzzyNarrow (no slot spans rows: fewer registers, more waves per SIMD) and for
 // DENSE = kFuzzyDense; the host takes the narrow one where the cut keeps every list that short, and also where lists
 // beyond kFuzzyDense may exist: those go to blend_backward_fuzzy_long_kernel, which then is the faster one for the lists
 // of 17 to 32 fragments as well (measured; slots of 64 lanes lost against it too).
-constexpr int kFuzzyLongColumn = 6;   // background row, column 6, as bits: 2 home + whether the workgroup has a list for the wave-per-list kernel
+constexpr int kFuzzyLongColumn = 6;   // background row, column 6: the workgroup has a list for the wave-per-list kernel
 // The wave-per-list kernel is launched kFuzzyReplicas times over (grid.y): replica r takes every kFuzzyReplicas-th long
 // list of a wave's pixels. Long lists cluster (where a surface is seen edge-on a whole strip of pixels holds hundreds
-// of fragments each), and a wave takes its lists one after the other. Replica 0 adds its background sums to the row
-// the dense kernel left for the workgroup; the others write rows of their own, which fold_background_rows_kernel adds up
-// into kFuzzyFoldRows rows right behind the per-workgroup ones, so that the sum over the rows stays short:
-// [workgroups] [kFuzzyFoldRows] [replica 1: workgroups] [replica 2: workgroups] ...
+// of fragments each), and a wave takes its lists one after the other. A workgroup of any replica adds the background up over all
+// its lists and writes it to a row of its own, of kLongRow floats; fold_background_rows_kernel adds those up into kFuzzyFoldRows
+// rows right behind the dense kernel's, so that the sum over the rows stays short:
+// [workgroups of the dense kernel] [kFuzzyFoldRows] [replica 0: workgroups] [replica 1: workgroups] ...
 // Most workgroups have no such list, so one of this kernel looks at kFuzzyStride of the dense kernel's, whose lists it takes one
 // workgroup after the other. Two views of 1237x701 without a cut: 88 us with 4 replicas and a workgroup for each, 88 with 4 or 8
 // looked at (what lasts is the waves with the most lists), 80 with 8 replicas and 8 looked at, 90 with 16 replicas.
 constexpr int kFuzzyReplicas   = 8;
 constexpr int kFuzzyFoldRows   = 256;
+constexpr int kLongRow         = 4;
 constexpr int kFuzzyStride     = 8;  // tiles' workgroups of the dense kernel that one of the second kernel looks at
-static_assert(kFuzzyStride * kBackgroundRow <= kWave, "a wave looks at them, and clears their rows, at once");
+static_assert(kFuzzyStride <= kWave && kLongRow >= VETRAST_MAX_CHANNELS, "a wave looks at them at once");
+// Room for the rows of the second kernel, in rows of kBackgroundRow floats for a workgroup that the dense kernel may have (every layer
+// split): what callers have reserved.
+constexpr int kLongRoom        = 3;
 
 template <int C, int DENSE>
 __device__ __forceinline__ void blend_backward_fuzzy(const BackwardPass& a, float depth_accept)
@@ -1017,10 +1021,8 @@ __device__ __forceinline__ void blend_backward_fuzzy(const BackwardPass& a, floa
     float* row = a.background_partial + (size_t)px.home * kBackgroundRow;
     if (threadIdx.x <= C) row[threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
     if (threadIdx.x == C + 1)
-    {
-        const float any = (red[0][C + 1] + red[1][C + 1]) + (red[2][C + 1] + red[3][C + 1]);
-        a.background_partial[(size_t)blockIdx.x * kBackgroundRow + kFuzzyLongColumn] = __uint_as_float((px.home << 1) | (any != 0.f ? 1u : 0u));
-    }
+        a.background_partial[(size_t)blockIdx.x * kBackgroundRow + kFuzzyLongColumn] =
+            (red[0][C + 1] + red[1][C + 1]) + (red[2][C + 1] + red[3][C + 1]);
 }
 
 template <int C, int DENSE>
@@ -1054,27 +1056,27 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
     __shared__ float red[kWaves][C];
     const uint32_t replica = blockIdx.y;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    // kFuzzyStride of the dense kernel's workgroups: lanes 8 k .. 8 k + 7 stand for the k-th of them, this grid's size apart
-    const uint32_t all      = a.tiles.regions_per_xcd * a.tiles.groups_per_region * kXcds;
-    const uint32_t own      = blockIdx.x + (uint32_t)(lane / kBackgroundRow) * gridDim.x;
-    const bool there        = lane < kFuzzyStride * kBackgroundRow && own < all;
-    const uint32_t own_state = there ? __float_as_uint(a.background_partial[(size_t)own * kBackgroundRow + kFuzzyLongColumn]) : 0u;
-    const size_t replica_rows = replica == 0u ? 0 : (size_t)kFuzzyFoldRows + (size_t)replica * all;
-    if (wave == 0 && there && replica != 0u && (own_state & 1u) == 0u)
-        a.background_partial[(replica_rows + (own_state >> 1)) * kBackgroundRow + lane % kBackgroundRow] = 0.f;
-    uint64_t with_list = __ballot((own_state & 1u) != 0u && lane % kBackgroundRow == 0);  // the same in all waves
-  for (; with_list != 0ull; with_list &= with_list - 1ull)
-  {
-    const int from       = __ffsll((unsigned long long)with_list) - 1;
-    const uint32_t home  = (uint32_t)__builtin_amdgcn_readlane((int)own_state, from) >> 1;
-    float* row_mine      = a.background_partial + (replica_rows + home) * kBackgroundRow;
-    const TilePixel px   = tile_pixel(a.tiles, a.ly, blockIdx.x + (uint32_t)(from / kBackgroundRow) * gridDim.x);
-    const FuzzyPixel f = fuzzy_pixel<C>(a, px);
-    float4* partial_l  = a.partial;  // (records are addressed by gradient_record)
-    const bool with_background = !a.use_environment_map;
+    // lane k stands for the k-th of kFuzzyStride workgroups of the dense kernel, this grid's size apart
+    const uint32_t all = a.tiles.regions_per_xcd * a.tiles.groups_per_region * kXcds;
+    const uint32_t own = blockIdx.x + (uint32_t)lane * gridDim.x;
+    const bool there   = lane < kFuzzyStride && own < all;
+    uint64_t with_list = __ballot(there && a.background_partial[(size_t)own * kBackgroundRow + kFuzzyLongColumn] != 0.f);  // the same in all waves
+    float* row = a.background_partial + ((size_t)all + kFuzzyFoldRows) * kBackgroundRow + ((size_t)replica * gridDim.x + blockIdx.x) * kLongRow;
+    if (with_list == 0ull)
+    {
+        if (threadIdx.x < (uint32_t)kLongRow) row[threadIdx.x] = 0.f;
+        return;
+    }
     float bg_grad[C];  // summed over the wave at the end: every lane adds what it computes for lane 0's sake once
 #pragma unroll
     for (int ci = 0; ci < C; ++ci) bg_grad[ci] = 0.f;
+  for (; with_list != 0ull; with_list &= with_list - 1ull)
+  {
+    const int from     = __ffsll((unsigned long long)with_list) - 1;
+    const TilePixel px = tile_pixel(a.tiles, a.ly, blockIdx.x + (uint32_t)from * gridDim.x);
+    const FuzzyPixel f = fuzzy_pixel<C>(a, px);
+    float4* partial_l  = a.partial;  // (records are addressed by gradient_record)
+    const bool with_background = !a.use_environment_map;
     auto everywhere = [&](float v, int src) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), src)); };
 
     uint64_t todo = __ballot(f.n > dense_max);
@@ -1360,6 +1362,7 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
             }
         }
     }
+  }
 #pragma unroll
     for (int ci = 0; ci < C; ++ci)
     {
@@ -1367,18 +1370,8 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
         if (lane == 0) red[wave][ci] = s;
     }
     __syncthreads();
-    if (threadIdx.x < (uint32_t)kBackgroundRow)
-    {
-        const float sum = threadIdx.x < C ? (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]) : 0.f;
-        if (replica == 0u)
-        {
-            if (threadIdx.x < C) row_mine[threadIdx.x] += sum;
-        }
-        else
-            row_mine[threadIdx.x] = sum;
-    }
-    __syncthreads();  // (the next one uses the array again)
-  }
+    if (threadIdx.x < (uint32_t)kLongRow)
+        row[threadIdx.x] = threadIdx.x < C ? (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]) : 0.f;
 }
 
 template <int C>
@@ -1395,21 +1388,21 @@ __global__ void __launch_bounds__(kBlock) blend_backward_fuzzy_long_views_kernel
     blend_backward_fuzzy_long<C>(views.v[blockIdx.z], depth_accept, dense_max);
 }
 
-// Adds `num_rows` rows of kBackgroundRow floats up into kFuzzyFoldRows rows: workgroup j takes rows j, j + 256, ... in a
-// fixed order (32 threads per column, each every 32nd of the workgroup's rows, then the 32 partial sums one after the other).
+// Adds `num_rows` rows of kLongRow floats up into kFuzzyFoldRows rows of kBackgroundRow: workgroup j takes rows j, j + 256, ... in a
+// fixed order (64 threads per column, each every 64th of the workgroup's rows, then the 64 partial sums one after the other).
 __device__ __forceinline__ void fold_background_rows(const float* __restrict__ rows, int num_rows, float* __restrict__ folded)
 {
-    __shared__ float part[kBlock / kBackgroundRow][kBackgroundRow];
-    const int column = threadIdx.x % kBackgroundRow, sub = threadIdx.x / kBackgroundRow;
+    constexpr int kThreads = kBlock / kLongRow;
+    __shared__ float part[kThreads][kLongRow];
+    const int column = threadIdx.x % kLongRow, sub = threadIdx.x / kLongRow;
     float sum = 0.f;
-    for (int r = blockIdx.x + kFuzzyFoldRows * sub; r < num_rows; r += kFuzzyFoldRows * (kBlock / kBackgroundRow))
-        sum += rows[(size_t)r * kBackgroundRow + column];
+    for (int r = blockIdx.x + kFuzzyFoldRows * sub; r < num_rows; r += kFuzzyFoldRows * kThreads) sum += rows[(size_t)r * kLongRow + column];
     part[sub][column] = sum;
     __syncthreads();
     if (threadIdx.x < (uint32_t)kBackgroundRow)
     {
         float total = 0.f;
-        for (int k = 0; k < kBlock / kBackgroundRow; ++k) total += part[k][threadIdx.x];
+        for (int k = 0; threadIdx.x < (uint32_t)kLongRow && k < kThreads; ++k) total += part[k][threadIdx.x];
         folded[(size_t)blockIdx.x * kBackgroundRow + threadIdx.x] = total;
     }
 }

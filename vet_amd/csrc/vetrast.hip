@@ -616,8 +616,8 @@ int vetrast_workspace_layout_for_mode(int32_t N, int32_t B, int32_t L, int32_t w
     // (the 2x2 splat's block is no smaller than a record for each corner would make it, which is what callers have reserved)
     at = std::max(at, shared_base + align_up(cap * kRecordRoom, kAlign));
     lay->background_partial_base = at;
-    // (the FUZZY_BLEND kernel that takes a wave per list keeps rows per replica and kFuzzyFoldRows rows they are folded into)
-    at += align_up(((size_t)tile_grid(make_tile_map(t, nullptr, true)) * kFuzzyReplicas + kFuzzyFoldRows) * kBackgroundRow * sizeof(float), kAlign);
+    // (the FUZZY_BLEND kernel that takes a wave per list keeps rows of its own and kFuzzyFoldRows rows they are folded into)
+    at += align_up(((size_t)tile_grid(make_tile_map(t, nullptr, true)) * (1 + kLongRoom) + kFuzzyFoldRows) * kBackgroundRow * sizeof(float), kAlign);
     const size_t backward_block = align_up(at, kAlign) - shared_base;
     lay->lane_scratch_stride    = std::max(forward_block, backward_block);
     lay->forward_only_bytes     = shared_base + lay->lane_scratch_stride * (lanes - 1) + forward_block;
@@ -1042,24 +1042,25 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
                     if (beyond_dense)
                     {
                         const uint32_t dense_max = (uint32_t)(wide ? kFuzzyDense : kFuzzyNarrow);
-                        // the rows of replicas 1 .. into kFuzzyFoldRows rows behind the per-workgroup ones
+                        // the second kernel's rows into kFuzzyFoldRows rows behind the dense one's
+                        const unsigned long_x = fuzzy_long_grid(tiles);
                         PerView<FoldArgs> folds{};
                         for (int k = 0; k < count; ++k)
                         {
                             folds.v[k].rows     = views.v[k].background_partial + ((size_t)kFuzzyFoldRows + tiles_x) * kBackgroundRow;
-                            folds.v[k].num_rows = (int)((kFuzzyReplicas - 1) * tiles_x);
+                            folds.v[k].num_rows = (int)(kFuzzyReplicas * long_x);
                             folds.v[k].folded   = views.v[k].background_partial + (size_t)tiles_x * kBackgroundRow;
                         }
                         if (one)
                         {
-                            hipLaunchKernelGGL(blend_backward_fuzzy_long_kernel<kC>, dim3(fuzzy_long_grid(tiles), kFuzzyReplicas), blk, 0, stream, bp,
+                            hipLaunchKernelGGL(blend_backward_fuzzy_long_kernel<kC>, dim3(long_x, kFuzzyReplicas), blk, 0, stream, bp,
                                                accept, dense_max);
                             hipLaunchKernelGGL(fold_background_rows_kernel, dim3(kFuzzyFoldRows), blk, 0, stream, folds.v[0].rows,
                                                folds.v[0].num_rows, folds.v[0].folded);
                         }
                         else
                         {
-                            hipLaunchKernelGGL(blend_backward_fuzzy_long_views_kernel<kC>, dim3(fuzzy_long_grid(tiles), kFuzzyReplicas, (unsigned)count),
+                            hipLaunchKernelGGL(blend_backward_fuzzy_long_views_kernel<kC>, dim3(long_x, kFuzzyReplicas, (unsigned)count),
                                                blk, 0, stream, views, accept, dense_max);
                             hipLaunchKernelGGL(fold_background_rows_views_kernel, dim3(kFuzzyFoldRows, (unsigned)count), blk, 0,
                                                stream, folds);
