@@ -1,6 +1,6 @@
-"""GPU parity of the per-pixel backward kernels where the regions of the screen are cut into parts that different XCDs take: up to
-64 regions in a launch, or a layer 0 that may blend four fragments a pixel; one more region, and one fragment less, on the other
-side. The FUZZY_BLEND kernel for long lists looks at every eighth workgroup or so of these grids. Every pixel's records must be there, and the sums over pixels must come out whichever workgroup added them up."""
+"""GPU parity of the per-pixel backward kernels where the regions of the screen are cut into parts that different XCDs take, and where
+they stay whole (test_region_rule_cpu.py has the rule). Every pixel's records must be there, and the sums over pixels must come out
+whichever workgroup added them up."""
 import numpy as np
 import pytest
 import torch
@@ -12,11 +12,14 @@ from vet_amd.rasterizer import DeviceScene, make_params
 pytestmark = pytest.mark.gpu
 
 
-# (width, height, layers, points, cut): 1 region of 5, 3, 2 and 1 layers; 8, 9, 64 and 65 regions; long lists, 66 regions
+# (width, height, layers, points, cut): 1 region of 5, 3, 2 and 1 layers; 8, 9, 64 and 65 regions; long lists, 66 regions; four layers with 4, 12
+# and 16 regions (parts, parts, whole), 16 in rows of eight with lists below and from the line on, five layers with strips of split tiles
 @pytest.mark.parametrize("mode", [1, 2, 3])
 @pytest.mark.parametrize("w,h,layers,points,cut", [(171, 133, 5, 20_000, -1), (61, 57, 3, 3_000, 40), (31, 30, 2, 3_000, -1), (16, 9, 1, 500, 16),
                                                    (250, 118, 3, 20_000, 16), (180, 190, 3, 20_000, -1), (512, 511, 3, 30_000, 16),
-                                                   (832, 316, 3, 30_000, 16), (350, 176, 2, 260_000, 3), (350, 176, 2, 260_000, 20)])
+                                                   (832, 316, 3, 30_000, 16), (350, 176, 2, 260_000, 3), (350, 176, 2, 260_000, 20),
+                                                   (203, 155, 4, 40_000, -1), (500, 371, 4, 20_000, 16), (500, 386, 4, 20_000, 16), (1021, 131, 4, 30_000, 16),
+                                                   (1021, 131, 4, 150_000, 16), (290, 270, 5, 120_000, 12)])
 def test_every_region_is_taken(mode, w, h, layers, points, cut, rasterizer, oracle):
     print(f"[case] region parts: mode {mode}, {w}x{h}, {layers} layers, {points} points, cut {cut}", flush=True)
     scene = synthetic.config2(num_points=points, seed=w, w=w, h=h, num_layers=layers, K=cut)

@@ -404,19 +404,13 @@ __device__ __forceinline__ size_t gradient_record(int point_major, int N, int L,
 // round-robin to the 8 XCDs (each with its own L2), so workgroup b belongs to XCD b % 8 and takes slot b / 8 of that
 // XCD's run of regions (region r goes to XCD r % 8): what one layer's tiles pulled into the XCD's L2 is still there
 // when the next layer's tiles of the region ask for the same points.
-// Where a launch has few regions, or its lists may be long, an XCD's regions hold a multiple of another's fragments (up to
-// 8 times, for one region), and the kernel lasts as long as the fullest XCD. There a region is cut into parts
-// (parts_log: 4^parts_log of them) and its part (x, y) is given to the XCD x + 3 y further on; on row by row of eight regions
-// every XCD then has each part of one of them. Per-pixel kernel, whole regions against 16 parts (us, kernel traces on one card):
-// six 228x228 crops of 5 layers 59 -> 40, 9.5 million points in 813x436 167 -> 139, two 602x267 crops of 3 million points 81 -> 52,
-// four 512x512 crops with the 2x2 splat 92 -> 84, ten million points at 1080p 545 -> 521. Everywhere it would cost
-// more than it gives, since a cache line of an image then belongs to several XCDs: four town views 387 -> 402, benchmark frame 107 ->
-// 111, two FUZZY_BLEND views of 1237x701 91 -> 94 (64 parts: 417, 114, 96; 4 parts: 392, 108, 92). Hence kPartsRegions, between the
-// four crops' 64 regions and those views' 120, and kPartsListLength, between the 2x2 splat's 3.9 fragments a pixel at
-// 1080p (152 either way) and the ten million points' 4.8.
+// Where that leaves an XCD's regions with a multiple of another's fragments (up to 8 times, for one region) the kernel lasts as
+// long as the fullest XCD, and a region is cut into parts (parts_log: 4^parts_log of them), whose part (x, y) is given to the XCD
+// x + 3 y further on; of a row of eight regions every XCD then has each part of one of them. (One region's 16 parts fall on the
+// XCDs unevenly, one to three each.) 4, 16 and 64 parts of every region, us, against whole ones: four town views 392, 402, 417 / 387,
+// benchmark frame 108, 111, 114 / 107, two FUZZY_BLEND views of 1237x701 92, 94, 96 / 91, ten million points 528, 520, 525 / 544.
+// region_rule.h has the rule and what it was measured on.
 constexpr int kXcds = 8;
-constexpr uint32_t kPartsRegions  = 64;   // regions of all views of a launch
-constexpr double kPartsListLength = 4.0;  // fragments a pixel of layer 0 may blend
 // A layer whose pixels hold long lists is split: a workgroup then owns one 16x4 strip of a tile and each of its waves
 // one row of 16 pixels (lanes 16..63 carry no pixel, only fragments), so that such a layer (few pixels, many fragments)
 // is spread over four times as many waves, each with a quarter of the rounds to run one after the other.

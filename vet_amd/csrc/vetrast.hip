@@ -18,6 +18,7 @@
 #include "build_kernels.h"
 #include "backward_kernels.h"
 #include "lift_kernels.h"
+#include "region_rule.h"
 
 using namespace vetrast;
 
@@ -291,8 +292,8 @@ size_t pixel_gradient_base(const vetrast_workspace_layout& lay)
     return align_up(lay.partial_base + (size_t)lay.fragment_capacity / (size_t)lay.hits_per_layer * kRecordRoom, kAlign);
 }
 
-// `views`: of a launch, see kPartsRegions.
-TileMap make_tile_map(const LayerTable& ly, const double* list_bound = nullptr, bool split_all = false, int views = 1)
+// `list`: fragments a pixel of layer 0 may blend, see regions_in_parts.
+TileMap make_tile_map(const LayerTable& ly, const double* list_bound = nullptr, bool split_all = false, double list = 0.0)
 {
     TileMap m;
     std::memset(&m, 0, sizeof(m));
@@ -308,7 +309,7 @@ TileMap make_tile_map(const LayerTable& ly, const double* list_bound = nullptr, 
     uint32_t tiles      = 0;
     for (int k = 0; k < ly.L; ++k) tiles += 1u << (2 * k);
     m.tiles_per_region = tiles;
-    if (m.regions * (uint32_t)views <= kPartsRegions || (list_bound && list_bound[0] >= kPartsListLength)) m.parts_log = 2;
+    if (regions_in_parts(ly.L, m.regions_x, m.regions, list)) m.parts_log = 2;
     m.regions_per_xcd  = (m.regions + kXcds - 1) / kXcds;
     m.groups_per_region = 0;
     for (int l = 0; l < ly.L; ++l) m.groups_per_region += (1u << (2 * (ly.L - 1 - l))) * m.split[l];
@@ -920,7 +921,8 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
         list_bound[l] = (double)N * hits / ((double)ly.w[l] * ly.h[l]);
         if (p.debug_max_list_length > 0) list_bound[l] = std::min(list_bound[l], (double)p.debug_max_list_length);
     }
-    const TileMap tiles = make_tile_map(ly, list_bound, false, std::min(B, std::max(1, lay.view_lanes)));
+    const double list   = fragments_a_pixel_may_blend((double)N * hits, p.expected_fragments[0], ly.w[0], ly.h[0], p.debug_max_list_length);
+    const TileMap tiles = make_tile_map(ly, list_bound, false, list);
     void* ws            = a->workspace;
 
     // The per-point kernel overwrites every gradient row in the first view, so the zeros_like fills of
