@@ -12,6 +12,39 @@ from vet_amd.rasterizer import DeviceScene, make_params
 pytestmark = pytest.mark.gpu
 
 
+def background_weights(ref, scene, params):
+    """FUZZY_BLEND: the weight T of every pixel's background element and the length of its list, T in 64 bits: the product over the
+    list's buckets of one minus their mean confidence. A bucket ends where a depth leaves the range behind its first (in 32 bits, as the
+    rule has it)."""
+    offsets, fragments = ref.offsets[0].astype(np.int64), ref.fragments[0]
+    length = np.diff(offsets)
+    if params.debug_max_list_length > 0:
+        length = np.minimum(length, params.debug_max_list_length)
+    confidence = scene.confidence.reshape(-1).astype(np.float64)
+    t, total, count = np.ones(len(length)), np.zeros(len(length)), np.zeros(len(length))
+    first = np.zeros(len(length), np.float32)
+    for i in range(int(length.max())):
+        q = np.nonzero(length > i)[0]
+        key = fragments[offsets[q] + i]
+        depth = (key >> np.uint64(32)).astype(np.uint32).view(np.float32)
+        new = q[~(depth - first[q] < np.float32(params.depth_accept_blend))]
+        t[new] *= 1.0 - total[new] / np.maximum(count[new], 1)
+        total[new], count[new] = 0.0, 0
+        first[new] = depth[np.isin(q, new, assume_unique=True)]
+        total[q] += confidence[(key & np.uint64(0xFFFFFFFF)).astype(np.int64)]
+        count[q] += 1
+    return t * (1.0 - total / np.maximum(count, 1)), length
+
+
+def fuzzy_background(ref, scene, params, grad_out, channel):
+    """FUZZY_BLEND's background gradient, sum T g, in 64 bits, and how far 32 bits may be off. T: a list of n fragments in b <= n buckets takes
+    fewer than n + 3 b roundings of 2^-24, each of a number of at most one. The sum: fewer than 256 additions one after the
+    other (64 lists of a wave, 8 steps to its workgroup's sum, 65 where rows are folded, then as in the other modes)."""
+    weight, length = background_weights(ref, scene, params)
+    g = np.concatenate([t[0, channel].reshape(-1).astype(np.float64) for t in grad_out])
+    return (weight * g).sum(), 2.0**-24 * (256 * np.abs(weight * g).sum() + 4 * (length * np.abs(g)).sum())
+
+
 # (width, height, layers, points, cut): 1 region of 5, 3, 2 and 1 layers; 8, 9, 64 and 65 regions; long lists, 66 regions; four layers with 4, 12
 # and 16 regions (parts, parts, whole), 16 in rows of eight with lists below and from the line on, five layers with strips of split tiles
 @pytest.mark.parametrize("mode", [1, 2, 3])
@@ -35,11 +68,41 @@ def test_every_region_is_taken(mode, w, h, layers, points, cut, rasterizer, orac
         assert max_rel_err(got[key].cpu().numpy(), want[key]) <= 1e-4, key  # 32-bit sums in another order
     # A pixel adds T g to the background's gradient (not where the 2x2 splat's blend has stopped in front of it), in fewer than 64
     # additions one after the other (10 inside a workgroup, then rows), so it is off by at most 64 roundings of 2^-24 of sum |T g|.
-    # FUZZY_BLEND's T is not the forward pass's: there the check's own sum stands in, of T g with T <= 1, one pixel after the other.
     weights = [ref.weight[0, ref.layer_base(l): ref.layer_base(l) + gw * gh].reshape(gh, gw).astype(np.float64) for l, (gw, gh) in enumerate(ref.sizes)]
-    weights = [np.ones_like(t) if mode == 2 else np.where(t < np.float32(0.001), 0.0, t) if mode == 3 else t for t in weights]
-    additions = 64 + (sum(t.size for t in weights) if mode == 2 else 0)
+    weights = [np.where(t < np.float32(0.001), 0.0, t) if mode == 3 else t for t in weights]
     for c in range(scene.num_channels):
-        terms = [t * g[0, c] for t, g in zip(weights, grad_out)]
-        exact = float(want["background"][c]) if mode == 2 else sum(t.sum() for t in terms)
-        assert abs(float(got["background"][c]) - exact) <= additions * 2.0**-24 * sum(np.abs(t).sum() for t in terms)
+        if mode == 2:
+            exact, bound = fuzzy_background(ref, scene, params, grad_out, c)
+        else:
+            terms = [t * g[0, c] for t, g in zip(weights, grad_out)]
+            exact, bound = sum(t.sum() for t in terms), 64 * 2.0**-24 * sum(np.abs(t).sum() for t in terms)
+        assert abs(float(got["background"][c]) - exact) <= bound
+
+
+# (width, height, layers, points, cut): 66 regions of two layers; 4, 24 and 60 of four, one of five
+@pytest.mark.parametrize("w,h,layers,points,cut", [(350, 176, 2, 260_000, -1), (350, 176, 2, 260_000, 40), (203, 155, 4, 60_000, -1),
+                                                   (700, 500, 4, 200_000, -1), (1237, 701, 4, 300_000, -1), (171, 133, 5, 40_000, 64)])
+def test_every_long_list_is_taken(w, h, layers, points, cut, rasterizer, oracle):
+    """FUZZY_BLEND's second kernel, which looks for lists of more than 16 fragments among up to eight workgroups of the first, eight
+    times over: only their pixels have an upstream gradient, of 0.5 and more, and a depth range of 100 m leaves the
+    background a weight everywhere, so that one list left out or taken twice shows in the background's gradient."""
+    print(f"[case] long lists: {w}x{h}, {layers} layers, {points} points, cut {cut}", flush=True)
+    scene = synthetic.config2(num_points=points, seed=w, w=w, h=h, num_layers=layers, K=cut)
+    params = make_params(scene, render_mode=2, need_point_gradient=1, depth_accept_blend=100.0)
+    ref = oracle.forward(scene, params, num_threads=8)
+    weight, length = background_weights(ref, scene, params)
+    grad_out = [(0.5 + np.abs(g)) * (length[ref.layer_base(l): ref.layer_base(l) + g[0, 0].size].reshape(g.shape[2:]) > 16)
+                for l, g in enumerate(scene.grad_out())]
+    grad_out = [np.ascontiguousarray(g, dtype=np.float32) for g in grad_out]
+    want = oracle.backward(ref, grad_out, num_threads=8)
+    res = rasterizer.forward(DeviceScene(scene), params, save_for_backward=True)
+    got = rasterizer.backward(res, [torch.from_numpy(g).cuda() for g in grad_out])
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(got["point_count"].cpu().numpy(), want["point_count"])
+    for key in ("texture", "confidence", "points"):
+        assert max_rel_err(got[key].cpu().numpy(), want[key]) <= 1e-4, key  # 32-bit sums in another order
+    assert (length > 16).sum() >= 1000
+    for c in range(scene.num_channels):
+        exact, bound = fuzzy_background(ref, scene, params, grad_out, c)
+        assert bound < 0.5 * 0.5 * weight[length > 16].min()  # half of the least that a list adds
+        assert abs(float(got["background"][c]) - exact) <= bound
