@@ -70,6 +70,7 @@ struct BuildPass
     const uint32_t* crowded_counts;
     uint32_t crowded_capacity;
     uint32_t crowded_blocks;         // workgroups at the front of the grid that go through them
+    uint32_t blocks_in_runs;         // workgroups behind those that take their bins in runs (in_runs): whole groups of them, or none
     uint32_t num_bins;
     uint32_t shared_end;             // see CrowdedBins
     int N;
@@ -950,13 +951,16 @@ __device__ __forceinline__ void build_by_workgroup(BuildArgs& args, uint32_t bin
     }
 }
 
-// Consecutive workgroups run on different XCDs, each of which has its own L2. Workgroup k of `all` takes place k of this order
-// instead: of every kXcds * run places an XCD has `run` neighbouring ones, as far as whole groups of them go. What neighbouring bins
-// share (lines of the images and of the lists, descriptors of one block of points) is then in one L2: call of ten million points
-// 1610 -> 1604 us, four town views 996 -> 992, 2x2 splat at 1080p 542 -> 539 (219 -> 211 of the pass), a million points in
-// 1279x719 99.6 -> 97.7, where two runs differ by 0.1 % (the last: 1.4 %). Runs of 32 workgroups with uncrowded bins
-// measured the same as 8, of 4 crowded bins 214 us of the 2x2 splat's pass.
-constexpr uint32_t kWaveBinRun = 8, kCrowdedRun = 16;
+// Consecutive workgroups run on different XCDs, each of which has its own L2. Turn k of the `all` crowded bins goes to place k of this
+// order instead: of every kXcds * run places an XCD has `run` neighbouring ones, as far as whole groups of them go. What neighbouring bins
+// share (lines of the images and of the lists, descriptors of one block of points) is then in one L2. Us of the pass, in turn / in
+// runs: 2x2 splat at 1080p 223 / 220 (runs of 4: 214 where 16 took 211 on another card), dense cloud in it 451 / 441, ten million
+// points 447 / 444, surfaces in 960x540 66 / 65, two views with the 2x2 splat 590 / 575. Uncrowded bins take runs of 8 in launches of more
+// than kRunsFrom workgroups for them: 1237x701 (3560 of them) 35.8 / 34.4, with the 2x2 splat in 1279x719 54.9 / 53.7, ten million points
+// 444 / 441; with fewer, neighbours that hold much are one XCD's and nobody else's: a town in 640x360 (3080) 19.4 / 20.1, four crops of 512x512 (1024)
+// 278 / 281. How many there are comes as an argument: the size of the grid does not lie with the arguments, and waiting for
+// it as well cost every launch 0.3 us (480x270 with three layers 16.9 / 17.2).
+constexpr uint32_t kWaveBinRun = 8, kCrowdedRun = 16, kRunsFrom = 3200;
 __device__ __forceinline__ uint32_t in_runs(uint32_t k, uint32_t all, uint32_t run)
 {
     const uint32_t group = kXcds * run, first = k / group * group, in = k - first;
@@ -996,7 +1000,7 @@ __device__ __forceinline__ void bin_build(BuildArgs& a)
     const uint32_t wave = uniform(threadIdx.x / kWave);
     const BinRoom room  = {s_keys + wave * kWaveBinCap, s_places + wave * kPlaces, s_items + wave * kWaveBinCap,
                            s_t + wave * kWave, s_alpha + wave * kWave, s_depth + wave * kWave};
-    const uint32_t bin  = in_runs(blockIdx.x - a.crowded_blocks, gridDim.x - a.crowded_blocks, kWaveBinRun) * kWaves + wave;
+    const uint32_t bin  = in_runs(blockIdx.x - a.crowded_blocks, a.blocks_in_runs, kWaveBinRun) * kWaves + wave;
     if (bin < a.num_bins) build_by_wave<C, BILINEAR, FUZZY>(a, bin, room, lane);
 }
 

@@ -717,6 +717,7 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
     uint32_t shared_end = bins;
     if (p.debug_max_list_length > 0 && p.debug_max_list_length <= kWave)
         for (int l = L - 1; l >= 0 && ly.bin_shift[l] <= kSmallBinShift; --l) shared_end = ly.bin_base[l];
+    const uint32_t wave_blocks    = (bins + kBlock / kWave - 1) / (kBlock / kWave);  // a wave to each of the others
     const uint32_t crowded_blocks = std::min({kCrowdedBlocks, crowded_entries_most((size_t)lay.fragment_capacity), std::max((bins + 3) / 4, kCrowdedAtOnce)});
     for (int first = 0; first < B; first += lanes)
     {
@@ -787,6 +788,7 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
             bp.crowded_counts      = sa.crowded.counts;
             bp.crowded_capacity    = sa.crowded.capacity;
             bp.crowded_blocks      = crowded_blocks;
+            bp.blocks_in_runs      = wave_blocks > kRunsFrom ? wave_blocks / (kXcds * kWaveBinRun) * (kXcds * kWaveBinRun) : 0u;
             bp.num_bins            = bins;
             bp.shared_end          = shared_end;
             bp.N                   = N;
@@ -862,7 +864,7 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
         {
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BUILD);
             const BuildPass& bp = build.v[0];
-            const unsigned blocks = crowded_blocks + (bins + kBlock / kWave - 1) / (kBlock / kWave);
+            const unsigned blocks = crowded_blocks + wave_blocks;
             const dim3 g(blocks), gv(blocks, views_y);
             auto launch = [&](auto channels, auto bilinear, auto fuzzy) {
                 constexpr int kC         = decltype(channels)::value;
