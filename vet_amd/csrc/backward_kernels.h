@@ -537,9 +537,11 @@ constexpr int kFuzzyLongColumn = 6;   // background row, column 6: the workgroup
 // its lists and writes it to a row of its own, of kLongRow floats; fold_background_rows_kernel adds those up into kFuzzyFoldRows
 // rows right behind the dense kernel's, so that the sum over the rows stays short:
 // [workgroups of the dense kernel] [kFuzzyFoldRows] [replica 0: workgroups] [replica 1: workgroups] ...
-// Most workgroups have no such list, so one of this kernel looks at kFuzzyStride of the dense kernel's, whose lists it takes one
-// workgroup after the other. Two views of 1237x701 without a cut: 88 us with 4 replicas and a workgroup for each, 88 with 4 or 8
-// looked at (what lasts is the waves with the most lists), 80 with 8 replicas and 8 looked at, 90 with 16 replicas.
+// Most workgroups have no such list, so one of this kernel looks at up to kFuzzyStride of the dense kernel's (fuzzy_long_grid), whose
+// lists it takes one workgroup after the other. What lasts is the waves with the most lists. Two views of 1237x701 without a cut, us: 4
+// replicas and a workgroup for each 88, with 4 or 8 looked at 88; 8 replicas with 8 looked at 80, 16 replicas 90, with rows of 32 bytes for
+// each of the dense kernel's workgroups. With one row a workgroup, against 4 replicas and a workgroup for each (another card): 80
+// / 93, four of five 617x617 views 679 / 743, the fifth 247 / 333; both kernels together 700x500 131 / 151, 384x384 126 / 139, 203x155 91 / 117.
 constexpr int kFuzzyReplicas   = 8;
 constexpr int kFuzzyFoldRows   = 256;
 constexpr int kLongRow         = 4;
@@ -1070,299 +1072,299 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
     float bg_grad[C];  // summed over the wave at the end: every lane adds what it computes for lane 0's sake once
 #pragma unroll
     for (int ci = 0; ci < C; ++ci) bg_grad[ci] = 0.f;
-  for (; with_list != 0ull; with_list &= with_list - 1ull)
-  {
-    const int from     = __ffsll((unsigned long long)with_list) - 1;
-    const TilePixel px = tile_pixel(a.tiles, a.ly, blockIdx.x + (uint32_t)from * gridDim.x);
-    const FuzzyPixel f = fuzzy_pixel<C>(a, px);
-    float4* partial_l  = a.partial;  // (records are addressed by gradient_record)
-    const bool with_background = !a.use_environment_map;
-    auto everywhere = [&](float v, int src) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), src)); };
-
-    uint64_t todo = __ballot(f.n > dense_max);
-    for (uint32_t turn = 0; todo != 0ull; ++turn)
+    for (; with_list != 0ull; with_list &= with_list - 1ull)
     {
-        const int src = __ffsll((unsigned long long)todo) - 1;
-        todo &= todo - 1ull;
-        if (turn % (uint32_t)kFuzzyReplicas != replica) continue;
-        // the pixel, the same on every lane
-        const uint32_t n       = (uint32_t)__builtin_amdgcn_readlane((int)f.n, src);
-        const uint64_t* list   = a.fragments + (uint32_t)__builtin_amdgcn_readlane((int)f.off, src);
-        const bool do_point    = __builtin_amdgcn_readlane((int)f.do_point, src) != 0;
-        float g[4], ax[4], ay[4];
-#pragma unroll
-        for (int ci = 0; ci < 4; ++ci) g[ci] = everywhere(f.g[ci], src), ax[ci] = everywhere(f.ax[ci], src), ay[ci] = everywhere(f.ay[ci], src);
-        const float bx = everywhere(f.bx, src), by = everywhere(f.by, src);
+        const int from     = __ffsll((unsigned long long)with_list) - 1;
+        const TilePixel px = tile_pixel(a.tiles, a.ly, blockIdx.x + (uint32_t)from * gridDim.x);
+        const FuzzyPixel f = fuzzy_pixel<C>(a, px);
+        float4* partial_l  = a.partial;  // (records are addressed by gradient_record)
+        const bool with_background = !a.use_environment_map;
+        auto everywhere = [&](float v, int src) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), src)); };
 
-        // A list that fits one step needs no first pass: the total is known inside the step.
-        const bool one_step = n <= (uint32_t)kWave;
-        double total = 0.0;
-#pragma unroll 1
-        for (int pass = one_step ? 1 : 0; pass < 2; ++pass)
+        uint64_t todo = __ballot(f.n > dense_max);
+        for (uint32_t turn = 0; todo != 0ull; ++turn)
         {
-            // carried from step to step (the same on every lane)
-            float open_sums[C + 1];
+            const int src = __ffsll((unsigned long long)todo) - 1;
+            todo &= todo - 1ull;
+            if (turn % (uint32_t)kFuzzyReplicas != replica) continue;
+            // the pixel, the same on every lane
+            const uint32_t n       = (uint32_t)__builtin_amdgcn_readlane((int)f.n, src);
+            const uint64_t* list   = a.fragments + (uint32_t)__builtin_amdgcn_readlane((int)f.off, src);
+            const bool do_point    = __builtin_amdgcn_readlane((int)f.do_point, src) != 0;
+            float g[4], ax[4], ay[4];
 #pragma unroll
-            for (int v = 0; v <= C; ++v) open_sums[v] = 0.f;
-            uint32_t open_m = 0, open_start = 0;
-            float last_min = 0.f, A_front = 1.f;  // transmittance in front of the open bucket
-            double prefix  = 0.0;                 // bucket terms of the closed buckets
-#pragma unroll 1
-            for (uint32_t begin = 0; begin < n; begin += kWave)
-            {
-                const uint32_t valid = min((uint32_t)kWave, n - begin);
-                const bool last_step = begin + kWave >= n;
-                const bool has       = (uint32_t)lane < valid;
-                float depth = 0.f, conf = 0.f;
-                float t[4]  = {0.f, 0.f, 0.f, 0.f};
-                int id = -1;
-                if (has)
-                {
-                    const uint64_t key = list[begin + lane];
-                    depth              = __uint_as_float((uint32_t)(key >> 32));
-                    const int point    = (int)(uint32_t)key;
-                    int ti             = -1;
-                    if ((uint32_t)point < (uint32_t)a.N) ti = a.index ? a.index[point] : point;
-                    if ((uint32_t)ti < (uint32_t)a.N)
-                    {
-                        const float4 t4 = a.packed[2 * (size_t)ti];
-                        conf            = a.packed[2 * (size_t)ti + 1].x;
-                        t[0] = t4.x, t[1] = t4.y, t[2] = t4.z, t[3] = t4.w;
-                        id = point;
-                    }
-                }
-                // ---- bucket boundaries of this step (src/lib/rendering/RenderBackward.cu:706-714); element 0 of the
-                // list opens the first bucket whether or not it resets the range
-                // One trip per bucket, not per element: the elements that do not fit the open range are found by all
-                // lanes at once, the first of them opens the next bucket and sets the next range.
-                uint64_t heads = begin == 0 ? 1ull : 0ull;
-                for (uint64_t beyond = __ballot(has && !(depth - last_min < depth_accept)); beyond != 0ull;)
-                {
-                    const int i = __ffsll((unsigned long long)beyond) - 1;
-                    heads |= 1ull << i;
-                    last_min = everywhere(depth, i);
-                    beyond   = __ballot(has && lane > i && !(depth - last_min < depth_accept));
-                }
-                // the background (depth 1e5) behind the last fragment: one more element of the last bucket if that
-                // bucket's range reaches it, else a bucket of its own
-                const bool bg_joins = last_step && with_background && (100000.f - last_min < depth_accept);
+            for (int ci = 0; ci < 4; ++ci) g[ci] = everywhere(f.g[ci], src), ax[ci] = everywhere(f.ax[ci], src), ay[ci] = everywhere(f.ay[ci], src);
+            const float bx = everywhere(f.bx, src), by = everywhere(f.by, src);
 
-                // ---- a bucket that was open and has no element in this step closes in front of it
-                if (open_m != 0u && (heads & 1ull))
+            // A list that fits one step needs no first pass: the total is known inside the step.
+            const bool one_step = n <= (uint32_t)kWave;
+            double total = 0.0;
+#pragma unroll 1
+            for (int pass = one_step ? 1 : 0; pass < 2; ++pass)
+            {
+                // carried from step to step (the same on every lane)
+                float open_sums[C + 1];
+#pragma unroll
+                for (int v = 0; v <= C; ++v) open_sums[v] = 0.f;
+                uint32_t open_m = 0, open_start = 0;
+                float last_min = 0.f, A_front = 1.f;  // transmittance in front of the open bucket
+                double prefix  = 0.0;                 // bucket terms of the closed buckets
+#pragma unroll 1
+                for (uint32_t begin = 0; begin < n; begin += kWave)
                 {
-                    const float inv   = 1.f / (float)open_m;
-                    const float bconf = open_sums[C] * inv;
-                    float dot = 0.f, x = 0.f;
-#pragma unroll
-                    for (int ci = 0; ci < C; ++ci)
+                    const uint32_t valid = min((uint32_t)kWave, n - begin);
+                    const bool last_step = begin + kWave >= n;
+                    const bool has       = (uint32_t)lane < valid;
+                    float depth = 0.f, conf = 0.f;
+                    float t[4]  = {0.f, 0.f, 0.f, 0.f};
+                    int id = -1;
+                    if (has)
                     {
-                        const float tb = open_sums[ci] * inv;
-                        dot += tb * g[ci];
-                        x += ((g[ci] * tb) * A_front) * bconf;
-                    }
-                    if (pass == 0)
-                        total += (double)x;
-                    else
-                    {
-                        prefix += (double)x;
-                        const float S     = (float)(total - prefix);
-                        const float gconf = (dot * A_front) * inv - S / ((1.f - bconf) + 1e-9f);
-                        float gt[4]       = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int ci = 0; ci < C; ++ci) gt[ci] = ((A_front * bconf) * g[ci]) * inv;
-                        for (uint32_t e = open_start + lane; e < begin; e += kWave)
+                        const uint64_t key = list[begin + lane];
+                        depth              = __uint_as_float((uint32_t)(key >> 32));
+                        const int point    = (int)(uint32_t)key;
+                        int ti             = -1;
+                        if ((uint32_t)point < (uint32_t)a.N) ti = a.index ? a.index[point] : point;
+                        if ((uint32_t)ti < (uint32_t)a.N)
                         {
-                            const int point = (int)(uint32_t)list[e];
-                            int ti          = -1;
-                            if ((uint32_t)point < (uint32_t)a.N) ti = a.index ? a.index[point] : point;
-                            if ((uint32_t)ti >= (uint32_t)a.N) continue;
-                            partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, point)] = make_float4(gt[0], gt[1], gt[2], gt[3]);
-                            reinterpret_cast<float*>(&partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, point) + 1])[0] = gconf;
+                            const float4 t4 = a.packed[2 * (size_t)ti];
+                            conf            = a.packed[2 * (size_t)ti + 1].x;
+                            t[0] = t4.x, t[1] = t4.y, t[2] = t4.z, t[3] = t4.w;
+                            id = point;
                         }
                     }
-                    A_front = (1.f - bconf) * A_front;
-                    open_m  = 0u;
-#pragma unroll
-                    for (int v = 0; v <= C; ++v) open_sums[v] = 0.f;
-                }
+                    // ---- bucket boundaries of this step (src/lib/rendering/RenderBackward.cu:706-714); element 0 of the
+                    // list opens the first bucket whether or not it resets the range
+                    // One trip per bucket, not per element: the elements that do not fit the open range are found by all
+                    // lanes at once, the first of them opens the next bucket and sets the next range.
+                    uint64_t heads = begin == 0 ? 1ull : 0ull;
+                    for (uint64_t beyond = __ballot(has && !(depth - last_min < depth_accept)); beyond != 0ull;)
+                    {
+                        const int i = __ffsll((unsigned long long)beyond) - 1;
+                        heads |= 1ull << i;
+                        last_min = everywhere(depth, i);
+                        beyond   = __ballot(has && lane > i && !(depth - last_min < depth_accept));
+                    }
+                    // the background (depth 1e5) behind the last fragment: one more element of the last bucket if that
+                    // bucket's range reaches it, else a bucket of its own
+                    const bool bg_joins = last_step && with_background && (100000.f - last_min < depth_accept);
 
-                // ---- this lane's bucket inside the step
-                const uint64_t upto  = heads & (lane == kWave - 1 ? ~0ull : (2ull << lane) - 1ull);
-                const bool joined    = upto == 0ull;  // belongs to the bucket that was open when the step began
-                const uint32_t first = joined ? 0u : 63u - (uint32_t)__clzll((long long)upto);
-                const uint64_t later = lane == kWave - 1 ? 0ull : heads >> (lane + 1);
-                uint32_t next        = later ? (uint32_t)lane + (uint32_t)__ffsll((unsigned long long)later) : valid;
-                next                 = min(next, valid);
-                const uint32_t dist  = (uint32_t)lane - first;
-                const bool closes    = has && (next < valid || last_step);  // the bucket ends in this step
-                const bool tail      = has && next == valid;                // the last bucket of the step
-                // sums over the bucket's elements of this step: inclusive scan from its first lane, read at its last
-                float sums[C + 1];
-                sums[C] = conf;
-#pragma unroll
-                for (int ci = 0; ci < C; ++ci) sums[ci] = t[ci];
-                const int last_lane = has ? (int)next - 1 : lane;
-#pragma unroll
-                for (int v = 0; v <= C; ++v)
-                {
-                    float x = sums[v];
-#pragma unroll
-                    for (int d = 1; d < kWave; d <<= 1)
+                    // ---- a bucket that was open and has no element in this step closes in front of it
+                    if (open_m != 0u && (heads & 1ull))
                     {
-                        const float o = __shfl_up(x, d, kWave);
-                        if (dist >= (uint32_t)d) x += o;
-                    }
-                    sums[v] = __shfl(x, last_lane, kWave);
-                    if (joined) sums[v] = open_sums[v] + sums[v];
-                }
-                uint32_t m = has ? (next - first) + (joined ? open_m : 0u) : 1u;
-                if (bg_joins && tail)
-                {
-                    sums[C] += 1.f;
-#pragma unroll
-                    for (int ci = 0; ci < C; ++ci) sums[ci] += a.background[ci];
-                    m += 1u;
-                }
-                const float inv   = 1.f / (float)m;
-                const float bconf = sums[C] * inv;
-                float dot = 0.f;
-#pragma unroll
-                for (int ci = 0; ci < C; ++ci) dot += (sums[ci] * inv) * g[ci];
-                // transmittance in front: product of (1 - mean confidence) over the buckets that close in this step in
-                // front of this one, times what was in front of the step
-                const bool closing_lane = closes && lane == last_lane;
-                float P = closing_lane ? 1.f - bconf : 1.f;
-#pragma unroll
-                for (int d = 1; d < kWave; d <<= 1)
-                {
-                    const float o = __shfl_up(P, d, kWave);
-                    if (lane >= d) P *= o;
-                }
-                const float P_before = __shfl(P, first > 0u ? (int)first - 1 : lane, kWave);
-                const float A        = first > 0u ? A_front * P_before : A_front;
-                const float P_end    = everywhere(P, (int)valid - 1);  // over all buckets that close in this step
-                float x = 0.f;
-#pragma unroll
-                for (int ci = 0; ci < C; ++ci) x += ((g[ci] * (sums[ci] * inv)) * A) * bconf;
-                // Terms of the buckets that close in this step, summed from the back: a bucket needs the terms of the
-                // buckets BEHIND it, and taking them as (all) - (those in front) would cancel to rounding noise deep in
-                // a list, where what is left behind is a millionth of what lies in front.
-                float X = closing_lane ? x : 0.f;
-#pragma unroll
-                for (int d = 1; d < kWave; d <<= 1)
-                {
-                    const float o = __shfl_down(X, d, kWave);
-                    if (lane + d < kWave) X += o;
-                }
-                const float X_end = everywhere(X, 0);  // all of them
-                if (one_step)
-                {
-                    // what the first pass would have left, from the same terms in the same order
-                    total = (double)X_end;
-                    if (with_background && !bg_joins)
-                    {
-                        float xb = 0.f;
-#pragma unroll
-                        for (int ci = 0; ci < C; ++ci) xb += ((g[ci] * a.background[ci]) * (A_front * P_end)) * 1.f;
-                        total += (double)xb;
-                    }
-                }
-                if (pass == 1)
-                {
-                    // behind this lane's bucket inside the step
-                    // (the exchange is made by every lane, then the lanes with nothing behind them drop what they got)
-                    const float X_next   = __shfl(X, min(last_lane + 1, kWave - 1), kWave);
-                    const float X_behind = last_lane + 1 < kWave ? X_next : 0.f;
-                    float gp0 = 0.f, gp1 = 0.f;
-                    if (has && id >= 0 && do_point)
-                    {
-                        float dR_dpx = bx, dR_dpy = by;
+                        const float inv   = 1.f / (float)open_m;
+                        const float bconf = open_sums[C] * inv;
+                        float dot = 0.f, x = 0.f;
 #pragma unroll
                         for (int ci = 0; ci < C; ++ci)
                         {
-                            dR_dpx += t[ci] * ax[ci];
-                            dR_dpy += t[ci] * ay[ci];
+                            const float tb = open_sums[ci] * inv;
+                            dot += tb * g[ci];
+                            x += ((g[ci] * tb) * A_front) * bconf;
                         }
-                        gp0 = dR_dpx / (float)C;
-                        gp1 = dR_dpy / (float)C;
-                    }
-                    // ... and behind the step: both sums are made of the same float terms, so this difference is exact
-                    const float S     = X_behind + (float)(total - (prefix + (double)X_end));
-                    const float gconf = (dot * A) * inv - S / ((1.f - bconf) + 1e-9f);
-                    float gt[4]       = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int ci = 0; ci < C; ++ci) gt[ci] = ((A * bconf) * g[ci]) * inv;
-                    if (has && id >= 0)
-                    {
-                        if (closes)
-                        {
-                            partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, id)]     = make_float4(gt[0], gt[1], gt[2], gt[3]);
-                            partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, id) + 1] = make_float4(gconf, gp0, gp1, 0.f);
-                        }
+                        if (pass == 0)
+                            total += (double)x;
                         else
                         {
-                            // the bucket stays open: its part of the record follows when it closes
-                            float* rec = reinterpret_cast<float*>(&partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, id) + 1]);
-                            rec[1] = gp0, rec[2] = gp1, rec[3] = 0.f;
-                        }
-                    }
-                    // the elements an earlier step left with a bucket that closes here
-                    const bool joined_closes = open_m != 0u && __builtin_amdgcn_readlane((int)(closes && joined), 0) != 0;
-                    if (joined_closes)
-                    {
-                        float gt0[4];
+                            prefix += (double)x;
+                            const float S     = (float)(total - prefix);
+                            const float gconf = (dot * A_front) * inv - S / ((1.f - bconf) + 1e-9f);
+                            float gt[4]       = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                        for (int ci = 0; ci < 4; ++ci) gt0[ci] = everywhere(gt[ci], 0);
-                        const float gconf0 = everywhere(gconf, 0);
-                        for (uint32_t e = open_start + lane; e < begin; e += kWave)
+                            for (int ci = 0; ci < C; ++ci) gt[ci] = ((A_front * bconf) * g[ci]) * inv;
+                            for (uint32_t e = open_start + lane; e < begin; e += kWave)
+                            {
+                                const int point = (int)(uint32_t)list[e];
+                                int ti          = -1;
+                                if ((uint32_t)point < (uint32_t)a.N) ti = a.index ? a.index[point] : point;
+                                if ((uint32_t)ti >= (uint32_t)a.N) continue;
+                                partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, point)] = make_float4(gt[0], gt[1], gt[2], gt[3]);
+                                reinterpret_cast<float*>(&partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, point) + 1])[0] = gconf;
+                            }
+                        }
+                        A_front = (1.f - bconf) * A_front;
+                        open_m  = 0u;
+#pragma unroll
+                        for (int v = 0; v <= C; ++v) open_sums[v] = 0.f;
+                    }
+
+                    // ---- this lane's bucket inside the step
+                    const uint64_t upto  = heads & (lane == kWave - 1 ? ~0ull : (2ull << lane) - 1ull);
+                    const bool joined    = upto == 0ull;  // belongs to the bucket that was open when the step began
+                    const uint32_t first = joined ? 0u : 63u - (uint32_t)__clzll((long long)upto);
+                    const uint64_t later = lane == kWave - 1 ? 0ull : heads >> (lane + 1);
+                    uint32_t next        = later ? (uint32_t)lane + (uint32_t)__ffsll((unsigned long long)later) : valid;
+                    next                 = min(next, valid);
+                    const uint32_t dist  = (uint32_t)lane - first;
+                    const bool closes    = has && (next < valid || last_step);  // the bucket ends in this step
+                    const bool tail      = has && next == valid;                // the last bucket of the step
+                    // sums over the bucket's elements of this step: inclusive scan from its first lane, read at its last
+                    float sums[C + 1];
+                    sums[C] = conf;
+#pragma unroll
+                    for (int ci = 0; ci < C; ++ci) sums[ci] = t[ci];
+                    const int last_lane = has ? (int)next - 1 : lane;
+#pragma unroll
+                    for (int v = 0; v <= C; ++v)
+                    {
+                        float x = sums[v];
+#pragma unroll
+                        for (int d = 1; d < kWave; d <<= 1)
                         {
-                            const int point = (int)(uint32_t)list[e];
-                            int ti          = -1;
-                            if ((uint32_t)point < (uint32_t)a.N) ti = a.index ? a.index[point] : point;
-                            if ((uint32_t)ti >= (uint32_t)a.N) continue;
-                            partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, point)] = make_float4(gt0[0], gt0[1], gt0[2], gt0[3]);
-                            reinterpret_cast<float*>(&partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, point) + 1])[0] = gconf0;
+                            const float o = __shfl_up(x, d, kWave);
+                            if (dist >= (uint32_t)d) x += o;
+                        }
+                        sums[v] = __shfl(x, last_lane, kWave);
+                        if (joined) sums[v] = open_sums[v] + sums[v];
+                    }
+                    uint32_t m = has ? (next - first) + (joined ? open_m : 0u) : 1u;
+                    if (bg_joins && tail)
+                    {
+                        sums[C] += 1.f;
+#pragma unroll
+                        for (int ci = 0; ci < C; ++ci) sums[ci] += a.background[ci];
+                        m += 1u;
+                    }
+                    const float inv   = 1.f / (float)m;
+                    const float bconf = sums[C] * inv;
+                    float dot = 0.f;
+#pragma unroll
+                    for (int ci = 0; ci < C; ++ci) dot += (sums[ci] * inv) * g[ci];
+                    // transmittance in front: product of (1 - mean confidence) over the buckets that close in this step in
+                    // front of this one, times what was in front of the step
+                    const bool closing_lane = closes && lane == last_lane;
+                    float P = closing_lane ? 1.f - bconf : 1.f;
+#pragma unroll
+                    for (int d = 1; d < kWave; d <<= 1)
+                    {
+                        const float o = __shfl_up(P, d, kWave);
+                        if (lane >= d) P *= o;
+                    }
+                    const float P_before = __shfl(P, first > 0u ? (int)first - 1 : lane, kWave);
+                    const float A        = first > 0u ? A_front * P_before : A_front;
+                    const float P_end    = everywhere(P, (int)valid - 1);  // over all buckets that close in this step
+                    float x = 0.f;
+#pragma unroll
+                    for (int ci = 0; ci < C; ++ci) x += ((g[ci] * (sums[ci] * inv)) * A) * bconf;
+                    // Terms of the buckets that close in this step, summed from the back: a bucket needs the terms of the
+                    // buckets BEHIND it, and taking them as (all) - (those in front) would cancel to rounding noise deep in
+                    // a list, where what is left behind is a millionth of what lies in front.
+                    float X = closing_lane ? x : 0.f;
+#pragma unroll
+                    for (int d = 1; d < kWave; d <<= 1)
+                    {
+                        const float o = __shfl_down(X, d, kWave);
+                        if (lane + d < kWave) X += o;
+                    }
+                    const float X_end = everywhere(X, 0);  // all of them
+                    if (one_step)
+                    {
+                        // what the first pass would have left, from the same terms in the same order
+                        total = (double)X_end;
+                        if (with_background && !bg_joins)
+                        {
+                            float xb = 0.f;
+#pragma unroll
+                            for (int ci = 0; ci < C; ++ci) xb += ((g[ci] * a.background[ci]) * (A_front * P_end)) * 1.f;
+                            total += (double)xb;
                         }
                     }
-                    if (last_step && with_background && lane == (int)valid - 1)
+                    if (pass == 1)
                     {
-                        // the background's share: an element of the last bucket, or a bucket of its own behind all
-                        const float scale = bg_joins ? A * bconf : (A_front * P_end) * 1.f;
-                        const float share = bg_joins ? inv : 1.f;
+                        // behind this lane's bucket inside the step
+                        // (the exchange is made by every lane, then the lanes with nothing behind them drop what they got)
+                        const float X_next   = __shfl(X, min(last_lane + 1, kWave - 1), kWave);
+                        const float X_behind = last_lane + 1 < kWave ? X_next : 0.f;
+                        float gp0 = 0.f, gp1 = 0.f;
+                        if (has && id >= 0 && do_point)
+                        {
+                            float dR_dpx = bx, dR_dpy = by;
 #pragma unroll
-                        for (int ci = 0; ci < C; ++ci) bg_grad[ci] += (scale * g[ci]) * share;
+                            for (int ci = 0; ci < C; ++ci)
+                            {
+                                dR_dpx += t[ci] * ax[ci];
+                                dR_dpy += t[ci] * ay[ci];
+                            }
+                            gp0 = dR_dpx / (float)C;
+                            gp1 = dR_dpy / (float)C;
+                        }
+                        // ... and behind the step: both sums are made of the same float terms, so this difference is exact
+                        const float S     = X_behind + (float)(total - (prefix + (double)X_end));
+                        const float gconf = (dot * A) * inv - S / ((1.f - bconf) + 1e-9f);
+                        float gt[4]       = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int ci = 0; ci < C; ++ci) gt[ci] = ((A * bconf) * g[ci]) * inv;
+                        if (has && id >= 0)
+                        {
+                            if (closes)
+                            {
+                                partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, id)]     = make_float4(gt[0], gt[1], gt[2], gt[3]);
+                                partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, id) + 1] = make_float4(gconf, gp0, gp1, 0.f);
+                            }
+                            else
+                            {
+                                // the bucket stays open: its part of the record follows when it closes
+                                float* rec = reinterpret_cast<float*>(&partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, id) + 1]);
+                                rec[1] = gp0, rec[2] = gp1, rec[3] = 0.f;
+                            }
+                        }
+                        // the elements an earlier step left with a bucket that closes here
+                        const bool joined_closes = open_m != 0u && __builtin_amdgcn_readlane((int)(closes && joined), 0) != 0;
+                        if (joined_closes)
+                        {
+                            float gt0[4];
+#pragma unroll
+                            for (int ci = 0; ci < 4; ++ci) gt0[ci] = everywhere(gt[ci], 0);
+                            const float gconf0 = everywhere(gconf, 0);
+                            for (uint32_t e = open_start + lane; e < begin; e += kWave)
+                            {
+                                const int point = (int)(uint32_t)list[e];
+                                int ti          = -1;
+                                if ((uint32_t)point < (uint32_t)a.N) ti = a.index ? a.index[point] : point;
+                                if ((uint32_t)ti >= (uint32_t)a.N) continue;
+                                partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, point)] = make_float4(gt0[0], gt0[1], gt0[2], gt0[3]);
+                                reinterpret_cast<float*>(&partial_l[2 * gradient_record(a.point_major_records, a.N, a.ly.L, px.l, point) + 1])[0] = gconf0;
+                            }
+                        }
+                        if (last_step && with_background && lane == (int)valid - 1)
+                        {
+                            // the background's share: an element of the last bucket, or a bucket of its own behind all
+                            const float scale = bg_joins ? A * bconf : (A_front * P_end) * 1.f;
+                            const float share = bg_joins ? inv : 1.f;
+#pragma unroll
+                            for (int ci = 0; ci < C; ++ci) bg_grad[ci] += (scale * g[ci]) * share;
+                        }
                     }
-                }
-                // ---- what the next step inherits
-                if (pass == 0)
-                    total += (double)X_end;
-                else
-                    prefix += (double)X_end;
-                if (last_step)
-                {
-                    if (pass == 0 && with_background && !bg_joins)
+                    // ---- what the next step inherits
+                    if (pass == 0)
+                        total += (double)X_end;
+                    else
+                        prefix += (double)X_end;
+                    if (last_step)
                     {
-                        float xb = 0.f;
+                        if (pass == 0 && with_background && !bg_joins)
+                        {
+                            float xb = 0.f;
 #pragma unroll
-                        for (int ci = 0; ci < C; ++ci) xb += ((g[ci] * a.background[ci]) * (A_front * P_end)) * 1.f;
-                        total += (double)xb;
+                            for (int ci = 0; ci < C; ++ci) xb += ((g[ci] * a.background[ci]) * (A_front * P_end)) * 1.f;
+                            total += (double)xb;
+                        }
                     }
-                }
-                else
-                {
-                    // the last bucket of the step stays open (valid = 64 here)
-                    const bool all_joined   = heads == 0ull;
-                    const uint32_t open_pos = all_joined ? 0u : 63u - (uint32_t)__clzll((long long)heads);
+                    else
+                    {
+                        // the last bucket of the step stays open (valid = 64 here)
+                        const bool all_joined   = heads == 0ull;
+                        const uint32_t open_pos = all_joined ? 0u : 63u - (uint32_t)__clzll((long long)heads);
 #pragma unroll
-                    for (int v = 0; v <= C; ++v) open_sums[v] = everywhere(sums[v], kWave - 1);
-                    open_m     = (uint32_t)kWave - open_pos + (all_joined ? open_m : 0u);
-                    open_start = all_joined ? open_start : begin + open_pos;
-                    A_front    = A_front * P_end;
+                        for (int v = 0; v <= C; ++v) open_sums[v] = everywhere(sums[v], kWave - 1);
+                        open_m     = (uint32_t)kWave - open_pos + (all_joined ? open_m : 0u);
+                        open_start = all_joined ? open_start : begin + open_pos;
+                        A_front    = A_front * P_end;
+                    }
                 }
             }
         }
     }
-  }
 #pragma unroll
     for (int ci = 0; ci < C; ++ci)
     {

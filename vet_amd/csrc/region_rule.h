@@ -22,7 +22,8 @@ namespace vetrast
 //   with 2, 127 / 113 with 3.8; two town views of 960x540 139 / 120 with 1.1, of 2000x1080 2 to 4 % slower up to 2.8.
 // * One, four or seven (modulo 8) give it a diagonal or every other row's half: 1100x600 31 / 33 with 0.8, 102 / 97 with 3.2; 1080p
 //   146 / 145 with 1.2, 224 / 220 with 2.4, 192 / 186 with 3.2, 242 / 234 with 4.2, ten million points in it 553 / 530, but four town
-//   views with list 1.1 387 / 402. 512x512 26 / 28 with 2.4, 31 / 35 with 3.3, four crops of that size level with 3.9.
+//   views with list 1.1 387 / 402. 512x512 26 / 28 with 2.4, 31 / 35 with 3.3; four crops of that size with the 2x2 splat
+//   157 / 162 with 3.9, 257 / 254 with 7.8, where many points are dropped by radius 91 / 89; in FULL_BLEND 183 / 176 with 3.9.
 // * Two, three, five or six spread whatever lies together by themselves: 700x500 37 / 41 with 3.7, 84 / 83 with 6, 102 / 95 with 10;
 //   640x360 31 / 31 with 3.3, 61 / 57 with 8.6; 1237x701 36 / 41 with 0.8, 65 / 69 with 3.1, 167 / 168 with 5.2, 208 / 203 with 8.6.
 constexpr int kPartsLayers            = 4;   // at least
