@@ -5,19 +5,20 @@
 // those tests have a foregone answer: in one image row the pixels a cell covers are a run whose ends can be computed.
 // So the work here goes by rows instead of pixels:
 //   1. lift_prefix_kernel: per image row the running sum (double) of sum_c |loss|, so that the sum over a run of pixels is
-//      one difference of two entries.
-//   2. lift_cells_kernel: a workgroup takes 32 cells, projects their corners and sets up, per triangle and for the outline
-//      of the 8 corners, where their edges cross a row; then every lane takes one ROW of one of the cells. Pixels that
+//      one difference of two entries. Beside that, workgroups of their own look for the cells whose box the image shows.
+//   2. lift_cells_kernel: a workgroup takes 32 of those cells, projects their corners and sets up, per triangle and for the
+//      outline of the 8 corners, where their edges cross a row; then every lane takes one ROW of one of the cells. Pixels that
 //      lie inside a triangle by more than the rounding error of the test are counted as a run, pixels outside the outline
 //      by more than that are left out, and the few in between get the literal test of the reference. The counts are the
 //      literal ones, pixel for pixel.
 // Measured (146 k cells of 0.25 m, 1080p, 121 M covered pixels, the camera inside the grid): 0.87 ms per call with a test per
-// pixel (bound by its ~200 vector instructions per 64 pixels), 0.22 ms by rows (running sums 13 us, rows 143 us, the
-// cells next to the camera that are tested pixel by pixel 63 us). The rows take 37 M wave instructions a view of three 1080p
-// views of 176 k cells, 61 us of them, and took 138 us: a wave waited 62 % of its life, with 12 waves on a compute unit, as
-// many as the cells' bounds in LDS leave with 128 threads to 32 cells. Hence 256 threads, triangles and outlines set up
-// side by side, and waves that go through their rows without waiting for each other: 99 us. (16 cells with 128 or 256
-// threads, 32 with 384 or 512: a fifth slower; 64 with 512: the same.)
+// pixel (bound by its ~200 vector instructions per 64 pixels), 0.22 ms by rows.
+// Bound by vector instructions (32 M of wave instructions a view of three 1080p views of 176 k cells, 55 of the cells kernel's 86 us)
+// and the round trips of a row's two running sums. A third of the cells is in the image: with the others in the workgroups too,
+// set up by as many idle lanes, it took 43 M and 103 us, cells of 0.15 m 385 a call (now 259), of 1 m 78 (now 56: there are few of
+// them, which are dealt to more workgroups then, kLiftLeast; with 768 or 1792 for it the same). Looking for them costs the running
+// sums' kernel 1 us (13.4 and 14.2; 17.2 when every cell of a stretch came from a cache line of its own).
+// The LDS of 7 workgroups (a bound is two floats; with three, 6 fit: 99 us). 16 cells to a workgroup 92 us, with 128 threads 112.
 #pragma once
 #include "common.h"
 #include "forward_kernels.h"
@@ -27,7 +28,8 @@ namespace vetrast
 constexpr int kLiftLargeCell    = 4096;  // boxes of more pixels are counted in the header (a diagnostic of the interface)
 constexpr int kLiftHeader       = 256;   // bytes: DeviceView (160), the count of large cells at 176, flag word at 192
 constexpr int kLiftBlock        = 256;   // threads of a workgroup of the cells kernel
-constexpr int kLiftCells        = 32;    // its cells
+constexpr int kLiftCells        = 32;    // its cells, at most
+constexpr uint32_t kLiftLeast   = 1024;  // workgroups that take the cells, if there are so many
 constexpr int kLiftSetup        = 4;     // threads that set a cell's triangles up, and as many its outline
 constexpr int kLiftSetupAll     = kLiftCells * kLiftSetup;
 static_assert(kLiftSetupAll % kWave == 0 && kLiftBlock >= 2 * kLiftSetupAll, "triangles and outlines are set up by different waves");
@@ -42,6 +44,8 @@ constexpr int kLiftPlainAtOnce  = 8;     // cells in work at a time
 constexpr float kLiftThin       = 0.05f; // smallest angle (about) of a triangle that is not a sliver
 constexpr int kLiftOpen         = 8;     // open pixels of a row that go to the list; a row with more is left to a wave
 constexpr int kLiftOpenPixels   = 128;   // the list of a wave; it is worked off when half full (a lane tests what does not fit)
+constexpr uint32_t kLiftNone    = 0x80000000u;  // (there are no more than 2^30 cells)
+constexpr uint32_t kLiftRun     = 4;     // neighbouring cells that go to one stretch together
 constexpr int kLiftOpenRows     = 128;   // such rows a workgroup keeps (a lane finishes what does not fit)
 // A cell whose open rows of more than kLiftWideRow columns add up to more than kLiftWideWork and more than one in
 // kLiftWideShare of its box's pixels is tested pixel by pixel by lift_plain_kernel: next to the camera the lines of slivers
@@ -79,9 +83,21 @@ struct LiftPass
     // [num_cells] each, written for cells left to lift_plain_kernel and, with several bands, for every cell:
     double* cell_sums;      // sum of the bands so far
     uint32_t* plain_state;  // 0, or first image row that is lift_plain_kernel's + 1 in bits 8.., below them its finished shares
-    int32_t* plain_count;   // pixels lift_plain_kernel has counted
+    // Cells the image shows, found by the first band's lift_prefix_kernel. The cells are dealt to stretches, kLiftRun neighbours
+    // at a time (lift_cell_of_stretch), and column k of stretch c is the place [k * stretches + c] of this array: the stretch's
+    // cells that are seen, and in its last column kLiftNone | how many these are, unless all are.
+    uint32_t* seen;         // [num_cells]
+    uint32_t stretches;     // a multiple of kWave
+    uint32_t prefix_groups; // workgroups of lift_prefix_kernel that add up
     double* sums;       // running sums of the band, see lift_sum_at; null: the image is too wide for one band to hold a row
 };
+
+// Workgroups that share the cells of a group of stretches.
+__host__ __device__ __forceinline__ uint32_t lift_shares(uint32_t cells, uint32_t groups)
+{
+    const uint32_t full = (cells + kLiftCells - 1u) / kLiftCells, least = (kLiftLeast + groups - 1u) / groups;
+    return full > least ? full : (cells < least ? cells : least);
+}
 
 // Where the sum of the pixels [0, x) of image row y is, 0 <= x <= width. The entry of x = 0 is zero, with the sign bit set
 // where the row has pixels so dim that rounding may have swallowed them.
@@ -107,12 +123,83 @@ __device__ __forceinline__ float lift_pixel_error(const LiftPass& a, int x, int 
 constexpr int kLiftPrefixBlock = kLiftRows * kWave;
 constexpr int kLiftPerLane     = 16;
 constexpr int kLiftStep        = kLiftPerLane * kWave;
+
+// Cell k of a stretch, or a number beyond the last cell. Neighbours share cache lines; what is left at the end is dealt one by one,
+// so that a stretch has no more places than cells.
+__device__ __forceinline__ uint32_t lift_cell_of_stretch(uint32_t k, uint32_t stretch, uint32_t stretches, uint32_t cells)
+{
+    const uint32_t in_runs = cells / (kLiftRun * stretches) * kLiftRun;  // cells of a stretch that come in runs
+    return k < in_runs ? (k / kLiftRun * stretches + stretch) * kLiftRun + k % kLiftRun : k * stretches + stretch;
+}
+
+// Workgroup c of these takes stretch c of the cells, a thread per cell: is one of its corners behind the camera, or its pixel
+// box outside the image (src/lib/rendering/RenderForward.cu:679-728)? The others are written down, turned by a share of their
+// number that grows from stretch to stretch: cells of one column then lie all over the grid.
+__device__ __forceinline__ void lift_find_cells(const LiftPass& a, const DeviceView& view, uint32_t stretch)
+{
+    __shared__ uint32_t s_seen[kLiftPrefixBlock / kWave];
+    const uint32_t all  = (uint32_t)a.num_cells, cell = lift_cell_of_stretch(threadIdx.x, stretch, a.stretches, all);
+    const uint32_t own  = threadIdx.x * a.stretches + stretch;  // the place of column threadIdx.x (these are all below 2^31)
+    const int lane      = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    bool seen           = cell < all;
+    if (seen)
+    {
+        const float* mn = a.bb_min + 3 * (size_t)cell;
+        const float* ln = a.bb_length + 3 * (size_t)cell;
+        const float m[3] = {mn[0], mn[1], mn[2]}, n[3] = {ln[0], ln[1], ln[2]};
+        float max_x = -10000000.f, max_y = -10000000.f, min_x = 10000000.f, min_y = 10000000.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+        {
+            float4 p;
+            p.x = m[0] + n[0] * (float)(i & 1);
+            p.y = m[1] + n[1] * (float)(i >> 1 & 1);
+            p.z = m[2] + n[2] * (float)(i >> 2);
+            p.w = 0.f;
+            Projected o;
+            if (!project_point(view, p, o))
+            {
+                seen = false;
+                continue;
+            }
+            max_x = fmaxf(o.ipx, max_x), max_y = fmaxf(o.ipy, max_y);
+            min_x = fminf(o.ipx, min_x), min_y = fminf(o.ipy, min_y);
+        }
+        const float border = (float)a.border, right = (float)(a.width - a.border), bottom = (float)(a.height - a.border);
+        seen = seen && !(max_x < border || min_x >= right || max_y < border || min_y >= bottom);
+    }
+    const uint64_t here = __ballot(seen);
+    if (lane == 0) s_seen[wave] = (uint32_t)__popcll(here);
+    __syncthreads();
+    uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(here >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)here, 0u)), found = 0;
+    for (int w = 0; w < kLiftPrefixBlock / kWave; ++w)
+    {
+        if (w < wave) rank += s_seen[w];
+        found += s_seen[w];
+    }
+    const uint32_t turn = stretch % kWave * found / kWave;
+    if (seen)
+    {
+        const uint32_t column = rank + turn < found ? rank + turn : rank + turn - found;
+        a.seen[column * a.stretches + stretch] = cell;
+    }
+    if (threadIdx.x >= found && own < all && own + a.stretches >= all) a.seen[own] = kLiftNone | found;
+}
+
 __global__ void __launch_bounds__(kLiftPrefixBlock) lift_prefix_kernel(LiftPass a, ViewSource src, const double* __restrict__ poses_se3,
                                                                        const float* __restrict__ intrinsics)
 {
     // (a place is left free behind a lane's, or all lanes would store to one bank)
     __shared__ double s_sum[kLiftStep * kLiftRows + kWave];
-    if (a.first && blockIdx.x == gridDim.x - 1 && threadIdx.x == kLiftPrefixBlock - 1)
+    if (blockIdx.x >= a.prefix_groups)  // (the first band's only)
+    {
+        bool distorted = false;
+        DeviceView v   = make_device_view(src, poses_se3, intrinsics, distorted);
+        v.has_dist     = 0u;
+        lift_find_cells(a, v, blockIdx.x - a.prefix_groups);
+        return;
+    }
+    if (a.first && blockIdx.x == a.prefix_groups - 1u && threadIdx.x == kLiftPrefixBlock - 1)
     {
         bool distorted = false;
         DeviceView v   = make_device_view(src, poses_se3, intrinsics, distorted);
@@ -271,11 +358,25 @@ __device__ __forceinline__ void cell_footprint(const LiftPass& a, int64_t cell, 
     f.x_size = (int)(fminf(max_x, (float)(a.width - a.border)) - f.min_x);
 }
 
-// A bound on x in image row y: x >= or <= slope * (y - y0) + x0.
+// A bound on x in an image row: x >= or <= slope * (row - the cell's first row) + x0.
 struct RowBound
 {
+    float slope, x0;
+    __device__ __forceinline__ float at(float row) const { return slope * row + x0; }
+};
+// The same through a point (x0, y0), as it is set up.
+struct LineBound
+{
     float slope, y0, x0;
-    __device__ __forceinline__ float at(float y) const { return slope * (y - y0) + x0; }
+    // Moved to the cell's first row, and by what that and evaluating it there may be off in x, to the larger or the smaller side. That
+    // is below 5 units in the last place of slope times the height of the box: as if the edge lay 8 of them, 2^-21 of the height,
+    // higher or lower.
+    __device__ __forceinline__ float off(float height) const { return fabsf(slope) * (height * 4.7683716e-7f); }
+    __device__ __forceinline__ RowBound from(float first_row, float height, bool larger) const
+    {
+        const float moved = off(height);
+        return {slope, (slope * (first_row - y0) + x0) + (larger ? moved : -moved)};
+    }
 };
 
 struct LiftCell
@@ -286,7 +387,7 @@ struct LiftCell
     int x_skip;          // a column between them that the reference's rounding of column + origin passes over, or INT_MAX
     RowBound outline[kLiftOutlineMax];
     RowBound tri[kLiftTriangleMax][3];                        // per triangle: a left, a right bound and one of either kind
-    RowBound sliver[kLiftSliverMax];     // lines of thin triangles, and
+    RowBound sliver[kLiftSliverMax];     // lines of thin triangles (x0 is the image row of one that is flat), and
     float sliver_width[kLiftSliverMax];  // their half width in columns, or -(half width in rows)
     uint32_t left_mask;                  // bit t: the third bound of triangle t is a left one; bit 8 + k: outline[k] is
     int num_outline, num_tri, num_sliver;
@@ -297,7 +398,7 @@ struct LiftCell
 
 // Bounds of the half-plane c1 (x - bx) - dx (y - by) >= e0. False where the edge is so flat that the bound says nothing
 // about a single row.
-__device__ __forceinline__ bool half_plane(float c1, float dx, float bx, float by, float e0, float flat, RowBound& r,
+__device__ __forceinline__ bool half_plane(float c1, float dx, float bx, float by, float e0, float flat, LineBound& r,
                                            bool& is_left)
 {
     if (fabsf(c1) <= flat) return false;
@@ -344,8 +445,34 @@ __device__ __forceinline__ void leave_to_plain_kernel(const LiftPass& a, int64_t
 {
     a.plain_cell[atomicAdd(a.num_plain, 1u)] = (uint32_t)cell;
     a.cell_sums[cell]   = sum;
-    a.plain_count[cell] = 0;
     a.plain_state[cell] = (uint32_t)(a.y0 + 1) << 8;  // (an image has less than 2^24 rows)
+}
+
+// The cells of share `part` of a group of kWave neighbouring stretches: their cells that are seen, one stretch's after the
+// other's, are dealt to as many shares as they fill, every so many-th of them to one, or to more where there are few cells.
+// False if there is no such share. Every thread of the workgroup must call.
+__device__ __forceinline__ bool lift_cells_of_share(const LiftPass& a, uint32_t group, uint32_t part, uint32_t (&cells)[kLiftCells])
+{
+    const uint32_t lane = threadIdx.x & (kWave - 1), all = (uint32_t)a.num_cells, stretch = group * kWave + lane;
+    const uint32_t columns = stretch < all ? (all - stretch + a.stretches - 1u) / a.stretches : 0u;
+    uint32_t found         = 0u;
+    if (columns != 0u)
+    {
+        const uint32_t last = a.seen[(columns - 1u) * a.stretches + stretch];
+        found               = (last & kLiftNone) != 0u ? last & ~kLiftNone : columns;
+    }
+    const uint32_t behind = wave_inclusive_scan(found, (int)lane);  // place behind the last of the lane's stretch
+    const uint32_t total  = (uint32_t)__builtin_amdgcn_readlane((int)behind, kWave - 1);
+    const uint32_t shares = lift_shares(total, a.stretches / kWave);
+    if (part >= shares) return false;  // (the same for all waves)
+    const uint32_t at = part + lane * shares;
+    uint32_t of       = 0u;  // stretches that end in front of place `at`
+#pragma unroll
+    for (uint32_t step = kWave / 2; step >= 1u; step >>= 1)
+        if ((uint32_t)__shfl((int)behind, (int)(of + step - 1u), kWave) <= at) of += step;
+    const uint32_t column = at - ((uint32_t)__shfl((int)behind, (int)of, kWave) - (uint32_t)__shfl((int)found, (int)of, kWave));
+    if (threadIdx.x < kLiftCells) cells[threadIdx.x] = at < total ? a.seen[column * a.stretches + group * kWave + of] : kLiftNone;
+    return true;
 }
 
 __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
@@ -358,12 +485,15 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     __shared__ uint32_t s_large;
     __shared__ bool s_left[kLiftCells];  // the cell is lift_plain_kernel's
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    __shared__ uint32_t s_cells[kLiftCells];  // cells of the workgroup, or kLiftNone
+    const uint32_t groups = a.stretches / kWave;
+    if (!lift_cells_of_share(a, blockIdx.x % groups, blockIdx.x / groups, s_cells)) return;
     if (lane == 0) s_num_pixels[wave] = 0;
     if (tid == 0) s_num_open = 0, s_large = 0u;
     __syncthreads();
     // ---- set-up: kLiftSetup threads per cell for its triangles, as many in other waves for its outline; both look at the box
-    // first. The workgroup's cells lie far apart in the grid (cells next to the camera cover hundreds of rows and are
-    // neighbours in it), so every workgroup gets about the same number of rows.
+    // first. The workgroup's cells are seen, all of them, and lie far apart in the grid (cells next to the camera cover hundreds of
+    // rows and are neighbours in it), so every workgroup gets about the same number of rows.
     const bool outlines = tid >= kLiftSetupAll;  // the same in a wave
     const int slot = tid / kLiftSetup % kLiftCells, part = tid % kLiftSetup;
     bool seen      = false;
@@ -371,15 +501,15 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     if (tid < 2 * kLiftSetupAll)
     {
         LiftCell& f        = s_cell[slot];
-        const int64_t cell = (int64_t)slot * gridDim.x + blockIdx.x;
-        const bool left    = !a.first && cell < a.num_cells && a.plain_state[cell] != 0u;  // by an earlier band
-        bool behind        = cell >= a.num_cells || left;
+        const uint32_t cell = s_cells[slot];
+        const bool left    = !a.first && cell != kLiftNone && a.plain_state[cell] != 0u;  // by an earlier band
+        bool behind        = cell == kLiftNone || left;
         float max_x = -10000000.f, max_y = -10000000.f, min_x = 10000000.f, min_y = 10000000.f;
         float far = 0.f;  // largest coordinate
         if (!behind)
         {
-            const float* mn = a.bb_min + 3 * cell;
-            const float* ln = a.bb_length + 3 * cell;
+            const float* mn = a.bb_min + 3 * (size_t)cell;
+            const float* ln = a.bb_length + 3 * (size_t)cell;
             const float m[3] = {mn[0], mn[1], mn[2]}, n[3] = {ln[0], ln[1], ln[2]};
 #pragma unroll
             for (int u = 0; u < 8 / kLiftSetup; ++u)
@@ -519,29 +649,30 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
                         const float by = at_longest == 0 ? y[1] : at_longest == 1 ? y[2] : y[0];
                         const float ax = at_longest == 0 ? x[0] : at_longest == 1 ? x[1] : x[2];
                         const float ay = at_longest == 0 ? y[0] : at_longest == 1 ? y[1] : y[2];
-                        RowBound r;
+                        LineBound r;
+                        RowBound line;
                         bool is_left;
                         float half_width;
                         const float c1 = ay - by, dx = ax - bx;
                         if (half_plane(c1, dx, bx, by, 0.f, flat, r, is_left))
-                            half_width = err / fabsf(c1) + slack;
+                            half_width = (err / fabsf(c1) + slack) + 2.f * r.off(reach_y), line = r.from(f.min_y, reach_y, true);
                         else
-                            r.slope = 0.f, r.x0 = 0.f, r.y0 = by, half_width = -(err + flat * reach_x) / fmaxf(fabsf(dx), 1e-12f);
+                            line = {0.f, by}, half_width = -(err + flat * reach_x) / fmaxf(fabsf(dx), 1e-12f);
                         const int at = atomicAdd(&f.num_sliver, 1);
-                        if (at < kLiftSliverMax) f.sliver[at] = r, f.sliver_width[at] = half_width;
+                        if (at < kLiftSliverMax) f.sliver[at] = line, f.sliver_width[at] = half_width;
                     }
                     if (area > 4.f * err)
                     {
                         RowBound bound[3];  // a left one, a right one, one of either kind
                         bool have_left = false, have_right = false, third_is_left = true;
-                        bound[0] = {0.f, 0.f, -1e9f};
-                        bound[1] = {0.f, 0.f, 1e9f};
-                        bound[2] = {0.f, 0.f, -1e9f};
+                        bound[0] = {0.f, -1e9f};
+                        bound[1] = {0.f, 1e9f};
+                        bound[2] = {0.f, -1e9f};
 #pragma unroll
                         for (int k = 0; k < 3; ++k)
                         {
                             const float bx = x[(k + 1) % 3], by = y[(k + 1) % 3], c1 = y[k] - by, dx = x[k] - bx;
-                            RowBound r;
+                            LineBound r;
                             bool is_left = true;
                             if (half_plane(c1, dx, bx, by, err, flat, r, is_left))
                                 r.x0 += is_left ? slack : -slack;
@@ -558,12 +689,13 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
                                 is_left   = !have_left || have_right;
                                 if (!is_left) r.slope = -r.slope, r.x0 = -r.x0;
                             }
+                            const RowBound b = r.from(f.min_y, reach_y, is_left);
                             if (is_left && !have_left)
-                                bound[0] = r, have_left = true;
+                                bound[0] = b, have_left = true;
                             else if (!is_left && !have_right)
-                                bound[1] = r, have_right = true;
+                                bound[1] = b, have_right = true;
                             else
-                                bound[2] = r, third_is_left = is_left;
+                                bound[2] = b, third_is_left = is_left;
                         }
                         const int at = atomicAdd(&f.num_tri, 1);
                         if (at < kLiftTriangleMax)
@@ -589,13 +721,13 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
                     }
                     const float near = 8.f * err + 0.01f * (fabsf(c1) + fabsf(dx));
                     const float out  = margin * (fabsf(c1) + fabsf(dx)) + 4.f * err;
-                    RowBound r;
+                    LineBound r;
                     bool is_left;
                     auto keep = [&]() {
                         r.x0 += is_left ? -slack : slack;
                         const int at = atomicAdd(&f.num_outline, 1);
                         if (at >= kLiftOutlineMax) return;
-                        f.outline[at] = r;
+                        f.outline[at] = r.from(f.min_y, reach_y, !is_left);
                         if (is_left) atomicOr(&f.left_mask, 256u << at);
                     };
                     if (lowest > -near && half_plane(c1, dx, bx, by, lowest - out, flat, r, is_left)) keep();
@@ -630,15 +762,14 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
         const int y = (int)((float)(r - s_start[slot]) + f.min_y);
         // the box lies inside the bordered image by construction; the guard keeps a row outside the band from being read
         if (y < a.y0 || y >= a.y1) return;
-        const float fy = (float)y;
+        const float fy = (float)y, row = fy - f.min_y;
         // columns that may be covered
         const uint32_t left_mask = f.left_mask;
         float lo = (float)f.xs, hi = (float)f.xe;
         const int edges = f.num_sliver <= kLiftSliverMax ? min(f.num_outline, kLiftOutlineMax) : 0;
         for (int k = 0; k < edges; ++k)
         {
-            const RowBound r = f.outline[k];
-            const float v    = r.at(fy);
+            const float v    = f.outline[k].at(row);
             const bool left  = (left_mask >> (8 + k)) & 1u;
             lo = fmaxf(lo, left ? v : lo);
             hi = fminf(hi, left ? hi : v);
@@ -651,7 +782,7 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
             const float width   = f.sliver_width[k];
             if (width >= 0.f)
             {
-                const float v = line.at(fy);
+                const float v = line.at(row);
                 const float c0 = fmaxf(ceilf(v - width), (float)f.xs), c1 = fminf(floorf(v + width), (float)f.xe);
                 if (c0 <= c1)  // (an empty range grows to the columns of the line)
                 {
@@ -659,7 +790,7 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
                     x     = min(x, (int)c0);
                 }
             }
-            else if (fabsf(fy - line.y0) <= -width)
+            else if (fabsf(fy - line.x0) <= -width)
                 x = f.xs, x_end = f.xe + 1;
         }
         if (x >= x_end) return;
@@ -672,8 +803,8 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
             from[t] = 0x7FFFFFFF, to[t] = 0;
             if (t < triangles)
             {
-                const float v = f.tri[t][2].at(fy);
-                float l = f.tri[t][0].at(fy), h = f.tri[t][1].at(fy);
+                const float v = f.tri[t][2].at(row);
+                float l = f.tri[t][0].at(row), h = f.tri[t][1].at(row);
                 if ((left_mask >> t) & 1u)
                     l = fmaxf(l, v);
                 else
@@ -805,8 +936,8 @@ __global__ void __launch_bounds__(kLiftBlock) lift_cells_kernel(LiftPass a)
     __syncthreads();
     if (tid < kLiftCells)
     {
-        const int64_t cell = (int64_t)tid * gridDim.x + blockIdx.x;
-        if (cell >= a.num_cells || s_left[tid]) return;
+        const uint32_t cell = s_cells[tid];
+        if (cell == kLiftNone || s_left[tid]) return;
         const double in_front = a.first ? 0.0 : a.cell_sums[cell];
         if (s_cell[tid].wide > 0)
         {
@@ -864,14 +995,13 @@ __global__ void __launch_bounds__(kBlock) lift_plain_kernel(LiftPass a)
             if (count > 0)
             {
                 atomicAdd(&a.cell_sums[cell], sum);
-                atomicAdd(&a.plain_count[cell], count);
+                atomicAdd(&a.access_count[cell], count);
             }
             __threadfence();
             if ((atomicAdd(&a.plain_state[cell], 1u) & 0xFFu) == (uint32_t)kLiftPlainShare - 1u)
             {
                 __threadfence();
                 const double all = atomicAdd(&a.cell_sums[cell], 0.0);
-                a.access_count[cell] += atomicAdd(&a.plain_count[cell], 0);
                 a.value[cell] = (float)((double)a.value[cell] + all);
             }
         }

@@ -49,8 +49,8 @@ inline size_t align_up(size_t v, size_t a)
 }
 
 // Bytes of error-lifting scratch for num_cells cells: header (camera constants, counters, flag word), per cell the sum of
-// the bands so far (images that take several) and what lift_plain_kernel needs of the cells that are left to it (their
-// list, rows and finished shares, counted pixels), the running sums of a band of image rows.
+// the bands so far (images that take several), what lift_plain_kernel needs of the cells that are left to it (their
+// list, rows and finished shares) and its place among the cells that are seen, the running sums of a band of image rows.
 constexpr size_t align_up_c(size_t v, size_t a) { return (v + a - 1) / a * a; }
 constexpr size_t lift_workspace_bytes_for(size_t num_cells, size_t num_sums)
 {
@@ -436,7 +436,7 @@ void launch_lift(const vetrast_lift_args* a, char* ws, size_t num_sums, hipStrea
     lp.cell_sums         = reinterpret_cast<double*>(at);
     lp.plain_cell        = reinterpret_cast<uint32_t*>(at + doubles);
     lp.plain_state       = reinterpret_cast<uint32_t*>(at + doubles + words);
-    lp.plain_count       = reinterpret_cast<int32_t*>(at + doubles + 2 * words);
+    lp.seen              = reinterpret_cast<uint32_t*>(at + doubles + 2 * words);
     lp.sums              = reinterpret_cast<double*>(at + doubles + 3 * words);
 
     ViewSource src;
@@ -447,6 +447,10 @@ void launch_lift(const vetrast_lift_args* a, char* ws, size_t num_sums, hipStrea
     for (int j = 0; j < 5; ++j) src.crop[j] = v.crop_transform[j];
     for (int j = 0; j < 4; ++j) src.rot[j] = v.crop_rotation[j];
 
+    // cells in stretches of at most a workgroup's threads, kWave of which lift_cells_kernel looks at together
+    lp.stretches = (uint32_t)((a->num_cells + kWave * kLiftPrefixBlock - 1) / (kWave * kLiftPrefixBlock)) * kWave;
+    const unsigned groups_of_cells = lp.stretches / kWave, columns = (unsigned)((a->num_cells + lp.stretches - 1) / lp.stretches);
+    const unsigned shares = lift_shares(columns * kWave, groups_of_cells);  // as if all were seen
     // rows a cell can cover, in bands whose running sums fit their room
     const int64_t top = std::min<int64_t>(a->border_pixels, a->height), bottom = std::max<int64_t>(top, (int64_t)a->height - a->border_pixels);
     int64_t band = (int64_t)(num_sums / ((size_t)a->width + 1)) / kLiftRows * kLiftRows;
@@ -460,9 +464,10 @@ void launch_lift(const vetrast_lift_args* a, char* ws, size_t num_sums, hipStrea
         lp.first = y == top ? 1 : 0;
         lp.last  = lp.y1 == bottom ? 1 : 0;
         const unsigned groups = lp.sums ? (unsigned)std::max(1, (lp.y1 - lp.y0 + kLiftRows - 1) / kLiftRows) : 1u;
-        hipLaunchKernelGGL(lift_prefix_kernel, dim3(groups), dim3(kLiftPrefixBlock), 0, stream, lp, src, a->poses_se3, a->intrinsics);
-        hipLaunchKernelGGL(lift_cells_kernel, dim3((unsigned)((a->num_cells + kLiftCells - 1) / kLiftCells)), dim3(kLiftBlock), 0,
-                           stream, lp);
+        lp.prefix_groups      = groups;
+        hipLaunchKernelGGL(lift_prefix_kernel, dim3(groups + (lp.first ? lp.stretches : 0u)), dim3(kLiftPrefixBlock), 0, stream, lp, src,
+                           a->poses_se3, a->intrinsics);
+        hipLaunchKernelGGL(lift_cells_kernel, dim3(shares * groups_of_cells), dim3(kLiftBlock), 0, stream, lp);
         y += band;
     } while (y < bottom);
     hipLaunchKernelGGL(lift_plain_kernel, dim3(kLiftPlainShare, kLiftPlainAtOnce), dim3(kBlock), 0, stream, lp);
