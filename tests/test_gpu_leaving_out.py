@@ -1,0 +1,72 @@
+"""The rough look that launches of several views take at a point before they project it: points around the edges of the image and
+the reach of its coarsest layer, on both sides of the camera plane and next to it, far away and not finite, with crops that are
+skewed, turned, mirrored and far from the image centre. Whatever it leaves out would not have left a fragment: the lists are the
+oracle's."""
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import kept_mask
+from vet_amd import abi, synthetic
+from vet_amd.rasterizer import DeviceScene, make_params
+
+pytestmark = pytest.mark.gpu
+
+_TURN = (np.cos(0.4), -np.sin(0.4), np.sin(0.4), np.cos(0.4))
+_VIEWS = {
+    "plain": [dict(), dict()],
+    "crops": [dict(crop_transform=(1.0, 1.0, -900.0, 40.0, 0.0)), dict(crop_transform=(3.0, 0.25, 12.5, -7.25, 0.3))],
+    "turned": [dict(crop_rotation=_TURN), dict(crop_transform=(-1.5, 2.0, 150.0, -60.0, -0.2), crop_rotation=_TURN)],
+}
+
+
+def _points(view, rng, n):
+    """Points whose image position lies on and around the edges of the frame and of the coarsest layer's reach."""
+    w, h = view.w, view.h
+    edges_x, edges_y = [-9.0, -0.5, 0.0, w / 2, w - 0.5, w + 9.0, 4.0 * w], [-9.0, -0.5, 0.0, h / 2, h - 0.5, h + 9.0, -3.0 * h]
+    u = rng.choice(edges_x, n) + rng.choice([0.0, 1e-4, -1e-4, 0.3, -0.3], n)
+    v = rng.choice(edges_y, n) + rng.choice([0.0, 1e-4, -1e-4, 0.3, -0.3], n)
+    z = rng.choice([1e-5, 1e-2, 0.7, 1.0, 30.0, 1e4, -1e-5, -0.5, -40.0], n)
+    r, c = np.array(view.crop_rotation, np.float64).reshape(2, 2), view.crop_transform
+    centre = np.array([w // 2, h // 2], np.float64)
+    p = (np.stack([u, v], 1) - centre) @ r + centre  # inverse of a rotation
+    y = (p[:, 1] - c[3]) / c[1]
+    x = (p[:, 0] - c[2] - c[4] * y) / c[0]
+    return x, y, z
+
+
+@pytest.mark.parametrize("mode", [abi.RENDER_FULL_BLEND, abi.RENDER_BILINEAR_BLEND])
+@pytest.mark.parametrize("kind", sorted(_VIEWS))
+def test_nothing_that_leaves_a_fragment(kind, mode, rasterizer, oracle):
+    print(f"[case] leaving out: {kind} mode {mode}", flush=True)
+    scene = synthetic.tiny_scene(num_points=6000, K=8, seed=7)
+    w, h = scene.views[0].w, scene.views[0].h
+    scene.views = [synthetic.ViewSpec(w, h, image_index=scene.views[0].image_index, **f) for f in _VIEWS[kind]]
+    rng = np.random.RandomState(3)
+    n = scene.num_points
+    q, t = scene.poses_se3[scene.views[0].image_index][:4], scene.poses_se3[scene.views[0].image_index][4:7]
+    k = scene.intrinsics[scene.views[0].camera_index].astype(np.float64)
+    at = [_points(v, rng, n // 2) for v in scene.views]
+    x, y, z = (np.concatenate([a[i] for a in at]) for i in range(3))
+    ny = (y - k[3]) / k[1]
+    nx = (x - k[2] - k[4] * ny) / k[0]
+    cam = np.stack([nx * z, ny * z, z], 1)
+    rot = np.array([[1 - 2 * (q[1] ** 2 + q[2] ** 2), 2 * (q[0] * q[1] - q[3] * q[2]), 2 * (q[0] * q[2] + q[3] * q[1])],
+                    [2 * (q[0] * q[1] + q[3] * q[2]), 1 - 2 * (q[0] ** 2 + q[2] ** 2), 2 * (q[1] * q[2] - q[3] * q[0])],
+                    [2 * (q[0] * q[2] - q[3] * q[1]), 2 * (q[1] * q[2] + q[3] * q[0]), 1 - 2 * (q[0] ** 2 + q[1] ** 2)]])
+    position = scene.position.copy()
+    position[: len(cam), :3] = ((cam - t) @ rot).astype(np.float32)
+    position[5, :3], position[6, 0], position[7, 2] = 1e30, np.inf, np.nan
+    scene.position = position
+    params = make_params(scene, render_mode=mode)
+    res = rasterizer.forward(DeviceScene(scene), params)
+    torch.cuda.synchronize()
+    ref = oracle.forward(scene, params)
+    total = 0
+    for b in range(2):
+        off = ref.offsets[b].astype(np.int64)
+        np.testing.assert_array_equal(res.offsets(b), off)
+        kept = kept_mask(off, scene.max_list_length)
+        np.testing.assert_array_equal(res.fragments(b)[kept], ref.fragments[b, : int(off[-1])][kept])
+        total += int(off[-1])
+    assert total > 1000  # points on both sides of the edges are in the lists

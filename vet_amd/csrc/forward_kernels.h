@@ -91,8 +91,36 @@ __device__ __forceinline__ DeviceView make_device_view(const ViewSource& s, cons
     for (int j = 0; j < 4; ++j) v.rot[j] = s.rot[j];
     v.ccx = (float)(s.w / 2);
     v.ccy = (float)(s.h / 2);
-    for (int j = 0; j < 3; ++j) v.pad[j] = 0.f;
+    v.can_leave_out = 0u;
+    v.off_by_size = v.off = 0.f;
     return v;
+}
+
+// Fills in what surely_outside looks at, in place of the distortion coefficients of a camera that is used without them. Image
+// position = A (vx / vz, vy / vz) + b with A = crop rotation x crop transform x K, so image position times depth is linear in the
+// point: A (rows 0 and 1 of its view position) + b depth. `size` adds up the magnitudes of all factors and terms that the projection
+// rounds on its way, each of them less than 20 times by 2^-24 of itself, as these rows do; 2^-14 of it is 50 times that.
+__device__ __forceinline__ void prepare_leaving_out(DeviceView& v, float width, float height)
+{
+    const float k00 = v.crop[0] * v.fx, k01 = v.crop[0] * v.s + v.crop[4] * v.fy, k11 = v.crop[1] * v.fy;
+    const float a[2][2] = {{v.rot[0] * k00, v.rot[0] * k01 + v.rot[1] * k11}, {v.rot[2] * k00, v.rot[2] * k01 + v.rot[3] * k11}};
+    const float mx = (v.crop[0] * v.cx + v.crop[4] * v.cy) + v.crop[2] - v.ccx, my = v.crop[1] * v.cy + v.crop[3] - v.ccy;
+    const float b[2] = {v.rot[0] * mx + v.rot[1] * my + v.ccx, v.rot[2] * mx + v.rot[3] * my + v.ccy};
+    float largest = 0.f;
+    for (int j = 0; j < 9; ++j) largest = fmaxf(largest, fabsf(v.r[j]));
+    const float turn = fabsf(v.rot[0]) + fabsf(v.rot[1]) + fabsf(v.rot[2]) + fabsf(v.rot[3]) + 1.f;
+    const float crop = fabsf(v.crop[0]) + fabsf(v.crop[1]) + fabsf(v.crop[4]) + 1.f;
+    const float size = turn * (crop * (fabsf(v.fx) + fabsf(v.fy) + fabsf(v.s) + fabsf(v.cx) + fabsf(v.cy)) + fabsf(v.crop[2]) + fabsf(v.crop[3]) +
+                               2.f * (fabsf(v.ccx) + fabsf(v.ccy))) + width + height + (float)(2 << VETRAST_MAX_LAYERS);
+    for (int i = 0; i < 2; ++i)
+    {
+        for (int j = 0; j < 3; ++j) v.image_row[i][j] = a[i][0] * v.r[j] + a[i][1] * v.r[3 + j] + b[i] * v.r[6 + j];
+        v.image_row[i][3] = a[i][0] * v.t[0] + a[i][1] * v.t[1] + b[i] * v.t[2];
+    }
+    const float far = fabsf(v.t[0]) + fabsf(v.t[1]) + fabsf(v.t[2]);
+    v.off_by_size   = 6.1035156e-5f * size * (3.f * largest);
+    v.off           = 6.1035156e-5f * size * far + 1e-30f;
+    v.can_leave_out = size < 1e15f && largest < 1e3f && far < 1e15f ? 1u : 0u;  // (nothing overflows, see surely_outside)
 }
 
 // One thread per view fills its camera constants; non-zero distortion coefficients raise flag bit 0 unless the caller
@@ -135,6 +163,7 @@ __global__ void __launch_bounds__(kBlock) prepare_views_kernel(PrepareViewsArgs 
         atomicOr(flags, 1u);  // refused: the call renders the camera without distortion and says so
         v.has_dist = 0u;
     }
+    if (!allow_distortion) prepare_leaving_out(v, (float)args.src[k].w, (float)args.src[k].h);
     views[first_view + k] = v;
 }
 
@@ -698,8 +727,10 @@ __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* _
     if (packs) store_packed_row(pack, slot, row, row_confidence);
 }
 
-// The pass for one view: fetch, projection, and the above.
-template <int HITS>
+// The pass for one view: fetch, projection, and the above. LEAVE_OUT: points are looked at roughly first (surely_outside). Launches of
+// several views do, which mostly are crops that see a tenth of the cloud: four crops of two million points 69.8 and 65.5 us (four town
+// views, bound by their atomics, 182 either way); a full frame sees half of it, 33 us either way.
+template <int HITS, bool LEAVE_OUT>
 __device__ __forceinline__ void bin_scatter(const ViewPass& a, uint32_t* __restrict__ bin_counts,
                                             const ScatterTargets& out, const PackJob& pack)
 {
@@ -709,7 +740,13 @@ __device__ __forceinline__ void bin_scatter(const ViewPass& a, uint32_t* __restr
     const int i = (a.point_order != nullptr && slot < a.N) ? a.point_order[slot] : slot;
     Projected p;
     p.ipx = p.ipy = p.z = p.radius = 0.f;
-    const bool visible = (uint32_t)i < (uint32_t)a.N && !point_is_skipped(a, i) && project_point(*a.view, a.position[i], p);
+    bool visible = (uint32_t)i < (uint32_t)a.N && !point_is_skipped(a, i);
+    if (visible)
+    {
+        const float4 position = a.position[i];
+        const float reach     = (float)(1 << (a.ly.L - 1)) + 1.f;
+        visible = !(LEAVE_OUT && surely_outside(*a.view, (float)a.ly.w[0], (float)a.ly.h[0], reach, position)) && project_point(*a.view, position, p);
+    }
     scatter_projected<HITS>(a, bin_counts, out, pack, slot, i, visible, p);
 }
 
@@ -717,7 +754,7 @@ template <int HITS>
 __global__ void __launch_bounds__(kBlock, kScatterWaves<HITS>) bin_scatter_kernel(ViewPass a, uint32_t* __restrict__ bin_counts,
                                                               ScatterTargets out, PackJob pack)
 {
-    bin_scatter<HITS>(a, bin_counts, out, pack);
+    bin_scatter<HITS, false>(a, bin_counts, out, pack);
 }
 
 struct ScatterArgs
@@ -738,7 +775,7 @@ template <int HITS>
 __global__ void __launch_bounds__(kBlock, kScatterWaves<HITS>) bin_scatter_views_kernel(PerView<ScatterArgs> views)
 {
     const ScatterArgs& v = views.v[blockIdx.y];
-    bin_scatter<HITS>(v.view, v.bin_counts, v.out, v.pack);
+    bin_scatter<HITS, true>(v.view, v.bin_counts, v.out, v.pack);
 }
 
 // The interleave as a launch of its own, for a caller that keeps the records across calls while texture and confidence
