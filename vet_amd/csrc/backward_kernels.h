@@ -2040,7 +2040,7 @@ struct CameraPass
 };
 static_assert(kViewLanes <= kBlock / kWave, "a wave per view of a round");
 
-__global__ void __launch_bounds__(kBlock) reduce_camera_kernel(CameraPass a)
+__device__ __forceinline__ void reduce_camera(const CameraPass& a)
 {
     __shared__ double red[kBlock / kWave][kCameraRow];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -2101,17 +2101,34 @@ __global__ void __launch_bounds__(kBlock) reduce_camera_kernel(CameraPass a)
 // Division of the accumulated position gradient by the number of contributing fragments.
 // mode 1: row i of the [N,4] buffer by count[i]. mode 2: the reference's literal behaviour, which walks the same
 // memory as N vec3 (src/lib/rendering/PointRenderer.cu:1072-1090,1278-1279), i.e. flat elements 3i..3i+2 by count[i].
-__global__ void __launch_bounds__(kBlock) normalize_point_gradient_kernel(float* __restrict__ grad_points,
-                                                                           const float* __restrict__ count, int N,
-                                                                           int mode)
+__device__ __forceinline__ void normalize_point_gradient(float* __restrict__ grad_points, const float* __restrict__ count, int N, int mode, int i)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     const float c = count[i];
     if (!(c > 0.f)) return;
     const size_t base = (mode == 2 ? 3 : 4) * (size_t)i;
 #pragma unroll
     for (int k = 0; k < 3; ++k) grad_points[base + k] = grad_points[base + k] / c;
+}
+
+__global__ void __launch_bounds__(kBlock) normalize_point_gradient_kernel(float* __restrict__ grad_points, const float* __restrict__ count,
+                                                                           int N, int mode)
+{
+    normalize_point_gradient(grad_points, count, N, mode, (int)(blockIdx.x * blockDim.x + threadIdx.x));
+}
+
+// The camera gradients, by the launch's first workgroup, and behind a call's last round the division of the position gradients by the
+// others beside it: neither waits for the other, and the camera rows are one workgroup's chain (four crops of two million points 8.9 and
+// 5.8 us one after the other, 9.1 together; a crop of 60 thousand 5.6 and 3.8, together 6.0). Without cameras the division has a kernel
+// of its own, whose 21 registers are a third of this one's (ten million points 51 and 56 us). The rows folded here as well, by workgroups the last of
+// which goes on with the sums, took 22 us where the three launches took 19: each of them writes its L2 back for it.
+__global__ void __launch_bounds__(kBlock) finish_gradients_kernel(CameraPass camera, float* __restrict__ grad_points, const float* __restrict__ count,
+                                                                   int N, int mode)
+{
+    if (blockIdx.x == 0)
+        reduce_camera(camera);
+    else
+        normalize_point_gradient(grad_points, count, N, mode, (int)((blockIdx.x - 1u) * blockDim.x + threadIdx.x));
 }
 
 }  // namespace vetrast

@@ -1182,6 +1182,7 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             else
                 with_channels(std::integral_constant<int, 4>{});
         }
+        const bool divide = g->grad_points && p.point_gradient_normalization != 0 && N > 0 && last == B;
         if (want_camera)
         {
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_GATHER);
@@ -1216,7 +1217,14 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             cp.normalize             = (p.camera_gradient_normalization && last == B) ? 1 : 0;
             cp.num_poses             = a->num_poses;
             cp.num_cameras           = a->num_cameras;
-            hipLaunchKernelGGL(reduce_camera_kernel, dim3(1), dim3(kBlock), 0, stream, cp);
+            hipLaunchKernelGGL(finish_gradients_kernel, dim3(1u + (divide ? (unsigned)grid_for(N) : 0u)), dim3(kBlock), 0, stream, cp, g->grad_points,
+                               g->grad_point_count, N, p.point_gradient_normalization);
+        }
+        else if (divide)
+        {
+            ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_POST);
+            hipLaunchKernelGGL(normalize_point_gradient_kernel, dim3(grid_for(N)), dim3(kBlock), 0, stream, g->grad_points, g->grad_point_count, N,
+                               p.point_gradient_normalization);
         }
         for (int v = first; N == 0 && v < last; ++v)
         {
@@ -1226,12 +1234,6 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
                                background_rows_count, C, g->grad_background, g->grad_confidence, 0, v > 0 ? 1 : 0,
                                p.texture_abs ? a->background : nullptr);
         }
-    }
-    if (g->grad_points && p.point_gradient_normalization != 0 && N > 0)
-    {
-        ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_POST);
-        hipLaunchKernelGGL(normalize_point_gradient_kernel, dim3(grid_for(N)), dim3(kBlock), 0, stream,
-                           g->grad_points, g->grad_point_count, N, p.point_gradient_normalization);
     }
     VET_HIP(ctx, hipGetLastError());
     return VETRAST_OK;
