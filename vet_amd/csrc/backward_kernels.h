@@ -469,23 +469,30 @@ struct FuzzyPixel
     float g[4], ax[4], ay[4], bx, by;  // upstream gradient; position heuristic in slope / offset form
 };
 
-template <int C>
-__device__ __forceinline__ FuzzyPixel fuzzy_pixel(const BackwardPass& a, const TilePixel& px)
+// Its list; the rest is zero.
+__device__ __forceinline__ FuzzyPixel fuzzy_list(const BackwardPass& a, const TilePixel& px)
 {
     FuzzyPixel f;
     f.n = f.off = 0, f.do_point = false, f.bx = f.by = 0.f;
 #pragma unroll
     for (int ci = 0; ci < 4; ++ci) f.g[ci] = f.ax[ci] = f.ay[ci] = 0.f;
     if (!px.active) return f;
+    f.off = a.offsets[px.q];
+    f.n   = a.offsets[px.q + 1] - f.off;
+    if (a.K > 0) f.n = min(f.n, (uint32_t)a.K);
+    return f;
+}
+
+// The rest, of a pixel inside the image.
+template <int C>
+__device__ __forceinline__ void fuzzy_samples(const BackwardPass& a, const TilePixel& px, FuzzyPixel& f)
+{
     const int l = px.l, lw = a.ly.w[l], lh = a.ly.h[l];
     const size_t plane   = (size_t)lw * lh;
     const uint32_t local = px.local;
     const float* G       = a.grad_out[l];
 #pragma unroll
     for (int ci = 0; ci < C; ++ci) f.g[ci] = G[ci * plane + local];
-    f.off = a.offsets[px.q];
-    f.n   = a.offsets[px.q + 1] - f.off;
-    if (a.K > 0) f.n = min(f.n, (uint32_t)a.K);
     f.do_point = a.need_point_gradient && f.n > 0 && interior_pixel(px.x, px.y, lw, lh);
     if (f.do_point)
     {
@@ -504,7 +511,6 @@ __device__ __forceinline__ FuzzyPixel fuzzy_pixel(const BackwardPass& a, const T
             f.by += 0.5f * (Iy0 * Gy0 - Iy1 * Gy1);
         }
     }
-    return f;
 }
 
 // Lists of up to kFuzzyDense fragments are laid out densely, one lane per FRAGMENT, as in blend_backward_kernel; what is
@@ -542,6 +548,9 @@ constexpr int kFuzzyLongColumn = 6;   // background row, column 6: the workgroup
 // replicas and a workgroup for each 88, with 4 or 8 looked at 88; 8 replicas with 8 looked at 80, 16 replicas 90, with rows of 32 bytes for
 // each of the dense kernel's workgroups. With one row a workgroup, against 4 replicas and a workgroup for each (another card): 80
 // / 93, four of five 617x617 views 679 / 743, the fifth 247 / 333; both kernels together 700x500 131 / 151, 384x384 126 / 139, 203x155 91 / 117.
+// A replica looks at the samples around its own lists' pixels only, and not at all at a tile where it has none (77 us of the two views
+// until then, 73 with it); the scans of a step are moves between registers (68; through the LDS crossbar they were chains of six exchanges).
+// With that, 16 replicas take 72 us, 4 workgroups looked at 73, 2 of them 82.
 constexpr int kFuzzyReplicas   = 8;
 constexpr int kFuzzyFoldRows   = 256;
 constexpr int kLongRow         = 4;
@@ -575,8 +584,9 @@ __device__ __forceinline__ void blend_backward_fuzzy(const BackwardPass& a, floa
     for (int ci = 0; ci < C; ++ci) bg_grad[ci] = 0.f;
     uint32_t n;
     {
-        const FuzzyPixel f = fuzzy_pixel<C>(a, px);
-        n                  = f.n;
+        FuzzyPixel f = fuzzy_list(a, px);
+        if (px.active) fuzzy_samples<C>(a, px, f);
+        n = f.n;
         // an empty list: the background is the only bucket, one element of confidence 1 with nothing in front of it
         if (px.active && n == 0 && with_background)
 #pragma unroll
@@ -1051,6 +1061,33 @@ __global__ void __launch_bounds__(kBlock) blend_backward_fuzzy_views_kernel(PerV
 // its total inside its one step and is processed once). The elements of a bucket that was
 // still open at the end of their step get the position part of their record there and the bucket's part when it
 // closes, from a loop over their keys. Grid: fuzzy_long_grid x kFuzzyReplicas.
+// Sum over the lanes from `dist` lanes below up to this one (dist <= lane), in moves between registers: inside a row of 16 lanes, then
+// from the last lane of a row to the next row, then from the lower half to the upper one. Every lane of the wave must be active.
+__device__ __forceinline__ float sum_from(float v, uint32_t dist, int lane)
+{
+    auto add = [&](uint32_t from, bool same) { v += same ? __uint_as_float(from) : 0.f; };
+    add(dpp_shifted<0x111, 0xF>(__float_as_uint(v)), dist >= 1u);
+    add(dpp_shifted<0x112, 0xF>(__float_as_uint(v)), dist >= 2u);
+    add(dpp_shifted<0x114, 0xF>(__float_as_uint(v)), dist >= 4u);
+    add(dpp_shifted<0x118, 0xF>(__float_as_uint(v)), dist >= 8u);
+    add(dpp_shifted<0x142, 0xA>(__float_as_uint(v)), dist > (uint32_t)(lane & 15));
+    add(dpp_shifted<0x143, 0xC>(__float_as_uint(v)), dist > (uint32_t)(lane & 31));
+    return v;
+}
+// Product over the lanes up to this one; lanes a move leaves without a source multiply with one.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_or_one(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0x3F800000, __float_as_int(v), CTRL, ROW_MASK, 0xF, false));
+}
+__device__ __forceinline__ float product_up_to(float v)
+{
+    v *= dpp_or_one<0x111, 0xF>(v), v *= dpp_or_one<0x112, 0xF>(v);
+    v *= dpp_or_one<0x114, 0xF>(v), v *= dpp_or_one<0x118, 0xF>(v);
+    v *= dpp_or_one<0x142, 0xA>(v), v *= dpp_or_one<0x143, 0xC>(v);
+    return v;
+}
+
 template <int C>
 __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a, float depth_accept, uint32_t dense_max)
 {
@@ -1069,6 +1106,7 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
         if (threadIdx.x < (uint32_t)kLongRow) row[threadIdx.x] = 0.f;
         return;
     }
+    auto reversed = [&](float v) { return __uint_as_float(lane_xor<63>(__float_as_uint(v), lane)); };
     float bg_grad[C];  // summed over the wave at the end: every lane adds what it computes for lane 0's sake once
 #pragma unroll
     for (int ci = 0; ci < C; ++ci) bg_grad[ci] = 0.f;
@@ -1076,17 +1114,21 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
     {
         const int from     = __ffsll((unsigned long long)with_list) - 1;
         const TilePixel px = tile_pixel(a.tiles, a.ly, blockIdx.x + (uint32_t)from * gridDim.x);
-        const FuzzyPixel f = fuzzy_pixel<C>(a, px);
+        FuzzyPixel f       = fuzzy_list(a, px);
+        // this replica's lists; only their pixels are looked at further
+        const uint64_t longer = __ballot(f.n > dense_max);
+        const uint32_t turn   = __builtin_amdgcn_mbcnt_hi((uint32_t)(longer >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)longer, 0u));
+        const bool mine       = f.n > dense_max && turn % (uint32_t)kFuzzyReplicas == replica;
+        uint64_t todo         = __ballot(mine);
+        if (todo == 0ull) continue;
+        if (mine) fuzzy_samples<C>(a, px, f);
         float4* partial_l  = a.partial;  // (records are addressed by gradient_record)
         const bool with_background = !a.use_environment_map;
         auto everywhere = [&](float v, int src) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), src)); };
 
-        uint64_t todo = __ballot(f.n > dense_max);
-        for (uint32_t turn = 0; todo != 0ull; ++turn)
+        for (; todo != 0ull; todo &= todo - 1ull)
         {
             const int src = __ffsll((unsigned long long)todo) - 1;
-            todo &= todo - 1ull;
-            if (turn % (uint32_t)kFuzzyReplicas != replica) continue;
             // the pixel, the same on every lane
             const uint32_t n       = (uint32_t)__builtin_amdgcn_readlane((int)f.n, src);
             const uint64_t* list   = a.fragments + (uint32_t)__builtin_amdgcn_readlane((int)f.off, src);
@@ -1207,14 +1249,7 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
 #pragma unroll
                     for (int v = 0; v <= C; ++v)
                     {
-                        float x = sums[v];
-#pragma unroll
-                        for (int d = 1; d < kWave; d <<= 1)
-                        {
-                            const float o = __shfl_up(x, d, kWave);
-                            if (dist >= (uint32_t)d) x += o;
-                        }
-                        sums[v] = __shfl(x, last_lane, kWave);
+                        sums[v] = __shfl(sum_from(sums[v], dist, lane), last_lane, kWave);
                         if (joined) sums[v] = open_sums[v] + sums[v];
                     }
                     uint32_t m = has ? (next - first) + (joined ? open_m : 0u) : 1u;
@@ -1233,13 +1268,7 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
                     // transmittance in front: product of (1 - mean confidence) over the buckets that close in this step in
                     // front of this one, times what was in front of the step
                     const bool closing_lane = closes && lane == last_lane;
-                    float P = closing_lane ? 1.f - bconf : 1.f;
-#pragma unroll
-                    for (int d = 1; d < kWave; d <<= 1)
-                    {
-                        const float o = __shfl_up(P, d, kWave);
-                        if (lane >= d) P *= o;
-                    }
+                    const float P = product_up_to(closing_lane ? 1.f - bconf : 1.f);
                     const float P_before = __shfl(P, first > 0u ? (int)first - 1 : lane, kWave);
                     const float A        = first > 0u ? A_front * P_before : A_front;
                     const float P_end    = everywhere(P, (int)valid - 1);  // over all buckets that close in this step
@@ -1249,13 +1278,8 @@ __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a,
                     // Terms of the buckets that close in this step, summed from the back: a bucket needs the terms of the
                     // buckets BEHIND it, and taking them as (all) - (those in front) would cancel to rounding noise deep in
                     // a list, where what is left behind is a millionth of what lies in front.
-                    float X = closing_lane ? x : 0.f;
-#pragma unroll
-                    for (int d = 1; d < kWave; d <<= 1)
-                    {
-                        const float o = __shfl_down(X, d, kWave);
-                        if (lane + d < kWave) X += o;
-                    }
+                    // (as a sum from the front with the lanes the other way round)
+                    const float X = reversed(sum_from(reversed(closing_lane ? x : 0.f), (uint32_t)lane, lane));
                     const float X_end = everywhere(X, 0);  // all of them
                     if (one_step)
                     {
