@@ -478,32 +478,39 @@ torch::autograd::variable_list PointRender::backward(torch::autograd::AutogradCo
     torch::Tensor g_texture    = torch::empty_like(texture);
     torch::Tensor g_confidence = torch::empty_like(confidence);
     torch::Tensor g_background = torch::empty_like(background_color);
-    torch::Tensor g_points, g_point_count;
+    // The counts of the three normalised gradients are this call's own: one allocation for all of them.
+    const bool points_need_grad = ctx->saved_data["points_need_grad"].toBool(), pose_needs_grad = ctx->saved_data["pose_need_grad"].toBool();
+    const bool intr_needs_grad  = ctx->saved_data["intr_need_grad"].toBool();
+    const int64_t F             = ctx->saved_data["num_poses"].toInt();
+    const int64_t point_counts = points_need_grad ? points.size(0) : 0, pose_counts = pose_needs_grad ? F : 0;
+    const int64_t intr_counts  = intr_needs_grad ? intrinsics.size(0) : 0;
+    torch::Tensor counts;
+    if (point_counts + pose_counts + intr_counts > 0) counts = torch::empty({point_counts + pose_counts + intr_counts}, points.options());
+    float* next_count = counts.defined() ? counts.data_ptr<float>() : nullptr;
+    torch::Tensor g_points;
     g.grad_texture    = g_texture.data_ptr<float>();
     g.grad_confidence = g_confidence.data_ptr<float>();
     g.grad_background = g_background.data_ptr<float>();
-    if (ctx->saved_data["points_need_grad"].toBool())
+    if (points_need_grad)
     {
         g_points           = torch::empty_like(points);
-        g_point_count      = torch::empty({points.size(0)}, points.options());
         g.grad_points      = g_points.data_ptr<float>();
-        g.grad_point_count = g_point_count.data_ptr<float>();
+        g.grad_point_count = next_count;
+        next_count += point_counts;
     }
-    torch::Tensor g_pose, g_pose_count, g_intrinsics, g_intrinsics_count;
-    if (ctx->saved_data["pose_need_grad"].toBool())  // PointRenderer.cu:287-293
+    torch::Tensor g_pose, g_intrinsics;
+    if (pose_needs_grad)  // PointRenderer.cu:287-293
     {
-        const int64_t F      = ctx->saved_data["num_poses"].toInt();
-        g_pose               = torch::empty({F, 6}, points.options().dtype(torch::kFloat64));
-        g_pose_count         = torch::empty({F}, points.options());
-        g.grad_pose          = g_pose.data_ptr<double>();
-        g.grad_pose_count    = g_pose_count.data_ptr<float>();
+        g_pose            = torch::empty({F, 6}, points.options().dtype(torch::kFloat64));
+        g.grad_pose       = g_pose.data_ptr<double>();
+        g.grad_pose_count = next_count;
+        next_count += pose_counts;
     }
-    if (ctx->saved_data["intr_need_grad"].toBool())  // PointRenderer.cu:295-300
+    if (intr_needs_grad)  // PointRenderer.cu:295-300
     {
         g_intrinsics            = torch::empty_like(intrinsics);
-        g_intrinsics_count      = torch::empty({intrinsics.size(0)}, intrinsics.options());
         g.grad_intrinsics       = g_intrinsics.data_ptr<float>();
-        g.grad_intrinsics_count = g_intrinsics_count.data_ptr<float>();
+        g.grad_intrinsics_count = next_count;
     }
     check_status(vetrast_backward(info->cache->ctx, &g, current_stream()), "backward");
 

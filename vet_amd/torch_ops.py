@@ -6,6 +6,7 @@ import torch  # noqa: F401  (libtorch must be loaded before the extension)
 
 _PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "vetrast_torch.so")
 _mod = None
+_no_index = torch.empty(0, dtype=torch.int32)  # stands for "no texture index"; on the host, so that no call allocates on the device
 
 
 def load():
@@ -33,7 +34,7 @@ def blend_point_cloud(texture, background_color, points, pose_tangents, intrinsi
     no_envmap_at_points, the default) or appended as channels (cat_env_to_color). Needs output_background_mask.
     """
     if t_index is None:
-        t_index = torch.empty(0, dtype=torch.int32, device=points.device)
+        t_index = _no_index
     return load().blend_point_cloud(texture, background_color, points, pose_tangents, intrinsics, confidence, poses_se3,
                                     t_index, [list(map(float, v)) for v in views], int(num_layers), bool(train),
                                     {k: float(v) for k, v in params.items()}, environment)
