@@ -1,7 +1,7 @@
 """The rough look that launches of several views take at a point before they project it: points around the edges of the image and
 the reach of its coarsest layer, on both sides of the camera plane and next to it, far away and not finite, with crops that are
 skewed, turned, mirrored and far from the image centre. Whatever it leaves out would not have left a fragment: the lists are the
-oracle's."""
+oracle's, and some of their fragments are of points as far outside the image as a pixel of the coarsest layer reaches."""
 import numpy as np
 import pytest
 import torch
@@ -20,12 +20,18 @@ _VIEWS = {
 }
 
 
-def _points(view, rng, n):
-    """Points whose image position lies on and around the edges of the frame and of the coarsest layer's reach."""
+def _edges(size, layers):
+    """Coordinates inside the image and at its edges, half and all of a coarsest pixel outside (as far as one hit and the 2x2 splat
+    reach), a pixel further, and far away."""
+    r = 2.0 ** (layers - 1)
+    return [-r - 1, -r, -r / 2, -0.5, 0.0, size / 2, size - 0.5, size, size + r / 2, size + r, size + r + 1]
+
+
+def _points(view, layers, rng, n):
+    """Points whose image position lies on and around these."""
     w, h = view.w, view.h
-    edges_x, edges_y = [-9.0, -0.5, 0.0, w / 2, w - 0.5, w + 9.0, 4.0 * w], [-9.0, -0.5, 0.0, h / 2, h - 0.5, h + 9.0, -3.0 * h]
-    u = rng.choice(edges_x, n) + rng.choice([0.0, 1e-4, -1e-4, 0.3, -0.3], n)
-    v = rng.choice(edges_y, n) + rng.choice([0.0, 1e-4, -1e-4, 0.3, -0.3], n)
+    u = rng.choice(_edges(w, layers) + [4.0 * w], n) + rng.choice([0.0, 1e-4, -1e-4, 0.3, -0.3], n)
+    v = rng.choice(_edges(h, layers) + [-3.0 * h], n) + rng.choice([0.0, 1e-4, -1e-4, 0.3, -0.3], n)
     z = rng.choice([1e-5, 1e-2, 0.7, 1.0, 30.0, 1e4, -1e-5, -0.5, -40.0], n)
     r, c = np.array(view.crop_rotation, np.float64).reshape(2, 2), view.crop_transform
     centre = np.array([w // 2, h // 2], np.float64)
@@ -35,18 +41,28 @@ def _points(view, rng, n):
     return x, y, z
 
 
+def _furthest(oracle, scene, ref, b, hits):
+    """How many pixels outside the image the furthest point is that has left a fragment in view b."""
+    view = scene.views[b]
+    prepared = oracle.prepare_view(scene.poses_se3[view.image_index], scene.intrinsics[view.camera_index])
+    total = int(ref.offsets[b, -1])
+    ids = np.unique((ref.fragments[b, :total] & np.uint64(0xFFFFFFFF)).astype(np.int64) >> (2 if hits == 4 else 0))
+    at = np.array([oracle.project_point(prepared, ref.views[b], scene.position[i])[1][:2] for i in ids], np.float64)
+    return max(-at.min(), (at - [view.w, view.h]).max())
+
+
 @pytest.mark.parametrize("mode", [abi.RENDER_FULL_BLEND, abi.RENDER_BILINEAR_BLEND])
 @pytest.mark.parametrize("kind", sorted(_VIEWS))
-def test_nothing_that_leaves_a_fragment(kind, mode, rasterizer, oracle):
-    print(f"[case] leaving out: {kind} mode {mode}", flush=True)
-    scene = synthetic.tiny_scene(num_points=6000, K=8, seed=7)
-    w, h = scene.views[0].w, scene.views[0].h
+@pytest.mark.parametrize("layers,w,h", [(1, 25, 17), (3, 24, 16), (5, 83, 61)])
+def test_nothing_that_leaves_a_fragment(layers, w, h, kind, mode, rasterizer, oracle):
+    print(f"[case] leaving out: {kind} mode {mode} {w}x{h} {layers} layers", flush=True)
+    scene = synthetic.tiny_scene(num_points=6000, w=w, h=h, num_layers=layers, K=8, seed=7)
     scene.views = [synthetic.ViewSpec(w, h, image_index=scene.views[0].image_index, **f) for f in _VIEWS[kind]]
     rng = np.random.RandomState(3)
     n = scene.num_points
     q, t = scene.poses_se3[scene.views[0].image_index][:4], scene.poses_se3[scene.views[0].image_index][4:7]
     k = scene.intrinsics[scene.views[0].camera_index].astype(np.float64)
-    at = [_points(v, rng, n // 2) for v in scene.views]
+    at = [_points(v, layers, rng, n // 2) for v in scene.views]
     x, y, z = (np.concatenate([a[i] for a in at]) for i in range(3))
     ny = (y - k[3]) / k[1]
     nx = (x - k[2] - k[4] * ny) / k[0]
@@ -62,11 +78,14 @@ def test_nothing_that_leaves_a_fragment(kind, mode, rasterizer, oracle):
     res = rasterizer.forward(DeviceScene(scene), params)
     torch.cuda.synchronize()
     ref = oracle.forward(scene, params)
+    hits = 4 if mode == abi.RENDER_BILINEAR_BLEND else 1
+    reach = 2.0 ** (layers - 1) * (1.0 if hits == 4 else 0.5)
     total = 0
-    for b in range(2):
+    for b in range(len(scene.views)):
         off = ref.offsets[b].astype(np.int64)
         np.testing.assert_array_equal(res.offsets(b), off)
         kept = kept_mask(off, scene.max_list_length)
         np.testing.assert_array_equal(res.fragments(b)[kept], ref.fragments[b, : int(off[-1])][kept])
         total += int(off[-1])
-    assert total > 1000  # points on both sides of the edges are in the lists
+        assert reach - 0.31 < _furthest(oracle, scene, ref, b, hits) <= reach
+    assert total > 300  # points on both sides of the edges are in the lists
