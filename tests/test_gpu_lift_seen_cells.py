@@ -3,6 +3,7 @@ stretches and the 4 neighbours that stay together in one. Counts are whole numbe
 rounded once, as the oracle's is."""
 import numpy as np
 import pytest
+import torch
 
 from tests.test_gpu_lift_rows import _both, _camera, _lift
 from vet_amd import synthetic
@@ -30,3 +31,37 @@ def test_no_cell_is_seen(rasterizer):
     poses, intr = _camera(w, h, (0.0, 0.0, -5.0))
     val, cnt = _lift(rasterizer, mn, ln, ViewSpec(w, h), poses, intr, synthetic.error_image(1, 3, h, w), 0)
     assert not val.any() and not cnt.any()
+
+
+def _left_to_the_plain_kernel(workspace, cells):
+    """First image rows of the bands from which on cells were tested pixel by pixel."""
+    up = lambda b: (b + 255) // 256 * 256  # noqa: E731
+    words = workspace.cpu().numpy().view(np.uint32)
+    listed = 256 + up(8 * cells)
+    state  = listed + up(4 * cells)
+    which  = words[listed // 4 : listed // 4 + words[180 // 4]]
+    return (words[state // 4 + which] >> 8).astype(np.int64) - 1
+
+
+# An image of three bands of rows: the first one's list of seen cells, several groups of stretches long, serves the others, where cells
+# next to the camera's lower side turn out to have too many wide open rows.
+@pytest.mark.parametrize("cells", [20000, 33000])
+def test_list_of_seen_cells_serves_all_bands(cells, rasterizer, oracle):
+    print(f"[case] lift {cells} cells, three bands", flush=True)
+    w, h, border = 2000, 4400, 16
+    mn, ln = synthetic.cell_grid(np.array([[-1.15, -1.15, -1.15], [1.12, 1.12, 1.12]]), 0.07)
+    keep = np.sort(np.argsort(np.linalg.norm(mn + ln / 2, axis=1), kind="stable")[:cells])
+    mn, ln = mn[keep], ln[keep]
+    planes = np.unique(mn[:, 2])
+    poses, intr = _camera(w, h, (0.013, -0.007, 0.01 - float(planes[len(planes) // 2])), 0.3, f=0.52 * w)
+    img = synthetic.error_image(cells, 2, h, w)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (mn, ln, poses, intr, img)]
+    val, cnt = torch.zeros(cells, device="cuda"), torch.zeros(cells, dtype=torch.int32, device="cuda")
+    workspace = rasterizer.lift_error(dev[0], dev[1], val, cnt, ViewSpec(w, h), dev[2], dev[3], dev[4], border_pixels=border)
+    torch.cuda.synchronize()
+    want_v, want_c = np.zeros(cells, np.float32), np.zeros(cells, np.int32)
+    oracle.lift_error(mn, ln, want_v, want_c, ViewSpec(w, h), poses, intr, img, border_pixels=border, num_threads=16)
+    assert 0.02 * cells < (want_c > 0).sum() < 0.6 * cells
+    assert (_left_to_the_plain_kernel(workspace, cells) > border).any()
+    np.testing.assert_array_equal(cnt.cpu().numpy(), want_c)
+    np.testing.assert_allclose(val.cpu().numpy(), want_v, rtol=1e-6, atol=1e-9)
