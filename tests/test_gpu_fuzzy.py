@@ -262,3 +262,27 @@ def test_long_buckets_against_a_float64_evaluation(rasterizer, oracle):
         print(f"  {key}: library vs float64 {lib_err:.2e}, oracle vs float64 {oracle_err:.2e}", flush=True)
         assert lib_err <= 5e-5, key
         assert oracle_err <= 1e-3, key
+
+
+@pytest.mark.parametrize("points,bucket", [(4000, 1), (12000, 1), (9000, 8)])
+def test_long_lists_of_many_buckets_against_a_float64_evaluation(points, bucket, rasterizer):
+    """Lists of up to several steps of a wave, in buckets of about `bucket` fragments that close inside a step or at its end: sums over the
+    lanes of a bucket, products over the buckets in front and sums over those behind. Confidences are low, so that something is left
+    behind all of them. What is in front of a bucket is a product of as many factors as there are buckets, each of them a rounded
+    difference and each product rounded: 2^-23 a bucket, relative to the largest gradients as the other bars (observed up to 5.7e-5)."""
+    scene = synthetic.tiny_scene(num_points=points, K=-1, seed=109 + bucket)
+    scene.confidence = (0.05 * scene.confidence).astype(np.float32)
+    if bucket > 1:
+        _levels(scene, step=2.0 * bucket * scene.views[0].w * scene.views[0].h / (16 * points))
+    params = make_params(scene, need_point_gradient=0, depth_accept_blend=0.008 if bucket > 1 else 1e-4, **MODE)
+    res = rasterizer.forward(DeviceScene(scene), params, save_for_backward=True)
+    grad_out = scene.grad_out()
+    got = rasterizer.backward(res, [torch.from_numpy(g).cuda() for g in grad_out], want_points=False)
+    torch.cuda.synchronize()
+    longest = int(np.diff(res.offsets(0)).max())
+    assert longest > 100
+    model = dict(zip(("texture", "confidence", "background"), _float64_model(scene, res, grad_out, params.depth_accept_blend)))
+    for key, want in model.items():
+        err = max_rel_err(got[key].cpu().numpy().astype(np.float64), want)
+        print(f"  {key}: library vs float64 {err:.2e}, longest list {longest}", flush=True)
+        assert err <= longest * 2.0 ** -23, key
