@@ -46,7 +46,7 @@ struct DeviceView
         float image_row[2][4];  // else, where can_leave_out: image x and y times depth as linear functions of the point
     };
     uint32_t has_dist;        // some coefficient is not zero and the caller has switched distortion on
-    uint32_t can_leave_out;   // see surely_outside
+    uint32_t can_leave_out;   // image_row is there, see surely_outside
     float off_by_size, off;   // what image_row and the projection's own rounding may be off: times |x| + |y| + |z|, and at least
 };
 static_assert(sizeof(DeviceView) == 40 * 4, "DeviceView is 40 floats");

@@ -124,7 +124,7 @@ __device__ __forceinline__ void prepare_leaving_out(DeviceView& v, float width, 
 }
 
 // One thread per view fills its camera constants; non-zero distortion coefficients raise flag bit 0 unless the caller
-// has switched distortion on.
+// has switched distortion on. leave_out (not with distortion): with what surely_outside looks at.
 // Workgroups beyond the first zero the per-bin counters of all views (n4 uint4 elements).
 __global__ void __launch_bounds__(kBlock) prepare_views_kernel(PrepareViewsArgs args, int first_view, int num_views,
                                                                 const double* __restrict__ poses_se3,
@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(kBlock) prepare_views_kernel(PrepareViewsArgs 
                                                                 uint32_t* __restrict__ flags,
                                                                 uint4* __restrict__ counters4, size_t n4,
                                                                 const float* __restrict__ background, int channels,
-                                                                int texture_abs, int allow_distortion)
+                                                                int texture_abs, int allow_distortion, int leave_out)
 {
     if (blockIdx.x > 0)
     {
@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(kBlock) prepare_views_kernel(PrepareViewsArgs 
         atomicOr(flags, 1u);  // refused: the call renders the camera without distortion and says so
         v.has_dist = 0u;
     }
-    if (!allow_distortion) prepare_leaving_out(v, (float)args.src[k].w, (float)args.src[k].h);
+    if (leave_out) prepare_leaving_out(v, (float)args.src[k].w, (float)args.src[k].h);
     views[first_view + k] = v;
 }
 
@@ -727,9 +727,7 @@ __device__ __forceinline__ void scatter_projected(const ViewPass& a, uint32_t* _
     if (packs) store_packed_row(pack, slot, row, row_confidence);
 }
 
-// The pass for one view: fetch, projection, and the above. LEAVE_OUT: points are looked at roughly first (surely_outside). Launches of
-// several views do, which mostly are crops that see a tenth of the cloud: four crops of two million points 69.8 and 65.5 us (four town
-// views, bound by their atomics, 182 either way); a full frame sees half of it, 33 us either way.
+// The pass for one view: fetch, projection, and the above. LEAVE_OUT: points are looked at roughly first (surely_outside).
 template <int HITS, bool LEAVE_OUT>
 __device__ __forceinline__ void bin_scatter(const ViewPass& a, uint32_t* __restrict__ bin_counts,
                                             const ScatterTargets& out, const PackJob& pack)
@@ -750,11 +748,11 @@ __device__ __forceinline__ void bin_scatter(const ViewPass& a, uint32_t* __restr
     scatter_projected<HITS>(a, bin_counts, out, pack, slot, i, visible, p);
 }
 
-template <int HITS>
+template <int HITS, bool LEAVE_OUT>
 __global__ void __launch_bounds__(kBlock, kScatterWaves<HITS>) bin_scatter_kernel(ViewPass a, uint32_t* __restrict__ bin_counts,
                                                               ScatterTargets out, PackJob pack)
 {
-    bin_scatter<HITS, false>(a, bin_counts, out, pack);
+    bin_scatter<HITS, LEAVE_OUT>(a, bin_counts, out, pack);
 }
 
 struct ScatterArgs
@@ -771,11 +769,11 @@ struct ScatterArgs
 // pass waits for its atomics, not for memory, and more, shorter threads hide more of that. Workgroups of the views
 // taking turns, instead of all of one view before those of the next, is slower as well, by a tenth for crops and by
 // half for full frames.)
-template <int HITS>
+template <int HITS, bool LEAVE_OUT>
 __global__ void __launch_bounds__(kBlock, kScatterWaves<HITS>) bin_scatter_views_kernel(PerView<ScatterArgs> views)
 {
     const ScatterArgs& v = views.v[blockIdx.y];
-    bin_scatter<HITS, true>(v.view, v.bin_counts, v.out, v.pack);
+    bin_scatter<HITS, LEAVE_OUT>(v.view, v.bin_counts, v.out, v.pack);
 }
 
 // The interleave as a launch of its own, for a caller that keeps the records across calls while texture and confidence

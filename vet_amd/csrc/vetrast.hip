@@ -657,6 +657,24 @@ bool views_see_little(const vetrast_params& p, int N, int hits)
     }
     return expected < (double)N * hits * p.num_layers / 3.0;
 }
+
+// Whether the scatter pass looks at a point roughly before it projects it (surely_outside): where the caller expects less than a tenth of
+// the fragments of all points in every layer (radius drop-out empties some of them: the fullest one says what is seen). The look takes the
+// projection away from waves that see nothing and costs the others a few per cent. Time of the pass with it / without, for two hundred
+// thousand to five million points in one, two or four views: crops that see a hundredth of the cloud 0.88 to 1.02, a thirtieth 0.92 to 1.00, a
+// sixteenth 0.92 to 1.00, an eighth 0.96 to 1.05; whole frames of a town, a sixth, 1.00 to 1.05; of a scene half of which is seen 0.98 to
+// 1.06, of a cloud that is seen whole 1.01 to 1.05. A caller who has not said what to expect of several views mostly has crops: these take
+// 0.95 to 1.03 then, such frames 1.00 to 1.06.
+bool few_points_are_seen(const vetrast_params& p, int N, int B, int hits)
+{
+    float fullest = 0.f;
+    for (int l = 0; l < p.num_layers; ++l)
+    {
+        if (!(p.expected_fragments[l] > 0.f)) return B > 1;
+        fullest = std::max(fullest, p.expected_fragments[l]);
+    }
+    return (double)fullest * 10.0 < (double)N * hits;
+}
 }  // namespace
 
 int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* stream_)
@@ -679,6 +697,7 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
     float4* packed       = own_pack ? ws_ptr<float4>(ws, lay.packed_base)
                                     : reinterpret_cast<float4*>(const_cast<float*>(a->packed_descriptors));
     DeviceView* views   = ws_ptr<DeviceView>(ws, lay.views_base);
+    const bool leave_out = !p.allow_distortion && few_points_are_seen(p, N, B, hits);
 
     {
         ScopeTimer tm(ctx, stream, VETRAST_SCOPE_PREPARE);
@@ -703,7 +722,7 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
             }
             hipLaunchKernelGGL(prepare_views_kernel, dim3(1 + (first == 0 ? zero_blocks : 0)), dim3(kBlock), 0, stream, pv,
                                first, cnt, a->poses_se3, a->intrinsics, views, flags, counters4, n4, a->background, C,
-                               p.texture_abs, p.allow_distortion);
+                               p.texture_abs, p.allow_distortion, leave_out ? 1 : 0);
         }
     }
 
@@ -820,14 +839,18 @@ int vetrast_forward(vetrast_ctx* ctx, const vetrast_forward_args* a, void* strea
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_COUNT);
             const ScatterArgs& sc = scatter.v[0];
             const dim3 g(grid_for(N)), gv(grid_for(N), views_y);
-            if (hits == 1 && one)
-                hipLaunchKernelGGL(bin_scatter_kernel<1>, g, blk, 0, stream, sc.view, sc.bin_counts, sc.out, sc.pack);
-            else if (hits == 1)
-                hipLaunchKernelGGL(bin_scatter_views_kernel<1>, gv, blk, 0, stream, scatter);
-            else if (one)
-                hipLaunchKernelGGL(bin_scatter_kernel<4>, g, blk, 0, stream, sc.view, sc.bin_counts, sc.out, sc.pack);
+            auto launch = [&](auto hits_c, auto leave_out_c) {
+                constexpr int kHits      = decltype(hits_c)::value;
+                constexpr bool kLeaveOut = decltype(leave_out_c)::value;
+                if (one)
+                    hipLaunchKernelGGL((bin_scatter_kernel<kHits, kLeaveOut>), g, blk, 0, stream, sc.view, sc.bin_counts, sc.out, sc.pack);
+                else
+                    hipLaunchKernelGGL((bin_scatter_views_kernel<kHits, kLeaveOut>), gv, blk, 0, stream, scatter);
+            };
+            if (hits == 1)
+                leave_out ? launch(std::integral_constant<int, 1>{}, std::true_type{}) : launch(std::integral_constant<int, 1>{}, std::false_type{});
             else
-                hipLaunchKernelGGL(bin_scatter_views_kernel<4>, gv, blk, 0, stream, scatter);
+                leave_out ? launch(std::integral_constant<int, 4>{}, std::true_type{}) : launch(std::integral_constant<int, 4>{}, std::false_type{});
         }
         {
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_SCAN);
