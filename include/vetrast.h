@@ -148,7 +148,8 @@ typedef enum vetrast_scope
     VETRAST_SCOPE_BACKWARD_PREPARE, /* "Prepare Backward": zero-fill of gradient buffers */
     VETRAST_SCOPE_BACKWARD_BLEND,   /* "BlendBackwards", per-pixel part */
     VETRAST_SCOPE_BACKWARD_GATHER,  /* "BlendBackwards", per-point sum of the stored fragment gradients */
-    VETRAST_SCOPE_BACKWARD_POST,    /* "Post Process Gradient" */
+    VETRAST_SCOPE_BACKWARD_POST,    /* "Post Process Gradient" (a launch of its own while profiling; else a call with camera
+                                       gradients does it beside them) */
     VETRAST_SCOPE_LIFT_ERROR,       /* vetrast_lift_error (the reference times FillSceneGridWithLoss in no scope) */
     VETRAST_SCOPE_COUNT_
 } vetrast_scope;

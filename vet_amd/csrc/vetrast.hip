@@ -1206,6 +1206,8 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
                 with_channels(std::integral_constant<int, 4>{});
         }
         const bool divide = g->grad_points && p.point_gradient_normalization != 0 && N > 0 && last == B;
+        // beside the camera gradients, unless their times are asked for one by one (the same code either way)
+        const bool divide_beside = divide && want_camera && !ctx->profiling;
         if (want_camera)
         {
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_GATHER);
@@ -1240,10 +1242,10 @@ int vetrast_backward(vetrast_ctx* ctx, const vetrast_backward_args* g, void* str
             cp.normalize             = (p.camera_gradient_normalization && last == B) ? 1 : 0;
             cp.num_poses             = a->num_poses;
             cp.num_cameras           = a->num_cameras;
-            hipLaunchKernelGGL(finish_gradients_kernel, dim3(1u + (divide ? (unsigned)grid_for(N) : 0u)), dim3(kBlock), 0, stream, cp, g->grad_points,
+            hipLaunchKernelGGL(finish_gradients_kernel, dim3(1u + (divide_beside ? (unsigned)grid_for(N) : 0u)), dim3(kBlock), 0, stream, cp, g->grad_points,
                                g->grad_point_count, N, p.point_gradient_normalization);
         }
-        else if (divide)
+        if (divide && !divide_beside)
         {
             ScopeTimer tm(ctx, stream, VETRAST_SCOPE_BACKWARD_POST);
             hipLaunchKernelGGL(normalize_point_gradient_kernel, dim3(grid_for(N)), dim3(kBlock), 0, stream, g->grad_points, g->grad_point_count, N,
