@@ -80,7 +80,7 @@ struct LiftPass
     uint32_t* flags;
     uint32_t* num_plain;    // cells left to lift_plain_kernel
     uint32_t* plain_cell;   // their numbers
-    // [num_cells] each, written for cells left to lift_plain_kernel and, with several bands, for every cell:
+    // [num_cells] each, written for cells left to lift_plain_kernel and, with several bands, for every cell that is seen:
     double* cell_sums;      // sum of the bands so far
     uint32_t* plain_state;  // 0, or first image row that is lift_plain_kernel's + 1 in bits 8.., below them its finished shares
     // Cells the image shows, found by the first band's lift_prefix_kernel. The cells are dealt to stretches, kLiftRun neighbours
