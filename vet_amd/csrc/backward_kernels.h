@@ -1049,20 +1049,9 @@ __global__ void __launch_bounds__(kBlock) blend_backward_fuzzy_views_kernel(PerV
     blend_backward_fuzzy<C, DENSE>(views.v[blockIdx.y], depth_accept);
 }
 
-// The lists blend_backward_fuzzy_kernel left out (more than `dense_max` fragments), one after the other, each by the
-// whole wave: 64 consecutive fragments per step, front to back, one lane per fragment. The bucket boundaries of a step
-// are found by a loop over its buckets that every lane runs alike (the rule is sequential, but it needs the depths
-// only: all lanes test their depth against the open range at once, the first that fails opens the next bucket); sums
-// over a bucket, the transmittance product over the buckets in front and the running sum of the bucket
-// terms are scans over the lanes. What crosses a step boundary is carried in registers: the open bucket (sums, number
-// of elements, first element), the depth its range started at, the transmittance in front of it and the sum of the
-// bucket terms so far. A bucket's gradient needs the sum of the terms of all LATER buckets, so the list is processed
-// twice: the first pass only adds up the terms, the second has the total and writes (a list of up to 64 fragments has
-// its total inside its one step and is processed once). The elements of a bucket that was
-// still open at the end of their step get the position part of their record there and the bucket's part when it
-// closes, from a loop over their keys. Grid: fuzzy_long_grid x kFuzzyReplicas.
-// Sum over the lanes from `dist` lanes below up to this one (dist <= lane), in moves between registers: inside a row of 16 lanes, then
-// from the last lane of a row to the next row, then from the lower half to the upper one. Every lane of the wave must be active.
+// Scans of the kernel below, in moves between registers: inside a row of 16 lanes, then from the last lane of a row to the next row, then
+// from the lower half to the upper one. Every lane of the wave must be active.
+// Sum over the lanes from the first one of this lane's segment, `dist` lanes below, up to this one.
 __device__ __forceinline__ float sum_from(float v, uint32_t dist, int lane)
 {
     auto add = [&](uint32_t from, bool same) { v += same ? __uint_as_float(from) : 0.f; };
@@ -1088,6 +1077,18 @@ __device__ __forceinline__ float product_up_to(float v)
     return v;
 }
 
+// The lists blend_backward_fuzzy_kernel left out (more than `dense_max` fragments), one after the other, each by the
+// whole wave: 64 consecutive fragments per step, front to back, one lane per fragment. The bucket boundaries of a step
+// are found by a loop over its buckets that every lane runs alike (the rule is sequential, but it needs the depths
+// only: all lanes test their depth against the open range at once, the first that fails opens the next bucket); sums
+// over a bucket, the transmittance product over the buckets in front and the running sum of the bucket
+// terms are scans over the lanes. What crosses a step boundary is carried in registers: the open bucket (sums, number
+// of elements, first element), the depth its range started at, the transmittance in front of it and the sum of the
+// bucket terms so far. A bucket's gradient needs the sum of the terms of all LATER buckets, so the list is processed
+// twice: the first pass only adds up the terms, the second has the total and writes (a list of up to 64 fragments has
+// its total inside its one step and is processed once). The elements of a bucket that was
+// still open at the end of their step get the position part of their record there and the bucket's part when it
+// closes, from a loop over their keys. Grid: fuzzy_long_grid x kFuzzyReplicas.
 template <int C>
 __device__ __forceinline__ void blend_backward_fuzzy_long(const BackwardPass& a, float depth_accept, uint32_t dense_max)
 {
