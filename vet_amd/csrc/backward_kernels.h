@@ -2143,8 +2143,8 @@ __global__ void __launch_bounds__(kBlock) normalize_point_gradient_kernel(float*
 }
 
 // The camera gradients, by the launch's first workgroup, and behind a call's last round the division of the position gradients by the
-// others beside it: neither waits for the other, and the camera rows are one workgroup's chain (four crops of two million points 8.9 and
-// 5.8 us one after the other, 9.1 together; a crop of 60 thousand 5.6 and 3.8, together 6.0). Without cameras the division has a kernel
+// others beside it: neither waits for the other, and the camera rows are one workgroup's chain (four crops of two million points 7.2 and
+// 5.0 us one after the other, 9.0 together; a crop of 60 thousand 5.3 and 3.5, together 5.3; medians of a kernel trace). Without cameras the division has a kernel
 // of its own, whose 21 registers are a third of this one's (ten million points 51 and 56 us). The rows folded here as well, by workgroups the last of
 // which goes on with the sums, took 22 us where the three launches took 19: each of them writes its L2 back for it.
 __global__ void __launch_bounds__(kBlock) finish_gradients_kernel(CameraPass camera, float* __restrict__ grad_points, const float* __restrict__ count,
