@@ -13,7 +13,7 @@
 //      literal ones, pixel for pixel.
 // Measured (146 k cells of 0.25 m, 1080p, 121 M covered pixels, the camera inside the grid): 0.87 ms per call with a test per
 // pixel (bound by its ~200 vector instructions per 64 pixels), 0.20 ms by rows.
-// Bound by vector instructions (32 M of wave instructions a view of three 1080p views of 176 k cells, 55 of the cells kernel's 86 us)
+// Bound by vector instructions (32 M of wave instructions a view of three 1080p views of 176 k cells, 52 of the cells kernel's 86 us)
 // and the round trips of a row's two running sums. A third of the cells is in the image: with the others in the workgroups too,
 // set up by as many idle lanes, it took 43 M and 103 us, cells of 0.15 m 385 a call (now 259), of 1 m 78 (now 56: there are few of
 // them, which are dealt to more workgroups then, kLiftLeast; with 768 or 1792 for it the same). Looking for them costs the running
